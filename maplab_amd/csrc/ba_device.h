@@ -105,7 +105,7 @@ struct DevTopology {
 // batches with their slot and pair lists, and for every upper block of S
 // the partial slots (segment * kTileBlocks + thread) summed into it, in order.
 struct SchurTilesDev {
-  int32_t n_segs;
+  int32_t n_segs, n_uslot;
   const int32_t* seg_order;
   const int4* segs;
   const uint32_t* seg_thread;

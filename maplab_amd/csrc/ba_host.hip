@@ -598,7 +598,7 @@ int build_topology(mlba_handle* h) {
   SchurTilesDev& d = h->tdev;
   d.n_segs = h->n_segs; d.seg_order = h->t_seg_order.p; d.segs = h->t_segs.p; d.seg_thread = h->t_seg_thread.p;
   d.batches = h->t_batches.p; d.slots = h->t_slots.p; d.batch_off = h->t_batch_off.p; d.pairs = h->t_pairs.p;
-  d.uslot_ptr = h->t_uslot_ptr.p; d.uslot = h->t_uslot.p;
+  d.uslot_ptr = h->t_uslot_ptr.p; d.uslot = h->t_uslot.p; d.n_uslot = (int32_t)uslot.size();
   HIP_OK(hipStreamSynchronize(h->stream));
   return MLBA_OK;
 }

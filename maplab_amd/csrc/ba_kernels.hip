@@ -753,7 +753,13 @@ __global__ __launch_bounds__(kTileBlocks) __attribute__((amdgpu_waves_per_eu(2))
 // part order, listed per upper block), plus on S_ii the direct observation
 // term C_i (sum Jo^T Jo) C_i and the LM diagonal D^2 / radius; written to
 // S_ij and S_ji = S_ij^T. One thread per entry; the first six threads of a
-// diagonal block also sum the rhs of its row.
+// diagonal block also sum the rhs of its row. A work-group of seven 36-thread
+// groups takes seven blocks, or with kWide one block whose slots k, k + 7, ...
+// group k sums, the seven sums then added in group order: a small system has
+// few blocks of many slots each.
+constexpr int kFinalizeGroups = 7;
+
+template <bool kWide>
 __global__ __launch_bounds__(252) void k_schur_finalize(int32_t nub, const int4* __restrict__ ublk,
                                                         const int32_t* __restrict__ uslot_ptr,
                                                         const int32_t* __restrict__ uslot,
@@ -763,19 +769,22 @@ __global__ __launch_bounds__(252) void k_schur_finalize(int32_t nub, const int4*
                                                         const double* __restrict__ pose_jtj, double inv_mu,
                                                         double min_diag, double max_diag, double* __restrict__ S,
                                                         double* __restrict__ rhs) {
-  const int u = blockIdx.x * 7 + threadIdx.x / 36, e = threadIdx.x % 36;
-  if (u >= nub) return;
+  __shared__ double red[kWide ? kFinalizeGroups : 1][kPartEntries];
+  const int grp = threadIdx.x / 36, e = threadIdx.x % 36;
+  const int u = kWide ? (int)blockIdx.x : (int)blockIdx.x * kFinalizeGroups + grp;
+  if (u >= nub) return;  // kWide: nub work-groups, none leaves here
+  constexpr int st = kWide ? kFinalizeGroups : 1;
   const int4 ub = ublk[u];
-  const int kb = uslot_ptr[u], ke = uslot_ptr[u + 1];
+  const int kb = uslot_ptr[u] + (kWide ? grp : 0), ke = uslot_ptr[u + 1];
   const bool rhs_entry = ub.z == ub.w && e < 6;
   double v = 0.0, g = 0.0;
   int k = kb;
   // Four slots' loads in flight at a time; the sums keep slot order.
-  for (; k + 4 <= ke; k += 4) {
+  for (; k + 3 * st < ke; k += 4 * st) {
     const double* p0 = partial + (size_t)uslot[k] * kPartEntries;
-    const double* p1 = partial + (size_t)uslot[k + 1] * kPartEntries;
-    const double* p2 = partial + (size_t)uslot[k + 2] * kPartEntries;
-    const double* p3 = partial + (size_t)uslot[k + 3] * kPartEntries;
+    const double* p1 = partial + (size_t)uslot[k + st] * kPartEntries;
+    const double* p2 = partial + (size_t)uslot[k + 2 * st] * kPartEntries;
+    const double* p3 = partial + (size_t)uslot[k + 3 * st] * kPartEntries;
     const double a0 = p0[e], a1 = p1[e], a2 = p2[e], a3 = p3[e];
     v += a0;
     v += a1;
@@ -789,10 +798,22 @@ __global__ __launch_bounds__(252) void k_schur_finalize(int32_t nub, const int4*
       g += b3;
     }
   }
-  for (; k < ke; ++k) {
+  for (; k < ke; k += st) {
     const double* p = partial + (size_t)uslot[k] * kPartEntries;
     v += p[e];
     if (rhs_entry) g += p[36 + e];
+  }
+  if (kWide) {
+    red[grp][e] = v;
+    if (e < 6) red[grp][36 + e] = g;
+    __syncthreads();
+    if (grp > 0) return;
+    v = red[0][e];
+    g = rhs_entry ? red[0][36 + e] : 0.0;
+    for (int q = 1; q < kFinalizeGroups; ++q) {
+      v += red[q][e];
+      if (rhs_entry) g += red[q][36 + e];
+    }
   }
   const int r = e / 6, c = e % 6;
   if (ub.z == ub.w) {
@@ -1588,8 +1609,14 @@ void launch_schur_blocks(hipStream_t s, const DevTopology& t, const SchurTilesDe
                          int32_t items_per_wg, int32_t xcd_map) {
   if (t.Pvar <= 0 || nub <= 0) return;
   launch_schur_tiles(s, d, gw, gr0, lm_acc, lm_z, partial, items_per_wg, xcd_map);
-  k_schur_finalize<<<(nub + 6) / 7, 252, 0, s>>>(nub, ublk, d.uslot_ptr, d.uslot, partial, pose_scale, pose_diag,
-                                                 pose_jtj, inv_mu, min_diag, max_diag, S, rhs);
+  // kWide from 24 slots a block on: below that its groups have too few slots
+  // each to hide their latency behind one another.
+  if (d.n_uslot >= 24 * (int64_t)nub)
+    k_schur_finalize<true><<<nub, 252, 0, s>>>(nub, ublk, d.uslot_ptr, d.uslot, partial, pose_scale, pose_diag,
+                                               pose_jtj, inv_mu, min_diag, max_diag, S, rhs);
+  else
+    k_schur_finalize<false><<<(nub + kFinalizeGroups - 1) / kFinalizeGroups, 252, 0, s>>>(
+        nub, ublk, d.uslot_ptr, d.uslot, partial, pose_scale, pose_diag, pose_jtj, inv_mu, min_diag, max_diag, S, rhs);
 }
 void launch_landmark_quality(hipStream_t s, const DevTopology& t, const double* vert, const double* vR,
                              const double* lm, int32_t min_observers, double min_angle_deg, double max_dist,

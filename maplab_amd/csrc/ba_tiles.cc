@@ -102,6 +102,14 @@ bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const in
   }
   const int64_t n_visits = (int64_t)visits.size();
   T.visits = n_visits;
+  // A segment runs its batches one after the other, so a small system is cut
+  // into about as many segments as work-groups run at once (two on each of
+  // 256 CUs); above 512 x kSegmentSlots staged blocks the length that fills
+  // the last round of work-groups best is fixed. Build of S (two kernels) with
+  // segments of 5120 blocks and cut so: 10 keyframes 130 -> 27 us (2 -> 39
+  // segments), 25 keyframes 203 -> 47, 60 keyframes 206 -> 74, 150 keyframes
+  // 249 -> 211; 300 and more unchanged.
+  int64_t segment_slots = kSegmentSlots;
   {
     int64_t staged = 0, npairs = 0;
     for (const Visit& v : visits) {
@@ -110,6 +118,7 @@ bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const in
     }
     T.slots.reserve(2 * staged);
     T.pairs.reserve(npairs + npairs / 64 + 64);
+    segment_slots = std::min<int64_t>(kSegmentSlots, staged / kSegmentTarget);
   }
   auto is_anchor = [&](int g) { return T.g_inc[T.g_inc_ptr[g]] < 0; };
   // Batches (LDS-sized groups of visits) with their slot lists and pair
@@ -239,7 +248,7 @@ bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const in
       T.staged += slots;
       seg_slots += slots;
       const int32_t nbatch = (int32_t)(T.batches.size() / 4);
-      if (v == ve || seg_slots >= kSegmentSlots || nbatch - seg_batch >= kSegmentBatches) {
+      if (v == ve || seg_slots >= segment_slots || nbatch - seg_batch >= kSegmentBatches) {
         close_segment(seg_batch, nbatch, I, J);
         seg_batch = nbatch;
         seg_slots = 0;

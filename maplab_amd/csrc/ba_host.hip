@@ -1169,6 +1169,7 @@ int minimize(mlba_handle* h, const mlba_options* o, double initial_radius, mlba_
       launch_block_inverse(s, h->Pvar, h->diag_pos.p, h->S.p, h->Minv.p, h->fail.p);
       HIP_OK(hipGetLastError());
       int pcg_iters = 0;
+      bool pcg_small = false;  // iteration count read with the step's scalars
       if (h->Pvar > 0 && (o->pcg_preconditioner == MLBA_PRECOND_BLOCK_JACOBI ||
                           o->pcg_preconditioner == MLBA_PRECOND_LEARNED)) {
         KernelTimer kt(h, MLBA_KERNEL_PCG);
@@ -1181,13 +1182,19 @@ int minimize(mlba_handle* h, const mlba_options* o, double initial_radius, mlba_
         const int32_t nritz = ritz_count(o);
         if ((rc = ritz_merge(h))) return rc;
         const int32_t nr_used = nritz > 0 ? h->ritz_nr : 0;
-        int32_t& est = h->pcg_last_iters[nr_used > 0 ? 1 : 0];
-        pcg_iters = launch_pcg_deflated(s, pcg_buffers(h, nr_used, nritz > 0), o->pcg_relative_tolerance,
-                                        o->pcg_max_iterations, est > 0 ? est : kPcgPoll,
-                                        est > 0 ? kPcgPollAfter : kPcgPoll, nullptr, 0);
-        if (pcg_iters < 0) return set_err(h, MLBA_EDEVICE, "PCG launch failed");
-        est = pcg_iters;
-        ritz_after_solve(h, nritz, pcg_iters);
+        const PcgBuffers B = pcg_buffers(h, nr_used, nritz > 0);
+        if ((pcg_small = pcg_small_applies(B))) {
+          if (!launch_pcg_small(s, B, o->pcg_relative_tolerance, o->pcg_max_iterations))
+            return set_err(h, MLBA_EDEVICE, "PCG launch failed");
+          h->ritz_nr = 0;  // no coarse space to recycle columns for
+        } else {
+          int32_t& est = h->pcg_last_iters[nr_used > 0 ? 1 : 0];
+          pcg_iters = launch_pcg_deflated(s, B, o->pcg_relative_tolerance, o->pcg_max_iterations,
+                                          est > 0 ? est : kPcgPoll, est > 0 ? kPcgPollAfter : kPcgPoll, nullptr, 0);
+          if (pcg_iters < 0) return set_err(h, MLBA_EDEVICE, "PCG launch failed");
+          est = pcg_iters;
+          ritz_after_solve(h, nritz, pcg_iters);
+        }
       }
       launch_unscale_poses(s, h->Pvar, h->px.p, h->pose_scale.p, h->w.p, h->parts_w.p);
       int32_t nbs = 0;
@@ -1225,6 +1232,7 @@ int minimize(mlba_handle* h, const mlba_options* o, double initial_radius, mlba_
       if ((rc = ritz_queue_vectors(h))) return rc;
       HIP_OK(hipEventSynchronize(h->scal_ev));
       collect_events(h);
+      if (pcg_small) pcg_iters = pcg_state_iterations(h->pcg_host);
       const int32_t fail_h = *fail_pinned;
       if (sm) sm->linear_solver_seconds += now_s() - t_ls;
       const double* sc = h->scal_host;

@@ -994,6 +994,132 @@ __global__ __launch_bounds__(kGroupBlock) void k_defl_partials(PcgArgs a, int32_
   if (a.reduce1) sum_partials_if_last(a, &last, red);
 }
 
+// Plain block-Jacobi PCG of a small system in one work-group, for systems
+// without a coarse space (the automatic space starts at 32 vertices). A
+// system of 10 keyframes needs about 40 iterations, and as two launches each
+// they cost 10.5 us an iteration on MI355X (launch and two dependent rounds
+// of global loads, not the 54 x 54 product): 450 us a solve, 3.6 ms of the
+// 6.3 ms that 10 LM iterations took (2.7 ms with this). Here S stays in
+// registers, dense: wave w holds columns 12 w .. 12 w + 11 of rows lane,
+// lane + 64 and lane + 128 (36 doubles a thread, which is what 1024 threads
+// leave room for and why 31 vertices are the limit); the waves' sums of a row
+// meet in LDS, and wave 0 keeps the vectors, so an iteration is two barriers.
+// Sums run in a fixed order.
+constexpr int kSmallVertices = 31;
+constexpr int kSmallRows = 192;
+constexpr int kSmallWaves = 16;
+constexpr int kSmallCols = kSmallRows / kSmallWaves;  // two blocks of columns a wave
+constexpr int kSmallRowsPerLane = kSmallRows / 64;
+
+__global__ __launch_bounds__(64 * kSmallWaves) void k_pcg_small(PcgArgs a, double tol, int32_t max_iters) {
+  __shared__ double red[kSmallWaves][kSmallRows];
+  __shared__ double ps[kSmallRows], rs[kSmallRows], xs[kSmallRows], Ms[6][kSmallRows];
+  __shared__ int16_t pos[32][32];
+  __shared__ int stop;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n = a.n6, P = a.Pvar;
+  const int bi = tid >> 5;  // block row
+  pos[bi][tid & 31] = -1;
+  __syncthreads();
+  if (bi < P)
+    for (int kb = a.row_ptr[bi] + (tid & 31); kb < a.row_ptr[bi + 1]; kb += 32) pos[bi][a.col_var[kb]] = (int16_t)kb;
+  __syncthreads();
+  double s[kSmallRowsPerLane][kSmallCols];
+#pragma unroll
+  for (int j = 0; j < kSmallRowsPerLane; ++j) {
+    const int row = lane + 64 * j;
+#pragma unroll
+    for (int h = 0; h < kSmallCols / 6; ++h) {
+      const int kb = row < n ? pos[row / 6][kSmallCols / 6 * wave + h] : -1;
+      const double* sb = a.S + (size_t)36 * max(kb, 0) + 6 * (row % 6);
+#pragma unroll
+      for (int c = 0; c < 6; ++c) s[j][6 * h + c] = kb >= 0 ? sb[c] : 0.0;
+    }
+  }
+  // Wave 0's vectors (rows lane + 64 j) live in LDS, the registers are S's;
+  // z takes red[0], which holds wave 0's own sums only between the barriers.
+  double rz = 0.0, rr = 0.0, tol2 = 0.0;
+  auto apply_minv = [&]() {
+    // rs is written and read by wave 0 alone.
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    double t0 = 0.0, t1 = 0.0;
+#pragma unroll
+    for (int j = 0; j < kSmallRowsPerLane; ++j) {
+      const int row = lane + 64 * j, base = row - row % 6;
+      double v = 0.0;
+#pragma unroll
+      for (int c = 0; c < 6; ++c) v += Ms[c][row] * rs[base + c];
+      red[0][row] = v;
+      const double rv = rs[row];
+      t0 += rv * v;
+      t1 += rv * rv;
+    }
+    rz = wave_sum(t0);
+    rr = wave_sum(t1);
+  };
+  if (wave == 0) {
+    for (int row = lane; row < kSmallRows; row += 64) {
+      xs[row] = ps[row] = 0.0;
+      rs[row] = row < n ? a.b[row] : 0.0;
+      for (int c = 0; c < 6; ++c) Ms[c][row] = row < n ? a.Minv[(size_t)6 * row + c] : 0.0;
+    }
+    apply_minv();
+    tol2 = tol * tol * rr;
+  }
+  double rz_prev = 0.0;
+  int k = 0;
+  while (true) {
+    if (wave == 0) {
+      const bool end = k == 0 ? (rr <= 0.0 || max_iters <= 0 || rr <= tol2) : (rr <= tol2 || k >= max_iters);
+      const double beta = k > 0 ? rz / rz_prev : 0.0;
+      rz_prev = rz;
+#pragma unroll
+      for (int j = 0; j < kSmallRowsPerLane; ++j) ps[lane + 64 * j] = red[0][lane + 64 * j] + beta * ps[lane + 64 * j];
+      if (lane == 0) stop = end;
+    }
+    __syncthreads();
+    if (stop) break;  // the same value in every thread
+    double acc[kSmallRowsPerLane] = {};
+#pragma unroll
+    for (int c = 0; c < kSmallCols; ++c) {
+      const double pc = ps[kSmallCols * wave + c];
+#pragma unroll
+      for (int j = 0; j < kSmallRowsPerLane; ++j) acc[j] += s[j][c] * pc;
+    }
+#pragma unroll
+    for (int j = 0; j < kSmallRowsPerLane; ++j) red[wave][lane + 64 * j] = acc[j];
+    __syncthreads();
+    if (wave == 0) {
+      double q[kSmallRowsPerLane], t = 0.0;
+#pragma unroll
+      for (int j = 0; j < kSmallRowsPerLane; ++j) {
+        q[j] = 0.0;
+#pragma unroll 4
+        for (int w = 0; w < kSmallWaves; ++w) q[j] += red[w][lane + 64 * j];
+        t += ps[lane + 64 * j] * q[j];
+      }
+      const double alpha = rz / wave_sum(t);
+#pragma unroll
+      for (int j = 0; j < kSmallRowsPerLane; ++j) {
+        const int row = lane + 64 * j;
+        xs[row] += alpha * ps[row];
+        rs[row] -= alpha * q[j];
+      }
+      apply_minv();
+    }
+    ++k;
+  }
+  if (wave == 0) {
+    for (int row = lane; row < n; row += 64) a.x[row] = xs[row];
+    if (lane == 0) {
+      a.st->iters = k;
+      a.st->done = 1;
+      a.st->defl_ok = 0;
+    }
+  }
+}
+
 // Clears the convergence flag and lifts the iteration limit so that one more
 // iteration runs (kernel timing only).
 __global__ void k_pcg_reopen(PcgState* st) {
@@ -1144,6 +1270,20 @@ static void launch_spmv(hipStream_t s, const PcgArgs& a, int32_t k, const double
   else
     k_pcg_spmv<false><<<a.Pvar, 256, 0, s>>>(a, k, p_prev, p_cur);
 }
+
+bool pcg_small_applies(const PcgBuffers& B) {
+  return B.K == 0 && B.kmat == nullptr && B.Pvar > 0 && B.Pvar <= kSmallVertices;
+}
+
+bool launch_pcg_small(hipStream_t s, const PcgBuffers& B, double tol, int32_t max_iters) {
+  if (!pcg_small_applies(B)) return false;
+  const PcgArgs a = make_args(B);
+  k_pcg_small<<<1, 64 * kSmallWaves, 0, s>>>(a, tol, max_iters);
+  return hipGetLastError() == hipSuccess &&
+         hipMemcpyAsync(B.state_host, a.st, sizeof(PcgState), hipMemcpyDeviceToHost, s) == hipSuccess;
+}
+
+int32_t pcg_state_iterations(const void* state_host) { return static_cast<const PcgState*>(state_host)->iters; }
 
 // Deflated PCG solve of S y = b. The host polls the state after `first`
 // iterations, then every `poll` iterations. With `probe` (three events),

@@ -33,6 +33,19 @@ __device__ inline double wave_reduce(double v, double identity, Op op) {
   return __hiloint2double(hi, lo);
 }
 
+// The same within each row of 16 lanes; result in all 16. Every lane of the
+// row must be active.
+template <typename Op>
+__device__ inline double row_reduce(double v, double identity, Op op) {
+  v = op(v, dpp_move<0xB1>(v, identity));   // quad_perm [1, 0, 3, 2]
+  v = op(v, dpp_move<0x4E>(v, identity));   // quad_perm [2, 3, 0, 1]
+  v = op(v, dpp_move<0x141>(v, identity));  // row_half_mirror
+  return op(v, dpp_move<0x140>(v, identity));  // row_mirror
+}
+__device__ inline double row_min(double v) {
+  return row_reduce(v, __builtin_inf(), [](double a, double b) { return fmin(a, b); });
+}
+
 __device__ inline double wave_sum(double v) {
   return wave_reduce(v, 0.0, [](double a, double b) { return a + b; });
 }

@@ -169,7 +169,8 @@ typedef struct mlba_options {
   int32_t pcg_ritz_vectors;               /* recycled Ritz vectors added to the deflation space:
                                              0 automatic (16), -1 none, else r (<= 16) */
   int32_t jacobian_fp32;                  /* 1: the robust-corrected Jacobians are rounded to FP32 and
-                                             stored so (88 instead of 160 bytes per observation);
+                                             stored so, with the rounding remainder in BF16 (80 instead of 96
+                                             bytes per observation);
                                              every product of them, S, the PCG, residuals, costs and
                                              LM scalars stay FP64, and S remains the Schur complement
                                              of J'J of that one rounded Jacobian (positive

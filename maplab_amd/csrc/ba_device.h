@@ -10,29 +10,54 @@
 namespace mlba {
 
 constexpr int kObsTile = 256;        // observations per linearization tile
-constexpr int kObsRecord = 20;       // doubles per observation record: r(2) Jl(2x3) Jo(2x6)
+// Observation record (96 bytes): the robust-corrected residual r (2), its
+// Jacobian K = d r / d p_I (2x3) with respect to the landmark in the observer's
+// IMU frame, and p_I. The Jacobians of the residual's blocks follow from them
+// and the vertex: J_landmark = K G with G = d p_I / d p_B (landmark_to_imu),
+// J_observer = K [|q|^2 [p_I]x | -R_I_M].
+constexpr int kObsRecord = 12;       // doubles: r K p_I, one unused
 
-// The record with FP32 Jacobians (residual kept in FP64): 88 bytes.
+// The record with the Jacobian in FP32 and the remainder of the rounding in
+// BF16 (32 significant bits together): 80 bytes. K alone carries what J_landmark
+// and J_observer used to round separately, 18 entries whose roundings partly
+// cancelled; with K in FP32 only, solves ended 1.3 times as far from the FP64
+// ones as those did.
 struct Rec32 {
   double r[2];
-  float J[18];  // Jl (2x3) then Jo (2x6)
+  double p[3];
+  float K[6];
+  uint16_t lo[6];
+  uint32_t unused;
 };
+__host__ __device__ inline float bf16_value(uint16_t b) {
+  union { uint32_t u; float f; } v;
+  v.u = (uint32_t)b << 16;
+  return v.f;
+}
+// The nearest BF16 (ties to even) of a finite value.
+__host__ __device__ inline uint16_t bf16_round(float x) {
+  union { float f; uint32_t u; } v;
+  v.f = x;
+  return (uint16_t)((v.u + 0x7FFFu + ((v.u >> 16) & 1u)) >> 16);
+}
 
-// Read access to observation record x: entry k as in the FP64 layout
-// (0..1 residual, 2..7 Jl, 8..19 Jo).
 template <bool kF32>
 struct RecView;
 template <>
 struct RecView<false> {
-  const double* p;
-  __host__ __device__ RecView(const void* base, size_t x) : p(static_cast<const double*>(base) + kObsRecord * x) {}
-  __host__ __device__ double operator[](int k) const { return p[k]; }
+  const double* q;
+  __host__ __device__ RecView(const void* base, size_t x) : q(static_cast<const double*>(base) + kObsRecord * x) {}
+  __host__ __device__ double r(int k) const { return q[k]; }
+  __host__ __device__ double K(int k) const { return q[2 + k]; }
+  __host__ __device__ double p(int k) const { return q[8 + k]; }
 };
 template <>
 struct RecView<true> {
-  const Rec32* p;
-  __host__ __device__ RecView(const void* base, size_t x) : p(static_cast<const Rec32*>(base) + x) {}
-  __host__ __device__ double operator[](int k) const { return k < 2 ? p->r[k] : static_cast<double>(p->J[k - 2]); }
+  const Rec32* q;
+  __host__ __device__ RecView(const void* base, size_t x) : q(static_cast<const Rec32*>(base) + x) {}
+  __host__ __device__ double r(int k) const { return q->r[k]; }
+  __host__ __device__ double K(int k) const { return static_cast<double>(q->K[k]) + static_cast<double>(bf16_value(q->lo[k])); }
+  __host__ __device__ double p(int k) const { return q->p[k]; }
 };
 constexpr int kLmAcc = 18;           // V(6) V_mission(6) g(3) g_mission(3)
 constexpr int kLmZ = 9;              // Z(6, upper triangle) and a copy of g(3), read together per incidence

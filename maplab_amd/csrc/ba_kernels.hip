@@ -102,14 +102,32 @@ __global__ void k_vertex_prep(int32_t P, const double* __restrict__ vert, double
 
 struct ObsEval {
   double r[2];
-  double Jl[6];   // d r / d p_B, row-major 2x3
-  double Jo[12];  // observer tangent [rot 3 | pos 3], row-major 2x6
-  double rho0;
+  double K[6];   // d r / d p_I, row-major 2x3
+  double G[9];   // d p_I / d p_B
+  double pI[3];  // the landmark in the observer's IMU frame
   bool failed;
 };
 
-// Residual and Jacobians of one observation (visual-error-term-inl.h:13-379,
-// evaluated directly in the tangent space of the observer pose).
+// G = d p_I / d p_B of a pose-coupled observation by vertex v of a landmark
+// anchored in vertex a: R_I_M R_M_B, over the mission frames for kGlobal.
+__device__ inline void landmark_to_imu(const DevTopology& t, int32_t type, int32_t a, int32_t v, const double* Ra,
+                                       const double* Rv, double* G) {
+  double H[9];  // d p_M / d p_B
+  for (int i = 0; i < 3; ++i)
+    for (int j = 0; j < 3; ++j) H[i * 3 + j] = Ra[j * 3 + i];
+  if (type == kTypeGlobal) {
+    const double* TL = t.mission_T + 12 * t.vertex_mission[a];
+    const double* TM = t.mission_T + 12 * t.vertex_mission[v];
+    double T1[9];
+    mat3_mul(TL, H, T1);  // R_G_LM R_LM_B
+    for (int i = 0; i < 3; ++i)
+      for (int j = 0; j < 3; ++j) H[i * 3 + j] = TM[i] * T1[j] + TM[3 + i] * T1[3 + j] + TM[6 + i] * T1[6 + j];
+  }
+  mat3_mul(Rv, H, G);
+}
+
+// Residual of one observation and the factors of its Jacobians
+// (visual-error-term-inl.h:13-379).
 template <bool kJac>
 __device__ inline void eval_observation(const DevTopology& t, int o, const double* __restrict__ vert,
                                         const double* __restrict__ vR, const double* __restrict__ lm,
@@ -120,20 +138,19 @@ __device__ inline void eval_observation(const DevTopology& t, int o, const doubl
   const int32_t l = t.obs_landmark[o];
   const int32_t v = t.obs_vertex[o];
   const double* pB = lm + 3 * l;
-  double pI[3];
-  double G[9];  // d p_I / d p_B
-  const double* Rv = vR + 12 * v;
+  double* pI = e.pI;
   if (type == kTypeKeyframe) {
     pI[0] = pB[0]; pI[1] = pB[1]; pI[2] = pB[2];
+    if (kJac)
+      for (int i = 0; i < 9; ++i) e.G[i] = (i % 4 == 0) ? 1.0 : 0.0;
   } else {
+    const double* Rv = vR + 12 * v;
     const int32_t a = t.lm_anchor[l];
     const double* Ra = vR + 12 * a;        // R_B_LM
     const double* pa = vert + 7 * a + 4;   // p_LM_B
     double pM[3];
     mat3t_vec(Ra, pB, pM);
     pM[0] += pa[0]; pM[1] += pa[1]; pM[2] += pa[2];
-    double H[9];  // d p_M / d p_B
-    if (kJac) for (int i = 0; i < 3; ++i) for (int j = 0; j < 3; ++j) H[i * 3 + j] = Ra[j * 3 + i];
     if (type == kTypeGlobal) {
       const double* TL = t.mission_T + 12 * t.vertex_mission[a];
       const double* TM = t.mission_T + 12 * t.vertex_mission[v];
@@ -141,19 +158,11 @@ __device__ inline void eval_observation(const DevTopology& t, int o, const doubl
       mat3_vec(TL, pM, pG);
       for (int i = 0; i < 3; ++i) d[i] = pG[i] + TL[9 + i] - TM[9 + i];
       mat3t_vec(TM, d, pM);
-      if (kJac) {
-        double T1[9], T2[9];
-        mat3_mul(TL, H, T1);  // R_G_LM R_LM_B
-        for (int i = 0; i < 3; ++i)
-          for (int j = 0; j < 3; ++j)
-            T2[i * 3 + j] = TM[i] * T1[j] + TM[3 + i] * T1[3 + j] + TM[6 + i] * T1[6 + j];
-        for (int i = 0; i < 9; ++i) H[i] = T2[i];
-      }
     }
     const double* pv = vert + 7 * v + 4;
     const double dm[3] = {pM[0] - pv[0], pM[1] - pv[1], pM[2] - pv[2]};
     mat3_vec(Rv, dm, pI);
-    if (kJac) mat3_mul(Rv, H, G);
+    if (kJac) landmark_to_imu(t, type, a, v, Ra, Rv, e.G);
   }
   double pC[3];
   mat3_vec(cam.R_C_I, pI, pC);
@@ -171,30 +180,29 @@ __device__ inline void eval_observation(const DevTopology& t, int o, const doubl
   }
   if (!kJac) return;
   if (e.failed) {
-    for (int i = 0; i < 6; ++i) e.Jl[i] = 0.0;
-    for (int i = 0; i < 12; ++i) e.Jo[i] = 0.0;
+    for (int i = 0; i < 6; ++i) e.K[i] = 0.0;
+    for (int i = 0; i < 3; ++i) pI[i] = 0.0;
     return;
   }
-  // K = (d kp / d p_C) * sigma^-1 * R_C_I : d r / d p_I (2x3)
-  double K[6];
+  // K = (d kp / d p_C) * sigma^-1 * R_C_I.
   for (int r = 0; r < 2; ++r)
     for (int c = 0; c < 3; ++c)
-      K[r * 3 + c] = sinv * (jp[r * 3] * cam.R_C_I[c] + jp[r * 3 + 1] * cam.R_C_I[3 + c] +
-                             jp[r * 3 + 2] * cam.R_C_I[6 + c]);
-  if (type == kTypeKeyframe) {
-    for (int i = 0; i < 6; ++i) e.Jl[i] = K[i];
-    for (int i = 0; i < 12; ++i) e.Jo[i] = 0.0;
-    return;
-  }
+      e.K[r * 3 + c] = sinv * (jp[r * 3] * cam.R_C_I[c] + jp[r * 3 + 1] * cam.R_C_I[3 + c] +
+                               jp[r * 3 + 2] * cam.R_C_I[6 + c]);
+}
+
+// The observer's tangent Jacobian (2x6, [rot 3 | pos 3]) from an observation
+// record: rotation |q|^2 (K_r x p_I), position -K_r R_I_M. Rv is the vertex's
+// 12-double rotation record.
+template <class Rec>
+__device__ inline void observer_jacobian(const Rec& rec, const double* Rv, double* Jo) {
+  const double n2 = Rv[9];
   for (int r = 0; r < 2; ++r) {
-    const double* k = K + 3 * r;
-    for (int c = 0; c < 3; ++c) e.Jl[r * 3 + c] = k[0] * G[c] + k[1] * G[3 + c] + k[2] * G[6 + c];
-    // rotation: |q|^2 * (K_r x p_I); position: -K_r R_I_M
-    const double n2 = Rv[9];
-    e.Jo[r * 6 + 0] = n2 * (k[1] * pI[2] - k[2] * pI[1]);
-    e.Jo[r * 6 + 1] = n2 * (k[2] * pI[0] - k[0] * pI[2]);
-    e.Jo[r * 6 + 2] = n2 * (k[0] * pI[1] - k[1] * pI[0]);
-    for (int c = 0; c < 3; ++c) e.Jo[r * 6 + 3 + c] = -(k[0] * Rv[c] + k[1] * Rv[3 + c] + k[2] * Rv[6 + c]);
+    const double k0 = rec.K(3 * r), k1 = rec.K(3 * r + 1), k2 = rec.K(3 * r + 2);
+    Jo[r * 6 + 0] = n2 * (k1 * rec.p(2) - k2 * rec.p(1));
+    Jo[r * 6 + 1] = n2 * (k2 * rec.p(0) - k0 * rec.p(2));
+    Jo[r * 6 + 2] = n2 * (k0 * rec.p(1) - k1 * rec.p(0));
+    for (int c = 0; c < 3; ++c) Jo[r * 6 + 3 + c] = -(k0 * Rv[c] + k1 * Rv[3 + c] + k2 * Rv[6 + c]);
   }
 }
 
@@ -206,14 +214,22 @@ __device__ inline double loss_scale(const DevLoss& loss, int32_t type, double si
   return 1.0;
 }
 
-// Per observation: robust-corrected residual and Jacobians into obs_rec;
+// Per observation: robust-corrected residual and Jacobian K into obs_rec;
 // per landmark: V = sum Jl'Jl, V_mission (pose-coupled observations only),
 // g = sum Jl'r, g_mission; per tile: cost and fixed cost.
 //
-// With kF32 the Jacobians are rounded to FP32 right after the correction and
-// every later product (V, g here; J'J, W, the model cost in the readers)
-// uses the rounded values, so S stays the Schur complement of J'J of one
-// Jacobian; records are Rec32 (residual in FP64).
+// With kF32 K is rounded (Rec32) right after the correction and every later
+// product (V, g here; J'J, W, the model cost in the readers) uses the rounded
+// values, so S stays the Schur complement of J'J of one Jacobian; records are
+// Rec32 (residual and p_I in FP64).
+//
+// The landmark sums meet in LDS: nine values per observation (V and g), value-
+// major; thread (run, value) adds its landmark's run of observations in order,
+// the pose-coupled ones and the store vertex's own separately, so all 256
+// threads share the sums (a run's first thread alone adding 18 values left
+// nine tenths of the tile idle).
+constexpr int kLinVals = 9;  // V (6), g (3)
+
 template <bool kJac, bool kF32 = false>
 __global__ __launch_bounds__(kObsTile) void k_linearize(DevTopology t, const double* __restrict__ vert,
                                                          const double* __restrict__ vR,
@@ -223,28 +239,33 @@ __global__ __launch_bounds__(kObsTile) void k_linearize(DevTopology t, const dou
                                                          double* __restrict__ lm_acc,
                                                          double* __restrict__ split_part,
                                                          double* __restrict__ tile_cost) {
-  __shared__ double red[kJac ? kObsTile * kLmAcc : 1];
-  __shared__ int32_t seg[kJac ? kObsTile : 1];
+  __shared__ double red[kJac ? kLinVals : 1][kJac ? kObsTile + 1 : 1];
+  __shared__ int32_t seg[kJac ? kObsTile : 1];    // landmark of each observation
+  __shared__ uint8_t own[kJac ? kObsTile : 1];    // made by the store vertex (not pose-coupled)
+  __shared__ int16_t head[kJac ? kObsTile + 1 : 1];  // first observation of each run
+  __shared__ int32_t wave_runs[4];
   __shared__ double lds4[4];
   const int tid = threadIdx.x;
   const int b = tile_begin[blockIdx.x], e = tile_begin[blockIdx.x + 1];
   const int o = b + tid;
-  double acc[kLmAcc];
-  for (int i = 0; i < kLmAcc; ++i) acc[i] = 0.0;
+  double acc[kLinVals];
+  for (int i = 0; i < kLinVals; ++i) acc[i] = 0.0;
   double cost = 0.0, fixed = 0.0;
   int32_t l = -1;
+  bool pose_coupled = true;
   if (o < e) {
     l = t.obs_landmark[o];
     const uint32_t flags = t.lm_flags[l];
-    ObsEval ev;
+    double rec[kObsRecord] = {};
     if (flags & kLmActive) {
+      ObsEval ev;
       eval_observation<kJac>(t, o, vert, vR, lm, ev);
       const int32_t meta = t.obs_meta[o];
       const int32_t type = obs_type(meta);
       const double s = ev.r[0] * ev.r[0] + ev.r[1] * ev.r[1];
       double rho[3];
       robust_loss(loss.type, loss_scale(loss, type, t.obs_sinv[o]), s, rho);
-      const bool pose_coupled = type != kTypeKeyframe;
+      pose_coupled = type != kTypeKeyframe;
       const bool has_var = !(flags & kLmConstant) ||
                            (pose_coupled && (obs_observer_var(meta) || t.vertex_var[t.lm_anchor[l]] >= 0));
       if (has_var) cost = 0.5 * rho[0]; else fixed = 0.5 * rho[0];
@@ -257,71 +278,85 @@ __global__ __launch_bounds__(kObsTile) void k_linearize(DevTopology t, const dou
           rs = sq1 / (1.0 - alpha);
           asq = alpha / s;
         }
-        double rr[2] = {ev.r[0] * rs, ev.r[1] * rs};
-        auto correct = [&](double* J, int cols) {
-          for (int c = 0; c < cols; ++c) {
-            const double rtj = J[c] * ev.r[0] + J[cols + c] * ev.r[1];
-            J[c] = sq1 * (J[c] - asq * ev.r[0] * rtj);
-            J[cols + c] = sq1 * (J[cols + c] - asq * ev.r[1] * rtj);
+        rec[0] = ev.r[0] * rs;
+        rec[1] = ev.r[1] * rs;
+        for (int c = 0; c < 3; ++c) {
+          const double rtj = ev.K[c] * ev.r[0] + ev.K[3 + c] * ev.r[1];
+          rec[2 + c] = sq1 * (ev.K[c] - asq * ev.r[0] * rtj);
+          rec[5 + c] = sq1 * (ev.K[3 + c] - asq * ev.r[1] * rtj);
+        }
+        if (kF32)
+          for (int i = 0; i < 6; ++i) {
+            const float hi = (float)rec[2 + i];
+            rec[2 + i] = (double)hi + (double)bf16_value(bf16_round((float)(rec[2 + i] - (double)hi)));
           }
-        };
-        correct(ev.Jl, 3);
-        if (pose_coupled) correct(ev.Jo, 6);
-        if (kF32) {
-          for (int i = 0; i < 6; ++i) ev.Jl[i] = (double)(float)ev.Jl[i];
-          for (int i = 0; i < 12; ++i) ev.Jo[i] = (double)(float)ev.Jo[i];
-          Rec32* rec = static_cast<Rec32*>(obs_rec) + o;
-          rec->r[0] = rr[0]; rec->r[1] = rr[1];
-          for (int i = 0; i < 6; ++i) rec->J[i] = (float)ev.Jl[i];
-          for (int i = 0; i < 12; ++i) rec->J[6 + i] = (float)ev.Jo[i];
-        } else {
-          double* rec = static_cast<double*>(obs_rec) + (size_t)kObsRecord * o;
-          rec[0] = rr[0]; rec[1] = rr[1];
-          for (int i = 0; i < 6; ++i) rec[2 + i] = ev.Jl[i];
-          for (int i = 0; i < 12; ++i) rec[8 + i] = ev.Jo[i];
-        }
-        const double* J = ev.Jl;
-        double V[6], g[3];
-        V[0] = J[0] * J[0] + J[3] * J[3];
-        V[1] = J[0] * J[1] + J[3] * J[4];
-        V[2] = J[0] * J[2] + J[3] * J[5];
-        V[3] = J[1] * J[1] + J[4] * J[4];
-        V[4] = J[1] * J[2] + J[4] * J[5];
-        V[5] = J[2] * J[2] + J[5] * J[5];
-        for (int c = 0; c < 3; ++c) g[c] = J[c] * rr[0] + J[3 + c] * rr[1];
-        for (int i = 0; i < 6; ++i) acc[i] = V[i];
-        for (int i = 0; i < 3; ++i) acc[12 + i] = g[i];
-        if (pose_coupled) {
-          for (int i = 0; i < 6; ++i) acc[6 + i] = V[i];
-          for (int i = 0; i < 3; ++i) acc[15 + i] = g[i];
-        }
+        for (int i = 0; i < 3; ++i) rec[8 + i] = ev.pI[i];
+        double J[6];
+        for (int r = 0; r < 2; ++r)
+          for (int c = 0; c < 3; ++c)
+            J[r * 3 + c] = rec[2 + 3 * r] * ev.G[c] + rec[3 + 3 * r] * ev.G[3 + c] + rec[4 + 3 * r] * ev.G[6 + c];
+        acc[0] = J[0] * J[0] + J[3] * J[3];
+        acc[1] = J[0] * J[1] + J[3] * J[4];
+        acc[2] = J[0] * J[2] + J[3] * J[5];
+        acc[3] = J[1] * J[1] + J[4] * J[4];
+        acc[4] = J[1] * J[2] + J[4] * J[5];
+        acc[5] = J[2] * J[2] + J[5] * J[5];
+        for (int c = 0; c < 3; ++c) acc[6 + c] = J[c] * rec[0] + J[3 + c] * rec[1];
       }
-    } else if (kJac) {
+    }
+    if (kJac) {
       if (kF32) {
-        Rec32* rec = static_cast<Rec32*>(obs_rec) + o;
-        rec->r[0] = rec->r[1] = 0.0;
-        for (int i = 0; i < 18; ++i) rec->J[i] = 0.0f;
+        Rec32* out = static_cast<Rec32*>(obs_rec) + o;
+        for (int i = 0; i < 2; ++i) out->r[i] = rec[i];
+        for (int i = 0; i < 3; ++i) out->p[i] = rec[8 + i];
+        for (int i = 0; i < 6; ++i) {
+          const float hi = (float)rec[2 + i];  // the sum rounds back to its parts
+          out->K[i] = hi;
+          out->lo[i] = bf16_round((float)(rec[2 + i] - (double)hi));
+        }
       } else {
-        double* rec = static_cast<double*>(obs_rec) + (size_t)kObsRecord * o;
-        for (int i = 0; i < kObsRecord; ++i) rec[i] = 0.0;
+        // Records are 96 bytes and the array is 256-byte aligned.
+        double2* out = reinterpret_cast<double2*>(static_cast<double*>(obs_rec) + (size_t)kObsRecord * o);
+        for (int i = 0; i < kObsRecord / 2; ++i) out[i] = make_double2(rec[2 * i], rec[2 * i + 1]);
       }
     }
   }
   if (kJac) {
-    for (int i = 0; i < kLmAcc; ++i) red[tid * kLmAcc + i] = acc[i];
-    seg[tid] = (o < e) ? l : -1;
+    for (int i = 0; i < kLinVals; ++i) red[i][tid] = acc[i];
+    seg[tid] = l;
+    own[tid] = pose_coupled ? 0 : 1;
     __syncthreads();
-    // Segment heads reduce their landmark's run in a fixed order.
-    if (o < e && (tid == 0 || seg[tid - 1] != l)) {
-      double sum[kLmAcc];
-      for (int i = 0; i < kLmAcc; ++i) sum[i] = 0.0;
-      for (int k = tid; k < kObsTile && seg[k] == l; ++k)
-        for (int i = 0; i < kLmAcc; ++i) sum[i] += red[k * kLmAcc + i];
+    // Runs of one landmark, in order: first observations into head.
+    const bool first = o < e && (tid == 0 || seg[tid - 1] != l);
+    const uint64_t mask = __ballot(first);
+    const int lane = tid & 63, wave = tid >> 6;
+    if (lane == 0) wave_runs[wave] = __popcll(mask);
+    __syncthreads();
+    int before = __popcll(mask & ((1ull << lane) - 1ull)), runs = 0;
+    for (int w = 0; w < 4; ++w) {
+      if (w < wave) before += wave_runs[w];
+      runs += wave_runs[w];
+    }
+    if (first) head[before] = (int16_t)tid;
+    if (tid == 0) head[runs] = (int16_t)(e - b);
+    __syncthreads();
+    for (int it = tid; it < runs * kLinVals; it += kObsTile) {
+      const int run = it / kLinVals, c = it - run * kLinVals;
+      const int k0 = head[run], k1 = head[run + 1];
+      double sum = 0.0, sum_own = 0.0;
+      for (int k = k0; k < k1; ++k) {
+        const double v = red[c][k];
+        if (own[k]) sum_own += v; else sum += v;
+      }
+      const int32_t lr = seg[k0];
       // A split landmark owns its tiles whole: the tile's sum goes to the
       // tile's slot, and k_split_sum adds the slots in tile order.
-      double* dst = (t.lm_flags[l] & kLmSplit) ? split_part + (size_t)kLmAcc * blockIdx.x
-                                               : lm_acc + (size_t)kLmAcc * l;
-      for (int i = 0; i < kLmAcc; ++i) dst[i] = sum[i];
+      double* dst = (t.lm_flags[lr] & kLmSplit) ? split_part + (size_t)kLmAcc * blockIdx.x
+                                                : lm_acc + (size_t)kLmAcc * lr;
+      // V, V_mission (6 each), then g, g_mission (3 each).
+      const int at = c < 6 ? c : 6 + c, step = c < 6 ? 6 : 3;
+      dst[at] = sum + sum_own;
+      dst[at + step] = sum;
     }
   }
   const double c_sum = block_sum256(cost, lds4);
@@ -365,14 +400,15 @@ __global__ __launch_bounds__(kRowThreads) void k_pose_rows(DevTopology t, const 
   const int ib = t.inc_ptr[i], ie = t.inc_ptr[i + 1];
   double g[6] = {0, 0, 0, 0, 0, 0}, d[6] = {0, 0, 0, 0, 0, 0}, jj[21];
   for (int k = 0; k < 21; ++k) jj[k] = 0.0;
+  const double* Rv = vR + 12 * t.var_vertex[i];
   for (int k = ib + threadIdx.x; k < ie; k += kRowThreads) {
     const int32_t x = t.inc[k];
     if (x >= 0) {
       const RecView<kF32> rec(obs_rec, x);
       double Jo[12];
-      for (int k2 = 0; k2 < 12; ++k2) Jo[k2] = rec[8 + k2];
+      observer_jacobian(rec, Rv, Jo);
       for (int c = 0; c < 6; ++c) {
-        g[c] += Jo[c] * rec[0] + Jo[6 + c] * rec[1];
+        g[c] += Jo[c] * rec.r(0) + Jo[6 + c] * rec.r(1);
         d[c] += Jo[c] * Jo[c] + Jo[6 + c] * Jo[6 + c];
       }
       int u = 0;
@@ -470,13 +506,6 @@ __global__ void k_landmark_prep(DevTopology t, const double* __restrict__ lm_acc
 
 // ------------------------------------------------------------ Schur complement
 
-// W' = Jl^T (Jo C) (3x6): landmark side unscaled, pose side scaled.
-template <class Rec>
-__device__ inline void wprime_obs(const Rec& rec, const double* cs, double* W) {
-  for (int a = 0; a < 3; ++a)
-    for (int c = 0; c < 6; ++c) W[a * 6 + c] = (rec[2 + a] * rec[8 + c] + rec[5 + a] * rec[14 + c]) * cs[c];
-}
-
 // Factor blocks of the reduced camera system
 //   S = F'F + D^2 - sum_l W_l' Z_l W_l,  rhs = F'r - sum_l W_l' Z_l g_l,
 // with Z_l = C_l (C_l V_l C_l + D_l^2)^-1 C_l from k_landmark_prep. An
@@ -514,8 +543,16 @@ __global__ __launch_bounds__(256) void k_schur_factors(
     double Wx[18], rx[6];
     if (x >= 0) {
       const RecView<kF32> rec(obs_rec, x);
-      wprime_obs(rec, cs, Wx);
-      for (int c = 0; c < 6; ++c) rx[c] = cs[c] * (rec[8 + c] * rec[0] + rec[14 + c] * rec[1]);
+      const int v = t.var_vertex[i], la = t.lm_anchor[t.obs_landmark[x]];
+      double Jo[12], G[9], Jl[6];
+      observer_jacobian(rec, vR + 12 * v, Jo);
+      landmark_to_imu(t, obs_type(t.obs_meta[x]), la, v, vR + 12 * la, vR + 12 * v, G);
+      for (int r = 0; r < 2; ++r)
+        for (int c = 0; c < 3; ++c)
+          Jl[r * 3 + c] = rec.K(3 * r) * G[c] + rec.K(3 * r + 1) * G[3 + c] + rec.K(3 * r + 2) * G[6 + c];
+      for (int a = 0; a < 3; ++a)
+        for (int c = 0; c < 6; ++c) Wx[a * 6 + c] = (Jl[a] * Jo[c] + Jl[3 + a] * Jo[6 + c]) * cs[c];
+      for (int c = 0; c < 6; ++c) rx[c] = cs[c] * (Jo[c] * rec.r(0) + Jo[6 + c] * rec.r(1));
     } else {
       const int32_t l = -1 - x;
       const int v = t.var_vertex[i];
@@ -1070,6 +1107,9 @@ __global__ void k_block_inverse(int32_t Pvar, const int32_t* __restrict__ diag_p
 // system, w = C_p y_p (per vertex) and u = C_l y_l = Z_l (g_l - sum W' y_p):
 // J y = Jl u + Jo w_o + Jl M w_a per observation and
 // model_cost_change = sum (J y)'r - |J y|^2 / 2 (ceres ComputeTrustRegionStep).
+// From the records, J y = K (s + G (u + M w_a)), s = |q|^2 p_I x w_rot -
+// R_I_M w_pos, G = R_I_M R_M_B, so the landmark side is taken in the landmark's
+// mission frame: the sums of R_M_I K'K s per landmark, then R_M_B' u once.
 // One work-group per linearization tile of whole landmarks: each observation
 // record is read once; the landmark sums are taken by the segment heads in a
 // fixed order. Tiles of landmarks split over several tiles are left to
@@ -1106,6 +1146,42 @@ __device__ inline void landmark_step(const DevTopology& t, int l, const double* 
   }
 }
 
+// Vector x between the landmark's mission frame and the observer's IMU frame
+// of a pose-coupled observation by vertex v: to_imu R_I_M (R_M_LM) x, else the
+// transpose.
+__device__ inline void rotate_observer(const DevTopology& t, int32_t type, int l, int v, const double* Rv, bool to_imu,
+                                       const double* x, double* out) {
+  double m[3];
+  if (type != kTypeGlobal) {
+    if (to_imu) mat3_vec(Rv, x, out);
+    else mat3t_vec(Rv, x, out);
+    return;
+  }
+  const double* TL = t.mission_T + 12 * t.vertex_mission[t.lm_anchor[l]];
+  const double* TM = t.mission_T + 12 * t.vertex_mission[v];
+  double g[3];
+  if (to_imu) {
+    mat3_vec(TL, x, g);
+    mat3t_vec(TM, g, m);
+    mat3_vec(Rv, m, out);
+  } else {
+    mat3t_vec(Rv, x, m);
+    mat3_vec(TM, m, g);
+    mat3t_vec(TL, g, out);
+  }
+}
+
+// s of an observation: |q|^2 p_I x w_rot - R_I_M w_pos (J_observer w = K s).
+template <class Rec>
+__device__ inline void observer_motion(const Rec& rec, const double* Rv, const double* wo, double* s) {
+  double rp[3];
+  mat3_vec(Rv, wo + 3, rp);
+  const double n2 = Rv[9];
+  s[0] = n2 * (rec.p(1) * wo[2] - rec.p(2) * wo[1]) - rp[0];
+  s[1] = n2 * (rec.p(2) * wo[0] - rec.p(0) * wo[2]) - rp[1];
+  s[2] = n2 * (rec.p(0) * wo[1] - rec.p(1) * wo[0]) - rp[2];
+}
+
 template <bool kF32>
 __global__ __launch_bounds__(kObsTile) void k_back_substitute(DevTopology t, const int32_t* __restrict__ tile_begin,
                                                               const double* __restrict__ vR,
@@ -1116,7 +1192,7 @@ __global__ __launch_bounds__(kObsTile) void k_back_substitute(DevTopology t, con
                                                               const double* __restrict__ w, double* __restrict__ u_out,
                                                               double* __restrict__ part) {
   __shared__ double red[kObsTile * 3];
-  __shared__ double ush[kObsTile * 6];  // u and M w_a at each segment head
+  __shared__ double ush[kObsTile * 6];  // u, and R_B_M' (u + M w_a), at each segment head
   __shared__ int32_t seg[kObsTile];
   __shared__ double lds4[4];
   const int tid = threadIdx.x;
@@ -1126,10 +1202,10 @@ __global__ __launch_bounds__(kObsTile) void k_back_substitute(DevTopology t, con
     return;
   }
   const int o = b + tid;
-  int32_t l = -1;
+  int32_t l = -1, v = 0, type = kTypeKeyframe;
   uint32_t flags = 0;
-  double r[2] = {0, 0}, jl[6], jw[2] = {0, 0}, c[3] = {0, 0, 0};
-  bool coupled = false, ovar = false;
+  double K[6], s[3] = {0, 0, 0}, c[3] = {0, 0, 0}, r[2] = {0, 0};
+  const double* Rv = vR;
   if (o < e) {
     l = t.obs_landmark[o];
     flags = t.lm_flags[l];
@@ -1138,19 +1214,19 @@ __global__ __launch_bounds__(kObsTile) void k_back_substitute(DevTopology t, con
   if (active) {
     const RecView<kF32> rec(obs_rec, o);
     const int32_t meta = t.obs_meta[o];
-    coupled = obs_type(meta) != kTypeKeyframe;
-    ovar = coupled && obs_observer_var(meta);
-    r[0] = rec[0];
-    r[1] = rec[1];
-    for (int k = 0; k < 6; ++k) jl[k] = rec[2 + k];
-    if (ovar) {
-      const double* wo = w + 6 * t.vertex_var[t.obs_vertex[o]];
-      for (int rr = 0; rr < 2; ++rr) {
-        double s = 0.0;
-        for (int k = 0; k < 6; ++k) s += rec[8 + rr * 6 + k] * wo[k];
-        jw[rr] = s;
+    type = obs_type(meta);
+    for (int k = 0; k < 6; ++k) K[k] = rec.K(k);
+    r[0] = rec.r(0);
+    r[1] = rec.r(1);
+    if (type != kTypeKeyframe) {
+      v = t.obs_vertex[o];
+      Rv = vR + 12 * v;
+      if (obs_observer_var(meta)) {
+        observer_motion(rec, Rv, w + 6 * t.vertex_var[v], s);
+        const double j0 = K[0] * s[0] + K[1] * s[1] + K[2] * s[2], j1 = K[3] * s[0] + K[4] * s[1] + K[5] * s[2];
+        const double kj[3] = {-(K[0] * j0 + K[3] * j1), -(K[1] * j0 + K[4] * j1), -(K[2] * j0 + K[5] * j1)};
+        rotate_observer(t, type, l, v, Rv, false, kj, c);
       }
-      for (int a = 0; a < 3; ++a) c[a] = -(jl[a] * jw[0] + jl[3 + a] * jw[1]);
     }
   }
   for (int k = 0; k < 3; ++k) red[tid * 3 + k] = c[k];
@@ -1159,27 +1235,36 @@ __global__ __launch_bounds__(kObsTile) void k_back_substitute(DevTopology t, con
   double uu = 0.0;
   if (active && (tid == 0 || seg[tid - 1] != l)) {
     const double* acc = lm_acc + (size_t)kLmAcc * l;
-    double tv[3] = {acc[12], acc[13], acc[14]};
+    const double* Ra = vR + 12 * t.lm_anchor[l];
+    double sum[3] = {0, 0, 0}, tv[3];
     for (int k = tid; k < kObsTile && seg[k] == l; ++k)
-      for (int a = 0; a < 3; ++a) tv[a] += red[k * 3 + a];
-    double u[3], Mwa[3];
+      for (int a = 0; a < 3; ++a) sum[a] += red[k * 3 + a];
+    mat3_vec(Ra, sum, tv);
+    for (int a = 0; a < 3; ++a) tv[a] += acc[12 + a];
+    double u[3], Mwa[3], um[3];
     landmark_step(t, l, vR, lm, lm_acc, lm_z, w, tv, u, Mwa);
     uu = u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
     for (int a = 0; a < 3; ++a) {
       u_out[3 * l + a] = u[a];
       ush[tid * 6 + a] = u[a];
-      ush[tid * 6 + 3 + a] = Mwa[a];
+      Mwa[a] += u[a];
     }
+    mat3t_vec(Ra, Mwa, um);
+    for (int a = 0; a < 3; ++a) ush[tid * 6 + 3 + a] = um[a];
   }
   __syncthreads();
   double mcc = 0.0;
   if (active) {
     const int h = t.lm_begin[l] - b;
-    double lu[3];
-    for (int a = 0; a < 3; ++a) lu[a] = ush[h * 6 + a] + (coupled ? ush[h * 6 + 3 + a] : 0.0);
-    double jy[2];
-    for (int rr = 0; rr < 2; ++rr) jy[rr] = jl[rr * 3] * lu[0] + jl[rr * 3 + 1] * lu[1] + jl[rr * 3 + 2] * lu[2] + jw[rr];
-    mcc = jy[0] * r[0] + jy[1] * r[1] - 0.5 * (jy[0] * jy[0] + jy[1] * jy[1]);
+    double y[3];
+    if (type == kTypeKeyframe) {
+      for (int a = 0; a < 3; ++a) y[a] = ush[h * 6 + a];
+    } else {
+      rotate_observer(t, type, l, v, Rv, true, &ush[h * 6 + 3], y);
+      for (int a = 0; a < 3; ++a) y[a] += s[a];
+    }
+    const double j0 = K[0] * y[0] + K[1] * y[1] + K[2] * y[2], j1 = K[3] * y[0] + K[4] * y[1] + K[5] * y[2];
+    mcc = j0 * r[0] + j1 * r[1] - 0.5 * (j0 * j0 + j1 * j1);
   }
   const double s1 = block_sum256(mcc, lds4);
   const double s2 = block_sum256(uu, lds4);
@@ -1207,38 +1292,49 @@ __global__ __launch_bounds__(256) void k_back_substitute_split(DevTopology t, in
     const int l = split_ids[k];
     const int lb = t.lm_begin[l], le = t.lm_begin[l + 1];
     const double* acc = lm_acc + (size_t)kLmAcc * l;
-    double tv[3] = {acc[12], acc[13], acc[14]};
+    const double* Ra = vR + 12 * t.lm_anchor[l];
+    double sum[3] = {0, 0, 0}, tv[3];
     for (int o = lb; o < le; ++o) {
-      const int32_t meta = t.obs_meta[o];
-      if (obs_type(meta) == kTypeKeyframe || !obs_observer_var(meta)) continue;
+      const int32_t meta = t.obs_meta[o], type = obs_type(meta);
+      if (type == kTypeKeyframe || !obs_observer_var(meta)) continue;
       const RecView<kF32> rec(obs_rec, o);
-      const double* wo = w + 6 * t.vertex_var[t.obs_vertex[o]];
-      double jw[2];
-      for (int rr = 0; rr < 2; ++rr) {
-        double s = 0.0;
-        for (int c = 0; c < 6; ++c) s += rec[8 + rr * 6 + c] * wo[c];
-        jw[rr] = s;
-      }
-      for (int a = 0; a < 3; ++a) tv[a] -= rec[2 + a] * jw[0] + rec[5 + a] * jw[1];
+      const int v = t.obs_vertex[o];
+      double s[3], c[3];
+      observer_motion(rec, vR + 12 * v, w + 6 * t.vertex_var[v], s);
+      const double j0 = rec.K(0) * s[0] + rec.K(1) * s[1] + rec.K(2) * s[2];
+      const double j1 = rec.K(3) * s[0] + rec.K(4) * s[1] + rec.K(5) * s[2];
+      const double kj[3] = {-(rec.K(0) * j0 + rec.K(3) * j1), -(rec.K(1) * j0 + rec.K(4) * j1),
+                            -(rec.K(2) * j0 + rec.K(5) * j1)};
+      rotate_observer(t, type, l, v, vR + 12 * v, false, kj, c);
+      for (int a = 0; a < 3; ++a) sum[a] += c[a];
     }
-    double u[3], Mwa[3];
+    mat3_vec(Ra, sum, tv);
+    for (int a = 0; a < 3; ++a) tv[a] += acc[12 + a];
+    double u[3], Mwa[3], um[3];
     landmark_step(t, l, vR, lm, lm_acc, lm_z, w, tv, u, Mwa);
     uu = u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
-    for (int a = 0; a < 3; ++a) u_out[3 * l + a] = u[a];
+    for (int a = 0; a < 3; ++a) {
+      u_out[3 * l + a] = u[a];
+      Mwa[a] += u[a];
+    }
+    mat3t_vec(Ra, Mwa, um);
     for (int o = lb; o < le; ++o) {
-      const int32_t meta = t.obs_meta[o];
+      const int32_t meta = t.obs_meta[o], type = obs_type(meta);
       const RecView<kF32> rec(obs_rec, o);
-      const bool coupled = obs_type(meta) != kTypeKeyframe;
-      double lu[3];
-      for (int a = 0; a < 3; ++a) lu[a] = u[a] + (coupled ? Mwa[a] : 0.0);
-      double jy[2];
-      for (int rr = 0; rr < 2; ++rr) jy[rr] = rec[2 + rr * 3] * lu[0] + rec[3 + rr * 3] * lu[1] + rec[4 + rr * 3] * lu[2];
-      if (coupled && obs_observer_var(meta)) {
-        const double* wo = w + 6 * t.vertex_var[t.obs_vertex[o]];
-        for (int rr = 0; rr < 2; ++rr)
-          for (int c = 0; c < 6; ++c) jy[rr] += rec[8 + rr * 6 + c] * wo[c];
+      double y[3] = {u[0], u[1], u[2]};
+      if (type != kTypeKeyframe) {
+        const int v = t.obs_vertex[o];
+        const double* Rv = vR + 12 * v;
+        rotate_observer(t, type, l, v, Rv, true, um, y);
+        if (obs_observer_var(meta)) {
+          double s[3];
+          observer_motion(rec, Rv, w + 6 * t.vertex_var[v], s);
+          for (int a = 0; a < 3; ++a) y[a] += s[a];
+        }
       }
-      mcc += jy[0] * rec[0] + jy[1] * rec[1] - 0.5 * (jy[0] * jy[0] + jy[1] * jy[1]);
+      const double j0 = rec.K(0) * y[0] + rec.K(1) * y[1] + rec.K(2) * y[2];
+      const double j1 = rec.K(3) * y[0] + rec.K(4) * y[1] + rec.K(5) * y[2];
+      mcc += j0 * rec.r(0) + j1 * rec.r(1) - 0.5 * (j0 * j0 + j1 * j1);
     }
   }
   const double s1 = block_sum256(mcc, lds4);

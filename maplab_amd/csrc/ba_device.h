@@ -59,8 +59,10 @@ struct RecView<true> {
   __host__ __device__ double K(int k) const { return static_cast<double>(q->K[k]) + static_cast<double>(bf16_value(q->lo[k])); }
   __host__ __device__ double p(int k) const { return q->p[k]; }
 };
-constexpr int kLmAcc = 18;           // V(6) V_mission(6) g(3) g_mission(3)
-constexpr int kLmZ = 9;              // Z(6, upper triangle) and a copy of g(3), read together per incidence
+constexpr int kLmAcc = 18;           // V_own(6) V_mission(6) g(3) g_mission(3); V = V_own + V_mission
+constexpr int kLmZ = 10;             // T(6, lower triangle, Z = T'T), T g(3), one unused
+constexpr int kLmAnchor = 18;        // anchor's factor: U(9), the negated self product(6), rhs(3)
+constexpr int kFactor = 12;          // factor block: P(3x3), p_I(3)
 
 // A batch of independent scalar reductions (k_reduce_many), 1..kMaxReduceBatch
 // of them.

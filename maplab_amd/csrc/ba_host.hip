@@ -46,18 +46,18 @@ void launch_pose_rows(hipStream_t s, const DevTopology& t, const double* vert, c
 void launch_jacobi_scaling(hipStream_t s, int32_t Pvar, int32_t L, int32_t use, const double* pose_diag,
                            const double* lm_acc, double* pose_scale, double* lm_scale);
 void launch_landmark_prep(hipStream_t s, const DevTopology& t, const double* lm_acc, const double* lm_scale,
-                          double inv_mu, double min_diag, double max_diag, double* lm_z, int32_t* fail);
+                          double inv_mu, double min_diag, double max_diag, double* lm_z, double* lm_anc,
+                          int32_t* fail);
 void launch_schur_factors(hipStream_t s, const DevTopology& t, int32_t n_g, const int32_t* g_row,
                           const int32_t* g_inc_ptr, const int32_t* g_inc, const double* vR, const double* lm,
-                          const double* obs_rec, const double* lm_acc, const double* pose_scale, double* gw,
-                          double* gr0, bool f32 = false);
+                          const double* obs_rec, double* gf, double* gk, bool f32 = false);
 void launch_schur_blocks(hipStream_t s, const DevTopology& t, const SchurTilesDev& d, int32_t nub, const int4* ublk,
-                         const double* gw, const double* gr0, const double* lm_acc, const double* lm_z,
-                         const double* pose_scale, const double* pose_diag, const double* pose_jtj, double inv_mu,
-                         double min_diag, double max_diag, double* partial, double* S, double* rhs,
+                         const double* gf, const double* gk, const double* lm_z, const double* lm_anc,
+                         const double* vR, const double* pose_scale, const double* pose_diag, const double* pose_jtj,
+                         double inv_mu, double min_diag, double max_diag, double* partial, double* S, double* rhs,
                          int32_t items_per_wg, int32_t xcd_map);
-void launch_schur_tiles(hipStream_t s, const SchurTilesDev& d, const double* gw, const double* gr0,
-                        const double* lm_acc, const double* lm_z, double* partial, int32_t items_per_wg,
+void launch_schur_tiles(hipStream_t s, const SchurTilesDev& d, const double* gf, const double* gk,
+                        const double* lm_z, const double* lm_anc, double* partial, int32_t items_per_wg,
                         int32_t xcd_map);
 bool schur_items_per_wg_supported(int32_t n);
 int32_t calib_entries();
@@ -188,7 +188,7 @@ struct mlba_handle {
   mlba_preconditioner_stats lp_stats{};
   DBuf<uint32_t> lm_flags;
   DBuf<uint8_t> lm_bad;                 // outlier flags of the last rejection pass
-  DBuf<double> lm, lm_cand, lm_acc, lm_scale, lm_z, lm_u;
+  DBuf<double> lm, lm_cand, lm_acc, lm_scale, lm_z, lm_anc, lm_u;
   DBuf<double> vert, vert_cand, vR, vR_cand;
   DBuf<int32_t> vertex_mission_d, vertex_var, var_vertex;
   DBuf<DevCamera> cams, cams_cand;
@@ -205,7 +205,7 @@ struct mlba_handle {
   DBuf<uint16_t> t_batch_off, t_pairs;
   DBuf<int32_t> t_uslot_ptr, t_uslot;   // partial slots of every upper block
   DBuf<int32_t> t_seg_order;            // segments in dispatch order
-  DBuf<double> gw, gr0;                 // per-linearization factor blocks (W or A_l, r0)
+  DBuf<double> gf, gk;                  // per-linearization factor blocks (P, p) and their k
   DBuf<double> schur_partial;           // kTilePartial per segment
   std::vector<int4> h_segs;             // host copy of the segments (dispatch order)
   // Dispatch schedule of k_schur_tiles (mlba_autotune): tile rows per band of
@@ -571,8 +571,8 @@ int build_topology(mlba_handle* h) {
   const size_t vb = (Pvar + 255) / 256 + 1;
   bool ok = h->tile_cost.alloc(2 * T) && h->tile_cost2.alloc(2 * T) && h->S.alloc(36 * (size_t)h->nnzb) &&
             h->split_part.alloc(h->n_split ? kLmAcc * T : 1) &&
-            h->gw.alloc(18 * std::max<size_t>(st.g_row.size(), 1)) &&
-            h->gr0.alloc(6 * std::max<size_t>(st.g_row.size(), 1)) &&
+            h->gf.alloc(kFactor * std::max<size_t>(st.g_row.size(), 1)) &&
+            h->gk.alloc(3 * std::max<size_t>(st.g_row.size(), 1)) &&
             h->schur_partial.alloc((size_t)kTilePartial * std::max(h->n_segs, 1)) &&
             h->pose_jtj.alloc(36 * (size_t)std::max(Pvar, 1)) &&
             h->rhs.alloc(V6) && h->pose_grad.alloc(V6) && h->pose_diag.alloc(V6) && h->pose_scale.alloc(V6) &&
@@ -899,12 +899,11 @@ DevLoss make_loss(const mlba_options* o) {
 // Linearize at the current state: residual records, landmark reductions,
 // vertex-row gradient and diag(F'F). Leaves cost / fixed cost / gradient
 // max norm in the scalar slots (device).
-// Per-linearization Schur factors (W, r0 of every factor block, anchor maps);
-// needs the Jacobi scaling of the solve.
+// Per-linearization Schur factors (P, p and k of every factor block).
 void schur_factors(mlba_handle* h) {
   KernelTimer kt(h, MLBA_KERNEL_SCHUR_FACTORS);
   launch_schur_factors(h->stream, h->topo, h->n_g, h->g_row.p, h->g_inc_ptr.p, h->g_inc.p, h->vR.p, h->lm.p,
-                       h->obs_rec.p, h->lm_acc.p, h->pose_scale.p, h->gw.p, h->gr0.p, h->f32_jac);
+                       h->obs_rec.p, h->gf.p, h->gk.p, h->f32_jac);
 }
 
 int linearize(mlba_handle* h, const mlba_options* o) {
@@ -1157,12 +1156,12 @@ int minimize(mlba_handle* h, const mlba_options* o, double initial_radius, mlba_
       {
         KernelTimer kt(h, MLBA_KERNEL_LANDMARK_PREP);
         launch_landmark_prep(s, h->topo, h->lm_acc.p, h->lm_scale.p, inv_mu, o->min_lm_diagonal,
-                             o->max_lm_diagonal, h->lm_z.p, h->fail.p);
+                             o->max_lm_diagonal, h->lm_z.p, h->lm_anc.p, h->fail.p);
       }
       {
         KernelTimer kt(h, MLBA_KERNEL_SCHUR_BLOCKS);
-        launch_schur_blocks(s, h->topo, h->tdev, h->n_upper, h->ublk.p, h->gw.p, h->gr0.p, h->lm_acc.p, h->lm_z.p,
-                            h->pose_scale.p, h->pose_diag.p, h->pose_jtj.p, inv_mu, o->min_lm_diagonal,
+        launch_schur_blocks(s, h->topo, h->tdev, h->n_upper, h->ublk.p, h->gf.p, h->gk.p, h->lm_z.p, h->lm_anc.p,
+                            h->vR.p, h->pose_scale.p, h->pose_diag.p, h->pose_jtj.p, inv_mu, o->min_lm_diagonal,
                             o->max_lm_diagonal, h->schur_partial.p, h->S.p, h->rhs.p, h->sched_waves,
                             h->sched_xcd);
       }
@@ -1521,7 +1520,7 @@ int32_t mlba_create(const mlba_problem_desc* d, mlba_handle** out) {
     return fail_out(rc);
   const bool ok = h->obs_rec.alloc((size_t)kObsRecord * N) && h->vert_cand.alloc(7 * (size_t)P) &&
                   h->vR.alloc(12 * (size_t)P) && h->vR_cand.alloc(12 * (size_t)P) && h->lm_cand.alloc(3 * (size_t)L) &&
-                  h->lm_acc.alloc((size_t)kLmAcc * L) && h->lm_scale.alloc(3 * (size_t)L) &&
+                  h->lm_acc.alloc((size_t)kLmAcc * L) && h->lm_anc.alloc((size_t)kLmAnchor * L) && h->lm_scale.alloc(3 * (size_t)L) &&
                   h->lm_z.alloc(kLmZ * (size_t)L) && h->lm_u.alloc(3 * (size_t)L) && h->scal.alloc(kNumSlots) &&
                   h->fail.alloc(1) && h->pcg_state.alloc(pcg_state_bytes());
   if (!ok) { h->err = "device allocation failed"; return fail_out(MLBA_ENOMEM); }
@@ -1812,9 +1811,9 @@ int build_rcs(mlba_handle* h, const mlba_options* o, double radius) {
   HIP_OK(hipMemsetAsync(h->fail.p, 0, sizeof(int32_t), s));
   const double inv_mu = 1.0 / radius;
   launch_landmark_prep(s, h->topo, h->lm_acc.p, h->lm_scale.p, inv_mu, o->min_lm_diagonal, o->max_lm_diagonal,
-                       h->lm_z.p, h->fail.p);
-  launch_schur_blocks(s, h->topo, h->tdev, h->n_upper, h->ublk.p, h->gw.p, h->gr0.p, h->lm_acc.p, h->lm_z.p,
-                      h->pose_scale.p, h->pose_diag.p, h->pose_jtj.p, inv_mu, o->min_lm_diagonal,
+                       h->lm_z.p, h->lm_anc.p, h->fail.p);
+  launch_schur_blocks(s, h->topo, h->tdev, h->n_upper, h->ublk.p, h->gf.p, h->gk.p, h->lm_z.p, h->lm_anc.p,
+                      h->vR.p, h->pose_scale.p, h->pose_diag.p, h->pose_jtj.p, inv_mu, o->min_lm_diagonal,
                       o->max_lm_diagonal, h->schur_partial.p, h->S.p, h->rhs.p, h->sched_waves, h->sched_xcd);
   HIP_OK(hipGetLastError());
   return MLBA_OK;
@@ -2468,7 +2467,7 @@ int32_t mlba_autotune(mlba_handle* h, const mlba_options* o, int32_t repeats, ml
     schur_factors(h);
     HIP_OK(hipMemsetAsync(h->fail.p, 0, sizeof(int32_t), s));
     launch_landmark_prep(s, h->topo, h->lm_acc.p, h->lm_scale.p, 1.0 / o->initial_trust_region_radius,
-                         o->min_lm_diagonal, o->max_lm_diagonal, h->lm_z.p, h->fail.p);
+                         o->min_lm_diagonal, o->max_lm_diagonal, h->lm_z.p, h->lm_anc.p, h->fail.p);
     HIP_OK(hipGetLastError());
     hipEvent_t e0, e1;
     HIP_OK(hipEventCreate(&e0));
@@ -2477,11 +2476,11 @@ int32_t mlba_autotune(mlba_handle* h, const mlba_options* o, int32_t repeats, ml
       return set_err(h, MLBA_EDEVICE, "hipEventCreate failed");
     }
     auto time_items = [&]() -> double {
-      launch_schur_tiles(s, h->tdev, h->gw.p, h->gr0.p, h->lm_acc.p, h->lm_z.p, h->schur_partial.p, h->sched_waves,
+      launch_schur_tiles(s, h->tdev, h->gf.p, h->gk.p, h->lm_z.p, h->lm_anc.p, h->schur_partial.p, h->sched_waves,
                          h->sched_xcd);  // warm
       (void)hipEventRecord(e0, s);
       for (int k = 0; k < repeats; ++k)
-        launch_schur_tiles(s, h->tdev, h->gw.p, h->gr0.p, h->lm_acc.p, h->lm_z.p, h->schur_partial.p,
+        launch_schur_tiles(s, h->tdev, h->gf.p, h->gk.p, h->lm_z.p, h->lm_anc.p, h->schur_partial.p,
                            h->sched_waves, h->sched_xcd);
       (void)hipEventRecord(e1, s);
       (void)hipEventSynchronize(e1);
@@ -2597,11 +2596,11 @@ int32_t mlba_time_kernels(mlba_handle* h, const mlba_options* o, int32_t repeats
   HIP_OK(hipMemsetAsync(h->fail.p, 0, sizeof(int32_t), s));
   t->landmark_prep_ms = timed([&] {
     launch_landmark_prep(s, h->topo, h->lm_acc.p, h->lm_scale.p, inv_mu, o->min_lm_diagonal, o->max_lm_diagonal,
-                         h->lm_z.p, h->fail.p);
+                         h->lm_z.p, h->lm_anc.p, h->fail.p);
   });
   t->schur_blocks_ms = timed([&] {
-    launch_schur_blocks(s, h->topo, h->tdev, h->n_upper, h->ublk.p, h->gw.p, h->gr0.p, h->lm_acc.p, h->lm_z.p,
-                        h->pose_scale.p, h->pose_diag.p, h->pose_jtj.p, inv_mu, o->min_lm_diagonal,
+    launch_schur_blocks(s, h->topo, h->tdev, h->n_upper, h->ublk.p, h->gf.p, h->gk.p, h->lm_z.p, h->lm_anc.p,
+                        h->vR.p, h->pose_scale.p, h->pose_diag.p, h->pose_jtj.p, inv_mu, o->min_lm_diagonal,
                         o->max_lm_diagonal, h->schur_partial.p, h->S.p, h->rhs.p, h->sched_waves, h->sched_xcd);
   });
   t->block_inverse_ms = timed([&] { launch_block_inverse(s, h->Pvar, h->diag_pos.p, h->S.p, h->Minv.p, h->fail.p); });

@@ -35,9 +35,10 @@ namespace mlba {
 
 // ------------------------------------------------------------ utilities
 
-// Inverse of a symmetric positive definite 3x3 matrix given as
-// (xx xy xz yy yz zz); returns false when not positive definite.
-__device__ inline bool spd3_inverse(const double* a, double* out) {
+// L^-1 (rows i00; i10 i11; i20 i21 i22) of the Cholesky factor L of a symmetric
+// positive definite 3x3 matrix given as (xx xy xz yy yz zz); returns false
+// when not positive definite.
+__device__ inline bool spd3_inverse_factor(const double* a, double* out) {
   const double l00 = sqrt(a[0]);
   if (!(l00 > 0.0)) return false;
   const double l10 = a[1] / l00, l20 = a[2] / l00;
@@ -51,15 +52,25 @@ __device__ inline bool spd3_inverse(const double* a, double* out) {
   const double i00 = 1.0 / l00, i11 = 1.0 / l11, i22 = 1.0 / l22;
   const double i10 = -l10 * i00 * i11;
   const double i21 = -l21 * i11 * i22;
-  const double i20 = -(l20 * i00 + l21 * i10) * i22;
-  // (L^-1)^T L^-1, L^-1 lower with rows (i00), (i10 i11), (i20 i21 i22).
-  out[0] = i00 * i00 + i10 * i10 + i20 * i20;
-  out[1] = i10 * i11 + i20 * i21;
-  out[2] = i20 * i22;
-  out[3] = i11 * i11 + i21 * i21;
-  out[4] = i21 * i22;
-  out[5] = i22 * i22;
+  out[0] = i00;
+  out[1] = i10;
+  out[2] = i11;
+  out[3] = -(l20 * i00 + l21 * i10) * i22;
+  out[4] = i21;
+  out[5] = i22;
   return true;
+}
+
+// T x and T'x of a lower-triangular 3x3 T (rows t0; t1 t2; t3 t4 t5).
+__device__ inline void tri_vec(const double* t, const double* x, double* out) {
+  out[0] = t[0] * x[0];
+  out[1] = t[1] * x[0] + t[2] * x[1];
+  out[2] = t[3] * x[0] + t[4] * x[1] + t[5] * x[2];
+}
+__device__ inline void trit_vec(const double* t, const double* x, double* out) {
+  out[0] = t[0] * x[0] + t[1] * x[1] + t[3] * x[2];
+  out[1] = t[2] * x[1] + t[4] * x[2];
+  out[2] = t[5] * x[2];
 }
 
 __device__ inline void sym3_full(const double* s, double* m) {
@@ -215,8 +226,8 @@ __device__ inline double loss_scale(const DevLoss& loss, int32_t type, double si
 }
 
 // Per observation: robust-corrected residual and Jacobian K into obs_rec;
-// per landmark: V = sum Jl'Jl, V_mission (pose-coupled observations only),
-// g = sum Jl'r, g_mission; per tile: cost and fixed cost.
+// per landmark: sum Jl'Jl over the store vertex's own observations (V_own) and
+// over the pose-coupled ones (V_mission), g = sum Jl'r, g_mission; per tile: cost and fixed cost.
 //
 // With kF32 K is rounded (Rec32) right after the correction and every later
 // product (V, g here; J'J, W, the model cost in the readers) uses the rounded
@@ -353,9 +364,9 @@ __global__ __launch_bounds__(kObsTile) void k_linearize(DevTopology t, const dou
       // tile's slot, and k_split_sum adds the slots in tile order.
       double* dst = (t.lm_flags[lr] & kLmSplit) ? split_part + (size_t)kLmAcc * blockIdx.x
                                                 : lm_acc + (size_t)kLmAcc * lr;
-      // V, V_mission (6 each), then g, g_mission (3 each).
+      // V_own, V_mission (6 each), then g, g_mission (3 each).
       const int at = c < 6 ? c : 6 + c, step = c < 6 ? 6 : 3;
-      dst[at] = sum + sum_own;
+      dst[at] = c < 6 ? sum_own : sum + sum_own;
       dst[at + step] = sum;
     }
   }
@@ -464,128 +475,190 @@ __global__ void k_jacobi_scaling(int32_t Pvar, int32_t L, int32_t use, const dou
   if (i < 3 * L) {
     const int l = i / 3, c = i % 3;
     const int di = c == 0 ? 0 : (c == 1 ? 3 : 5);
-    lm_scale[i] = use ? 1.0 / (1.0 + sqrt(lm_acc[(size_t)kLmAcc * l + di])) : 1.0;
+    const double* V = lm_acc + (size_t)kLmAcc * l;
+    lm_scale[i] = use ? 1.0 / (1.0 + sqrt(V[di] + V[6 + di])) : 1.0;
   }
 }
 
 // ------------------------------------------------------------ landmark pivot
 
-// Z_l = C (C V C + D^2)^-1 C, D^2 = clamp(diag(C V C)) / mu (ceres
-// LevenbergMarquardtStrategy diagonal), followed by a copy of the landmark
-// gradient g_l, so that the per-incidence Schur factors read Z_l and g_l of
-// their (scattered) landmark from one 72-byte record. Zero for non-variable
-// landmarks.
+// T_l with Z_l = T'T = C (C V C + D^2)^-1 C, D^2 = clamp(diag(C V C)) / mu
+// (ceres LevenbergMarquardtStrategy diagonal), and T_l g_l, so that the Schur
+// factors read both from one record of their (scattered) landmark. Zero for
+// inactive and constant landmarks.
+//
+// For a landmark whose anchor vertex is variable also the anchor's factor
+// (see the Schur complement below): U_a = T R with R = Z^-1 - V_mission =
+// V_own + D^2 / C^2 (formed so, not as a difference), the negated self product
+// -V_mission Z R and the rhs part -(g_mission - V_mission Z g). A constant
+// landmark has Z = 0, but its observations couple its anchor all the same:
+// T = e I with U_a = I / e gives those products exactly, and e = 1e-20 makes
+// the observations' own products vanish.
 __global__ void k_landmark_prep(DevTopology t, const double* __restrict__ lm_acc,
                                 const double* __restrict__ lm_scale, double inv_mu, double min_diag,
-                                double max_diag, double* __restrict__ lm_z, int32_t* __restrict__ fail) {
+                                double max_diag, double* __restrict__ lm_z, double* __restrict__ lm_anc,
+                                int32_t* __restrict__ fail) {
   const int l = blockIdx.x * blockDim.x + threadIdx.x;
   if (l >= t.L) return;
-  double* z = lm_z + kLmZ * l;
+  double* z = lm_z + (size_t)kLmZ * l;
+  double* an = lm_anc + (size_t)kLmAnchor * l;
   const uint32_t flags = t.lm_flags[l];
-  if (!(flags & kLmActive) || (flags & kLmConstant)) {
-    for (int i = 0; i < kLmZ; ++i) z[i] = 0.0;
-    return;
+  const double* acc = lm_acc + (size_t)kLmAcc * l;
+  const bool anchored = (flags & kLmAnchorVar) != 0;
+  double T[6] = {0, 0, 0, 0, 0, 0}, damp[3] = {0, 0, 0};
+  bool zero = !(flags & kLmActive);
+  if (!zero && !(flags & kLmConstant)) {
+    const double* c = lm_scale + 3 * l;
+    double A[6];
+    for (int i = 0; i < 6; ++i) A[i] = acc[i] + acc[6 + i];
+    A[0] *= c[0] * c[0]; A[1] *= c[0] * c[1]; A[2] *= c[0] * c[2];
+    A[3] *= c[1] * c[1]; A[4] *= c[1] * c[2]; A[5] *= c[2] * c[2];
+    const double d[3] = {fmin(fmax(A[0], min_diag), max_diag) * inv_mu, fmin(fmax(A[3], min_diag), max_diag) * inv_mu,
+                         fmin(fmax(A[5], min_diag), max_diag) * inv_mu};
+    A[0] += d[0];
+    A[3] += d[1];
+    A[5] += d[2];
+    if (spd3_inverse_factor(A, T)) {
+      T[0] *= c[0]; T[1] *= c[0]; T[2] *= c[1];
+      T[3] *= c[0]; T[4] *= c[1]; T[5] *= c[2];
+      for (int k = 0; k < 3; ++k) damp[k] = d[k] / (c[k] * c[k]);
+    } else {
+      atomicAdd(fail, 1);
+      for (int k = 0; k < 6; ++k) T[k] = 0.0;
+      zero = true;
+    }
   }
-  const double* V = lm_acc + (size_t)kLmAcc * l;
-  const double* c = lm_scale + 3 * l;
-  double A[6] = {c[0] * c[0] * V[0], c[0] * c[1] * V[1], c[0] * c[2] * V[2],
-                 c[1] * c[1] * V[3], c[1] * c[2] * V[4], c[2] * c[2] * V[5]};
-  A[0] += fmin(fmax(A[0], min_diag), max_diag) * inv_mu;
-  A[3] += fmin(fmax(A[3], min_diag), max_diag) * inv_mu;
-  A[5] += fmin(fmax(A[5], min_diag), max_diag) * inv_mu;
-  double inv[6];
-  if (!spd3_inverse(A, inv)) {
-    atomicAdd(fail, 1);
-    for (int i = 0; i < kLmZ; ++i) z[i] = 0.0;
-    return;
+  const double* g = acc + 12;
+  double y[3] = {0, 0, 0};
+  if (!zero) tri_vec(T, g, y);
+  const bool pinned = !zero && (flags & kLmConstant) && anchored;
+  constexpr double kPin = 1e-20;
+  if (pinned) T[0] = T[2] = T[5] = kPin;
+  for (int i = 0; i < 6; ++i) z[i] = T[i];
+  for (int i = 0; i < 3; ++i) z[6 + i] = y[i];
+  if (!anchored) return;
+  double U[9] = {}, X[6] = {}, h[3] = {};
+  if (!zero) {
+    const double* V = acc + 6;
+    const double* gm = acc + 15;
+    if (pinned) {
+      U[0] = U[4] = U[8] = 1.0 / kPin;
+      for (int i = 0; i < 6; ++i) X[i] = -V[i];
+      for (int i = 0; i < 3; ++i) h[i] = -gm[i];
+    } else {
+      double R[9], VM[9], B[9];
+      sym3_full(acc, R);
+      for (int k = 0; k < 3; ++k) R[4 * k] += damp[k];
+      sym3_full(V, VM);
+      for (int c = 0; c < 3; ++c) {  // U = T R, B = T V_mission, column by column
+        const double r[3] = {R[c], R[3 + c], R[6 + c]}, m[3] = {VM[c], VM[3 + c], VM[6 + c]};
+        double o[3];
+        tri_vec(T, r, o);
+        for (int k = 0; k < 3; ++k) U[3 * k + c] = o[k];
+        tri_vec(T, m, o);
+        for (int k = 0; k < 3; ++k) B[3 * k + c] = o[k];
+      }
+      double W[9];  // V_mission Z R = B'U
+      for (int r = 0; r < 3; ++r)
+        for (int c = 0; c < 3; ++c) W[3 * r + c] = B[r] * U[c] + B[3 + r] * U[3 + c] + B[6 + r] * U[6 + c];
+      X[0] = -W[0];
+      X[1] = -0.5 * (W[1] + W[3]);
+      X[2] = -0.5 * (W[2] + W[6]);
+      X[3] = -W[4];
+      X[4] = -0.5 * (W[5] + W[7]);
+      X[5] = -W[8];
+      for (int c = 0; c < 3; ++c) h[c] = B[c] * y[0] + B[3 + c] * y[1] + B[6 + c] * y[2] - gm[c];
+    }
   }
-  z[0] = c[0] * c[0] * inv[0]; z[1] = c[0] * c[1] * inv[1]; z[2] = c[0] * c[2] * inv[2];
-  z[3] = c[1] * c[1] * inv[3]; z[4] = c[1] * c[2] * inv[4]; z[5] = c[2] * c[2] * inv[5];
-  z[6] = V[12]; z[7] = V[13]; z[8] = V[14];
+  for (int i = 0; i < 9; ++i) an[i] = U[i];
+  for (int i = 0; i < 6; ++i) an[9 + i] = X[i];
+  for (int i = 0; i < 3; ++i) an[15 + i] = h[i];
 }
 
 // ------------------------------------------------------------ Schur complement
 
-// Factor blocks of the reduced camera system
-//   S = F'F + D^2 - sum_l W_l' Z_l W_l,  rhs = F'r - sum_l W_l' Z_l g_l,
-// with Z_l = C_l (C_l V_l C_l + D_l^2)^-1 C_l from k_landmark_prep. An
-// incidence x of variable vertex i is an observation by i whose residual
-// depends on the pose of i, or the anchor of a landmark l whose anchor
-// vertex i is variable (A_l = M_l C_i, the anchor map of the landmark):
-//   observation: W_x = Jl^T Jo C_i,  r0_x = C_i Jo^T r
-//   anchor:      W_x = V_LM,l A_l,   r0_x = A_l^T g_LM,l
-// and per LM iteration (Z_l depends on the damping)
-//   Q_x = [anchor: A_l^T] - W_x^T Z_l,  rhs_x = r0_x - W_x^T Z_l g_l
+// The reduced camera system
+//   S = F'F + D^2 - sum_l W_l' Z_l W_l,  rhs = F'r - sum_l W_l' Z_l g_l
 // (ceres' Schur eliminator, schur_eliminator_impl.h, restated on the
-// anchor-lifted blocks). S_ij sums, over the landmarks l seen from rows i and
-// j >= i, Q_x W_y + [x observation, y anchor] W_x^T A_l over l's incidences
-// x in row i and y in row j. Both terms are linear in the incidences of one
-// row, so the incidences of a landmark in one row are summed first into a
-// factor block (W, r0); an anchor is alone in its row and its block stores
-// A_l in place of W (the Schur kernel forms W = V_LM,l A_l next to it).
-// Factor blocks are stored landmark-major (rows ascending), per
-// linearization.
+// anchor-lifted blocks) from factors of the landmark-pose blocks. With
+// E(p) = [[p]x | -I] (3x6) and the row transform D_i = diag(|q_i|^2 I, R_i) C_i
+// of the vertex of row i (R_I_M, column scaling C_i), the Jacobians factor as
+//   J_observer C = K E(p_I) D_i                 (p_I: landmark in the IMU frame)
+//   J_anchor C   = -J_landmark E(p_B) D_a       (J_landmark times the anchor map)
+// and with P = J_landmark' K, summed over the observations of landmark l by
+// the vertex (they share p_I), and k = K'r, l's products with Z = T'T are
+//   S_ij -= D_i' E_i' (U_i' U_j) E_j D_j,       U = T P      (3x3)
+//   rhs_i += D_i' E_i' (k - U_i' T g)
+// The anchor a of l joins them with U_a = T R, R = Z^-1 - V_mission: an
+// observation x with the anchor gives W_x'(Z V_mission - I) A = -W_x' Z R A,
+// and the anchor with itself V_mission - V_mission Z V_mission =
+// V_mission Z R, which k_landmark_prep forms (as its rhs part). So a staged
+// factor is U and p (12 doubles) for both sides of every product, where the
+// plain blocks W and W'Z are 36, and a product is 27 + 72 multiply-adds with
+// 24 doubles read from LDS instead of 108 with 36. The row transforms are
+// applied once per block of S, by k_schur_finalize.
+// Factor blocks (P, p) and k are stored landmark-major (rows ascending), per
+// linearization. An anchor's block keeps p_B.
 template <bool kF32>
 __global__ __launch_bounds__(256) void k_schur_factors(
     DevTopology t, int32_t n_g, const int32_t* __restrict__ g_row, const int32_t* __restrict__ g_inc_ptr,
     const int32_t* __restrict__ g_inc, const double* __restrict__ vR, const double* __restrict__ lm,
-    const void* __restrict__ obs_rec, const double* __restrict__ lm_acc, const double* __restrict__ pose_scale,
-    double* __restrict__ gw, double* __restrict__ gr0) {
+    const void* __restrict__ obs_rec, double* __restrict__ gf, double* __restrict__ gk) {
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= n_g) return;
-  const int i = g_row[g];
-  const double* cs = pose_scale + 6 * i;
-  double W[18], r0[6];
-  for (int k = 0; k < 18; ++k) W[k] = 0.0;
-  for (int c = 0; c < 6; ++c) r0[c] = 0.0;
-  for (int m = g_inc_ptr[g]; m < g_inc_ptr[g + 1]; ++m) {
-    const int32_t x = g_inc[m];
-    double Wx[18], rx[6];
-    if (x >= 0) {
-      const RecView<kF32> rec(obs_rec, x);
-      const int v = t.var_vertex[i], la = t.lm_anchor[t.obs_landmark[x]];
-      double Jo[12], G[9], Jl[6];
-      observer_jacobian(rec, vR + 12 * v, Jo);
-      landmark_to_imu(t, obs_type(t.obs_meta[x]), la, v, vR + 12 * la, vR + 12 * v, G);
-      for (int r = 0; r < 2; ++r)
-        for (int c = 0; c < 3; ++c)
-          Jl[r * 3 + c] = rec.K(3 * r) * G[c] + rec.K(3 * r + 1) * G[3 + c] + rec.K(3 * r + 2) * G[6 + c];
-      for (int a = 0; a < 3; ++a)
-        for (int c = 0; c < 6; ++c) Wx[a * 6 + c] = (Jl[a] * Jo[c] + Jl[3 + a] * Jo[6 + c]) * cs[c];
-      for (int c = 0; c < 6; ++c) rx[c] = cs[c] * (Jo[c] * rec.r(0) + Jo[6 + c] * rec.r(1));
-    } else {
-      const int32_t l = -1 - x;
-      const int v = t.var_vertex[i];
-      const double* acc_l = lm_acc + (size_t)kLmAcc * l;
-      double M[18], A[18];
-      anchor_map(lm + 3 * l, vR + 12 * v, vR[12 * v + 9], M);
-      for (int a = 0; a < 3; ++a)
-        for (int c = 0; c < 6; ++c) A[a * 6 + c] = M[a * 6 + c] * cs[c];
-      const double* gLM = acc_l + 15;
-      for (int c = 0; c < 6; ++c) rx[c] = A[c] * gLM[0] + A[6 + c] * gLM[1] + A[12 + c] * gLM[2];
-      // The anchor's block keeps A_l; the Schur kernel forms W_x = V_LM,l A_l.
-      for (int k = 0; k < 18; ++k) Wx[k] = A[k];
+  const int m0 = g_inc_ptr[g], m1 = g_inc_ptr[g + 1];
+  double f[kFactor] = {}, k[3] = {0, 0, 0};
+  const int32_t x0 = g_inc[m0];
+  if (x0 < 0) {
+    const int32_t l = -1 - x0;
+    if (t.lm_flags[l] & kLmActive)
+      for (int c = 0; c < 3; ++c) f[9 + c] = lm[3 * l + c];
+  } else {
+    const int v = t.var_vertex[g_row[g]], la = t.lm_anchor[t.obs_landmark[x0]];
+    double G[9];
+    landmark_to_imu(t, obs_type(t.obs_meta[x0]), la, v, vR + 12 * la, vR + 12 * v, G);
+    for (int m = m0; m < m1; ++m) {
+      const RecView<kF32> rec(obs_rec, g_inc[m]);
+      for (int r = 0; r < 2; ++r) {
+        const double k0 = rec.K(3 * r), k1 = rec.K(3 * r + 1), k2 = rec.K(3 * r + 2), rr = rec.r(r);
+        for (int a = 0; a < 3; ++a) {
+          const double jl = k0 * G[a] + k1 * G[3 + a] + k2 * G[6 + a];
+          f[3 * a] += jl * k0;
+          f[3 * a + 1] += jl * k1;
+          f[3 * a + 2] += jl * k2;
+        }
+        k[0] += k0 * rr;
+        k[1] += k1 * rr;
+        k[2] += k2 * rr;
+      }
+      // A failed projection's record is zero, p_I included.
+      if (rec.p(0) != 0.0 || rec.p(1) != 0.0 || rec.p(2) != 0.0)
+        for (int c = 0; c < 3; ++c) f[9 + c] = rec.p(c);
     }
-    for (int k = 0; k < 18; ++k) W[k] += Wx[k];
-    for (int c = 0; c < 6; ++c) r0[c] += rx[c];
   }
-  double* w = gw + (size_t)18 * g;
-  for (int k = 0; k < 18; ++k) w[k] = W[k];
-  double* rr = gr0 + (size_t)6 * g;
-  for (int c = 0; c < 6; ++c) rr[c] = r0[c];
+  double2* out = reinterpret_cast<double2*>(gf + (size_t)kFactor * g);
+  for (int c = 0; c < kFactor / 2; ++c) out[c] = make_double2(f[2 * c], f[2 * c + 1]);
+  for (int c = 0; c < 3; ++c) gk[(size_t)3 * g + c] = k[c];
 }
 
-// LDS of one batch of a tile: the staged factor blocks (W and Q^T, both 3x6
-// row-major, and the rhs contribution r0 - W^T Z g on diagonal tiles), the
-// batch's pair list and the segment's batch words. Slot entries are
-// slot-minor (entry e of slot s at [e][s]), so the staging writes of
-// consecutive threads hit consecutive banks.
+// LDS of one round of a tile: the staged factors of one or two batches (U and
+// p), on diagonal tiles their rhs vectors and the anchors' self products, the
+// batches' pair lists and the segment's batch words. Entries are slot-minor,
+// the factor's in pairs of 16 bytes (row r of U and p_r are [2 r][s] and
+// [2 r + 1][s]), so that the staging writes of consecutive threads hit
+// consecutive banks and a product's 24 doubles are 12 reads.
 struct TileLds {
-  double f[2][18][kBatchSlots];  // [0] W, [1] Q^T = [anchor: A_l] - Z_l W
-  double r[6][kBatchSlots];
-  uint32_t pairs[kBatchPairs / 2];
+  union {
+    double2 f[kFactor / 2][2 * kBatchSlots];
+    struct {
+      double2 f[kFactor / 2][kBatchSlots];
+      double h[3][kBatchSlots];
+      double x[6][kBatchSlots];
+      uint8_t anchor[kBatchSlots];
+    } diag;
+  };
+  uint32_t pairs[2][kBatchPairs / 2];
   int4 bt[kSegmentBatches];
-  uint8_t anchor[kBatchSlots];
 };
 
 struct TileArgs {
@@ -593,90 +666,271 @@ struct TileArgs {
   const int2* slots;
   const uint16_t* batch_off;
   const uint32_t* pairs;  // the pair list as 32-bit words (batches start on a word)
-  const double* gw;
-  const double* gr0;
-  const double* lm_acc;
+  const double* gf;
+  const double* gk;
   const double* lm_z;
+  const double* lm_anc;
 };
 
-// A thread's index loads of one batch (two batches ahead): its slot's word,
-// its part's pair range and its share of the pair list.
+// A thread's part of a segment.
+struct TilePart {
+  int32_t tid, np, blk, part;
+};
+
+// A thread's index loads of one batch (two rounds ahead): its slot's word and
+// its part's pair range.
 struct TileIdx {
   int2 slot;
   int32_t pb, pe;
-  uint32_t pw[kPairWords];
 };
 
-// A thread's data loads of one batch (one batch ahead): its slot's factor
-// block (W, or A_l for an anchor's block) and r0, its landmark's pivot (Z,
-// g) and, for an anchor, V_LM; and the index words.
+// A thread's data loads of one batch (one round ahead): its slot's factor (P,
+// or U for an anchor, and p), its landmark's T, its share of the pair list; on
+// diagonal tiles T g, k (or the anchor's rhs) and the anchor's self product.
+template <bool kDiag>
 struct TileStage {
-  double w[18], z[9], v[6], r0[6];
-  int32_t pb, pe;
+  double f[kFactor], z[kDiag ? 9 : 6], h[kDiag ? 3 : 1], x[kDiag ? 6 : 1];
   uint32_t pw[kPairWords];
-  int2 slot;
+  TileIdx q;
 };
 
-__device__ inline void tile_idx(TileIdx& q, const TileArgs& ta, const int4& bt, int b, int tid, int blk, int part,
-                                int np) {
+__device__ inline void tile_idx(TileIdx& q, const TileArgs& ta, const int4& bt, int b, const TilePart& me) {
   q.slot = make_int2(-1, 0);
-  if (tid < bt.y) q.slot = ta.slots[bt.x + tid];
+  if (me.tid < bt.y) q.slot = ta.slots[bt.x + me.tid];
   q.pb = q.pe = 0;
-  if (np) {
+  if (me.np) {
     const uint16_t* off = ta.batch_off + (size_t)b * (kTileBlocks + 1);
-    q.pb = off[blk] + part;
-    q.pe = off[blk + 1];
+    q.pb = off[me.blk] + me.part;
+    q.pe = off[me.blk + 1];
   }
+}
+
+template <bool kDiag>
+__device__ inline void tile_data(TileStage<kDiag>& st, const TileIdx& q, const TileArgs& ta, const int4& bt, int tid) {
+  st.q = q;
   const int nw = (bt.w + 1) >> 1;
   const uint32_t* pw = ta.pairs + (bt.z >> 1);
 #pragma unroll
   for (int k = 0; k < kPairWords; ++k) {
     const int j = tid + k * kTileBlocks;
-    q.pw[k] = j < nw ? pw[j] : 0u;
+    st.pw[k] = j < nw ? pw[j] : 0u;
   }
-}
-
-__device__ inline void tile_data(TileStage& st, const TileIdx& q, const TileArgs& ta, bool diag) {
-  st.slot = q.slot;
-  st.pb = q.pb;
-  st.pe = q.pe;
-#pragma unroll
-  for (int k = 0; k < kPairWords; ++k) st.pw[k] = q.pw[k];
   if (q.slot.x < 0) return;
   const uint32_t lw = (uint32_t)q.slot.y;
-  const int l = (int)(lw & ~kSlotAnchor);
-  const double* wp = ta.gw + (size_t)18 * q.slot.x;
+  const size_t l = lw & ~kSlotAnchor;
+  const bool anc = (lw & kSlotAnchor) != 0;
+  const double* fp = ta.gf + (size_t)kFactor * q.slot.x;
+  const double* an = ta.lm_anc + kLmAnchor * l;
+  const double* up = anc ? an : fp;
 #pragma unroll
-  for (int e = 0; e < 18; ++e) st.w[e] = wp[e];
-  const double* zp = ta.lm_z + (size_t)kLmZ * l;
+  for (int e = 0; e < 9; ++e) st.f[e] = up[e];
 #pragma unroll
-  for (int e = 0; e < 9; ++e) st.z[e] = zp[e];
-  if (lw & kSlotAnchor) {
-    const double* vp = ta.lm_acc + (size_t)kLmAcc * l + 6;
+  for (int e = 9; e < kFactor; ++e) st.f[e] = fp[e];
+  const double* zp = ta.lm_z + kLmZ * l;
 #pragma unroll
-    for (int e = 0; e < 6; ++e) st.v[e] = vp[e];
-  }
-  if (diag) {
-    const double* rp = ta.gr0 + (size_t)6 * q.slot.x;
+  for (int e = 0; e < (kDiag ? 9 : 6); ++e) st.z[e] = zp[e];
+  if (kDiag) {
+    const double* hp = anc ? an + 15 : ta.gk + (size_t)3 * q.slot.x;
 #pragma unroll
-    for (int e = 0; e < 6; ++e) st.r0[e] = rp[e];
+    for (int e = 0; e < 3; ++e) st.h[e] = hp[e];
+    if (anc)
+#pragma unroll
+      for (int e = 0; e < 6; ++e) st.x[e] = an[9 + e];
   }
 }
 
-// One work item = one segment of a tile (I, J). Per batch: every thread
-// stages its slot's factor block in LDS (Q^T formed from W, Z and A) and its
-// share of the pair list, then each thread adds the products of its part of
-// its block's pairs in list order,
-//   Q_x W_y              (y not the anchor, or x the anchor too)
-//   W_x^T (Q^T_y)        (y the anchor of an observation x: Q_x W_y + W_x^T A_l)
-// both as sum_a Lt(a, r) Rt(a, c) over the rows of two 3x6 blocks; a part of
-// a diagonal block of a diagonal tile also adds the rhs of its pairs' block.
-// Loads are software-pipelined: while a batch's products run, the next
-// batch's data loads and the batch after that's index loads are in flight.
-// Each part's sums go to its own slot of the segment's partial. Work-groups
-// take items_per_wg consecutive items of the dispatch order; with xcd_map
-// each XCD walks a contiguous range of work-groups (work-group b runs on XCD
-// b mod 8). Neither changes a partial.
+// A batch's staged data into LDS: U = T P (an anchor's is ready), p, and on
+// diagonal tiles h = k - U'T g.
+template <bool kDiag>
+__device__ inline void tile_stage(TileLds& sh, const TileStage<kDiag>& st, int tid, int half) {
+#pragma unroll
+  for (int j = 0; j < kPairWords; ++j) sh.pairs[half][tid + j * kTileBlocks] = st.pw[j];
+  if (st.q.slot.x < 0) return;
+  const double* z = st.z;
+  const bool anc = ((uint32_t)st.q.slot.y & kSlotAnchor) != 0;
+  double u[9];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const double p0 = st.f[c], p1 = st.f[3 + c], p2 = st.f[6 + c];
+    u[c] = anc ? p0 : z[0] * p0;
+    u[3 + c] = anc ? p1 : z[1] * p0 + z[2] * p1;
+    u[6 + c] = anc ? p2 : z[3] * p0 + z[4] * p1 + z[5] * p2;
+  }
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    const double2 lo = make_double2(u[3 * r], u[3 * r + 1]), hi = make_double2(u[3 * r + 2], st.f[9 + r]);
+    if (kDiag) {
+      sh.diag.f[2 * r][tid] = lo;
+      sh.diag.f[2 * r + 1][tid] = hi;
+    } else {
+      sh.f[2 * r][half * kBatchSlots + tid] = lo;
+      sh.f[2 * r + 1][half * kBatchSlots + tid] = hi;
+    }
+  }
+  if (kDiag) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+      sh.diag.h[c][tid] = anc ? st.h[c] : st.h[c] - (u[c] * z[6] + u[3 + c] * z[7] + u[6 + c] * z[8]);
+#pragma unroll
+    for (int c = 0; c < 6; ++c) sh.diag.x[c][tid] = st.x[c];
+    sh.diag.anchor[tid] = anc ? 1 : 0;
+  }
+}
+
+// One segment of a tile. Per round (one batch on a diagonal tile, two on the
+// others): every thread stages its slot's factor of each batch in LDS and its
+// share of the pair lists, then each thread adds the products of its part of
+// its block's pairs in list order, one batch's after the other's in one loop: a
+// wave's loop lasts as long as its busiest part, and over two batches the
+// parts' shares are more even (a part has 1.9 pairs a batch, the busiest 6.6).
+// A part of a diagonal block of a diagonal tile also adds the rhs of its
+// pairs' factors. Loads are software-pipelined: while a round's products run,
+// the next round's data loads and the index loads of the one after that are in
+// flight. Each part's sums go to its own slot of the segment's partial.
+template <bool kDiag>
+__device__ inline void tile_segment(TileLds& sh, const TileArgs& ta, const int4& sg, uint32_t tw,
+                                    double* __restrict__ out_base) {
+  constexpr int kHalves = kDiag ? 1 : 2;
+  constexpr int kSlots = kHalves * kBatchSlots;
+  TilePart me;
+  me.tid = threadIdx.x;
+  me.np = seg_thread_parts(tw);
+  me.blk = seg_thread_block(tw);
+  me.part = seg_thread_part(tw);
+  const int tid = me.tid, np = me.np, nb = sg.y - sg.x;
+  const bool rhs_part = kDiag && np && me.blk / kTileBand == me.blk % kTileBand;
+  const double2(*fl)[kSlots] =
+      kDiag ? reinterpret_cast<const double2(*)[kSlots]>(sh.diag.f) : reinterpret_cast<const double2(*)[kSlots]>(sh.f);
+  // Sums of [p_i]x X [p_j]x, [p_i]x X, X [p_j]x and X over the pairs, X =
+  // U_i' U_j; of p_i x h and h.
+  double rr[9], rp[9], pr[9], pp[9], racc[kDiag ? 6 : 1];
+#pragma unroll
+  for (int e = 0; e < 9; ++e) rr[e] = rp[e] = pr[e] = pp[e] = 0.0;
+#pragma unroll
+  for (int c = 0; c < (kDiag ? 6 : 1); ++c) racc[c] = 0.0;
+  TileIdx q[kHalves];
+  TileStage<kDiag> st[kHalves];
+#pragma unroll
+  for (int h = 0; h < kHalves; ++h) {
+    if (h < nb) {
+      tile_idx(q[h], ta, sh.bt[h], sg.x + h, me);
+      tile_data(st[h], q[h], ta, sh.bt[h], tid);
+    } else {
+      q[h].slot = make_int2(-1, 0);
+      q[h].pb = q[h].pe = 0;
+      st[h].q = q[h];
+    }
+    if (kHalves + h < nb) tile_idx(q[h], ta, sh.bt[kHalves + h], sg.x + kHalves + h, me);
+  }
+  for (int k = 0; k < nb; k += kHalves) {
+    __syncthreads();
+    int n0 = 0, total = 0, b0 = 0, b1 = 0;
+#pragma unroll
+    for (int h = 0; h < kHalves; ++h) {
+      if (k + h < nb) {
+        tile_stage(sh, st[h], tid, h);
+        const int n = np && st[h].q.pe > st[h].q.pb ? (st[h].q.pe - st[h].q.pb + np - 1) / np : 0;
+        if (h == 0) {
+          n0 = n;
+          b0 = st[h].q.pb;
+        } else {
+          b1 = st[h].q.pb;
+        }
+        total += n;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < kHalves; ++h) {
+      const int kn = k + kHalves + h, kq = kn + kHalves;
+      if (kn < nb) tile_data(st[h], q[h], ta, sh.bt[kn], tid);
+      if (kq < nb) tile_idx(q[h], ta, sh.bt[kq], sg.x + kq, me);
+    }
+    for (int it = 0; it < total; ++it) {
+      const bool second = kHalves == 2 && it >= n0;
+      const int p = second ? b1 + (it - n0) * np : b0 + it * np;
+      const uint32_t w = reinterpret_cast<const uint16_t*>(sh.pairs[second ? 1 : 0])[p];
+      const int base = second ? kBatchSlots : 0;
+      const int x = base + (int)(w & 255u), y = base + (int)(w >> 8);
+      const double2 a0 = fl[0][x], a1 = fl[1][x], b0v = fl[0][y], b1v = fl[1][y];
+      const double2 a2 = fl[2][x], a3 = fl[3][x], b2v = fl[2][y], b3v = fl[3][y];
+      const double2 a4 = fl[4][x], a5 = fl[5][x], b4v = fl[4][y], b5v = fl[5][y];
+      double X[9];
+      X[0] = a0.x * b0v.x + a2.x * b2v.x + a4.x * b4v.x;
+      X[1] = a0.x * b0v.y + a2.x * b2v.y + a4.x * b4v.y;
+      X[2] = a0.x * b1v.x + a2.x * b3v.x + a4.x * b5v.x;
+      X[3] = a0.y * b0v.x + a2.y * b2v.x + a4.y * b4v.x;
+      X[4] = a0.y * b0v.y + a2.y * b2v.y + a4.y * b4v.y;
+      X[5] = a0.y * b1v.x + a2.y * b3v.x + a4.y * b5v.x;
+      X[6] = a1.x * b0v.x + a3.x * b2v.x + a5.x * b4v.x;
+      X[7] = a1.x * b0v.y + a3.x * b2v.y + a5.x * b4v.y;
+      X[8] = a1.x * b1v.x + a3.x * b3v.x + a5.x * b5v.x;
+      if (kDiag && x == y && sh.diag.anchor[x]) {
+        X[0] = sh.diag.x[0][x]; X[4] = sh.diag.x[3][x]; X[8] = sh.diag.x[5][x];
+        X[1] = X[3] = sh.diag.x[1][x];
+        X[2] = X[6] = sh.diag.x[2][x];
+        X[5] = X[7] = sh.diag.x[4][x];
+      }
+      const double px = a1.y, py = a3.y, pz = a5.y;
+      const double qx = b1v.y, qy = b3v.y, qz = b5v.y;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        pp[c] += X[c];
+        pp[3 + c] += X[3 + c];
+        pp[6 + c] += X[6 + c];
+        rp[c] += py * X[6 + c] - pz * X[3 + c];
+        rp[3 + c] += pz * X[c] - px * X[6 + c];
+        rp[6 + c] += px * X[3 + c] - py * X[c];
+      }
+      double Y[9];
+#pragma unroll
+      for (int r = 0; r < 3; ++r) {
+        Y[3 * r] = X[3 * r + 1] * qz - X[3 * r + 2] * qy;
+        Y[3 * r + 1] = X[3 * r + 2] * qx - X[3 * r] * qz;
+        Y[3 * r + 2] = X[3 * r] * qy - X[3 * r + 1] * qx;
+      }
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        pr[c] += Y[c];
+        pr[3 + c] += Y[3 + c];
+        pr[6 + c] += Y[6 + c];
+        rr[c] += py * Y[6 + c] - pz * Y[3 + c];
+        rr[3 + c] += pz * Y[c] - px * Y[6 + c];
+        rr[6 + c] += px * Y[3 + c] - py * Y[c];
+      }
+      if (kDiag && rhs_part) {
+        const double h0 = sh.diag.h[0][x], h1 = sh.diag.h[1][x], h2 = sh.diag.h[2][x];
+        racc[0] += py * h2 - pz * h1;
+        racc[1 % (kDiag ? 6 : 1)] += pz * h0 - px * h2;
+        racc[2 % (kDiag ? 6 : 1)] += px * h1 - py * h0;
+        racc[3 % (kDiag ? 6 : 1)] += h0;
+        racc[4 % (kDiag ? 6 : 1)] += h1;
+        racc[5 % (kDiag ? 6 : 1)] += h2;
+      }
+    }
+  }
+  if (np) {
+    // -E_i' X E_j and E_i' h, E' = [-[p]x; -I].
+    double* out = out_base + (size_t)tid * kPartEntries;
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        out[6 * r + c] = rr[3 * r + c];
+        out[6 * r + 3 + c] = -rp[3 * r + c];
+        out[6 * (3 + r) + c] = pr[3 * r + c];
+        out[6 * (3 + r) + 3 + c] = -pp[3 * r + c];
+      }
+    if (kDiag)
+#pragma unroll
+      for (int c = 0; c < 6; ++c) out[36 + c] = -racc[c % (kDiag ? 6 : 1)];
+  }
+}
+
+// One work item = one segment of a tile (I, J). Work-groups take items_per_wg
+// consecutive items of the dispatch order; with xcd_map each XCD walks a
+// contiguous range of work-groups (work-group b runs on XCD b mod 8). Neither
+// changes a partial.
 __global__ __launch_bounds__(kTileBlocks) __attribute__((amdgpu_waves_per_eu(2))) void k_schur_tiles(
     int32_t n_segs, int32_t items_per_wg, int32_t xcd_map, const int32_t* __restrict__ seg_order,
     const int4* __restrict__ segs, const uint32_t* __restrict__ seg_thread, TileArgs ta,
@@ -692,175 +946,116 @@ __global__ __launch_bounds__(kTileBlocks) __attribute__((amdgpu_waves_per_eu(2))
     if (si >= n_segs) break;
     const int sid = seg_order[si];
     const int4 sg = segs[sid];
-    const bool diag = sg.z == sg.w;
-    const int nb = sg.y - sg.x;
     const uint32_t tw = seg_thread[(size_t)sid * kTileBlocks + tid];
-    const int np = seg_thread_parts(tw), blk = seg_thread_block(tw), part = seg_thread_part(tw);
-    const bool rhs_part = diag && np && blk / kTileBand == blk % kTileBand;
     __syncthreads();
-    if (tid < nb) sh.bt[tid] = ta.batches[sg.x + tid];
+    if (tid < sg.y - sg.x) sh.bt[tid] = ta.batches[sg.x + tid];
     __syncthreads();
-    double acc[36], racc[6];
-#pragma unroll
-    for (int e = 0; e < 36; ++e) acc[e] = 0.0;
-#pragma unroll
-    for (int c = 0; c < 6; ++c) racc[c] = 0.0;
-    TileIdx q;
-    TileStage st;
-    tile_idx(q, ta, sh.bt[0], sg.x, tid, blk, part, np);
-    tile_data(st, q, ta, diag);
-    if (nb > 1) tile_idx(q, ta, sh.bt[1], sg.x + 1, tid, blk, part, np);
-    for (int k = 0; k < nb; ++k) {
-      __syncthreads();
-      if (st.slot.x >= 0) {
-        // Column by column: W (= V_LM A_l for an anchor, whose block holds
-        // A_l), Q^T = [anchor: A_l] - Z W and r0 - W^T Z g.
-        const double* z = st.z;
-        const double Z[9] = {z[0], z[1], z[2], z[1], z[3], z[4], z[2], z[4], z[5]};
-        const bool anc = ((uint32_t)st.slot.y & kSlotAnchor) != 0;
-        const double* v = st.v;
-        const double V[9] = {v[0], v[1], v[2], v[1], v[3], v[4], v[2], v[4], v[5]};
-        double zg[3];
-#pragma unroll
-        for (int a = 0; a < 3; ++a) zg[a] = Z[a * 3] * z[6] + Z[a * 3 + 1] * z[7] + Z[a * 3 + 2] * z[8];
-#pragma unroll
-        for (int c = 0; c < 6; ++c) {
-          const double b0 = st.w[c], b1 = st.w[6 + c], b2 = st.w[12 + c];
-          double w0 = b0, w1 = b1, w2 = b2;
-          if (anc) {
-            w0 = V[0] * b0 + V[1] * b1 + V[2] * b2;
-            w1 = V[3] * b0 + V[4] * b1 + V[5] * b2;
-            w2 = V[6] * b0 + V[7] * b1 + V[8] * b2;
-          }
-          const double q0 = Z[0] * w0 + Z[1] * w1 + Z[2] * w2;
-          const double q1 = Z[3] * w0 + Z[4] * w1 + Z[5] * w2;
-          const double q2 = Z[6] * w0 + Z[7] * w1 + Z[8] * w2;
-          sh.f[0][c][tid] = w0;
-          sh.f[0][6 + c][tid] = w1;
-          sh.f[0][12 + c][tid] = w2;
-          sh.f[1][c][tid] = anc ? b0 - q0 : -q0;
-          sh.f[1][6 + c][tid] = anc ? b1 - q1 : -q1;
-          sh.f[1][12 + c][tid] = anc ? b2 - q2 : -q2;
-          if (diag) sh.r[c][tid] = st.r0[c] - (w0 * zg[0] + w1 * zg[1] + w2 * zg[2]);
-        }
-        sh.anchor[tid] = anc ? 1 : 0;
-      }
-#pragma unroll
-      for (int j = 0; j < kPairWords; ++j) sh.pairs[tid + j * kTileBlocks] = st.pw[j];
-      const int pb = st.pb, pe = st.pe;
-      __syncthreads();
-      if (k + 1 < nb) tile_data(st, q, ta, diag);
-      if (k + 2 < nb) tile_idx(q, ta, sh.bt[k + 2], sg.x + k + 2, tid, blk, part, np);
-      const uint16_t* pl = reinterpret_cast<const uint16_t*>(sh.pairs);
-      for (int p = pb; p < pe; p += np) {
-        const uint32_t pr = pl[p];
-        const int x = (int)(pr & 255u), y = (int)(pr >> 8);
-        const int sel = (sh.anchor[y] && !sh.anchor[x]) ? 1 : 0;
-        const double* Lt = &sh.f[1 - sel][0][x];
-        const double* Rt = &sh.f[sel][0][y];
-#pragma unroll 1
-        for (int a = 0; a < 3; ++a) {
-          double l6[6], r6[6];
-#pragma unroll
-          for (int c = 0; c < 6; ++c) {
-            l6[c] = Lt[(a * 6 + c) * kBatchSlots];
-            r6[c] = Rt[(a * 6 + c) * kBatchSlots];
-          }
-#pragma unroll
-          for (int r = 0; r < 6; ++r)
-#pragma unroll
-            for (int c = 0; c < 6; ++c) acc[r * 6 + c] += l6[r] * r6[c];
-        }
-        if (rhs_part)
-#pragma unroll
-          for (int c = 0; c < 6; ++c) racc[c] += sh.r[c][x];
-      }
-    }
-    if (np) {
-      double* out = partial + (size_t)sid * kTilePartial + (size_t)tid * kPartEntries;
-#pragma unroll
-      for (int e = 0; e < 36; ++e) out[e] = acc[e];
-#pragma unroll
-      for (int c = 0; c < 6; ++c) out[36 + c] = racc[c];
-    }
+    double* out = partial + (size_t)sid * kTilePartial;
+    if (sg.z == sg.w)
+      tile_segment<true>(sh, ta, sg, tw, out);
+    else
+      tile_segment<false>(sh, ta, sg, tw, out);
   }
 }
 
-// S_ij = sum of the block's part slots (segments in segment order, parts in
-// part order, listed per upper block), plus on S_ii the direct observation
-// term C_i (sum Jo^T Jo) C_i and the LM diagonal D^2 / radius; written to
-// S_ij and S_ji = S_ij^T. One thread per entry; the first six threads of a
-// diagonal block also sum the rhs of its row. A work-group of seven 36-thread
-// groups takes seven blocks, or with kWide one block whose slots k, k + 7, ...
-// group k sums, the seven sums then added in group order: a small system has
-// few blocks of many slots each.
+// S_ij = D_i' (sum of the block's part slots) D_j (segments in segment order,
+// parts in part order, listed per upper block; D the row transforms), plus on
+// S_ii the direct observation term C_i (sum Jo^T Jo) C_i and the LM diagonal
+// D^2 / radius; written to S_ij and S_ji = S_ij^T. One thread per entry; the
+// first six threads of a diagonal block also sum the rhs of its row. A
+// work-group of seven 36-thread groups takes seven blocks, or with kWide one
+// block whose slots k, k + 7, ... group k sums, the seven sums then added in
+// group order: a small system has few blocks of many slots each.
 constexpr int kFinalizeGroups = 7;
 
 template <bool kWide>
-__global__ __launch_bounds__(252) void k_schur_finalize(int32_t nub, const int4* __restrict__ ublk,
+__global__ __launch_bounds__(252) void k_schur_finalize(DevTopology t, int32_t nub, const int4* __restrict__ ublk,
                                                         const int32_t* __restrict__ uslot_ptr,
                                                         const int32_t* __restrict__ uslot,
                                                         const double* __restrict__ partial,
+                                                        const double* __restrict__ vR,
                                                         const double* __restrict__ pose_scale,
                                                         const double* __restrict__ pose_diag,
                                                         const double* __restrict__ pose_jtj, double inv_mu,
                                                         double min_diag, double max_diag, double* __restrict__ S,
                                                         double* __restrict__ rhs) {
-  __shared__ double red[kWide ? kFinalizeGroups : 1][kPartEntries];
-  const int grp = threadIdx.x / 36, e = threadIdx.x % 36;
+  __shared__ double red[kFinalizeGroups][kPartEntries];
+  __shared__ double mid[kFinalizeGroups][36];
+  const int grp = threadIdx.x / 36, e = threadIdx.x % 36, r = e / 6, c = e % 6;
   const int u = kWide ? (int)blockIdx.x : (int)blockIdx.x * kFinalizeGroups + grp;
-  if (u >= nub) return;  // kWide: nub work-groups, none leaves here
+  const bool valid = u < nub;
   constexpr int st = kWide ? kFinalizeGroups : 1;
-  const int4 ub = ublk[u];
-  const int kb = uslot_ptr[u] + (kWide ? grp : 0), ke = uslot_ptr[u + 1];
-  const bool rhs_entry = ub.z == ub.w && e < 6;
+  const int4 ub = valid ? ublk[u] : make_int4(0, 0, 0, 1);
+  const bool diag = ub.z == ub.w, rhs_entry = diag && e < 6;
   double v = 0.0, g = 0.0;
-  int k = kb;
-  // Four slots' loads in flight at a time; the sums keep slot order.
-  for (; k + 3 * st < ke; k += 4 * st) {
-    const double* p0 = partial + (size_t)uslot[k] * kPartEntries;
-    const double* p1 = partial + (size_t)uslot[k + st] * kPartEntries;
-    const double* p2 = partial + (size_t)uslot[k + 2 * st] * kPartEntries;
-    const double* p3 = partial + (size_t)uslot[k + 3 * st] * kPartEntries;
-    const double a0 = p0[e], a1 = p1[e], a2 = p2[e], a3 = p3[e];
-    v += a0;
-    v += a1;
-    v += a2;
-    v += a3;
-    if (rhs_entry) {
-      const double b0 = p0[36 + e], b1 = p1[36 + e], b2 = p2[36 + e], b3 = p3[36 + e];
-      g += b0;
-      g += b1;
-      g += b2;
-      g += b3;
+  if (valid) {
+    const int ke = uslot_ptr[u + 1];
+    int k = uslot_ptr[u] + (kWide ? grp : 0);
+    // Four slots' loads in flight at a time; the sums keep slot order.
+    for (; k + 3 * st < ke; k += 4 * st) {
+      const double* p0 = partial + (size_t)uslot[k] * kPartEntries;
+      const double* p1 = partial + (size_t)uslot[k + st] * kPartEntries;
+      const double* p2 = partial + (size_t)uslot[k + 2 * st] * kPartEntries;
+      const double* p3 = partial + (size_t)uslot[k + 3 * st] * kPartEntries;
+      const double a0 = p0[e], a1 = p1[e], a2 = p2[e], a3 = p3[e];
+      v += a0;
+      v += a1;
+      v += a2;
+      v += a3;
+      if (rhs_entry) {
+        const double b0 = p0[36 + e], b1 = p1[36 + e], b2 = p2[36 + e], b3 = p3[36 + e];
+        g += b0;
+        g += b1;
+        g += b2;
+        g += b3;
+      }
+    }
+    for (; k < ke; k += st) {
+      const double* p = partial + (size_t)uslot[k] * kPartEntries;
+      v += p[e];
+      if (rhs_entry) g += p[36 + e];
     }
   }
-  for (; k < ke; k += st) {
-    const double* p = partial + (size_t)uslot[k] * kPartEntries;
-    v += p[e];
-    if (rhs_entry) g += p[36 + e];
-  }
+  red[grp][e] = v;
+  if (rhs_entry) red[grp][36 + e] = g;
+  __syncthreads();
   if (kWide) {
-    red[grp][e] = v;
-    if (e < 6) red[grp][36 + e] = g;
-    __syncthreads();
-    if (grp > 0) return;
-    v = red[0][e];
-    g = rhs_entry ? red[0][36 + e] : 0.0;
+    double a = red[0][e], b = rhs_entry ? red[0][36 + e] : 0.0;
     for (int q = 1; q < kFinalizeGroups; ++q) {
-      v += red[q][e];
-      if (rhs_entry) g += red[q][36 + e];
+      a += red[q][e];
+      if (rhs_entry) b += red[q][36 + e];
     }
+    __syncthreads();
+    red[grp][e] = a;
+    if (rhs_entry) red[grp][36 + e] = b;
+    __syncthreads();
   }
-  const int r = e / 6, c = e % 6;
-  if (ub.z == ub.w) {
-    const int i = ub.z;
+  // Sums times D_j from the right, then D_i' from the left.
+  const double* raw = red[grp];
+  const double* Ri = vR + 12 * t.var_vertex[ub.z];
+  const double* Rj = vR + 12 * (diag || !valid ? t.var_vertex[ub.z] : t.var_vertex[ub.w]);
+  double x;
+  if (c < 3) x = raw[e] * Rj[9];
+  else x = raw[6 * r + 3] * Rj[c - 3] + raw[6 * r + 4] * Rj[c] + raw[6 * r + 5] * Rj[3 + c];
+  mid[grp][e] = x;
+  __syncthreads();
+  if (!valid || (kWide && grp > 0)) return;
+  const double* m = mid[grp];
+  if (r < 3) v = m[e] * Ri[9];
+  else v = m[18 + c] * Ri[r - 3] + m[24 + c] * Ri[r] + m[30 + c] * Ri[3 + r];
+  const int i = ub.z, j = ub.w;
+  v *= pose_scale[6 * i + r] * pose_scale[6 * j + c];
+  if (diag) {
     v += pose_scale[6 * i + r] * pose_scale[6 * i + c] * pose_jtj[36 * i + e];
     if (r == c) {
       const double sc = pose_scale[6 * i + c];
       v += fmin(fmax(sc * sc * pose_diag[6 * i + c], min_diag), max_diag) * inv_mu;
     }
-    if (rhs_entry) rhs[6 * i + e] = g;
+    if (rhs_entry) {
+      const double* h = raw + 36;
+      const double y = e < 3 ? h[e] * Ri[9] : h[3] * Ri[e - 3] + h[4] * Ri[e] + h[5] * Ri[3 + e];
+      rhs[6 * i + e] = y * pose_scale[6 * i + e];
+    }
   }
   S[(size_t)36 * ub.x + e] = v;
   if (ub.y != ub.x) S[(size_t)36 * ub.y + c * 6 + r] = v;
@@ -1140,9 +1335,9 @@ __device__ inline void landmark_step(const DevTopology& t, int l, const double* 
       sym3_full(acc + 6, VLM);
       for (int a = 0; a < 3; ++a) tv[a] -= VLM[a * 3] * Mwa[0] + VLM[a * 3 + 1] * Mwa[1] + VLM[a * 3 + 2] * Mwa[2];
     }
-    double Z[9];
-    sym3_full(lm_z + kLmZ * l, Z);
-    for (int a = 0; a < 3; ++a) u[a] = Z[a * 3] * tv[0] + Z[a * 3 + 1] * tv[1] + Z[a * 3 + 2] * tv[2];
+    double y[3];
+    tri_vec(lm_z + (size_t)kLmZ * l, tv, y);
+    trit_vec(lm_z + (size_t)kLmZ * l, y, u);
   }
 }
 
@@ -1731,49 +1926,48 @@ void launch_jacobi_scaling(hipStream_t s, int32_t Pvar, int32_t L, int32_t use, 
   if (n > 0) k_jacobi_scaling<<<(n + 255) / 256, 256, 0, s>>>(Pvar, L, use, pose_diag, lm_acc, pose_scale, lm_scale);
 }
 void launch_landmark_prep(hipStream_t s, const DevTopology& t, const double* lm_acc, const double* lm_scale,
-                          double inv_mu, double min_diag, double max_diag, double* lm_z, int32_t* fail) {
+                          double inv_mu, double min_diag, double max_diag, double* lm_z, double* lm_anc,
+                          int32_t* fail) {
   if (t.L > 0)
-    k_landmark_prep<<<(t.L + 255) / 256, 256, 0, s>>>(t, lm_acc, lm_scale, inv_mu, min_diag, max_diag, lm_z, fail);
+    k_landmark_prep<<<(t.L + 255) / 256, 256, 0, s>>>(t, lm_acc, lm_scale, inv_mu, min_diag, max_diag, lm_z, lm_anc,
+                                                      fail);
 }
 void launch_schur_factors(hipStream_t s, const DevTopology& t, int32_t n_g, const int32_t* g_row,
                           const int32_t* g_inc_ptr, const int32_t* g_inc, const double* vR, const double* lm,
-                          const double* obs_rec, const double* lm_acc, const double* pose_scale, double* gw,
-                          double* gr0, bool f32) {
+                          const double* obs_rec, double* gf, double* gk, bool f32) {
   if (t.Pvar <= 0 || n_g <= 0) return;
   if (f32)
-    k_schur_factors<true><<<(n_g + 255) / 256, 256, 0, s>>>(t, n_g, g_row, g_inc_ptr, g_inc, vR, lm, obs_rec,
-                                                            lm_acc, pose_scale, gw, gr0);
+    k_schur_factors<true><<<(n_g + 255) / 256, 256, 0, s>>>(t, n_g, g_row, g_inc_ptr, g_inc, vR, lm, obs_rec, gf, gk);
   else
-    k_schur_factors<false><<<(n_g + 255) / 256, 256, 0, s>>>(t, n_g, g_row, g_inc_ptr, g_inc, vR, lm, obs_rec,
-                                                             lm_acc, pose_scale, gw, gr0);
+    k_schur_factors<false><<<(n_g + 255) / 256, 256, 0, s>>>(t, n_g, g_row, g_inc_ptr, g_inc, vR, lm, obs_rec, gf, gk);
 }
 bool schur_items_per_wg_supported(int32_t n) { return n == 1 || n == 2 || n == 4 || n == 8; }
-void launch_schur_tiles(hipStream_t s, const SchurTilesDev& d, const double* gw, const double* gr0,
-                        const double* lm_acc, const double* lm_z, double* partial, int32_t items_per_wg,
+void launch_schur_tiles(hipStream_t s, const SchurTilesDev& d, const double* gf, const double* gk,
+                        const double* lm_z, const double* lm_anc, double* partial, int32_t items_per_wg,
                         int32_t xcd_map) {
   if (d.n_segs <= 0) return;
   const int wgs = (d.n_segs + items_per_wg - 1) / items_per_wg;
   const int per_xcd = (wgs + 7) / 8;
-  const TileArgs ta{d.batches, d.slots, d.batch_off, reinterpret_cast<const uint32_t*>(d.pairs), gw, gr0, lm_acc,
-                    lm_z};
+  const TileArgs ta{d.batches, d.slots, d.batch_off, reinterpret_cast<const uint32_t*>(d.pairs), gf, gk, lm_z, lm_anc};
   k_schur_tiles<<<8 * per_xcd, kTileBlocks, 0, s>>>(d.n_segs, items_per_wg, xcd_map, d.seg_order, d.segs,
                                                      d.seg_thread, ta, partial);
 }
 void launch_schur_blocks(hipStream_t s, const DevTopology& t, const SchurTilesDev& d, int32_t nub, const int4* ublk,
-                         const double* gw, const double* gr0, const double* lm_acc, const double* lm_z,
-                         const double* pose_scale, const double* pose_diag, const double* pose_jtj, double inv_mu,
-                         double min_diag, double max_diag, double* partial, double* S, double* rhs,
+                         const double* gf, const double* gk, const double* lm_z, const double* lm_anc,
+                         const double* vR, const double* pose_scale, const double* pose_diag, const double* pose_jtj,
+                         double inv_mu, double min_diag, double max_diag, double* partial, double* S, double* rhs,
                          int32_t items_per_wg, int32_t xcd_map) {
   if (t.Pvar <= 0 || nub <= 0) return;
-  launch_schur_tiles(s, d, gw, gr0, lm_acc, lm_z, partial, items_per_wg, xcd_map);
+  launch_schur_tiles(s, d, gf, gk, lm_z, lm_anc, partial, items_per_wg, xcd_map);
   // kWide from 24 slots a block on: below that its groups have too few slots
   // each to hide their latency behind one another.
   if (d.n_uslot >= 24 * (int64_t)nub)
-    k_schur_finalize<true><<<nub, 252, 0, s>>>(nub, ublk, d.uslot_ptr, d.uslot, partial, pose_scale, pose_diag,
+    k_schur_finalize<true><<<nub, 252, 0, s>>>(t, nub, ublk, d.uslot_ptr, d.uslot, partial, vR, pose_scale, pose_diag,
                                                pose_jtj, inv_mu, min_diag, max_diag, S, rhs);
   else
     k_schur_finalize<false><<<(nub + kFinalizeGroups - 1) / kFinalizeGroups, 252, 0, s>>>(
-        nub, ublk, d.uslot_ptr, d.uslot, partial, pose_scale, pose_diag, pose_jtj, inv_mu, min_diag, max_diag, S, rhs);
+        t, nub, ublk, d.uslot_ptr, d.uslot, partial, vR, pose_scale, pose_diag, pose_jtj, inv_mu, min_diag, max_diag, S,
+        rhs);
 }
 void launch_landmark_quality(hipStream_t s, const DevTopology& t, const double* vert, const double* vR,
                              const double* lm, int32_t min_observers, double min_angle_deg, double max_dist,

@@ -102,14 +102,15 @@ bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const in
   }
   const int64_t n_visits = (int64_t)visits.size();
   T.visits = n_visits;
-  // A segment runs its batches one after the other, so a small system is cut
-  // into about as many segments as work-groups run at once (two on each of
-  // 256 CUs); above 512 x kSegmentSlots staged blocks the length that fills
-  // the last round of work-groups best is fixed. Build of S (two kernels) with
-  // segments of 5120 blocks and cut so: 10 keyframes 130 -> 27 us (2 -> 39
-  // segments), 25 keyframes 203 -> 47, 60 keyframes 206 -> 74, 150 keyframes
-  // 249 -> 211; 300 and more unchanged.
-  int64_t segment_slots = kSegmentSlots;
+  // A segment runs its batches one after the other, and about kSegmentTarget
+  // work-groups run at once (two on each of 256 CUs): the segments are sized
+  // for whole rounds of them, kSegmentSlots staged blocks or up to twice that
+  // each, and a system too small for one round of those is cut into one round
+  // of shorter ones. Build of S (two kernels) with segments of 5120 blocks and
+  // cut so: 10 keyframes 130 -> 27 us (2 -> 39 segments), 25 keyframes 203 ->
+  // 47, 60 keyframes 206 -> 74; with today's kernel 200 keyframes 234 -> 190,
+  // 300 keyframes 344 -> 294, 500 and more unchanged.
+  int64_t segment_slots = 0;
   {
     int64_t staged = 0, npairs = 0;
     for (const Visit& v : visits) {
@@ -118,7 +119,8 @@ bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const in
     }
     T.slots.reserve(2 * staged);
     T.pairs.reserve(npairs + npairs / 64 + 64);
-    segment_slots = std::min<int64_t>(kSegmentSlots, staged / kSegmentTarget);
+    const int64_t rounds = std::max<int64_t>(1, staged / ((int64_t)kSegmentTarget * kSegmentSlots));
+    segment_slots = staged / (kSegmentTarget * rounds);
   }
   auto is_anchor = [&](int g) { return T.g_inc[T.g_inc_ptr[g]] < 0; };
   // Batches (LDS-sized groups of visits) with their slot lists and pair

@@ -28,11 +28,11 @@ namespace mlba {
 
 constexpr int kTileBand = 16;                        // block rows (and columns) of a tile
 constexpr int kTileBlocks = kTileBand * kTileBand;   // blocks of a tile = threads of a work-group
-constexpr int kBatchSlots = 192;                     // factor blocks staged in LDS per batch (<= 256)
-constexpr int kSegmentSlots = 5120;                  // staged factor blocks per segment (about), at most
-constexpr int kSegmentTarget = 512;                  // segments a system is cut into when that makes them shorter
+constexpr int kBatchSlots = 256;                     // factor blocks staged in LDS per batch (<= 256)
+constexpr int kSegmentSlots = 5120;                  // staged factor blocks per segment of a large system, at least
+constexpr int kSegmentTarget = 512;                  // segments that run at once
 constexpr int kSegmentBatches = 64;                  // batches per segment, at most
-constexpr int kBatchPairs = 2048;                    // pairs per batch, at most
+constexpr int kBatchPairs = 2560;                    // pairs per batch, at most
 constexpr int kPairWords = kBatchPairs / 2 / kTileBlocks;  // 32-bit pair words a thread stages per batch
 constexpr int kPartEntries = 42;                     // a part's block (36) and rhs (6) sums
 constexpr int kTilePartial = kTileBlocks * kPartEntries;  // doubles of one segment's partial

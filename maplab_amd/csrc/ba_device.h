@@ -144,6 +144,13 @@ struct SchurTilesDev {
   const int32_t* uslot;
 };
 
+// Where k_evaluate_full writes the Jacobian blocks: block b of observation o
+// (2 x size, row-major) at block[b] + o * stride[b]; null: not wanted.
+struct EvalOut {
+  double* block[10];
+  int32_t stride[10];
+};
+
 // Loss of the whitened residual.
 struct DevLoss {
   int32_t type;      // 0 Huber (maplab), 1 Cauchy, 2 trivial

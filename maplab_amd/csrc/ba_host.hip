@@ -89,7 +89,7 @@ void launch_reduce(hipStream_t s, int32_t n, int32_t stride, int32_t offset, boo
                    double* out);
 void launch_evaluate_full(hipStream_t s, const DevTopology& t, const double* vert, const double* vR, const double* lm,
                           const double* baseframes, const double* cam_q, bool tangent, const int32_t* perm,
-                          double* res, double* jout, int32_t jstride, uint32_t mask);
+                          double* res, const EvalOut& jout, bool want_jac);
 }  // namespace mlba
 
 using namespace mlba;
@@ -1607,6 +1607,28 @@ int32_t mlba_landmark_quality(mlba_handle* h, const mlba_quality_options* o, uin
   return MLBA_OK;
 }
 
+// Jacobian blocks as the caller's arrays hold them: the wanted ones one after
+// the other from base, N x 2 x size each.
+static EvalOut eval_blocks(double* base, size_t N, const int* sizes, int nblocks, double* const* jacobians) {
+  EvalOut out{};
+  for (int b = 0; b < nblocks; ++b) {
+    if (!jacobians || !jacobians[b]) continue;
+    out.block[b] = base;
+    out.stride[b] = 2 * sizes[b];
+    base += N * (size_t)out.stride[b];
+  }
+  return out;
+}
+
+// Queues the copies of the wanted blocks into the caller's arrays.
+static int copy_eval_blocks(mlba_handle* h, const EvalOut& out, int nblocks, double* const* jacobians) {
+  for (int b = 0; b < nblocks; ++b)
+    if (out.block[b] && h->N)
+      HIP_OK(hipMemcpyAsync(jacobians[b], out.block[b], sizeof(double) * out.stride[b] * (size_t)h->N,
+                            hipMemcpyDeviceToHost, h->stream));
+  return MLBA_OK;
+}
+
 int32_t mlba_evaluate(mlba_handle* h, int32_t flags, const mlba_options* options, double* residuals,
                       double* const* jacobians, double* cost) {
   if (!h) return MLBA_EINVAL;
@@ -1616,19 +1638,17 @@ int32_t mlba_evaluate(mlba_handle* h, int32_t flags, const mlba_options* options
   static const int amb[10] = {3, 7, 7, 7, 7, 4, 3, 4, 4, 1};
   static const int tng[10] = {3, 6, 6, 6, 6, 3, 3, 4, 4, 1};
   const int* sz = tangent ? tng : amb;
-  int stride = 0;
-  uint32_t mask = 0;
-  for (int b = 0; b < 10; ++b) {
-    stride += 2 * sz[b];  // the device record always has room for block 9
-    if (b < nblocks && jacobians && jacobians[b]) mask |= 1u << b;
-  }
+  size_t width = 0;  // doubles of the wanted blocks of one observation
+  for (int b = 0; b < nblocks; ++b)
+    if (jacobians && jacobians[b]) width += 2 * (size_t)sz[b];
   hipStream_t s = h->stream;
   launch_vertex_prep(s, h->P, h->vert.p, h->vR.p);
   DBuf<double> res_d, jac_d;
   if (residuals && !res_d.alloc(2 * (size_t)h->N)) return set_err(h, MLBA_ENOMEM, "device allocation failed");
-  if (mask && !jac_d.alloc((size_t)stride * h->N)) return set_err(h, MLBA_ENOMEM, "device allocation failed");
+  if (width && !jac_d.alloc(width * h->N)) return set_err(h, MLBA_ENOMEM, "device allocation failed");
+  const EvalOut out = eval_blocks(jac_d.p, h->N, sz, nblocks, jacobians);
   launch_evaluate_full(s, h->topo, h->vert.p, h->vR.p, h->lm.p, h->baseframes.p, h->cam_q.p, tangent, h->perm_d.p,
-                       residuals ? res_d.p : nullptr, mask ? jac_d.p : nullptr, stride, mask);
+                       residuals ? res_d.p : nullptr, out, width != 0);
   if (cost) {
     mlba_options defaults;
     mlba_options_init(&defaults);
@@ -1641,27 +1661,13 @@ int32_t mlba_evaluate(mlba_handle* h, int32_t flags, const mlba_options* options
   HIP_OK(hipGetLastError());
   if (residuals)
     HIP_OK(hipMemcpyAsync(residuals, res_d.p, 2 * sizeof(double) * h->N, hipMemcpyDeviceToHost, s));
-  std::vector<double> jh;
-  if (mask) {
-    jh.resize((size_t)stride * h->N);
-    HIP_OK(hipMemcpyAsync(jh.data(), jac_d.p, jh.size() * sizeof(double), hipMemcpyDeviceToHost, s));
-  }
+  int rc = copy_eval_blocks(h, out, nblocks, jacobians);
+  if (rc) return rc;
   if (cost) {
-    int rc = read_scalars(h);
-    if (rc) return rc;
+    if ((rc = read_scalars(h))) return rc;
     *cost = h->scal_host[kCandCost] + h->scal_host[kCandFixed];
   }
   HIP_OK(hipStreamSynchronize(s));
-  if (mask) {
-    int off = 0;
-    for (int b = 0; b < nblocks; ++b) {
-      const int n = 2 * sz[b];
-      if (jacobians[b])
-        for (int o = 0; o < h->N; ++o)
-          std::memcpy(jacobians[b] + (size_t)o * n, jh.data() + (size_t)o * stride + off, n * sizeof(double));
-      off += n;
-    }
-  }
   return MLBA_OK;
 }
 
@@ -1722,8 +1728,10 @@ int32_t mlba_evaluate_noalloc(mlba_handle* h, int32_t flags, const mlba_options*
   double* jac_d = res_d + res_n;
   hipStream_t s = h->stream;
   launch_vertex_prep(s, h->P, h->vert.p, h->vR.p);
+  // The wanted blocks take no more than the room asked for.
+  const EvalOut out = eval_blocks(jac_d, h->N, sz, nblocks, jacobians);
   launch_evaluate_full(s, h->topo, h->vert.p, h->vR.p, h->lm.p, h->baseframes.p, h->cam_q.p, tangent, h->perm_d.p,
-                       residuals ? res_d : nullptr, mask ? jac_d : nullptr, stride, mask);
+                       residuals ? res_d : nullptr, out, mask != 0);
   if (cost) {
     mlba_options defaults;
     mlba_options_init(&defaults);
@@ -1736,17 +1744,7 @@ int32_t mlba_evaluate_noalloc(mlba_handle* h, int32_t flags, const mlba_options*
   HIP_OK(hipGetLastError());
   if (residuals && h->N)
     HIP_OK(hipMemcpyAsync(residuals, res_d, 2 * sizeof(double) * h->N, hipMemcpyDeviceToHost, s));
-  if (mask && h->N) {
-    // Block b of every record straight into the caller's row-major array.
-    int off = 0;
-    for (int b = 0; b < nblocks; ++b) {
-      const size_t n = 2 * (size_t)sz[b];
-      if (jacobians[b])
-        HIP_OK(hipMemcpy2DAsync(jacobians[b], n * sizeof(double), jac_d + off, (size_t)stride * sizeof(double),
-                                n * sizeof(double), (size_t)h->N, hipMemcpyDeviceToHost, s));
-      off += (int)n;
-    }
-  }
+  if (const int rc = copy_eval_blocks(h, out, nblocks, jacobians)) return rc;
   if (cost) {
     int rc = read_scalars(h);
     if (rc) return rc;
@@ -2118,9 +2116,16 @@ class CalibSolver {
     DevTopology tt = h->topo;
     tt.cams = cams;
     const int E = calib_entries();
+    // The calibration blocks 5 .. 9 inside one record per observation.
+    static const int kTangent[10] = {3, 6, 6, 6, 6, 3, 3, 4, 4, 1};
+    EvalOut rec{};
+    for (int b = 0, off = 0; b < 10; off += 2 * kTangent[b], ++b) {
+      if (!jac || b < 5) continue;
+      rec.block[b] = h->calib_rec.p + off;
+      rec.stride[b] = calib_record_stride();
+    }
     launch_evaluate_full(s, tt, h->vert.p, h->vR.p, h->lm.p, h->baseframes.p, cam_q, true, h->perm_d.p,
-                         h->calib_res.p, jac ? h->calib_rec.p : nullptr, calib_record_stride(),
-                         jac ? 0x3E0u : 0u);
+                         h->calib_res.p, rec, jac);
     launch_calib_normal(s, tt, h->perm_d.p, h->calib_res.p, h->calib_rec.p, make_loss(o_), !jac, h->calib_part.p,
                         h->calib_out.p);
     HIP_OK(hipGetLastError());

@@ -1673,15 +1673,16 @@ __global__ void k_reduce_many(ReduceBatch batch) {
 
 // Every Jacobian block of VisualReprojectionError::Evaluate
 // (visual-error-term-inl.h:184-367), in the caller's order, ambient or
-// tangent. Observation index is in the original (caller) order via perm.
+// tangent. Observation index is in the original (caller) order via perm. Each
+// block goes to an array of its own, as the caller has it, so that it is
+// copied out as it is.
 __global__ __launch_bounds__(256) void k_evaluate_full(DevTopology t, const double* __restrict__ vert,
                                                        const double* __restrict__ vR,
                                                        const double* __restrict__ lm,
                                                        const double* __restrict__ baseframes,
                                                        const double* __restrict__ cam_q, int32_t tangent,
                                                        const int32_t* __restrict__ perm, double* __restrict__ res,
-                                                       double* __restrict__ jout, int32_t jstride,
-                                                       uint32_t block_mask) {
+                                                       EvalOut jout, int32_t want_jac) {
   const int o = blockIdx.x * blockDim.x + threadIdx.x;
   if (o >= t.N) return;
   const int32_t meta = t.obs_meta[o];
@@ -1766,32 +1767,30 @@ __global__ __launch_bounds__(256) void k_evaluate_full(DevTopology t, const doub
     res[2 * oo] = failed ? 0.0 : (kp[0] - t.obs_kp[2 * o]) * sinv;
     res[2 * oo + 1] = failed ? 0.0 : (kp[1] - t.obs_kp[2 * o + 1]) * sinv;
   }
-  if (!jout) return;
+  if (!want_jac) return;
   // K = d r / d p_I = jp sinv R_C_I; Kc = jp sinv (d r / d p_C).
   double Kc[6], K[6];
   for (int k = 0; k < 6; ++k) Kc[k] = failed ? 0.0 : jp[k] * sinv;
   for (int r = 0; r < 2; ++r)
     for (int c = 0; c < 3; ++c)
       K[r * 3 + c] = Kc[r * 3] * cam.R_C_I[c] + Kc[r * 3 + 1] * cam.R_C_I[3 + c] + Kc[r * 3 + 2] * cam.R_C_I[6 + c];
-  // Block offsets inside the output record of this observation.
   // Block 9 (requested only with the xi flag) is d r / d xi of a
   // unified-projection camera.
   const int amb[10] = {3, 7, 7, 7, 7, 4, 3, 4, 4, 1};
   const int tng[10] = {3, 6, 6, 6, 6, 3, 3, 4, 4, 1};
-  double* rec = jout + (size_t)oo * jstride;
-  int offs[10];
-  int acc_off = 0;
-  for (int b = 0; b < 10; ++b) { offs[b] = acc_off; acc_off += 2 * (tangent ? tng[b] : amb[b]); }
+  auto at = [&](int b) { return jout.block[b] + (size_t)oo * jout.stride[b]; };
   auto zero_block = [&](int b) {
     const int n = 2 * (tangent ? tng[b] : amb[b]);
-    for (int k = 0; k < n; ++k) rec[offs[b] + k] = 0.0;
+    double* J = at(b);
+    for (int k = 0; k < n; ++k) J[k] = 0.0;
   };
   // Write J = Kx * D (2x3) into columns [c0, c0+3) of a block of width w.
   auto put3 = [&](int b, int c0, const double* Kx, const double* D, double scale) {
     const int w = tangent ? tng[b] : amb[b];
+    double* J = at(b);
     for (int r = 0; r < 2; ++r)
       for (int c = 0; c < 3; ++c)
-        rec[offs[b] + r * w + c0 + c] =
+        J[r * w + c0 + c] =
             scale * (Kx[r * 3] * D[c] + Kx[r * 3 + 1] * D[3 + c] + Kx[r * 3 + 2] * D[6 + c]);
   };
   // Rotation block: tangent = J_q |q|^2 ; ambient = J_q * 4 Jq(q)^T.
@@ -1800,17 +1799,18 @@ __global__ __launch_bounds__(256) void k_evaluate_full(DevTopology t, const doub
     for (int r = 0; r < 2; ++r)
       for (int c = 0; c < 3; ++c) Jr[r * 3 + c] = Kx[r * 3] * D[c] + Kx[r * 3 + 1] * D[3 + c] + Kx[r * 3 + 2] * D[6 + c];
     const int w = tangent ? tng[b] : amb[b];
+    double* J = at(b);
     if (tangent) {
       const double n2 = q[0] * q[0] + q[1] * q[1] + q[2] * q[2] + q[3] * q[3];
       for (int r = 0; r < 2; ++r)
-        for (int c = 0; c < 3; ++c) rec[offs[b] + r * w + c] = Jr[r * 3 + c] * n2;
+        for (int c = 0; c < 3; ++c) J[r * w + c] = Jr[r * 3 + c] * n2;
     } else {
       // 4 * 0.5 * [[w,-z,y],[z,w,-x],[-y,x,w],[-x,-y,-z]]^T (quaternion-param-jpl.cc:8-32)
       const double x = q[0], y = q[1], z = q[2], w4 = q[3];
       const double JqT[12] = {w4, z, -y, -x, -z, w4, x, -y, y, -x, w4, -z};  // 3x4
       for (int r = 0; r < 2; ++r)
         for (int c = 0; c < 4; ++c)
-          rec[offs[b] + r * w + c] =
+          J[r * w + c] =
               2.0 * (Jr[r * 3] * JqT[c] + Jr[r * 3 + 1] * JqT[4 + c] + Jr[r * 3 + 2] * JqT[8 + c]);
     }
   };
@@ -1819,16 +1819,15 @@ __global__ __launch_bounds__(256) void k_evaluate_full(DevTopology t, const doub
   const double* qGLM = baseframes + 7 * t.vertex_mission[a];
   const double* qGM = baseframes + 7 * t.vertex_mission[v];
   const double* qCI = cam_q + 7 * ci;
-  const int rot0 = tangent ? 0 : 0;
-  (void)rot0;
   for (int b = 0; b < 10; ++b) {
-    if (!((block_mask >> b) & 1u)) continue;
-    zero_block(b);
-    if (failed) continue;
+    if (!jout.block[b]) continue;
     const bool used = (b == 0) || (b == 5) || (b == 6) || (b == 7) || (b == 8) ||
                       (b == 9 && cam.model == kCameraUnifiedProjection) ||
                       ((b == 1 || b == 4) && type != kTypeKeyframe) || ((b == 2 || b == 3) && type == kTypeGlobal);
-    if (!used) continue;
+    if (failed || !used) {
+      zero_block(b);
+      continue;
+    }
     const int pc0 = tangent ? 3 : 4;  // column of the position part of a pose block
     switch (b) {
       case 0: put3(0, 0, K, D_pI_pB, 1.0); break;
@@ -1853,7 +1852,7 @@ __global__ __launch_bounds__(256) void k_evaluate_full(DevTopology t, const doub
       case 7: {
         // d kp / d (fu fv cu cv) at the distorted normalized point.
         const double u = (kp[0] - cam.intr[2]) / cam.intr[0], vv = (kp[1] - cam.intr[3]) / cam.intr[1];
-        double* J = rec + offs[7];
+        double* J = at(7);
         J[0] = u * sinv; J[1] = 0.0; J[2] = sinv; J[3] = 0.0;
         J[4] = 0.0; J[5] = vv * sinv; J[6] = 0.0; J[7] = sinv;
         break;
@@ -1861,7 +1860,7 @@ __global__ __launch_bounds__(256) void k_evaluate_full(DevTopology t, const doub
       case 8: {
         // d kp / d distortion at the undistorted normalized point (the
         // model's projection before distortion), rows x f.
-        double* J = rec + offs[8];
+        double* J = at(8);
         double den = pC[2];
         if (cam.model == kCameraUnifiedProjection)
           den += cam.xi * sqrt(pC[0] * pC[0] + pC[1] * pC[1] + pC[2] * pC[2]);
@@ -1878,8 +1877,8 @@ __global__ __launch_bounds__(256) void k_evaluate_full(DevTopology t, const doub
         // d kp / d xi (camera-unified-projection.cc:176-189).
         double kx[2], jx[6], jxi[2];
         project_unified(cam.xi, cam.dist_type, cam.intr, cam.dist, cam.width, cam.height, pC, kx, jx, jxi);
-        rec[offs[9]] = jxi[0] * sinv;
-        rec[offs[9] + 1] = jxi[1] * sinv;
+        at(9)[0] = jxi[0] * sinv;
+        at(9)[1] = jxi[1] * sinv;
         break;
       }
     }
@@ -2146,10 +2145,10 @@ void launch_calib_normal(hipStream_t s, const DevTopology& t, const int32_t* per
 
 void launch_evaluate_full(hipStream_t s, const DevTopology& t, const double* vert, const double* vR, const double* lm,
                           const double* baseframes, const double* cam_q, bool tangent, const int32_t* perm,
-                          double* res, double* jout, int32_t jstride, uint32_t mask) {
+                          double* res, const EvalOut& jout, bool want_jac) {
   if (t.N > 0)
     k_evaluate_full<<<(t.N + 255) / 256, 256, 0, s>>>(t, vert, vR, lm, baseframes, cam_q, tangent ? 1 : 0, perm, res,
-                                                      jout, jstride, mask);
+                                                      jout, want_jac ? 1 : 0);
 }
 
 // ------------------------------------------------------------ outlier rejection

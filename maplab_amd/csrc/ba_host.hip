@@ -408,35 +408,72 @@ int build_topology(mlba_handle* h) {
       if (flags[l] & kLmAnchorVar) inc[fill[vertex_var[h->lm_anchor[l]]]++] = -1 - l;
   }
   h->n_inc = (int32_t)inc.size();
-  // Block structure of S: row i couples with every variable vertex of every
-  // landmark it touches.
-  std::vector<int32_t> row_ptr(Pvar + 1, 0), col_var, diag_pos(Pvar, 0);
+  // Factor blocks and the work decomposition of the sums of S (ba_tiles.h).
+  SchurTiles st;
   {
-    std::vector<int32_t> mark(Pvar, -1), cols;
+    std::string terr;
+    if (!build_schur_tiles(Pvar, L, inc_ptr.data(), inc.data(), h->s_landmark.data(), &st, &terr))
+      return set_err(h, MLBA_ENOMEM, terr);
+  }
+  // Block structure of S: row i couples with the row of every factor block of
+  // every landmark it has one of. Incidence pairs (x in row i, y in row j >= i,
+  // same landmark) summed into each upper block: two factor blocks of a
+  // landmark multiply their incidence counts. Rows are independent.
+  std::vector<int32_t> row_ptr(Pvar + 1, 0), col_var, diag_pos(Pvar, 0);
+  std::vector<int32_t> upair;
+  int64_t total_pairs = 0;
+  {
+    const int64_t n_g = (int64_t)st.g_row.size();
+    std::vector<int32_t> row_g_ptr(Pvar + 1, 0), row_g(n_g), row_l(n_g);  // factor blocks and landmarks of each row
+    for (int64_t g = 0; g < n_g; ++g) row_g_ptr[st.g_row[g] + 1]++;
+    for (int i = 0; i < Pvar; ++i) row_g_ptr[i + 1] += row_g_ptr[i];
+    {
+      std::vector<int32_t> fill(row_g_ptr.begin(), row_g_ptr.end() - 1);
+      for (int l = 0; l < L; ++l)
+        for (int g = st.lm_g_ptr[l]; g < st.lm_g_ptr[l + 1]; ++g) {
+          const int k = fill[st.g_row[g]]++;
+          row_g[k] = g;
+          row_l[k] = l;
+        }
+    }
+    std::vector<std::vector<int32_t>> cols(Pvar), counts(Pvar);  // columns of a row; pairs of those >= the row
+    if (!parallel_ranges(Pvar, 4, [&](int64_t i0, int64_t i1) {
+          std::vector<int32_t> mark(Pvar, -1), pairs(Pvar, 0);
+          for (int i = (int)i0; i < (int)i1; ++i) {
+            std::vector<int32_t>& c = cols[i];
+            auto touch = [&](int j) {
+              if (mark[j] != i) {
+                mark[j] = i;
+                pairs[j] = 0;
+                c.push_back(j);
+              }
+            };
+            touch(i);
+            for (int k = row_g_ptr[i]; k < row_g_ptr[i + 1]; ++k) {
+              const int a = row_g[k], l = row_l[k];
+              const int ma = st.g_inc_ptr[a + 1] - st.g_inc_ptr[a];
+              for (int b = st.lm_g_ptr[l]; b < a; ++b) touch(st.g_row[b]);
+              for (int b = a; b < st.lm_g_ptr[l + 1]; ++b) {
+                const int j = st.g_row[b];
+                touch(j);
+                pairs[j] += ma * (st.g_inc_ptr[b + 1] - st.g_inc_ptr[b]);
+              }
+            }
+            std::sort(c.begin(), c.end());
+            for (int j : c)
+              if (j >= i) counts[i].push_back(pairs[j]);
+          }
+        }))
+      return set_err(h, MLBA_ENOMEM, "host allocation failed");
     h->max_row_blocks = 0;
     for (int i = 0; i < Pvar; ++i) {
-      cols.clear();
-      auto touch = [&](int j) {
-        if (mark[j] != i) { mark[j] = i; cols.push_back(j); }
-      };
-      touch(i);
-      int last_l = -1;
-      for (int k = inc_ptr[i]; k < inc_ptr[i + 1]; ++k) {
-        const int x = inc[k];
-        const int l = x >= 0 ? h->s_landmark[x] : -1 - x;
-        if (l == last_l) continue;
-        last_l = l;
-        for (int o = h->lm_begin[l]; o < h->lm_begin[l + 1]; ++o)
-          if (meta[o] & 4) touch(vertex_var[h->s_vertex[o]]);
-        if (flags[l] & kLmAnchorVar) touch(vertex_var[h->lm_anchor[l]]);
-      }
-      std::sort(cols.begin(), cols.end());
-      for (size_t k = 0; k < cols.size(); ++k)
-        if (cols[k] == i) diag_pos[i] = (int32_t)(col_var.size() + k);
-      col_var.insert(col_var.end(), cols.begin(), cols.end());
+      diag_pos[i] = (int32_t)(col_var.size() + cols[i].size() - counts[i].size());
+      col_var.insert(col_var.end(), cols[i].begin(), cols[i].end());
+      upair.insert(upair.end(), counts[i].begin(), counts[i].end());
       row_ptr[i + 1] = (int32_t)col_var.size();
-      h->max_row_blocks = std::max<int32_t>(h->max_row_blocks, (int32_t)cols.size());
+      h->max_row_blocks = std::max<int32_t>(h->max_row_blocks, (int32_t)cols[i].size());
     }
+    for (int32_t n : upair) total_pairs += n;
   }
   h->nnzb = (int32_t)col_var.size();
   h->hat_K = -1;
@@ -445,12 +482,10 @@ int build_topology(mlba_handle* h) {
   h->ritz_stage = 0;
   h->h_row_ptr = row_ptr;
   h->h_col_var = col_var;
-  // Upper blocks of S (row i, column j >= i, in row order) and the work
-  // decomposition of their sums (ba_tiles.h).
+  // Upper blocks of S (row i, column j >= i, in row order).
   std::vector<int4> ublk;
-  std::vector<int32_t> ubase(Pvar + 1, 0);
-  for (int i = 0; i < Pvar; ++i) {
-    ubase[i] = (int32_t)ublk.size();
+  ublk.reserve(upair.size());
+  for (int i = 0; i < Pvar; ++i)
     for (int k = diag_pos[i]; k < row_ptr[i + 1]; ++k) {
       const int j = col_var[k];
       int kt = k;
@@ -461,35 +496,7 @@ int build_topology(mlba_handle* h) {
       }
       ublk.push_back(make_int4(k, kt, i, j));
     }
-  }
-  ubase[Pvar] = (int32_t)ublk.size();
   h->n_upper = (int32_t)ublk.size();
-  SchurTiles st;
-  {
-    std::string terr;
-    if (!build_schur_tiles(Pvar, L, inc_ptr.data(), inc.data(), h->s_landmark.data(), &st, &terr))
-      return set_err(h, MLBA_ENOMEM, terr);
-  }
-  // Incidence pairs (x in row i, y in row j >= i, same landmark) summed into
-  // each upper block: two factor blocks of a landmark multiply their
-  // incidence counts.
-  std::vector<int32_t> upair(ublk.size(), 0);
-  int64_t total_pairs = 0;
-  for (int l = 0; l < L; ++l)
-    for (int a = st.lm_g_ptr[l]; a < st.lm_g_ptr[l + 1]; ++a) {
-      const int i = st.g_row[a];
-      const int ma = st.g_inc_ptr[a + 1] - st.g_inc_ptr[a];
-      const int32_t* cb = col_var.data() + diag_pos[i];
-      const int32_t* ce = col_var.data() + row_ptr[i + 1];
-      for (int b = a; b < st.lm_g_ptr[l + 1]; ++b) {
-        const int j = st.g_row[b];
-        const int32_t* f = std::lower_bound(cb, ce, j);
-        if (f == ce || *f != j) return set_err(h, MLBA_EINVAL, "internal: S block structure misses a landmark pair");
-        const int64_t m = (int64_t)ma * (st.g_inc_ptr[b + 1] - st.g_inc_ptr[b]);
-        upair[ubase[i] + (f - cb)] += (int32_t)m;
-        total_pairs += m;
-      }
-    }
   h->schur_pairs = total_pairs;
   h->n_g = (int32_t)st.g_row.size();
   h->nbands = st.nbands;

@@ -3,7 +3,9 @@
 #include "ba_tiles.h"
 
 #include <algorithm>
+#include <atomic>
 #include <limits>
+#include <thread>
 
 namespace mlba {
 
@@ -14,6 +16,35 @@ struct Run {
 };
 
 }  // namespace
+
+bool parallel_ranges(int64_t n, int64_t piece, const std::function<void(int64_t, int64_t)>& body) {
+  if (n <= 0) return true;
+  piece = std::max<int64_t>(piece, 1);
+  std::atomic<int64_t> next{0};
+  std::atomic<bool> ok{true};
+  auto work = [&]() {
+    for (int64_t b = next.fetch_add(piece); b < n; b = next.fetch_add(piece)) {
+      try {
+        body(b, std::min(n, b + piece));
+      } catch (...) {
+        ok = false;
+      }
+    }
+  };
+  const int64_t pieces = (n + piece - 1) / piece;
+  const int64_t hw = std::max(1u, std::thread::hardware_concurrency());
+  std::vector<std::thread> pool;
+  try {
+    const int64_t extra = std::min<int64_t>({pieces, hw, 8}) - 1;
+    pool.reserve((size_t)std::max<int64_t>(extra, 0));
+    for (int64_t t = 0; t < extra; ++t) pool.emplace_back(work);
+  } catch (...) {
+    // Fewer threads than wanted: the ones that run take all pieces.
+  }
+  work();
+  for (std::thread& t : pool) t.join();
+  return ok;
+}
 
 bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const int32_t* inc,
                        const int32_t* obs_landmark, SchurTiles* out, std::string* err) {
@@ -31,39 +62,56 @@ bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const in
     std::vector<int32_t> fill(lm_ptr.begin(), lm_ptr.end() - 1);
     for (int64_t k = 0; k < n_inc; ++k) lm_list[fill[lm_of(inc[k])]++] = (int32_t)k;
   }
-  // Factor blocks: the incidences of one landmark in one row.
-  std::vector<int32_t>& lm_g = T.lm_g_ptr;
-  lm_g.assign(L + 1, 0);
-  T.g_row.reserve(n_inc);
-  T.g_inc.reserve(n_inc);
-  for (int l = 0; l < L; ++l) {
-    int last = -1;
-    for (int m = lm_ptr[l]; m < lm_ptr[l + 1]; ++m) {
-      const int k = lm_list[m];
-      if (inc_row[k] != last) {
-        last = inc_row[k];
-        T.g_row.push_back(last);
-        T.g_inc_ptr.push_back((int32_t)T.g_inc.size());
+  // Factor blocks: the incidences of one landmark in one row. Landmarks are
+  // counted first, so that each has its place and pieces of them are filled
+  // independently.
+  constexpr int64_t kPiece = 4096;  // landmarks
+  UnsetVector<int32_t>& lm_g = T.lm_g_ptr;
+  lm_g.resize((size_t)L + 1);
+  lm_g[0] = 0;
+  std::atomic<bool> shared{false};
+  bool ok = parallel_ranges(L, kPiece, [&](int64_t l0, int64_t l1) {
+    for (int64_t l = l0; l < l1; ++l) {
+      int n = 0, last = -1;
+      for (int m = lm_ptr[l]; m < lm_ptr[l + 1]; ++m) {
+        const int row = inc_row[lm_list[m]];
+        // An anchor incidence is alone in its row: the anchor vertex's own
+        // observations of the landmark do not couple its pose.
+        if (row == last && (inc[lm_list[m]] < 0 || inc[lm_list[m - 1]] < 0)) shared = true;
+        n += row != last;
+        last = row;
       }
-      T.g_inc.push_back(inc[k]);
+      lm_g[l + 1] = n;
     }
-    lm_g[l + 1] = (int32_t)T.g_row.size();
+  });
+  if (shared) {
+    *err = "internal: an anchor incidence shares its row with observations";
+    return false;
   }
-  T.g_inc_ptr.push_back((int32_t)T.g_inc.size());
-  // An anchor incidence is alone in its row: the anchor vertex's own
-  // observations of the landmark do not couple its pose.
-  for (size_t g = 0; g + 1 < T.g_inc_ptr.size(); ++g) {
-    const int b = T.g_inc_ptr[g], e = T.g_inc_ptr[g + 1];
-    for (int k = b; k < e; ++k)
-      if (T.g_inc[k] < 0 && e - b != 1) {
-        *err = "internal: an anchor incidence shares its row with observations";
-        return false;
+  for (int l = 0; l < L; ++l) lm_g[l + 1] += lm_g[l];
+  const int64_t n_g = lm_g[L];
+  T.g_row.resize((size_t)n_g);
+  T.g_inc_ptr.resize((size_t)n_g + 1);
+  T.g_inc.resize((size_t)n_inc);
+  T.g_inc_ptr[n_g] = (int32_t)n_inc;
+  ok = ok && parallel_ranges(L, kPiece, [&](int64_t l0, int64_t l1) {
+    for (int64_t l = l0; l < l1; ++l) {
+      int g = lm_g[l], last = -1;
+      for (int m = lm_ptr[l]; m < lm_ptr[l + 1]; ++m) {
+        const int k = lm_list[m];
+        if (inc_row[k] != last) {
+          last = inc_row[k];
+          T.g_row[g] = last;
+          T.g_inc_ptr[g++] = m;
+        }
+        T.g_inc[m] = inc[k];
       }
-  }
+    }
+  });
   const int64_t nb = (Pvar + kTileBand - 1) / kTileBand;
   T.nbands = (int32_t)nb;
-  std::vector<Run> runs;
-  auto landmark_runs = [&](int l) {
+  // The runs of a landmark's factor blocks in one band.
+  auto landmark_runs = [&](int64_t l, std::vector<Run>& runs) {
     runs.clear();
     for (int g = lm_g[l]; g < lm_g[l + 1]; ++g) {
       const int band = T.g_row[g] / kTileBand;
@@ -73,34 +121,51 @@ bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const in
   };
   // Visits (landmark, first block in I, first in J, blocks in I, in J),
   // grouped by tile in (I, J) order, landmarks ascending in a tile (a
-  // landmark visits a tile at most once; only visited tiles exist).
+  // landmark visits a tile at most once; only visited tiles exist): a counting
+  // sort over pieces of the landmarks, each with counts of its own.
   struct Visit {
     int64_t key;  // I * nb + J
     int32_t l, gi, gj, ni, nj;
   };
-  std::vector<Visit> visits;
-  for (int l = 0; l < L; ++l) {
-    landmark_runs(l);
-    for (size_t a = 0; a < runs.size(); ++a)
-      for (size_t b = a; b < runs.size(); ++b) {
-        const bool diag = a == b;
-        visits.push_back(Visit{runs[a].band * nb + runs[b].band, l, runs[a].g, runs[b].g, runs[a].n,
-                               diag ? 0 : runs[b].n});
+  const int64_t keys = nb * nb;
+  const int64_t pieces = std::max<int64_t>(1, std::min<int64_t>({16, (L + kPiece - 1) / kPiece, (1 << 22) / std::max<int64_t>(keys, 1)}));
+  const int64_t span = (L + pieces - 1) / pieces;
+  std::vector<int64_t> at((size_t)(pieces * keys), 0);  // visits, then the place of the next, by piece and tile
+  ok = ok && parallel_ranges(pieces, 1, [&](int64_t p0, int64_t p1) {
+    std::vector<Run> runs;
+    for (int64_t q = p0; q < p1; ++q)
+      for (int64_t l = q * span; l < std::min<int64_t>(L, (q + 1) * span); ++l) {
+        landmark_runs(l, runs);
+        for (size_t a = 0; a < runs.size(); ++a)
+          for (size_t b = a; b < runs.size(); ++b) at[(size_t)(q * keys + runs[a].band * nb + runs[b].band)]++;
       }
-  }
-  {
-    // Stable LSD radix sort by key, 16 bits per pass (keys < nb^2).
-    std::vector<Visit> tmp(visits.size());
-    std::vector<int64_t> count(65537);
-    for (int shift = 0; shift < 64 && (nb * nb - 1) >> shift; shift += 16) {
-      std::fill(count.begin(), count.end(), 0);
-      for (const Visit& v : visits) count[((v.key >> shift) & 65535) + 1]++;
-      for (int k = 0; k < 65536; ++k) count[k + 1] += count[k];
-      for (const Visit& v : visits) tmp[count[(v.key >> shift) & 65535]++] = v;
-      visits.swap(tmp);
+  });
+  int64_t n_visits = 0;
+  for (int64_t k = 0; k < keys; ++k)
+    for (int64_t q = 0; q < pieces; ++q) {
+      const int64_t n = at[(size_t)(q * keys + k)];
+      at[(size_t)(q * keys + k)] = n_visits;
+      n_visits += n;
     }
+  UnsetVector<Visit> visits;
+  visits.resize((size_t)n_visits);
+  ok = ok && parallel_ranges(pieces, 1, [&](int64_t p0, int64_t p1) {
+    std::vector<Run> runs;
+    for (int64_t q = p0; q < p1; ++q)
+      for (int64_t l = q * span; l < std::min<int64_t>(L, (q + 1) * span); ++l) {
+        landmark_runs(l, runs);
+        for (size_t a = 0; a < runs.size(); ++a)
+          for (size_t b = a; b < runs.size(); ++b) {
+            const int64_t key = runs[a].band * nb + runs[b].band;
+            visits[(size_t)at[(size_t)(q * keys + key)]++] =
+                Visit{key, (int32_t)l, runs[a].g, runs[b].g, runs[a].n, a == b ? 0 : runs[b].n};
+          }
+      }
+  });
+  if (!ok) {
+    *err = "internal: the Schur decomposition failed";
+    return false;
   }
-  const int64_t n_visits = (int64_t)visits.size();
   T.visits = n_visits;
   // A segment runs its batches one after the other, and about kSegmentTarget
   // work-groups run at once (two on each of 256 CUs): the segments are sized
@@ -110,34 +175,87 @@ bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const in
   // cut so: 10 keyframes 130 -> 27 us (2 -> 39 segments), 25 keyframes 203 ->
   // 47, 60 keyframes 206 -> 74; with today's kernel 200 keyframes 234 -> 190,
   // 300 keyframes 344 -> 294, 500 and more unchanged.
-  int64_t segment_slots = 0;
-  {
-    int64_t staged = 0, npairs = 0;
-    for (const Visit& v : visits) {
-      staged += v.ni + v.nj;
-      npairs += v.nj ? (int64_t)v.ni * v.nj : (int64_t)v.ni * (v.ni + 1) / 2;
-    }
-    T.slots.reserve(2 * staged);
-    T.pairs.reserve(npairs + npairs / 64 + 64);
-    const int64_t rounds = std::max<int64_t>(1, staged / ((int64_t)kSegmentTarget * kSegmentSlots));
-    segment_slots = staged / (kSegmentTarget * rounds);
-  }
+  int64_t staged_all = 0;
+  for (const Visit& v : visits) staged_all += v.ni + v.nj;
+  const int64_t rounds = std::max<int64_t>(1, staged_all / ((int64_t)kSegmentTarget * kSegmentSlots));
+  const int64_t segment_slots = staged_all / (kSegmentTarget * rounds);
   auto is_anchor = [&](int g) { return T.g_inc[T.g_inc_ptr[g]] < 0; };
-  // Batches (LDS-sized groups of visits) with their slot lists and pair
-  // lists by block, and segments (runs of batches of one tile) with their
-  // thread parts.
-  std::vector<uint32_t> bp_block;
-  std::vector<uint16_t> bp_pair;
-  int32_t cnt[kTileBlocks + 1];
-  int64_t seg_cnt[kTileBlocks];
-  int parts[kTileBlocks];
-  auto close_segment = [&](int32_t b0, int32_t b1, int64_t I, int64_t J) {
-    T.segs.push_back(b0);
-    T.segs.push_back(b1);
-    T.segs.push_back((int32_t)I);
-    T.segs.push_back((int32_t)J);
+  auto pairs_of = [](const Visit& v) { return v.nj ? v.ni * v.nj : v.ni * (v.ni + 1) / 2; };
+  // Batches (LDS-sized groups of visits) and segments (runs of batches of one
+  // tile) of every visited tile, counted first: each tile's slots, pairs
+  // (batches start on a 32-bit word), batches and segments then have their
+  // place, and the tiles are filled independently of one another.
+  struct Tile {
+    int64_t v0, v1;                   // visits
+    int64_t slot, pair, batch, seg;   // first of each
+  };
+  std::vector<Tile> tiles;
+  int64_t n_slots = 0, n_pairs = 0, n_batches = 0, n_segs = 0;
+  for (int64_t v = 0; v < n_visits;) {
+    const int64_t key = visits[v].key;
+    tiles.push_back(Tile{v, v, n_slots, n_pairs, n_batches, n_segs});
+    int64_t seg_slots = 0, seg_batches = 0;
+    bool open = false;
+    while (v < n_visits && visits[v].key == key) {
+      int64_t slots = 0, np = 0;
+      for (; v < n_visits && visits[v].key == key; ++v) {
+        const int c = visits[v].ni + visits[v].nj;
+        if (slots + c > kBatchSlots) break;
+        slots += c;
+        np += pairs_of(visits[v]);
+      }
+      // A visit has at most 16 x 16 pairs over 32 slots (8 per slot), or
+      // 16 x 17 / 2 over 16 on a diagonal tile (8.5 per slot).
+      if (np > kBatchPairs) {
+        *err = "internal: a Schur batch has more pairs than its LDS holds";
+        return false;
+      }
+      n_slots += slots;
+      n_pairs += (np + 1) & ~(int64_t)1;
+      ++n_batches;
+      seg_slots += slots;
+      ++seg_batches;
+      open = true;
+      if (seg_slots >= segment_slots || seg_batches >= kSegmentBatches) {
+        ++n_segs;
+        seg_slots = seg_batches = 0;
+        open = false;
+      }
+    }
+    if (open) ++n_segs;
+    tiles.back().v1 = v;
+    T.tile_key.push_back(key);
+    T.tile_seg.push_back((int32_t)tiles.back().seg);
+    T.tile_seg.push_back((int32_t)n_segs);
+  }
+  const int64_t limit = std::numeric_limits<int32_t>::max();
+  if (n_slots > limit) {
+    *err = "reduced camera system has too many staged factor blocks";
+    return false;
+  }
+  if (n_pairs > limit) {
+    *err = "reduced camera system has too many factor pairs";
+    return false;
+  }
+  T.staged = n_slots;
+  T.slots.resize(2 * (size_t)n_slots);
+  T.pairs.resize((size_t)n_pairs);
+  T.batches.resize(4 * (size_t)n_batches);
+  T.batch_off.resize((size_t)n_batches * (kTileBlocks + 1));
+  T.segs.resize(4 * (size_t)n_segs);
+  T.seg_thread.resize((size_t)n_segs * kTileBlocks);
+  T.seg_block.resize((size_t)n_segs * kTileBlocks);
+  // Segment sg of tile (I, J): its batches and thread parts.
+  auto close_segment = [&](int64_t sg, int64_t b0, int64_t b1, int64_t I, int64_t J) {
+    int32_t* out = &T.segs[4 * (size_t)sg];
+    out[0] = (int32_t)b0;
+    out[1] = (int32_t)b1;
+    out[2] = (int32_t)I;
+    out[3] = (int32_t)J;
+    int64_t seg_cnt[kTileBlocks];
+    int parts[kTileBlocks];
     for (int k = 0; k < kTileBlocks; ++k) seg_cnt[k] = 0;
-    for (int32_t b = b0; b < b1; ++b) {
+    for (int64_t b = b0; b < b1; ++b) {
       const uint16_t* o = &T.batch_off[(size_t)b * (kTileBlocks + 1)];
       for (int k = 0; k < kTileBlocks; ++k) seg_cnt[k] += o[k + 1] - o[k];
     }
@@ -166,99 +284,78 @@ bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const in
       if (parts[best] >= 255) --nh;
       else std::push_heap(heap, heap + nh, lower);
     }
-    const size_t base = T.seg_thread.size();
-    T.seg_thread.resize(base + kTileBlocks, 0u);
-    T.seg_block.resize(base + kTileBlocks, 0);
+    uint32_t* thread = &T.seg_thread[(size_t)sg * kTileBlocks];
+    uint16_t* block = &T.seg_block[(size_t)sg * kTileBlocks];
+    for (int k = 0; k < kTileBlocks; ++k) {
+      thread[k] = 0u;
+      block[k] = 0;
+    }
     int t = 0;
     for (int k = 0; k < kTileBlocks; ++k) {
       if (!parts[k]) continue;
-      T.seg_block[base + k] = (uint16_t)(t | (parts[k] << 8));
-      for (int p = 0; p < parts[k]; ++p)
-        T.seg_thread[base + t++] = (uint32_t)k | ((uint32_t)p << 8) | ((uint32_t)parts[k] << 16);
+      block[k] = (uint16_t)(t | (parts[k] << 8));
+      for (int p = 0; p < parts[k]; ++p) thread[t++] = (uint32_t)k | ((uint32_t)p << 8) | ((uint32_t)parts[k] << 16);
     }
   };
-  for (int64_t tv = 0; tv < n_visits;) {
-    const int64_t key = visits[tv].key, I = key / nb, J = key % nb;
-    int64_t v = tv, ve = tv;
-    while (ve < n_visits && visits[ve].key == key) ++ve;
-    tv = ve;
+  auto fill_tile = [&](const Tile& tile) {
+    const int64_t key = visits[tile.v0].key, I = key / nb, J = key % nb;
     const bool diag = I == J;
-    const int32_t seg_first = (int32_t)(T.segs.size() / 4);
-    int32_t seg_batch = (int32_t)(T.batches.size() / 4);
-    int64_t seg_slots = 0;
-    while (v < ve) {
-      const int64_t bv = v;
-      int slots = 0;
-      while (v < ve) {
-        const int c = visits[v].ni + visits[v].nj;
-        if (slots + c > kBatchSlots) break;
-        slots += c;
-        ++v;
-      }
-      const size_t slot0 = T.slots.size() / 2;
-      if (slot0 + slots > (size_t)std::numeric_limits<int32_t>::max()) {
-        *err = "reduced camera system has too many staged factor blocks";
-        return false;
-      }
-      bp_block.clear();
-      bp_pair.clear();
-      int s = 0;
-      for (int64_t u = bv; u < v; ++u) {
-        const Visit& vr = visits[u];
+    int64_t slot = tile.slot, pair = tile.pair, batch = tile.batch, seg = tile.seg, seg_first = batch, seg_slots = 0;
+    uint16_t block[kBatchPairs], list[kBatchPairs];
+    int32_t cnt[kTileBlocks + 1];
+    for (int64_t v = tile.v0; v < tile.v1; ++batch) {
+      int s = 0, np = 0;
+      int32_t* out = &T.slots[2 * (size_t)slot];
+      for (; v < tile.v1; ++v) {
+        const Visit& vr = visits[v];
+        if (s + vr.ni + vr.nj > kBatchSlots) break;
         const int si = s, sj = diag ? s : s + vr.ni;
+        for (int a = 0; a < vr.ni + vr.nj; ++a) {
+          const int g = a < vr.ni ? vr.gi + a : vr.gj + a - vr.ni;
+          *out++ = g;
+          *out++ = vr.l | (int32_t)(is_anchor(g) ? kSlotAnchor : 0u);
+        }
+        const int nj = diag ? vr.ni : vr.nj, gj = diag ? vr.gi : vr.gj;
         for (int a = 0; a < vr.ni; ++a) {
-          T.slots.push_back(vr.gi + a);
-          T.slots.push_back(vr.l | (int32_t)(is_anchor(vr.gi + a) ? kSlotAnchor : 0u));
-        }
-        for (int b = 0; b < vr.nj; ++b) {
-          T.slots.push_back(vr.gj + b);
-          T.slots.push_back(vr.l | (int32_t)(is_anchor(vr.gj + b) ? kSlotAnchor : 0u));
-        }
-        const int nj = diag ? vr.ni : vr.nj;
-        const int gj = diag ? vr.gi : vr.gj;
-        for (int a = 0; a < vr.ni; ++a)
+          const int row = (int)(T.g_row[vr.gi + a] - I * kTileBand) * kTileBand;
           for (int b = diag ? a : 0; b < nj; ++b) {
-            bp_block.push_back((uint32_t)((T.g_row[vr.gi + a] - I * kTileBand) * kTileBand +
-                                          (T.g_row[gj + b] - J * kTileBand)));
-            bp_pair.push_back((uint16_t)((si + a) | ((sj + b) << 8)));
+            block[np] = (uint16_t)(row + (int)(T.g_row[gj + b] - J * kTileBand));
+            list[np++] = (uint16_t)((si + a) | ((sj + b) << 8));
           }
+        }
         s += vr.ni + vr.nj;
-      }
-      // A visit has at most 16 x 16 pairs over 32 slots (8 per slot), or
-      // 16 x 17 / 2 over 16 on a diagonal tile (8.5 per slot).
-      if (bp_pair.size() > (size_t)kBatchPairs) {
-        *err = "internal: a Schur batch has more pairs than its LDS holds";
-        return false;
       }
       // Stable counting sort of the batch's pairs by block.
       for (int k = 0; k <= kTileBlocks; ++k) cnt[k] = 0;
-      for (uint32_t b : bp_block) cnt[b + 1]++;
+      for (int k = 0; k < np; ++k) cnt[block[k] + 1]++;
       for (int k = 0; k < kTileBlocks; ++k) cnt[k + 1] += cnt[k];
-      if (T.pairs.size() % 2) T.pairs.push_back(0);  // batches start on a 32-bit word
-      const size_t pb = T.pairs.size();
-      if (pb + bp_pair.size() > (size_t)std::numeric_limits<int32_t>::max()) {
-        *err = "reduced camera system has too many factor pairs";
-        return false;
-      }
-      for (int k = 0; k <= kTileBlocks; ++k) T.batch_off.push_back((uint16_t)cnt[k]);
-      T.pairs.resize(pb + bp_pair.size());
-      for (size_t k = 0; k < bp_pair.size(); ++k) T.pairs[pb + cnt[bp_block[k]]++] = bp_pair[k];
-      T.batches.push_back((int32_t)slot0);
-      T.batches.push_back(slots);
-      T.batches.push_back((int32_t)pb);
-      T.batches.push_back((int32_t)bp_pair.size());
-      T.staged += slots;
-      seg_slots += slots;
-      const int32_t nbatch = (int32_t)(T.batches.size() / 4);
-      if (v == ve || seg_slots >= segment_slots || nbatch - seg_batch >= kSegmentBatches) {
-        close_segment(seg_batch, nbatch, I, J);
-        seg_batch = nbatch;
+      uint16_t* off = &T.batch_off[(size_t)batch * (kTileBlocks + 1)];
+      for (int k = 0; k <= kTileBlocks; ++k) off[k] = (uint16_t)cnt[k];
+      uint16_t* pl = &T.pairs[(size_t)pair];
+      for (int k = 0; k < np; ++k) pl[cnt[block[k]]++] = list[k];
+      if (np % 2) pl[np] = 0;
+      int32_t* bw = &T.batches[4 * (size_t)batch];
+      bw[0] = (int32_t)slot;
+      bw[1] = s;
+      bw[2] = (int32_t)pair;
+      bw[3] = np;
+      slot += s;
+      pair += (np + 1) & ~1;
+      seg_slots += s;
+      if (v == tile.v1 || seg_slots >= segment_slots || batch + 1 - seg_first >= kSegmentBatches) {
+        close_segment(seg++, seg_first, batch + 1, I, J);
+        seg_first = batch + 1;
         seg_slots = 0;
       }
     }
-    T.tile_key.push_back(key);
-    T.tile_seg.push_back(seg_first);
-    T.tile_seg.push_back((int32_t)(T.segs.size() / 4));
+  };
+  // The whole decomposition of 300 keyframes (1.2M observations, 8.4M pairs):
+  // 480 ms on one thread of an eight-core host, 69 ms on its eight.
+  if (!parallel_ranges((int64_t)tiles.size(), 1, [&](int64_t b, int64_t e) {
+        for (int64_t t = b; t < e; ++t) fill_tile(tiles[t]);
+      })) {
+    *err = "internal: the Schur decomposition failed";
+    return false;
   }
   return true;
 }

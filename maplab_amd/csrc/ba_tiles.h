@@ -21,7 +21,11 @@
 
 #include <stdint.h>
 
+#include <functional>
+#include <memory>
+#include <new>
 #include <string>
+#include <utility>
 #include <vector>
 
 namespace mlba {
@@ -45,19 +49,44 @@ constexpr int seg_thread_block(uint32_t w) { return (int)(w & 255u); }
 constexpr int seg_thread_part(uint32_t w) { return (int)((w >> 8) & 255u); }
 constexpr int seg_thread_parts(uint32_t w) { return (int)((w >> 16) & 255u); }
 
+// A vector whose resize leaves new elements unset: the large arrays are sized
+// once and filled by several threads.
+template <class T>
+struct UnsetAllocator : std::allocator<T> {
+  template <class U>
+  struct rebind {
+    using other = UnsetAllocator<U>;
+  };
+  template <class U>
+  void construct(U* p) noexcept {
+    ::new (static_cast<void*>(p)) U;
+  }
+  template <class U, class... A>
+  void construct(U* p, A&&... a) {
+    ::new (static_cast<void*>(p)) U(std::forward<A>(a)...);
+  }
+};
+template <class T>
+using UnsetVector = std::vector<T, UnsetAllocator<T>>;
+
+// Runs body(begin, end) over pieces of [0, n) on up to eight threads (the
+// caller's among them), pieces taken in order; rethrows nothing: returns false
+// when a piece threw.
+bool parallel_ranges(int64_t n, int64_t piece, const std::function<void(int64_t, int64_t)>& body);
+
 struct SchurTiles {
   int32_t nbands = 0;
-  std::vector<int32_t> g_row;       // row of each factor block (landmark-major, rows ascending)
-  std::vector<int32_t> g_inc_ptr;   // incidences summed into each factor block
-  std::vector<int32_t> g_inc;       // their codes (observation >= 0, anchor -1 - landmark)
-  std::vector<int32_t> lm_g_ptr;    // factor blocks of each landmark (L + 1)
-  std::vector<int32_t> slots;       // 2 per staged slot: factor block, landmark | kSlotAnchor
-  std::vector<int32_t> batches;     // 4 per batch: first slot, slots, first pair (even), pairs
-  std::vector<uint16_t> batch_off;  // kTileBlocks + 1 per batch: pair offsets of each block
-  std::vector<uint16_t> pairs;      // staged slots x | y << 8, by block, then visit
-  std::vector<int32_t> segs;        // 4 per segment: first batch, end batch, I, J
-  std::vector<uint32_t> seg_thread; // kTileBlocks per segment: the thread's part
-  std::vector<uint16_t> seg_block;  // kTileBlocks per segment: the block's parts
+  UnsetVector<int32_t> g_row;       // row of each factor block (landmark-major, rows ascending)
+  UnsetVector<int32_t> g_inc_ptr;   // incidences summed into each factor block
+  UnsetVector<int32_t> g_inc;       // their codes (observation >= 0, anchor -1 - landmark)
+  UnsetVector<int32_t> lm_g_ptr;    // factor blocks of each landmark (L + 1)
+  UnsetVector<int32_t> slots;       // 2 per staged slot: factor block, landmark | kSlotAnchor
+  UnsetVector<int32_t> batches;     // 4 per batch: first slot, slots, first pair (even), pairs
+  UnsetVector<uint16_t> batch_off;  // kTileBlocks + 1 per batch: pair offsets of each block
+  UnsetVector<uint16_t> pairs;      // staged slots x | y << 8, by block, then visit
+  UnsetVector<int32_t> segs;        // 4 per segment: first batch, end batch, I, J
+  UnsetVector<uint32_t> seg_thread; // kTileBlocks per segment: the thread's part
+  UnsetVector<uint16_t> seg_block;  // kTileBlocks per segment: the block's parts
   std::vector<int64_t> tile_key;    // visited tiles, ascending I * nbands + J
   std::vector<int32_t> tile_seg;    // 2 per visited tile: its segment range
   int64_t visits = 0;               // landmark tile visits

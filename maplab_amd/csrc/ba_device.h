@@ -75,6 +75,8 @@ constexpr int kMaxReduceBatch = 8;
 struct ReduceBatch {
   ReduceDesc d[kMaxReduceBatch];
   int32_t count;
+  int32_t* fail;     // nullable: failure counter, copied to fail_out and cleared
+  double* fail_out;
 };
 constexpr int kRowThreads = 256;     // threads of a reduced-camera-system row block
 

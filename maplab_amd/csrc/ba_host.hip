@@ -37,25 +37,26 @@ namespace mlba {
 void launch_vertex_prep(hipStream_t s, int32_t P, const double* vert, double* vR);
 void launch_linearize(hipStream_t s, bool jac, int32_t tiles, const DevTopology& t, const double* vert,
                       const double* vR, const double* lm, DevLoss loss, const int32_t* tile_begin, double* obs_rec,
-                      double* lm_acc, double* split_part, double* tile_cost, bool f32 = false);
+                      double* lm_acc, double* split_part, double* tile_cost, bool f32 = false,
+                      hipEvent_t stop = nullptr);
 void launch_split_sum(hipStream_t s, int32_t n, const int32_t* ids, const int32_t* split_tiles,
                       const double* split_part, double* lm_acc);
 void launch_pose_rows(hipStream_t s, const DevTopology& t, const double* vert, const double* vR, const double* lm,
                       const double* obs_rec, const double* lm_acc, double* pose_grad, double* pose_diag,
-                      double* pose_jtj, bool f32 = false);
+                      double* pose_jtj, bool f32 = false, hipEvent_t stop = nullptr);
 void launch_jacobi_scaling(hipStream_t s, int32_t Pvar, int32_t L, int32_t use, const double* pose_diag,
                            const double* lm_acc, double* pose_scale, double* lm_scale);
 void launch_landmark_prep(hipStream_t s, const DevTopology& t, const double* lm_acc, const double* lm_scale,
                           double inv_mu, double min_diag, double max_diag, double* lm_z, double* lm_anc,
-                          int32_t* fail);
+                          int32_t* fail, hipEvent_t stop = nullptr);
 void launch_schur_factors(hipStream_t s, const DevTopology& t, int32_t n_g, const int32_t* g_row,
                           const int32_t* g_inc_ptr, const int32_t* g_inc, const double* vR, const double* lm,
-                          const double* obs_rec, double* gf, double* gk, bool f32 = false);
+                          const double* obs_rec, double* gf, double* gk, bool f32 = false, hipEvent_t stop = nullptr);
 void launch_schur_blocks(hipStream_t s, const DevTopology& t, const SchurTilesDev& d, int32_t nub, const int4* ublk,
                          const double* gf, const double* gk, const double* lm_z, const double* lm_anc,
                          const double* vR, const double* pose_scale, const double* pose_diag, const double* pose_jtj,
                          double inv_mu, double min_diag, double max_diag, double* partial, double* S, double* rhs,
-                         int32_t items_per_wg, int32_t xcd_map);
+                         int32_t items_per_wg, int32_t xcd_map, hipEvent_t stop = nullptr);
 void launch_schur_tiles(hipStream_t s, const SchurTilesDev& d, const double* gf, const double* gk,
                         const double* lm_z, const double* lm_anc, double* partial, int32_t items_per_wg,
                         int32_t xcd_map);
@@ -68,20 +69,20 @@ void launch_landmark_quality(hipStream_t s, const DevTopology& t, const double* 
                              const double* lm, int32_t min_observers, double min_angle_deg, double max_dist,
                              double min_dist, double max_reproj_px, uint8_t* good);
 void launch_block_inverse(hipStream_t s, int32_t Pvar, const int32_t* diag_pos, const double* S, double* Minv,
-                          int32_t* fail);
+                          int32_t* fail, hipEvent_t stop = nullptr);
 int32_t pcg_max_lanczos();
 int32_t launch_back_substitute(hipStream_t s, const DevTopology& t, int32_t tiles, const int32_t* tile_begin,
                                int32_t n_split, const int32_t* split_ids, const double* vR, const double* lm,
                                const double* obs_rec, const double* lm_acc, const double* lm_z, const double* w,
-                               double* u, double* part, bool f32 = false);
-void launch_unscale_poses(hipStream_t s, int32_t Pvar, const double* y, const double* pose_scale, double* w,
-                          double* part);
-void launch_candidate(hipStream_t s, const DevTopology& t, const double* vert, const double* w, double* cand_v,
-                      double* cand_vR, double* part_v, const double* lm, const double* u, double* cand_l,
-                      double* part_l);
+                               double* u, double* part, bool f32 = false, hipEvent_t stop = nullptr);
+void launch_step_vertices(hipStream_t s, const DevTopology& t, const double* vert, const double* y,
+                          const double* pose_scale, double* w, double* cand_v, double* cand_vR, double* part_w,
+                          double* part_x, hipEvent_t stop = nullptr);
+void launch_candidate_landmarks(hipStream_t s, const DevTopology& t, const double* lm, const double* u, double* cand_l,
+                                double* part_l, hipEvent_t stop = nullptr);
 void launch_gradient_norm(hipStream_t s, const DevTopology& t, const double* vert, const double* pose_grad,
                           const double* lm_acc, double* part);
-bool launch_reduce_many(hipStream_t s, const ReduceBatch& batch);
+bool launch_reduce_many(hipStream_t s, const ReduceBatch& batch, hipEvent_t stop = nullptr);
 void launch_stream_copy(hipStream_t s, int64_t words, const void* src, void* dst);
 void launch_find_outliers(hipStream_t s, const DevTopology& t, const double* vert, const double* vR, const double* lm,
                           int32_t use_reproj, double max_reproj2, uint32_t* lm_flags, uint8_t* bad);
@@ -145,7 +146,7 @@ struct DBuf {
 };
 
 // Scalar slots of the reduction output array.
-enum Slot { kCost = 0, kFixed, kMcc, kUU, kWW, kXV, kXL, kCandCost, kCandFixed, kGradMax, kNumSlots };
+enum Slot { kCost = 0, kFixed, kMcc, kUU, kWW, kXV, kXL, kCandCost, kCandFixed, kGradMax, kFail, kPcgIters, kNumSlots };
 
 }  // namespace
 
@@ -242,7 +243,7 @@ struct mlba_handle {
   DBuf<int32_t> fail;
   DBuf<char> pcg_state;
   void* pcg_host = nullptr;
-  double* scal_host = nullptr;  // pinned: kNumSlots scalars, then the step's failure flag
+  double* scal_host = nullptr;  // pinned: kNumSlots scalars
   hipEvent_t scal_ev = nullptr;
   DevTopology topo{};
   SchurTilesDev tdev{};
@@ -589,7 +590,7 @@ int build_topology(mlba_handle* h) {
             h->parts_a.alloc(std::max<size_t>(Pvar, 2 * vb) + 1) && h->parts_b.alloc(2 * vb + 2) &&
             h->parts_l.alloc(2 * ((size_t)h->tiles + (size_t)(h->n_split + 255) / 256 + 1)) &&
             h->parts_c.alloc((size_t)(h->L + 255) / 256 + 1) &&
-            h->parts_v.alloc((size_t)(h->P + 255) / 256 + 1) && h->parts_w.alloc((6 * (size_t)Pvar + 255) / 256 + 1) &&
+            h->parts_v.alloc((size_t)(h->P + 255) / 256 + 1) && h->parts_w.alloc((size_t)(h->P + 255) / 256 + 1) &&
             h->parts_g.alloc(((size_t)Pvar + h->L + 255) / 256 + 1);
   if (!ok) return set_err(h, MLBA_ENOMEM, "device allocation failed");
   // The landmark step of inactive or observation-less landmarks stays zero.
@@ -610,9 +611,12 @@ int build_topology(mlba_handle* h) {
   return MLBA_OK;
 }
 
-// Kernel timing inside the LM loop: begin/end record an event pair on the
-// library stream; collect_events (after a stream synchronization) adds the
-// elapsed times to the summary.
+// Kernel timing inside the LM loop, only with a summary to fill: a timed span
+// runs from one event to the next, most of them stop events of the kernels
+// themselves (see launch in ba_kernels.hip); collect_events (after a stream
+// synchronization) adds the elapsed times to the summary. With a recorded pair
+// of events around every span, 10 LM iterations of a 10-keyframe map took 2.65
+// ms against 2.03 without any.
 hipEvent_t next_event(mlba_handle* h) {
   if (h->ev_next == h->ev_pool.size()) {
     hipEvent_t e;
@@ -621,23 +625,17 @@ hipEvent_t next_event(mlba_handle* h) {
   }
   return h->ev_pool[h->ev_next++];
 }
-struct KernelTimer {
-  mlba_handle* h;
-  int id;
-  hipEvent_t a = nullptr;
-  KernelTimer(mlba_handle* hh, int kid) : h(hh), id(kid) {
-    if (!h->ev_summary) return;
-    a = next_event(h);
-    if (a) (void)hipEventRecord(a, h->stream);
-  }
-  ~KernelTimer() {
-    if (!a) return;
-    hipEvent_t b = next_event(h);
-    if (!b) return;
-    (void)hipEventRecord(b, h->stream);
-    h->ev_pending.push_back({id, {a, b}});
-  }
-};
+// An event for a launch's stop argument (null without a summary).
+hipEvent_t stop_event(mlba_handle* h) { return h->ev_summary ? next_event(h) : nullptr; }
+// An event recorded here.
+hipEvent_t mark_event(mlba_handle* h) {
+  hipEvent_t e = stop_event(h);
+  if (e) (void)hipEventRecord(e, h->stream);
+  return e;
+}
+void time_span(mlba_handle* h, int id, hipEvent_t begin, hipEvent_t end) {
+  if (begin && end) h->ev_pending.push_back({id, {begin, end}});
+}
 void collect_events(mlba_handle* h) {
   if (h->ev_summary) {
     for (auto& p : h->ev_pending) {
@@ -907,26 +905,25 @@ DevLoss make_loss(const mlba_options* o) {
 // vertex-row gradient and diag(F'F). Leaves cost / fixed cost / gradient
 // max norm in the scalar slots (device).
 // Per-linearization Schur factors (P, p and k of every factor block).
-void schur_factors(mlba_handle* h) {
-  KernelTimer kt(h, MLBA_KERNEL_SCHUR_FACTORS);
+void schur_factors(mlba_handle* h, hipEvent_t stop = nullptr) {
   launch_schur_factors(h->stream, h->topo, h->n_g, h->g_row.p, h->g_inc_ptr.p, h->g_inc.p, h->vR.p, h->lm.p,
-                       h->obs_rec.p, h->gf.p, h->gk.p, h->f32_jac);
+                       h->obs_rec.p, h->gf.p, h->gk.p, h->f32_jac, stop);
 }
 
-int linearize(mlba_handle* h, const mlba_options* o) {
+// With `rotations`, the rotation records of the current vertices are formed
+// first (an accepted candidate brings its own). Returns the last event of the
+// linearization through `end`.
+int linearize(mlba_handle* h, const mlba_options* o, bool rotations = true, hipEvent_t* end = nullptr) {
   hipStream_t s = h->stream;
-  launch_vertex_prep(s, h->P, h->vert.p, h->vR.p);
-  {
-    KernelTimer kt(h, MLBA_KERNEL_LINEARIZE);
-    launch_linearize(s, true, h->tiles, h->topo, h->vert.p, h->vR.p, h->lm.p, make_loss(o), h->tile_begin.p,
-                     h->obs_rec.p, h->lm_acc.p, h->split_part.p, h->tile_cost.p, h->f32_jac);
-  }
+  if (rotations) launch_vertex_prep(s, h->P, h->vert.p, h->vR.p);
+  const hipEvent_t e0 = mark_event(h), e1 = stop_event(h), e2 = stop_event(h), e3 = stop_event(h);
+  launch_linearize(s, true, h->tiles, h->topo, h->vert.p, h->vR.p, h->lm.p, make_loss(o), h->tile_begin.p,
+                   h->obs_rec.p, h->lm_acc.p, h->split_part.p, h->tile_cost.p, h->f32_jac, e1);
+  time_span(h, MLBA_KERNEL_LINEARIZE, e0, e1);
   launch_split_sum(s, h->n_split, h->split_ids.p, h->split_tiles.p, h->split_part.p, h->lm_acc.p);
-  {
-    KernelTimer kt(h, MLBA_KERNEL_POSE_ROWS);
-    launch_pose_rows(s, h->topo, h->vert.p, h->vR.p, h->lm.p, h->obs_rec.p, h->lm_acc.p, h->pose_grad.p,
-                     h->pose_diag.p, h->pose_jtj.p, h->f32_jac);
-  }
+  launch_pose_rows(s, h->topo, h->vert.p, h->vR.p, h->lm.p, h->obs_rec.p, h->lm_acc.p, h->pose_grad.p,
+                   h->pose_diag.p, h->pose_jtj.p, h->f32_jac, e2);
+  time_span(h, MLBA_KERNEL_POSE_ROWS, e1, e2);
   const int gb = (h->Pvar + h->L + 255) / 256;
   launch_gradient_norm(s, h->topo, h->vert.p, h->pose_grad.p, h->lm_acc.p, h->parts_g.p);
   ReduceBatch rb{};
@@ -934,7 +931,8 @@ int linearize(mlba_handle* h, const mlba_options* o) {
   rb.d[1] = {h->tiles, 2, 1, 0, h->tile_cost.p, h->scal.p + kFixed};
   rb.d[2] = {gb, 1, 0, 1, h->parts_g.p, h->scal.p + kGradMax};
   rb.count = 3;
-  if (!launch_reduce_many(s, rb)) return set_err(h, MLBA_EINVAL, "internal: scalar reduction batch size");
+  if (!launch_reduce_many(s, rb, e3)) return set_err(h, MLBA_EINVAL, "internal: scalar reduction batch size");
+  if (end) *end = e3;
   HIP_OK(hipGetLastError());
   return MLBA_OK;
 }
@@ -1124,10 +1122,15 @@ int minimize(mlba_handle* h, const mlba_options* o, double initial_radius, mlba_
   h->f32_jac = o->jacobian_fp32 != 0;
   if ((rc = ensure_coarse_basis(h, o->pcg_coarse_nodes))) return rc;
   const double t_ev0 = now_s();
+  HIP_OK(hipMemsetAsync(h->fail.p, 0, sizeof(int32_t), s));  // each step hands it over and clears it
   if ((rc = linearize(h, o))) return rc;
   launch_jacobi_scaling(s, h->Pvar, h->L, o->use_jacobi_scaling, h->pose_diag.p, h->lm_acc.p, h->pose_scale.p,
                         h->lm_scale.p);
-  schur_factors(h);
+  {
+    const hipEvent_t e0 = mark_event(h), e1 = stop_event(h);
+    schur_factors(h, e1);
+    time_span(h, MLBA_KERNEL_SCHUR_FACTORS, e0, e1);
+  }
   if ((rc = read_scalars(h))) return rc;
   if (sm) sm->evaluate_seconds += now_s() - t_ev0;
   double x_cost = h->scal_host[kCost];
@@ -1150,7 +1153,6 @@ int minimize(mlba_handle* h, const mlba_options* o, double initial_radius, mlba_
     int consecutive_invalid = 0, iteration = 0;
     const int lb = (h->L + 255) / 256;
     const int pb = (h->P + 255) / 256;
-    const int wb = (6 * h->Pvar + 255) / 256;
     while (true) {
       const double t_iter = now_s();
       ++iteration;
@@ -1159,40 +1161,33 @@ int minimize(mlba_handle* h, const mlba_options* o, double initial_radius, mlba_
       const double inv_mu = 1.0 / radius;
       // Linear solve: Schur elimination + PCG on the reduced camera system.
       const double t_ls = now_s();
-      HIP_OK(hipMemsetAsync(h->fail.p, 0, sizeof(int32_t), s));
-      {
-        KernelTimer kt(h, MLBA_KERNEL_LANDMARK_PREP);
-        launch_landmark_prep(s, h->topo, h->lm_acc.p, h->lm_scale.p, inv_mu, o->min_lm_diagonal,
-                             o->max_lm_diagonal, h->lm_z.p, h->lm_anc.p, h->fail.p);
-      }
-      {
-        KernelTimer kt(h, MLBA_KERNEL_SCHUR_BLOCKS);
-        launch_schur_blocks(s, h->topo, h->tdev, h->n_upper, h->ublk.p, h->gf.p, h->gk.p, h->lm_z.p, h->lm_anc.p,
-                            h->vR.p, h->pose_scale.p, h->pose_diag.p, h->pose_jtj.p, inv_mu, o->min_lm_diagonal,
-                            o->max_lm_diagonal, h->schur_partial.p, h->S.p, h->rhs.p, h->sched_waves,
-                            h->sched_xcd);
-      }
-      launch_block_inverse(s, h->Pvar, h->diag_pos.p, h->S.p, h->Minv.p, h->fail.p);
+      const hipEvent_t e0 = mark_event(h), e_prep = stop_event(h), e_schur = stop_event(h), e_inv = stop_event(h);
+      launch_landmark_prep(s, h->topo, h->lm_acc.p, h->lm_scale.p, inv_mu, o->min_lm_diagonal, o->max_lm_diagonal,
+                           h->lm_z.p, h->lm_anc.p, h->fail.p, e_prep);
+      time_span(h, MLBA_KERNEL_LANDMARK_PREP, e0, e_prep);
+      launch_schur_blocks(s, h->topo, h->tdev, h->n_upper, h->ublk.p, h->gf.p, h->gk.p, h->lm_z.p, h->lm_anc.p,
+                          h->vR.p, h->pose_scale.p, h->pose_diag.p, h->pose_jtj.p, inv_mu, o->min_lm_diagonal,
+                          o->max_lm_diagonal, h->schur_partial.p, h->S.p, h->rhs.p, h->sched_waves, h->sched_xcd,
+                          e_schur);
+      time_span(h, MLBA_KERNEL_SCHUR_BLOCKS, e_prep, e_schur);
+      launch_block_inverse(s, h->Pvar, h->diag_pos.p, h->S.p, h->Minv.p, h->fail.p, e_inv);
       HIP_OK(hipGetLastError());
       int pcg_iters = 0;
       bool pcg_small = false;  // iteration count read with the step's scalars
       if (h->Pvar > 0 && (o->pcg_preconditioner == MLBA_PRECOND_BLOCK_JACOBI ||
                           o->pcg_preconditioner == MLBA_PRECOND_LEARNED)) {
-        KernelTimer kt(h, MLBA_KERNEL_PCG);
         if ((rc = lp_solve(h, o, o->pcg_preconditioner == MLBA_PRECOND_LEARNED, &pcg_iters))) return rc;
       } else if (h->Pvar > 0 && o->pcg_preconditioner == MLBA_PRECOND_LEARNED_DEFLATED) {
-        KernelTimer kt(h, MLBA_KERNEL_PCG);
         if ((rc = lp_deflated_solve(h, o, &pcg_iters))) return rc;
       } else if (h->Pvar > 0) {
-        KernelTimer kt(h, MLBA_KERNEL_PCG);
         const int32_t nritz = ritz_count(o);
         if ((rc = ritz_merge(h))) return rc;
         const int32_t nr_used = nritz > 0 ? h->ritz_nr : 0;
         const PcgBuffers B = pcg_buffers(h, nr_used, nritz > 0);
         if ((pcg_small = pcg_small_applies(B))) {
-          if (!launch_pcg_small(s, B, o->pcg_relative_tolerance, o->pcg_max_iterations))
+          if (!launch_pcg_small(s, B, o->pcg_relative_tolerance, o->pcg_max_iterations, h->scal.p + kPcgIters))
             return set_err(h, MLBA_EDEVICE, "PCG launch failed");
-          h->ritz_nr = 0;  // no coarse space to recycle columns for
+          h->ritz_nr = h->ritz_stage = 0;  // no coarse space to recycle columns for
         } else {
           int32_t& est = h->pcg_last_iters[nr_used > 0 ? 1 : 0];
           pcg_iters = launch_pcg_deflated(s, B, o->pcg_relative_tolerance, o->pcg_max_iterations,
@@ -1202,48 +1197,45 @@ int minimize(mlba_handle* h, const mlba_options* o, double initial_radius, mlba_
           ritz_after_solve(h, nritz, pcg_iters);
         }
       }
-      launch_unscale_poses(s, h->Pvar, h->px.p, h->pose_scale.p, h->w.p, h->parts_w.p);
-      int32_t nbs = 0;
-      {
-        KernelTimer kt(h, MLBA_KERNEL_BACK_SUBSTITUTE);
-        nbs = launch_back_substitute(s, h->topo, h->tiles, h->tile_begin.p, h->n_split, h->split_ids.p, h->vR.p,
-                                     h->lm.p, h->obs_rec.p, h->lm_acc.p, h->lm_z.p, h->w.p, h->lm_u.p,
-                                     h->parts_l.p, h->f32_jac);
-      }
+      const hipEvent_t e_pcg = mark_event(h);
+      if (h->Pvar > 0) time_span(h, MLBA_KERNEL_PCG, e_inv, e_pcg);
       // Candidate point and its cost; the step's scalars (model cost change,
       // step and state norms) and the cost in one batch of reductions.
-      launch_candidate(s, h->topo, h->vert.p, h->w.p, h->vert_cand.p, h->vR_cand.p, h->parts_v.p, h->lm.p,
-                       h->lm_u.p, h->lm_cand.p, h->parts_c.p);
-      {
-        KernelTimer kt(h, MLBA_KERNEL_COST);
-        launch_linearize(s, false, h->tiles, h->topo, h->vert_cand.p, h->vR_cand.p, h->lm_cand.p, make_loss(o),
-                         h->tile_begin.p, nullptr, nullptr, nullptr, h->tile_cost2.p);
-      }
+      const hipEvent_t e_vert = stop_event(h), e_back = stop_event(h), e_cand = stop_event(h), e_cost = stop_event(h);
+      launch_step_vertices(s, h->topo, h->vert.p, h->px.p, h->pose_scale.p, h->w.p, h->vert_cand.p, h->vR_cand.p,
+                           h->parts_w.p, h->parts_v.p, e_vert);
+      const int32_t nbs = launch_back_substitute(s, h->topo, h->tiles, h->tile_begin.p, h->n_split, h->split_ids.p,
+                                                 h->vR.p, h->lm.p, h->obs_rec.p, h->lm_acc.p, h->lm_z.p, h->w.p,
+                                                 h->lm_u.p, h->parts_l.p, h->f32_jac, e_back);
+      time_span(h, MLBA_KERNEL_BACK_SUBSTITUTE, e_vert, e_back);
+      launch_candidate_landmarks(s, h->topo, h->lm.p, h->lm_u.p, h->lm_cand.p, h->parts_c.p, e_cand);
+      launch_linearize(s, false, h->tiles, h->topo, h->vert_cand.p, h->vR_cand.p, h->lm_cand.p, make_loss(o),
+                       h->tile_begin.p, nullptr, nullptr, nullptr, h->tile_cost2.p, false, e_cost);
+      time_span(h, MLBA_KERNEL_COST, e_cand, e_cost);
       // The step's scalars and the candidate cost in one launch.
       ReduceBatch rb{};
       rb.d[0] = {nbs, 2, 0, 0, h->parts_l.p, h->scal.p + kMcc};
       rb.d[1] = {nbs, 2, 1, 0, h->parts_l.p, h->scal.p + kUU};
-      rb.d[2] = {wb, 1, 0, 0, h->parts_w.p, h->scal.p + kWW};
+      rb.d[2] = {pb, 1, 0, 0, h->parts_w.p, h->scal.p + kWW};
       rb.d[3] = {pb, 1, 0, 0, h->parts_v.p, h->scal.p + kXV};
       rb.d[4] = {lb, 1, 0, 0, h->parts_c.p, h->scal.p + kXL};
       rb.d[5] = {h->tiles, 2, 0, 0, h->tile_cost2.p, h->scal.p + kCandCost};
       rb.count = 6;
+      rb.fail = h->fail.p;
+      rb.fail_out = h->scal.p + kFail;
       if (!launch_reduce_many(s, rb)) return set_err(h, MLBA_EINVAL, "internal: scalar reduction batch size");
       HIP_OK(hipGetLastError());
-      int32_t* fail_pinned = reinterpret_cast<int32_t*>(h->scal_host + kNumSlots);
-      HIP_OK(hipMemcpyAsync(fail_pinned, h->fail.p, sizeof(int32_t), hipMemcpyDeviceToHost, s));
       HIP_OK(hipMemcpyAsync(h->scal_host, h->scal.p, kNumSlots * sizeof(double), hipMemcpyDeviceToHost, s));
       HIP_OK(hipEventRecord(h->scal_ev, s));
       // The recycling's host work and kernels go behind the step's cost.
       if ((rc = ritz_queue_vectors(h))) return rc;
       HIP_OK(hipEventSynchronize(h->scal_ev));
       collect_events(h);
-      if (pcg_small) pcg_iters = pcg_state_iterations(h->pcg_host);
-      const int32_t fail_h = *fail_pinned;
+      if (pcg_small) pcg_iters = (int)h->scal_host[kPcgIters];
       if (sm) sm->linear_solver_seconds += now_s() - t_ls;
       const double* sc = h->scal_host;
       const double mcc = sc[kMcc];
-      bool step_valid = fail_h == 0 && std::isfinite(mcc) && mcc > 0.0;
+      bool step_valid = sc[kFail] == 0.0 && std::isfinite(mcc) && mcc > 0.0;
       cur.linear_solver_iterations = pcg_iters;
       if (sm) sm->total_linear_solver_iterations += pcg_iters;
       cur.step_is_valid = step_valid;
@@ -1280,9 +1272,13 @@ int minimize(mlba_handle* h, const mlba_options* o, double initial_radius, mlba_
         if (cur.relative_decrease > o->min_relative_decrease) {
           std::swap(h->vert.p, h->vert_cand.p);
           std::swap(h->lm.p, h->lm_cand.p);
+          std::swap(h->vR.p, h->vR_cand.p);
           const double t_ev = now_s();
-          if ((rc = linearize(h, o))) return rc;
-          schur_factors(h);
+          hipEvent_t e_lin = nullptr;
+          if ((rc = linearize(h, o, false, &e_lin))) return rc;
+          const hipEvent_t e_fac = stop_event(h);
+          schur_factors(h, e_fac);
+          time_span(h, MLBA_KERNEL_SCHUR_FACTORS, e_lin, e_fac);
           if ((rc = read_scalars(h))) return rc;
           if (sm) sm->evaluate_seconds += now_s() - t_ev;
           x_cost = h->scal_host[kCost];
@@ -1532,7 +1528,7 @@ int32_t mlba_create(const mlba_problem_desc* d, mlba_handle** out) {
                   h->fail.alloc(1) && h->pcg_state.alloc(pcg_state_bytes());
   if (!ok) { h->err = "device allocation failed"; return fail_out(MLBA_ENOMEM); }
   if (hipHostMalloc(&h->pcg_host, pcg_state_bytes(), hipHostMallocDefault) != hipSuccess ||
-      hipHostMalloc((void**)&h->scal_host, (kNumSlots + 1) * sizeof(double), hipHostMallocDefault) != hipSuccess ||
+      hipHostMalloc((void**)&h->scal_host, kNumSlots * sizeof(double), hipHostMallocDefault) != hipSuccess ||
       hipEventCreateWithFlags(&h->scal_ev, hipEventDisableTiming) != hipSuccess) {
     h->err = "pinned host allocation failed";
     return fail_out(MLBA_ENOMEM);
@@ -2646,7 +2642,8 @@ int32_t mlba_time_kernels(mlba_handle* h, const mlba_options* o, int32_t repeats
     t->pcg_coarse_columns = 6 * (int64_t)std::max(h->hat_K, 0) + nr_used;
     t->pcg_window_columns = h->grp_width + nr_used;
   }
-  launch_unscale_poses(s, h->Pvar, h->px.p, h->pose_scale.p, h->w.p, h->parts_w.p);
+  launch_step_vertices(s, h->topo, h->vert.p, h->px.p, h->pose_scale.p, h->w.p, h->vert_cand.p, h->vR_cand.p,
+                       h->parts_w.p, h->parts_v.p);
   t->back_substitute_ms = timed([&] {
     (void)launch_back_substitute(s, h->topo, h->tiles, h->tile_begin.p, h->n_split, h->split_ids.p, h->vR.p,
                                  h->lm.p, h->obs_rec.p, h->lm_acc.p, h->lm_z.p, h->w.p, h->lm_u.p, h->parts_l.p,

@@ -19,13 +19,16 @@
 //   k_block_inverse   block-Jacobi preconditioner (6x6 inverses of diag(S))
 //   (ba_pcg.hip)      deflated block-Jacobi PCG on S
 //   k_back_substitute landmark step and the LM model cost change
-//   k_candidate       x (+) step for vertices (JPL Plus) and landmarks
+//   k_step_vertices   vertex step and x (+) step (JPL Plus)
+//   k_candidate_landmarks
 //   k_gradient_norm   max |x - Plus(x, -g)|
 //   k_evaluate_full   every reference Jacobian block (Evaluate parity API)
 // All reductions are fixed-order (per-tile partials summed by one block,
 // S blocks by one wave each, the tile sums of a landmark split over several
 // linearization tiles added in tile order), so results repeat bit for bit
 // run to run.
+#include <hip/hip_ext.h>
+
 #include "ba_device.h"
 #include "ba_math.h"
 #include "ba_reduce.h"
@@ -1537,38 +1540,28 @@ __global__ __launch_bounds__(256) void k_back_substitute_split(DevTopology t, in
   if (threadIdx.x == 0) { part[2 * blockIdx.x] = s1; part[2 * blockIdx.x + 1] = s2; }
 }
 
-// w = C_p y_p and |w|^2 partials.
-__global__ __launch_bounds__(256) void k_unscale_poses(int32_t Pvar, const double* __restrict__ y,
-                                                       const double* __restrict__ pose_scale,
-                                                       double* __restrict__ w, double* __restrict__ part) {
-  __shared__ double lds4[4];
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  double s = 0.0;
-  if (i < 6 * Pvar) {
-    const double v = y[i] * pose_scale[i];
-    w[i] = v;
-    s = v * v;
-  }
-  const double t = block_sum256(s, lds4);
-  if (threadIdx.x == 0) part[blockIdx.x] = t;
-}
-
-// Candidate state x (+) delta with delta = -w (vertices, JPL Plus) and
-// -u (landmarks); partials of |x|^2 over variable blocks.
-// Candidate vertex x [+] (-w) and its rotation record (as k_vertex_prep).
-__global__ __launch_bounds__(256) void k_candidate_vertices(DevTopology t, const double* __restrict__ vert,
-                                                            const double* __restrict__ w,
-                                                            double* __restrict__ cand, double* __restrict__ cand_vR,
-                                                            double* __restrict__ part) {
+// Vertex step w = C_p y_p, candidate vertices x [+] (-w) (JPL Plus) and their
+// rotation records (as k_vertex_prep); partials of |w|^2 and of |x|^2 over
+// variable vertices.
+__global__ __launch_bounds__(256) void k_step_vertices(DevTopology t, const double* __restrict__ vert,
+                                                       const double* __restrict__ y,
+                                                       const double* __restrict__ pose_scale, double* __restrict__ w,
+                                                       double* __restrict__ cand, double* __restrict__ cand_vR,
+                                                       double* __restrict__ part_w, double* __restrict__ part_x) {
   __shared__ double lds4[4];
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  double xx = 0.0;
+  double xx = 0.0, ww = 0.0;
   if (v < t.P) {
     const double* x = vert + 7 * v;
     double c[7];
     const int32_t j = t.vertex_var[v];
     if (j >= 0) {
-      const double* wv = w + 6 * j;
+      double wv[6];
+      for (int k = 0; k < 6; ++k) {
+        wv[k] = y[6 * j + k] * pose_scale[6 * j + k];
+        w[6 * j + k] = wv[k];
+        ww += wv[k] * wv[k];
+      }
       const double d[3] = {-wv[0], -wv[1], -wv[2]};
       quat_plus_jpl(x, d, c);
       c[4] = x[4] - wv[3];
@@ -1582,10 +1575,15 @@ __global__ __launch_bounds__(256) void k_candidate_vertices(DevTopology t, const
     for (int k = 0; k < 7; ++k) out[k] = c[k];
     vertex_rotation(c, cand_vR + 12 * v);
   }
-  const double s = block_sum256(xx, lds4);
-  if (threadIdx.x == 0) part[blockIdx.x] = s;
+  const double sw = block_sum256(ww, lds4);
+  const double sx = block_sum256(xx, lds4);
+  if (threadIdx.x == 0) {
+    part_w[blockIdx.x] = sw;
+    part_x[blockIdx.x] = sx;
+  }
 }
 
+// Candidate landmarks x - u; partials of |x|^2 over variable landmarks.
 __global__ __launch_bounds__(256) void k_candidate_landmarks(DevTopology t, const double* __restrict__ lm,
                                                              const double* __restrict__ u,
                                                              double* __restrict__ cand, double* __restrict__ part) {
@@ -1663,10 +1661,15 @@ __global__ void k_reduce(int32_t n, int32_t stride, int32_t offset, int32_t is_m
 }
 
 // Several independent reductions in one launch, work-group b computing
-// reduction b exactly as k_reduce does.
+// reduction b exactly as k_reduce does; the step's failure counter is handed
+// over and cleared with them.
 __global__ void k_reduce_many(ReduceBatch batch) {
   const ReduceDesc& d = batch.d[blockIdx.x];
   reduce_parts(d.n, d.stride, d.offset, d.is_max, d.parts, d.out);
+  if (batch.fail && blockIdx.x == 0 && threadIdx.x == 0) {
+    *batch.fail_out = (double)*batch.fail;
+    *batch.fail = 0;
+  }
 }
 
 // ------------------------------------------------------------ Evaluate API
@@ -1887,22 +1890,30 @@ __global__ __launch_bounds__(256) void k_evaluate_full(DevTopology t, const doub
 
 // ------------------------------------------------------------ launchers
 
+// One launch; with `stop`, that event completes with the kernel. An event tied
+// to its kernel's own completion costs a launch under 1 us, one recorded by
+// itself 3 us (a packet of its own in the queue).
+template <class... P, class... A>
+static void launch(hipStream_t s, hipEvent_t stop, void (*kernel)(P...), int grid, int block, A... args) {
+  if (stop)
+    hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(block), 0, s, nullptr, stop, 0, static_cast<P>(args)...);
+  else
+    kernel<<<grid, block, 0, s>>>(static_cast<P>(args)...);
+}
+// The stop event of a launcher that has nothing to launch.
+static void launch_nothing(hipStream_t s, hipEvent_t stop) {
+  if (stop) (void)hipEventRecord(stop, s);
+}
+
 void launch_vertex_prep(hipStream_t s, int32_t P, const double* vert, double* vR) {
   if (P > 0) k_vertex_prep<<<(P + 255) / 256, 256, 0, s>>>(P, vert, vR);
 }
 void launch_linearize(hipStream_t s, bool jac, int32_t tiles, const DevTopology& t, const double* vert,
                       const double* vR, const double* lm, DevLoss loss, const int32_t* tile_begin, double* obs_rec,
-                      double* lm_acc, double* split_part, double* tile_cost, bool f32) {
-  if (tiles <= 0) return;
-  if (jac && f32)
-    k_linearize<true, true><<<tiles, kObsTile, 0, s>>>(t, vert, vR, lm, loss, tile_begin, obs_rec, lm_acc,
-                                                       split_part, tile_cost);
-  else if (jac)
-    k_linearize<true><<<tiles, kObsTile, 0, s>>>(t, vert, vR, lm, loss, tile_begin, obs_rec, lm_acc, split_part,
-                                                 tile_cost);
-  else
-    k_linearize<false><<<tiles, kObsTile, 0, s>>>(t, vert, vR, lm, loss, tile_begin, obs_rec, lm_acc, split_part,
-                                                  tile_cost);
+                      double* lm_acc, double* split_part, double* tile_cost, bool f32, hipEvent_t stop) {
+  if (tiles <= 0) return launch_nothing(s, stop);
+  const auto kernel = jac ? (f32 ? &k_linearize<true, true> : &k_linearize<true, false>) : &k_linearize<false, false>;
+  launch(s, stop, kernel, tiles, kObsTile, t, vert, vR, lm, loss, tile_begin, obs_rec, lm_acc, split_part, tile_cost);
 }
 void launch_split_sum(hipStream_t s, int32_t n, const int32_t* ids, const int32_t* split_tiles,
                       const double* split_part, double* lm_acc) {
@@ -1910,14 +1921,10 @@ void launch_split_sum(hipStream_t s, int32_t n, const int32_t* ids, const int32_
 }
 void launch_pose_rows(hipStream_t s, const DevTopology& t, const double* vert, const double* vR, const double* lm,
                       const double* obs_rec, const double* lm_acc, double* pose_grad, double* pose_diag,
-                      double* pose_jtj, bool f32) {
-  if (t.Pvar <= 0) return;
-  if (f32)
-    k_pose_rows<true><<<t.Pvar, kRowThreads, 0, s>>>(t, vert, vR, lm, obs_rec, lm_acc, pose_grad, pose_diag,
-                                                     pose_jtj);
-  else
-    k_pose_rows<false><<<t.Pvar, kRowThreads, 0, s>>>(t, vert, vR, lm, obs_rec, lm_acc, pose_grad, pose_diag,
-                                                      pose_jtj);
+                      double* pose_jtj, bool f32, hipEvent_t stop) {
+  if (t.Pvar <= 0) return launch_nothing(s, stop);
+  launch(s, stop, f32 ? &k_pose_rows<true> : &k_pose_rows<false>, t.Pvar, kRowThreads, t, vert, vR, lm, obs_rec,
+         lm_acc, pose_grad, pose_diag, pose_jtj);
 }
 void launch_jacobi_scaling(hipStream_t s, int32_t Pvar, int32_t L, int32_t use, const double* pose_diag,
                            const double* lm_acc, double* pose_scale, double* lm_scale) {
@@ -1926,19 +1933,17 @@ void launch_jacobi_scaling(hipStream_t s, int32_t Pvar, int32_t L, int32_t use, 
 }
 void launch_landmark_prep(hipStream_t s, const DevTopology& t, const double* lm_acc, const double* lm_scale,
                           double inv_mu, double min_diag, double max_diag, double* lm_z, double* lm_anc,
-                          int32_t* fail) {
-  if (t.L > 0)
-    k_landmark_prep<<<(t.L + 255) / 256, 256, 0, s>>>(t, lm_acc, lm_scale, inv_mu, min_diag, max_diag, lm_z, lm_anc,
-                                                      fail);
+                          int32_t* fail, hipEvent_t stop) {
+  if (t.L <= 0) return launch_nothing(s, stop);
+  launch(s, stop, &k_landmark_prep, (t.L + 255) / 256, 256, t, lm_acc, lm_scale, inv_mu, min_diag, max_diag, lm_z,
+         lm_anc, fail);
 }
 void launch_schur_factors(hipStream_t s, const DevTopology& t, int32_t n_g, const int32_t* g_row,
                           const int32_t* g_inc_ptr, const int32_t* g_inc, const double* vR, const double* lm,
-                          const double* obs_rec, double* gf, double* gk, bool f32) {
-  if (t.Pvar <= 0 || n_g <= 0) return;
-  if (f32)
-    k_schur_factors<true><<<(n_g + 255) / 256, 256, 0, s>>>(t, n_g, g_row, g_inc_ptr, g_inc, vR, lm, obs_rec, gf, gk);
-  else
-    k_schur_factors<false><<<(n_g + 255) / 256, 256, 0, s>>>(t, n_g, g_row, g_inc_ptr, g_inc, vR, lm, obs_rec, gf, gk);
+                          const double* obs_rec, double* gf, double* gk, bool f32, hipEvent_t stop) {
+  if (t.Pvar <= 0 || n_g <= 0) return launch_nothing(s, stop);
+  launch(s, stop, f32 ? &k_schur_factors<true> : &k_schur_factors<false>, (n_g + 255) / 256, 256, t, n_g, g_row,
+         g_inc_ptr, g_inc, vR, lm, obs_rec, gf, gk);
 }
 bool schur_items_per_wg_supported(int32_t n) { return n == 1 || n == 2 || n == 4 || n == 8; }
 void launch_schur_tiles(hipStream_t s, const SchurTilesDev& d, const double* gf, const double* gk,
@@ -1955,18 +1960,15 @@ void launch_schur_blocks(hipStream_t s, const DevTopology& t, const SchurTilesDe
                          const double* gf, const double* gk, const double* lm_z, const double* lm_anc,
                          const double* vR, const double* pose_scale, const double* pose_diag, const double* pose_jtj,
                          double inv_mu, double min_diag, double max_diag, double* partial, double* S, double* rhs,
-                         int32_t items_per_wg, int32_t xcd_map) {
-  if (t.Pvar <= 0 || nub <= 0) return;
+                         int32_t items_per_wg, int32_t xcd_map, hipEvent_t stop) {
+  if (t.Pvar <= 0 || nub <= 0) return launch_nothing(s, stop);
   launch_schur_tiles(s, d, gf, gk, lm_z, lm_anc, partial, items_per_wg, xcd_map);
   // kWide from 24 slots a block on: below that its groups have too few slots
   // each to hide their latency behind one another.
-  if (d.n_uslot >= 24 * (int64_t)nub)
-    k_schur_finalize<true><<<nub, 252, 0, s>>>(t, nub, ublk, d.uslot_ptr, d.uslot, partial, vR, pose_scale, pose_diag,
-                                               pose_jtj, inv_mu, min_diag, max_diag, S, rhs);
-  else
-    k_schur_finalize<false><<<(nub + kFinalizeGroups - 1) / kFinalizeGroups, 252, 0, s>>>(
-        t, nub, ublk, d.uslot_ptr, d.uslot, partial, vR, pose_scale, pose_diag, pose_jtj, inv_mu, min_diag, max_diag, S,
-        rhs);
+  const bool wide = d.n_uslot >= 24 * (int64_t)nub;
+  launch(s, stop, wide ? &k_schur_finalize<true> : &k_schur_finalize<false>,
+         wide ? nub : (nub + kFinalizeGroups - 1) / kFinalizeGroups, 252, t, nub, ublk, d.uslot_ptr, d.uslot, partial,
+         vR, pose_scale, pose_diag, pose_jtj, inv_mu, min_diag, max_diag, S, rhs);
 }
 void launch_landmark_quality(hipStream_t s, const DevTopology& t, const double* vert, const double* vR,
                              const double* lm, int32_t min_observers, double min_angle_deg, double max_dist,
@@ -1986,8 +1988,9 @@ void launch_landmark_quality(hipStream_t s, const DevTopology& t, const double* 
     k_landmark_quality<false><<<(t.L + per - 1) / per, 64 * kQualityWaves, 0, s>>>(t, vert, vR, lm, q, good);
 }
 void launch_block_inverse(hipStream_t s, int32_t Pvar, const int32_t* diag_pos, const double* S, double* Minv,
-                          int32_t* fail) {
-  if (Pvar > 0) k_block_inverse<<<(Pvar + 63) / 64, 64, 0, s>>>(Pvar, diag_pos, S, Minv, fail);
+                          int32_t* fail, hipEvent_t stop) {
+  if (Pvar <= 0) return launch_nothing(s, stop);
+  launch(s, stop, &k_block_inverse, (Pvar + 63) / 64, 64, Pvar, diag_pos, S, Minv, fail);
 }
 
 // Part entries: 2 per tile, then 2 per block of 256 split landmarks; returns
@@ -1995,34 +1998,28 @@ void launch_block_inverse(hipStream_t s, int32_t Pvar, const int32_t* diag_pos, 
 int32_t launch_back_substitute(hipStream_t s, const DevTopology& t, int32_t tiles, const int32_t* tile_begin,
                                int32_t n_split, const int32_t* split_ids, const double* vR, const double* lm,
                                const double* obs_rec, const double* lm_acc, const double* lm_z, const double* w,
-                               double* u, double* part, bool f32) {
-  if (tiles > 0) {
-    if (f32)
-      k_back_substitute<true><<<tiles, kObsTile, 0, s>>>(t, tile_begin, vR, lm, obs_rec, lm_acc, lm_z, w, u, part);
-    else
-      k_back_substitute<false><<<tiles, kObsTile, 0, s>>>(t, tile_begin, vR, lm, obs_rec, lm_acc, lm_z, w, u, part);
-  }
+                               double* u, double* part, bool f32, hipEvent_t stop) {
   const int sb = (n_split + 255) / 256;
   double* part_split = part + 2 * (size_t)std::max(tiles, 0);
-  if (sb > 0) {
-    if (f32)
-      k_back_substitute_split<true><<<sb, 256, 0, s>>>(t, n_split, split_ids, vR, lm, obs_rec, lm_acc, lm_z, w, u,
-                                                       part_split);
-    else
-      k_back_substitute_split<false><<<sb, 256, 0, s>>>(t, n_split, split_ids, vR, lm, obs_rec, lm_acc, lm_z, w,
-                                                        u, part_split);
-  }
+  if (tiles <= 0 && sb <= 0) launch_nothing(s, stop);
+  if (tiles > 0)
+    launch(s, sb > 0 ? nullptr : stop, f32 ? &k_back_substitute<true> : &k_back_substitute<false>, tiles, kObsTile, t,
+           tile_begin, vR, lm, obs_rec, lm_acc, lm_z, w, u, part);
+  if (sb > 0)
+    launch(s, stop, f32 ? &k_back_substitute_split<true> : &k_back_substitute_split<false>, sb, 256, t, n_split,
+           split_ids, vR, lm, obs_rec, lm_acc, lm_z, w, u, part_split);
   return std::max(tiles, 0) + sb;
 }
-void launch_unscale_poses(hipStream_t s, int32_t Pvar, const double* y, const double* pose_scale, double* w,
-                          double* part) {
-  if (Pvar > 0) k_unscale_poses<<<(6 * Pvar + 255) / 256, 256, 0, s>>>(Pvar, y, pose_scale, w, part);
+void launch_step_vertices(hipStream_t s, const DevTopology& t, const double* vert, const double* y,
+                          const double* pose_scale, double* w, double* cand_v, double* cand_vR, double* part_w,
+                          double* part_x, hipEvent_t stop) {
+  if (t.P <= 0) return launch_nothing(s, stop);
+  launch(s, stop, &k_step_vertices, (t.P + 255) / 256, 256, t, vert, y, pose_scale, w, cand_v, cand_vR, part_w, part_x);
 }
-void launch_candidate(hipStream_t s, const DevTopology& t, const double* vert, const double* w, double* cand_v,
-                      double* cand_vR, double* part_v, const double* lm, const double* u, double* cand_l,
-                      double* part_l) {
-  if (t.P > 0) k_candidate_vertices<<<(t.P + 255) / 256, 256, 0, s>>>(t, vert, w, cand_v, cand_vR, part_v);
-  if (t.L > 0) k_candidate_landmarks<<<(t.L + 255) / 256, 256, 0, s>>>(t, lm, u, cand_l, part_l);
+void launch_candidate_landmarks(hipStream_t s, const DevTopology& t, const double* lm, const double* u, double* cand_l,
+                                double* part_l, hipEvent_t stop) {
+  if (t.L <= 0) return launch_nothing(s, stop);
+  launch(s, stop, &k_candidate_landmarks, (t.L + 255) / 256, 256, t, lm, u, cand_l, part_l);
 }
 void launch_gradient_norm(hipStream_t s, const DevTopology& t, const double* vert, const double* pose_grad,
                           const double* lm_acc, double* part) {
@@ -2033,9 +2030,9 @@ void launch_reduce(hipStream_t s, int32_t n, int32_t stride, int32_t offset, boo
                    double* out) {
   k_reduce<<<1, 256, 0, s>>>(n, stride, offset, is_max ? 1 : 0, parts, out);
 }
-bool launch_reduce_many(hipStream_t s, const ReduceBatch& batch) {
+bool launch_reduce_many(hipStream_t s, const ReduceBatch& batch, hipEvent_t stop) {
   if (batch.count < 1 || batch.count > kMaxReduceBatch) return false;  // caller reports it; nothing launched
-  k_reduce_many<<<batch.count, 256, 0, s>>>(batch);
+  launch(s, stop, &k_reduce_many, batch.count, 256, batch);
   return true;
 }
 // ------------------------------------------------------------ calibration

@@ -80,12 +80,10 @@ int launch_pcg_deflated(hipStream_t s, const PcgBuffers& B, double tol, int32_t 
                         int32_t poll, const hipEvent_t* probe, int32_t probe_reps);
 
 // Block-Jacobi PCG of a system without a coarse space (K = 0) and few enough
-// vertices for one work-group: one launch, no host poll. The state (its
-// iteration count) is copied to B.state_host on the stream and read with
-// pcg_state_iterations once the stream has passed it.
+// vertices for one work-group: one launch, no host poll. The iteration count
+// goes to iters_out (device).
 bool pcg_small_applies(const PcgBuffers& B);
-bool launch_pcg_small(hipStream_t s, const PcgBuffers& B, double tol, int32_t max_iters);
-int32_t pcg_state_iterations(const void* state_host);
+bool launch_pcg_small(hipStream_t s, const PcgBuffers& B, double tol, int32_t max_iters, double* iters_out);
 
 // Recycling the deflation space after a solve (m Lanczos vectors kept):
 // Rn = Zh' Y (r columns; Y is m x r, row-major, already divided by the

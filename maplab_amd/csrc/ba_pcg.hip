@@ -1011,7 +1011,8 @@ constexpr int kSmallWaves = 16;
 constexpr int kSmallCols = kSmallRows / kSmallWaves;  // two blocks of columns a wave
 constexpr int kSmallRowsPerLane = kSmallRows / 64;
 
-__global__ __launch_bounds__(64 * kSmallWaves) void k_pcg_small(PcgArgs a, double tol, int32_t max_iters) {
+__global__ __launch_bounds__(64 * kSmallWaves) void k_pcg_small(PcgArgs a, double tol, int32_t max_iters,
+                                                                double* __restrict__ iters_out) {
   __shared__ double red[kSmallWaves][kSmallRows];
   __shared__ double ps[kSmallRows], rs[kSmallRows], xs[kSmallRows], Ms[6][kSmallRows];
   __shared__ int16_t pos[32][32];
@@ -1112,11 +1113,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_pcg_small(PcgArgs a, doubl
   }
   if (wave == 0) {
     for (int row = lane; row < n; row += 64) a.x[row] = xs[row];
-    if (lane == 0) {
-      a.st->iters = k;
-      a.st->done = 1;
-      a.st->defl_ok = 0;
-    }
+    if (lane == 0) *iters_out = (double)k;
   }
 }
 
@@ -1275,15 +1272,11 @@ bool pcg_small_applies(const PcgBuffers& B) {
   return B.K == 0 && B.kmat == nullptr && B.Pvar > 0 && B.Pvar <= kSmallVertices;
 }
 
-bool launch_pcg_small(hipStream_t s, const PcgBuffers& B, double tol, int32_t max_iters) {
+bool launch_pcg_small(hipStream_t s, const PcgBuffers& B, double tol, int32_t max_iters, double* iters_out) {
   if (!pcg_small_applies(B)) return false;
-  const PcgArgs a = make_args(B);
-  k_pcg_small<<<1, 64 * kSmallWaves, 0, s>>>(a, tol, max_iters);
-  return hipGetLastError() == hipSuccess &&
-         hipMemcpyAsync(B.state_host, a.st, sizeof(PcgState), hipMemcpyDeviceToHost, s) == hipSuccess;
+  k_pcg_small<<<1, 64 * kSmallWaves, 0, s>>>(make_args(B), tol, max_iters, iters_out);
+  return hipGetLastError() == hipSuccess;
 }
-
-int32_t pcg_state_iterations(const void* state_host) { return static_cast<const PcgState*>(state_host)->iters; }
 
 // Deflated PCG solve of S y = b. The host polls the state after `first`
 // iterations, then every `poll` iterations. With `probe` (three events),

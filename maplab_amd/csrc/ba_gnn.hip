@@ -21,6 +21,7 @@
 #include <cmath>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "ba_learned.h"
@@ -158,13 +159,30 @@ __global__ __launch_bounds__(256) void k_mfma_gemm_tn(int32_t m_pad, int32_t kt,
   }
 }
 
-// out[e] = sum over chunks c (in order) of part[c][e], e < n; scale applied.
-__global__ void k_sum_chunks(int32_t chunks, int32_t n, const float* __restrict__ part, float* __restrict__ out) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n) return;
+// out[e] = sum over chunks of part[c][e], e < n: four threads an entry, thread
+// q adding chunks q, q + 4, ... in order, then the four sums in order. The
+// loads of one thread are independent, but a few dozen chunks added by one
+// thread each kept 17 us of latency in every one of 18 launches (20000 rows).
+constexpr int kSumParts = 4;
+__global__ __launch_bounds__(256) void k_sum_chunks(int32_t chunks, int32_t n, const float* __restrict__ part,
+                                                    float* __restrict__ out) {
+  __shared__ float red[kSumParts][64];
+  const int q = threadIdx.x >> 6, e = blockIdx.x * 64 + (threadIdx.x & 63);
   float s = 0.0f;
-  for (int c = 0; c < chunks; ++c) s += part[(size_t)c * n + e];
-  out[e] = s;
+  if (e < n) {
+    int c = q;
+    for (; c + 7 * kSumParts < chunks; c += 8 * kSumParts) {
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = part[(size_t)(c + k * kSumParts) * n + e];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) s += v[k];
+    }
+    for (; c < chunks; c += kSumParts) s += part[(size_t)c * n + e];
+  }
+  red[q][threadIdx.x & 63] = s;
+  __syncthreads();
+  if (q == 0 && e < n) out[e] = (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
 }
 
 // Column sums of a [rows x cols] matrix (BF16 or FP32) per chunk of 256
@@ -206,19 +224,59 @@ __global__ void k_gnn_degree(GnnGraph g, int32_t* __restrict__ deg) {
   deg[i] = d;
 }
 
-// agg_i = bf16(sum_e g_e y_src / deg_i) into HA[:, 64:128]; one wave per node.
+// Gate of every edge slot of one layer, used by the forward and the backward
+// aggregation (which read it once forwards and once through the reverse slot;
+// the exponential per edge and lane of both cost more than the sums).
+__global__ __launch_bounds__(256) void k_gnn_gates(int32_t slots, const float* __restrict__ ef,
+                                                   const float* __restrict__ a, const float* __restrict__ cg,
+                                                   float* __restrict__ gates) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e < slots) gates[e] = gate(ef, e, a, cg[0]);
+}
+
+// Four BF16 features of a row.
+__device__ inline void load_bf16x4(const uint16_t* __restrict__ p, float* v) {
+  const uint2 w = *reinterpret_cast<const uint2*>(p);
+  v[0] = from_bf16((uint16_t)(w.x & 0xFFFFu));
+  v[1] = from_bf16((uint16_t)(w.x >> 16));
+  v[2] = from_bf16((uint16_t)(w.y & 0xFFFFu));
+  v[3] = from_bf16((uint16_t)(w.y >> 16));
+}
+// Sum of v over the four rows of 16 lanes, in row order; result in every lane.
+__device__ inline float rows_sum(float v, int rl) {
+  float s = __shfl(v, rl);
+  s += __shfl(v, 16 + rl);
+  s += __shfl(v, 32 + rl);
+  return s + __shfl(v, 48 + rl);
+}
+
+// agg_i = bf16(sum_e g_e y_src / deg_i) into HA[:, 64:128]; one wave per node,
+// four edges at a time: each row of 16 lanes takes every fourth edge, a lane
+// four features of it (8-byte loads), and the rows' sums are added at the end.
 __global__ __launch_bounds__(64) void k_gnn_aggregate(GnnGraph g, const int32_t* __restrict__ deg,
-                                                      const uint16_t* __restrict__ y, const float* __restrict__ a,
-                                                      const float* __restrict__ cg, uint16_t* __restrict__ ha) {
-  const int i = blockIdx.x, f = threadIdx.x;
-  const float c = cg[0];
-  float s = 0.0f;
-  for (int e = g.row_ptr[i]; e < g.row_ptr[i + 1]; ++e) {
+                                                      const uint16_t* __restrict__ y, const float* __restrict__ gates,
+                                                      uint16_t* __restrict__ ha) {
+  const int i = blockIdx.x, lane = threadIdx.x, row = lane >> 4, rl = lane & 15;
+  const int e1 = g.row_ptr[i + 1];
+  float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+  for (int e = g.row_ptr[i] + row; e < e1; e += 4) {
     const int j = g.col[e];
     if (j == i) continue;
-    s += gate(g.edge_feat, e, a, c) * from_bf16(y[(size_t)j * kH + f]);
+    float v[4];
+    load_bf16x4(y + (size_t)j * kH + 4 * rl, v);
+    const float ge = gates[e];
+    for (int k = 0; k < 4; ++k) s[k] += ge * v[k];
   }
-  ha[(size_t)i * 2 * kH + kH + f] = to_bf16(deg[i] ? s / (float)deg[i] : 0.0f);
+  const float inv = (float)deg[i];
+  ushort4 out;
+  float r[4];
+  for (int k = 0; k < 4; ++k) r[k] = rows_sum(s[k], rl);
+  out.x = to_bf16(deg[i] ? r[0] / inv : 0.0f);
+  out.y = to_bf16(deg[i] ? r[1] / inv : 0.0f);
+  out.z = to_bf16(deg[i] ? r[2] / inv : 0.0f);
+  out.w = to_bf16(deg[i] ? r[3] / inv : 0.0f);
+  if (row == 0) *reinterpret_cast<ushort4*>(ha + (size_t)i * 2 * kH + kH + 4 * rl) = out;
 }
 
 // theta = h3 W_out + b_out (FP32); one thread per (node, term).
@@ -288,38 +346,56 @@ __global__ void k_gnn_output_wgrad(int32_t nodes, const uint16_t* __restrict__ h
 // Backward of the aggregation of node j (one wave): dy_j = bf16(sum over the
 // edges (dst i, src j) of g / deg_i dagg_i), and per node the partial
 // gradients of the gate parameters over the edges into j:
-// gpart[j] = (d a_g (3), d c_g) with dg_e = <dagg_j, y_src> / deg_j.
+// gpart[j] = (d a_g (3), d c_g) with dg_e = <dagg_j, y_src> / deg_j. Four edges
+// at a time as in k_gnn_aggregate, so that an edge's inner product is a sum
+// over 16 lanes and four of them are formed together.
 __global__ __launch_bounds__(64) void k_gnn_aggregate_back(GnnGraph g, int32_t m_pad, const int32_t* __restrict__ deg,
                                                            const uint16_t* __restrict__ y,
                                                            const float* __restrict__ dha,
-                                                           const float* __restrict__ a, const float* __restrict__ cg,
+                                                           const float* __restrict__ gates,
                                                            uint16_t* __restrict__ dy, float* __restrict__ gpart) {
-  const int j = blockIdx.x, f = threadIdx.x;
+  const int j = blockIdx.x, lane = threadIdx.x, row = lane >> 4, rl = lane & 15;
   if (j >= g.nodes) {
-    if (j < m_pad) dy[(size_t)j * kH + f] = 0;
+    if (j < m_pad) dy[(size_t)j * kH + lane] = 0;
     return;
   }
-  const float c = cg[0];
-  const int degj = deg[j];
-  const float dagg_j = dha[(size_t)j * 2 * kH + kH + f];
-  float s = 0.0f;
+  const float degj = (float)deg[j];
+  const float4 dj = *reinterpret_cast<const float4*>(dha + (size_t)j * 2 * kH + kH + 4 * rl);
+  float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   float ga[kLpEdgeFeatures + 1] = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int e = g.row_ptr[j]; e < g.row_ptr[j + 1]; ++e) {
+  const int e1 = g.row_ptr[j + 1];
+  // Every lane of a row runs the same edges: the row sums stay defined.
+  for (int e = g.row_ptr[j] + row; e < e1; e += 4) {
     const int i = g.col[e];
     if (i == j) continue;
     // Into i from j: the reverse slot, in row i.
-    const int er = g.rev[e];
-    s += gate(g.edge_feat, er, a, c) / (float)deg[i] * dha[(size_t)i * 2 * kH + kH + f];
+    const float w = gates[g.rev[e]] / (float)deg[i];
+    const float4 di = *reinterpret_cast<const float4*>(dha + (size_t)i * 2 * kH + kH + 4 * rl);
+    s[0] += w * di.x;
+    s[1] += w * di.y;
+    s[2] += w * di.z;
+    s[3] += w * di.w;
     // Edge e into j from i: d gate.
-    const float dg = wave_sum_f(dagg_j * from_bf16(y[(size_t)i * kH + f])) / (float)degj;
-    const float ge = gate(g.edge_feat, e, a, c);
+    float v[4];
+    load_bf16x4(y + (size_t)i * kH + 4 * rl, v);
+    const float dg = row_sum_f((dj.x * v[0] + dj.y * v[1]) + (dj.z * v[2] + dj.w * v[3])) / degj;
+    const float ge = gates[e];
     const float ds = dg * ge * (1.0f - ge);
     for (int k = 0; k < kLpEdgeFeatures; ++k) ga[k] += ds * g.edge_feat[(size_t)kLpEdgeFeatures * e + k];
     ga[kLpEdgeFeatures] += ds;
   }
-  dy[(size_t)j * kH + f] = to_bf16(s);
-  if (f < kLpEdgeFeatures + 1) gpart[(size_t)(kLpEdgeFeatures + 1) * j + f] = ga[f];
+  ushort4 out;
+  out.x = to_bf16(rows_sum(s[0], rl));
+  out.y = to_bf16(rows_sum(s[1], rl));
+  out.z = to_bf16(rows_sum(s[2], rl));
+  out.w = to_bf16(rows_sum(s[3], rl));
+  float gs[kLpEdgeFeatures + 1];
+  for (int k = 0; k <= kLpEdgeFeatures; ++k) gs[k] = rows_sum(ga[k], rl);
+  if (row == 0) *reinterpret_cast<ushort4*>(dy + (size_t)j * kH + 4 * rl) = out;
+  if (lane == 0)
+    *reinterpret_cast<float4*>(gpart + (size_t)(kLpEdgeFeatures + 1) * j) = make_float4(gs[0], gs[1], gs[2], gs[3]);
 }
+static_assert(kLpEdgeFeatures == 3 && kH == 64, "k_gnn_aggregate_back packs four gate gradients and 64 features");
 
 // dz = bf16(dh * [h > 0]) for h in HA[:, 0:64], dh in dHA[:, 0:64].
 __global__ void k_gnn_relu_back(int32_t nodes, int32_t m_pad, const uint16_t* __restrict__ ha,
@@ -368,6 +444,18 @@ __global__ void k_gnn_weights(const float* __restrict__ params, Layout L, uint16
   }
 }
 
+// Counts the slots whose column is out of range or whose reverse slot is not
+// the one of the transposed edge; one wave per row (row_ptr is valid).
+__global__ __launch_bounds__(64) void k_gnn_check(GnnGraph g, int32_t* __restrict__ bad) {
+  const int i = blockIdx.x;
+  int n = 0;
+  for (int e = g.row_ptr[i] + (int)threadIdx.x; e < g.row_ptr[i + 1]; e += 64) {
+    const int j = g.col[e], r = g.rev[e];
+    if (j < 0 || j >= g.nodes || r < 0 || r >= g.slots || g.col[r] != i || r < g.row_ptr[j] || r >= g.row_ptr[j + 1]) ++n;
+  }
+  if (n) atomicAdd(bad, n);
+}
+
 __global__ void k_adam(int32_t n, float lr, float c1, float c2, const float* __restrict__ g, float* __restrict__ p,
                        float* __restrict__ m, float* __restrict__ v) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -404,19 +492,41 @@ class GnnWorkspace {
   float* gpart = nullptr;          // m_pad x 4
   float* part = nullptr;           // chunks x 128 x 64
   int32_t* deg = nullptr;          // m_pad: edges into each node
-  std::vector<void*> allocs;
-  bool ok = true;
+  float* gates = nullptr;          // 3 x slots: edge gates of each layer
+  void* base = nullptr;            // one allocation, cleared, that everything above lies in
 
-  template <typename T>
-  T* get(size_t n) {
-    void* p = nullptr;
-    if (hipMalloc(&p, std::max<size_t>(n, 1) * sizeof(T)) != hipSuccess) { ok = false; return nullptr; }
-    (void)hipMemset(p, 0, std::max<size_t>(n, 1) * sizeof(T));
-    allocs.push_back(p);
-    return static_cast<T*>(p);
+  // Places every buffer from `at` on (256-byte aligned) and returns the end.
+  size_t place(char* at) {
+    const size_t M = m_pad;
+    size_t used = 0;
+    auto put = [&](auto& p, size_t n) {
+      p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(at ? at + used : nullptr);
+      used += (std::max<size_t>(n, 1) * sizeof(*p) + 255) & ~(size_t)255;
+    };
+    for (int l = 0; l < kGnnLayers; ++l) {
+      put(ha[l], M * 2 * kH);
+      put(y[l], M * kH);
+    }
+    put(h3, M * kH);
+    put(deg, M);
+    put(wm, kGnnLayers * kH * kH);
+    put(wu, kGnnLayers * 2 * kH * kH);
+    put(wmt, kGnnLayers * kH * kH);
+    put(wut, kGnnLayers * 2 * kH * kH);
+    put(gates, kGnnLayers * (size_t)slots);
+    if (training) {
+      put(dtheta, M * kLpTerms);
+      put(lpart, M);
+      put(dz, M * kH);
+      put(dy, M * kH);
+      put(dha, M * 2 * kH);
+      put(gpart, M * (kLpEdgeFeatures + 1));
+      put(part, (M / kChunk + 1) * 2 * kH * kH);
+    }
+    return used;
   }
   ~GnnWorkspace() {
-    for (void* p : allocs) (void)hipFree(p);
+    if (base) (void)hipFree(base);
   }
 };
 
@@ -426,27 +536,14 @@ GnnWorkspace* gnn_workspace_create(int32_t nodes, int32_t slots, bool for_traini
   w->slots = slots;
   w->m_pad = std::max(128, ((nodes + 127) / 128) * 128);
   w->training = for_training;
-  const size_t M = w->m_pad;
-  for (int l = 0; l < kGnnLayers; ++l) {
-    w->ha[l] = w->get<uint16_t>(M * 2 * kH);
-    w->y[l] = w->get<uint16_t>(M * kH);
+  const size_t bytes = w->place(nullptr);
+  if (hipMalloc(&w->base, bytes) != hipSuccess) {
+    w->base = nullptr;
+    delete w;
+    return nullptr;
   }
-  w->h3 = w->get<uint16_t>(M * kH);
-  w->deg = w->get<int32_t>(M);
-  w->wm = w->get<uint16_t>(kGnnLayers * kH * kH);
-  w->wu = w->get<uint16_t>(kGnnLayers * 2 * kH * kH);
-  w->wmt = w->get<uint16_t>(kGnnLayers * kH * kH);
-  w->wut = w->get<uint16_t>(kGnnLayers * 2 * kH * kH);
-  if (for_training) {
-    w->dtheta = w->get<float>(M * kLpTerms);
-    w->lpart = w->get<float>(M);
-    w->dz = w->get<uint16_t>(M * kH);
-    w->dy = w->get<uint16_t>(M * kH);
-    w->dha = w->get<float>(M * 2 * kH);
-    w->gpart = w->get<float>(M * (kLpEdgeFeatures + 1));
-    w->part = w->get<float>((M / kChunk + 1) * 2 * kH * kH);
-  }
-  if (!w->ok) { delete w; return nullptr; }
+  (void)hipMemset(w->base, 0, bytes);
+  (void)w->place(static_cast<char*>(w->base));
   return w;
 }
 
@@ -472,7 +569,7 @@ void gemm_tn(hipStream_t s, GnnWorkspace* w, int kt, int nt, const uint16_t* A, 
   const int chunks = (w->m_pad + kChunk - 1) / kChunk;
   k_mfma_gemm_tn<<<chunks, 256, 0, s>>>(w->m_pad, kt, nt, A, lda, B, ldb, w->part);
   const int n = 32 * kt * 32 * nt;
-  k_sum_chunks<<<(n + 255) / 256, 256, 0, s>>>(chunks, n, w->part, out);
+  k_sum_chunks<<<(n + 63) / 64, 256, 0, s>>>(chunks, n, w->part, out);
 }
 
 void col_sums(hipStream_t s, GnnWorkspace* w, int rows, int cols, const uint16_t* a16, const float* a32, int lda,
@@ -480,13 +577,13 @@ void col_sums(hipStream_t s, GnnWorkspace* w, int rows, int cols, const uint16_t
   const int chunks = (rows + kChunk - 1) / kChunk;
   if (chunks <= 0) { (void)hipMemsetAsync(out, 0, cols * sizeof(float), s); return; }
   k_col_partials<<<chunks, 128, 0, s>>>(rows, cols, a16, a32, lda, w->part);
-  k_sum_chunks<<<(cols + 255) / 256, 256, 0, s>>>(chunks, cols, w->part, out);
+  k_sum_chunks<<<(cols + 63) / 64, 256, 0, s>>>(chunks, cols, w->part, out);
 }
 
 }  // namespace
 
 bool gnn_forward(hipStream_t s, GnnWorkspace* w, const GnnGraph& g, const float* params, float* theta) {
-  if (!w || g.nodes != w->nodes) return false;
+  if (!w || g.nodes != w->nodes || g.slots != w->slots) return false;
   if (g.nodes == 0) return true;
   const Layout L = layout();
   k_gnn_weights<<<dim3((2 * kH * kH + 255) / 256, kGnnLayers), 256, 0, s>>>(params, L, w->wm, w->wu, w->wmt, w->wut);
@@ -495,7 +592,11 @@ bool gnn_forward(hipStream_t s, GnnWorkspace* w, const GnnGraph& g, const float*
   for (int l = 0; l < kGnnLayers; ++l) {
     gemm(s, w, kH, 2, w->ha[l], 2 * kH, w->wm + (size_t)l * kH * kH, params + L.b_m[l], false, w->y[l], nullptr, kH,
          0, false);
-    k_gnn_aggregate<<<g.nodes, kH, 0, s>>>(g, w->deg, w->y[l], params + L.a_g[l], params + L.c_g[l], w->ha[l]);
+    float* gates = w->gates + (size_t)l * w->slots;
+    if (g.slots > 0)
+      k_gnn_gates<<<(g.slots + 255) / 256, 256, 0, s>>>(g.slots, g.edge_feat, params + L.a_g[l], params + L.c_g[l],
+                                                        gates);
+    k_gnn_aggregate<<<g.nodes, kH, 0, s>>>(g, w->deg, w->y[l], gates, w->ha[l]);
     uint16_t* out = (l + 1 < kGnnLayers) ? w->ha[l + 1] : w->h3;
     const int ldo = (l + 1 < kGnnLayers) ? 2 * kH : kH;
     gemm(s, w, 2 * kH, 2, w->ha[l], 2 * kH, w->wu + (size_t)l * 2 * kH * kH, params + L.b_u[l], true, out, nullptr,
@@ -508,7 +609,7 @@ bool gnn_forward(hipStream_t s, GnnWorkspace* w, const GnnGraph& g, const float*
 
 bool gnn_loss_backward(hipStream_t s, GnnWorkspace* w, const GnnGraph& g, const float* params, const float* theta,
                        const float* qc, float inv_count, float* loss_out, float* grad) {
-  if (!w || !w->training || g.nodes != w->nodes) return false;
+  if (!w || !w->training || g.nodes != w->nodes || g.slots != w->slots) return false;
   const Layout L = layout();
   const int nodes = g.nodes, M = w->m_pad;
   if (hipMemsetAsync(grad, 0, kGnnParams * sizeof(float), s) != hipSuccess) return false;
@@ -520,7 +621,7 @@ bool gnn_loss_backward(hipStream_t s, GnnWorkspace* w, const GnnGraph& g, const 
     const int chunks = (nodes + kChunk - 1) / kChunk;
     const int n = kH * kLpTerms + kLpTerms;
     k_gnn_output_wgrad<<<chunks, 192, 0, s>>>(nodes, w->h3, w->dtheta, w->part);
-    k_sum_chunks<<<(n + 255) / 256, 256, 0, s>>>(chunks, n, w->part, grad + L.w_out);  // W_out then b_out
+    k_sum_chunks<<<(n + 63) / 64, 256, 0, s>>>(chunks, n, w->part, grad + L.w_out);  // W_out then b_out
   }
   k_gnn_output_back<<<M, kH, 0, s>>>(nodes, M, w->dtheta, params + L.w_out, w->h3, w->dz);
   for (int l = kGnnLayers - 1; l >= 0; --l) {
@@ -530,7 +631,7 @@ bool gnn_loss_backward(hipStream_t s, GnnWorkspace* w, const GnnGraph& g, const 
     // dHA = dz W_u' (FP32, 128 columns).
     gemm(s, w, kH, 4, w->dz, kH, w->wut + (size_t)l * 2 * kH * kH, nullptr, false, nullptr, w->dha, 2 * kH, 0, false);
     // Aggregation: dy and the gate parameter gradients.
-    k_gnn_aggregate_back<<<M, kH, 0, s>>>(g, M, w->deg, w->y[l], w->dha, params + L.a_g[l], params + L.c_g[l], w->dy,
+    k_gnn_aggregate_back<<<M, kH, 0, s>>>(g, M, w->deg, w->y[l], w->dha, w->gates + (size_t)l * w->slots, w->dy,
                                           w->gpart);
     col_sums(s, w, nodes, kLpEdgeFeatures + 1, nullptr, w->gpart, kLpEdgeFeatures + 1, grad + L.a_g[l]);  // a_g, c_g
     // y = h_{l-1} W_m + b_m: dW_m = h_{l-1}' dy, db_m = sum dy, dh_{l-1} += dy W_m'.
@@ -544,7 +645,7 @@ bool gnn_loss_backward(hipStream_t s, GnnWorkspace* w, const GnnGraph& g, const 
     const int chunks = (nodes + kChunk - 1) / kChunk;
     const int n = (kLpNodeFeatures + 1) * kH;
     k_gnn_input_back<<<chunks, kH, 0, s>>>(nodes, g.node_feat, w->ha[0], w->dha, w->part);
-    k_sum_chunks<<<(n + 255) / 256, 256, 0, s>>>(chunks, n, w->part, grad + L.w_in);  // W_in then b_in
+    k_sum_chunks<<<(n + 63) / 64, 256, 0, s>>>(chunks, n, w->part, grad + L.w_in);  // W_in then b_in
   }
   return hipGetLastError() == hipSuccess;
 }
@@ -601,12 +702,6 @@ struct DeviceDataset {
     double cnt = 0.0;
     for (int i = 0; i < d->nodes; ++i) {
       if (d->row_ptr[i + 1] < d->row_ptr[i]) return gnn_fail(MLBA_EINVAL, "dataset: row_ptr not monotone");
-      for (int e = d->row_ptr[i]; e < d->row_ptr[i + 1]; ++e) {
-        const int j = d->col[e], r = d->rev[e];
-        if (j < 0 || j >= d->nodes || r < 0 || r >= d->slots || d->col[r] != i || r < d->row_ptr[j] ||
-            r >= d->row_ptr[j + 1])
-          return gnn_fail(MLBA_EINVAL, "dataset: col / rev out of range or not the reverse slot");
-      }
       cnt += d->qc[5 * (size_t)i + 4] != 0.0f;
     }
     inv_count = cnt > 0 ? (float)(1.0 / cnt) : 0.0f;
@@ -620,6 +715,14 @@ struct DeviceDataset {
     qc = put(d->qc, (size_t)d->nodes * 5);
     if (!g.row_ptr || !g.col || !g.rev || !g.node_feat || !g.edge_feat || !qc)
       return gnn_fail(MLBA_ENOMEM, "dataset: device allocation failed");
+    // Nothing else reads col and rev before this has passed them.
+    int32_t* bad = put<int32_t>(nullptr, 1);
+    int32_t n_bad = 0;
+    if (!bad) return gnn_fail(MLBA_ENOMEM, "dataset: device allocation failed");
+    if (d->nodes > 0) mlba::k_gnn_check<<<d->nodes, 64, 0, nullptr>>>(g, bad);
+    if (hipMemcpy(&n_bad, bad, sizeof(n_bad), hipMemcpyDeviceToHost) != hipSuccess)
+      return gnn_fail(MLBA_EDEVICE, "dataset: check failed");
+    if (n_bad) return gnn_fail(MLBA_EINVAL, "dataset: col / rev out of range or not the reverse slot");
     return MLBA_OK;
   }
 };

@@ -72,6 +72,14 @@ __device__ inline float wave_sum_f(float v) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
+// The same within each row of 16 lanes; result in all 16.
+__device__ inline float row_sum_f(float v) {
+  v += dpp_move_f<0xB1>(v, 0.0f);
+  v += dpp_move_f<0x4E>(v, 0.0f);
+  v += dpp_move_f<0x141>(v, 0.0f);
+  return v + dpp_move_f<0x140>(v, 0.0f);
+}
+
 // Block-wide sum of one value for a 256-thread block; result valid in thread 0.
 __device__ inline double block_sum256(double v, double* lds4) {
   v = wave_sum(v);

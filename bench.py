@@ -97,7 +97,7 @@ def kernel_table(sm, kt, n_pcg_total):
             "launches": int(launches), "total_ms": round(sm.kernel_ms[abi.KERNEL_PCG], 4),
             "avg_ms": round(sm.kernel_ms[abi.KERNEL_PCG] / launches, 5), "pcg_iterations": int(n_pcg_total),
             "per_iteration_ms": round(it_ms, 5),
-            "note": "events around each whole solve: coarse-space set-up, both kernels of every iteration, "
+            "note": "events around each whole solve: coarse-space set-up, the kernels of every iteration, "
                     "launch gaps and the host convergence polls"}
     if kt.pcg_spmv_ms > 0 and n_pcg_total > 0:
         timing = ("mlba_time_kernels: events around a batch of back-to-back launches on the library stream "
@@ -106,7 +106,10 @@ def kernel_table(sm, kt, n_pcg_total):
         groups = (P + 41) // 42
         spmv_b = nnzb * 292 + P * 200 + P * 6 * gw * 8
         upd_b = P * 344 + P * 288 + P * 6 * gw * 8 + groups * gw * ne * 8 + groups * (3 + ne) * 8
-        for name, ms, b in (("k_pcg_spmv", kt.pcg_spmv_ms, spmv_b), ("k_pcg_update", kt.pcg_update_ms, upd_b)):
+        # One launch per iteration up to 2048 vertices, two above.
+        step_b = nnzb * 292 + P * (2 * 144 + 288 + 288) + P * 6 * gw * 8 + ne * ne * 8
+        two = (("k_pcg_spmv", kt.pcg_spmv_ms, spmv_b), ("k_pcg_update", kt.pcg_update_ms, upd_b))
+        for name, ms, b in two if kt.pcg_update_ms > 0 else (("k_pcg_step", kt.pcg_spmv_ms, step_b),):
             rows[name] = row_of(n_pcg_total, ms * n_pcg_total, b)
             rows[name]["timing"] = timing
     return rows
@@ -117,7 +120,7 @@ TRAFFIC_PROFILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "prof
 # Bench kernel row -> the kernel whose rocprofv3 FETCH_SIZE / WRITE_SIZE row
 # gives its HBM traffic (the Schur block build is dominated by its tile pass).
 TRAFFIC_KERNEL = {"k_schur_blocks": "mlba::k_schur_tiles", "k_pcg_spmv": "mlba::k_pcg_spmv<false>",
-                  "k_pcg_update": "mlba::k_pcg_update",
+                  "k_pcg_update": "mlba::k_pcg_update", "k_pcg_step": "mlba::k_pcg_step",
                   "k_schur_factors": "mlba::k_schur_factors<false>", "k_linearize": "mlba::k_linearize<true, false>",
                   "k_back_substitute": "mlba::k_back_substitute<false>"}
 

@@ -219,7 +219,7 @@ struct mlba_handle {
   DBuf<int32_t> hat_node, node_range, grp_lo, blk_hat, blk_rng;
   std::vector<int32_t> h_row_ptr, h_col_var;  // host copy of the S block structure
   int32_t grp_width = 0;                // hat columns of the per-group SW window
-  DBuf<double> hat_w, blk_w, defl_SR, defl_E, defl_Einv, defl_y, defl_cden, pcg_part2;
+  DBuf<double> hat_w, blk_w, defl_SR, defl_E, defl_Einv, defl_y, defl_cden, pcg_part2, pcg_step;
   int32_t hat_K = -1;  // coarse nodes of the current hat basis
   // Iterations of the last solve without and with recycled columns: the
   // length of the next such solve's first batch.
@@ -731,7 +731,7 @@ int ensure_coarse_basis(mlba_handle* h, int32_t requested) {
   if (!h->defl_SR.alloc(groups * gw * (size_t)(6 * gr)) ||
       !h->defl_E.alloc(std::max<size_t>(ne * ne, 1)) || !h->defl_Einv.alloc(std::max<size_t>(ne * ne + groups * gw * ne, 1)) ||
       !h->defl_y.alloc(std::max<size_t>(ne, 1)) || !h->defl_cden.alloc(std::max<size_t>(nr, 1)) ||
-      !h->pcg_part2.alloc((groups + 1) * (3 + ne)))
+      !h->pcg_part2.alloc((groups + 1) * (3 + ne)) || !h->pcg_step.alloc(std::max<size_t>(pcg_step_doubles(Pvar), 1)))
     return set_err(h, MLBA_ENOMEM, "device allocation failed");
   if (nr > 0) {
     const size_t n6 = 6 * (size_t)Pvar, zc = (size_t)pcg_max_lanczos();
@@ -779,7 +779,7 @@ PcgBuffers pcg_buffers(mlba_handle* h, int32_t nr, bool keep_lanczos) {
   B.blk_hat = h->blk_hat.p; B.blk_w = h->blk_w.p; B.blk_rng = h->blk_rng.p;
   B.SR = h->defl_SR.p; B.E = h->defl_E.p; B.Einv = h->defl_Einv.p; B.y = h->defl_y.p; B.cden = h->defl_cden.p;
   B.x = h->px.p; B.r = h->pr.p; B.z = h->pz.p; B.p0 = h->pp.p; B.p1 = h->pp2.p; B.q = h->pq.p;
-  B.part = h->pcg_part.p; B.part2 = h->pcg_part2.p; B.Zh = h->ritz_Zh.p; B.coef = h->ritz_coef.p;
+  B.part = h->pcg_part.p; B.part2 = h->pcg_part2.p; B.step = h->pcg_step.p; B.Zh = h->ritz_Zh.p; B.coef = h->ritz_coef.p;
   B.state_dev = h->pcg_state.p; B.state_host = h->pcg_host;
   return B;
 }
@@ -2620,8 +2620,9 @@ int32_t mlba_time_kernels(mlba_handle* h, const mlba_options* o, int32_t repeats
                                   o->pcg_relative_tolerance, o->pcg_max_iterations, kPcgPoll, kPcgPoll, nullptr, 0);
     });
     t->pcg_iterations = iters;
-    // One more iteration: each of its two kernels launched repeats x 8 times
-    // back to back between events (launch gaps included), averaged.
+    // One more iteration: each of its kernels (one: pcg_spmv, or two) launched
+    // repeats x 8 times back to back between events (launch gaps included),
+    // averaged.
     hipEvent_t pe[3];
     for (auto& e : pe) HIP_OK(hipEventCreate(&e));
     const int reps = std::max(1, repeats) * 8;
@@ -2635,7 +2636,7 @@ int32_t mlba_time_kernels(mlba_handle* h, const mlba_options* o, int32_t repeats
       HIP_OK(hipEventElapsedTime(&a, pe[0], pe[1]));
       HIP_OK(hipEventElapsedTime(&b, pe[1], pe[2]));
       t->pcg_spmv_ms = a / reps;
-      t->pcg_update_ms = b / reps;
+      t->pcg_update_ms = pcg_step_doubles(h->Pvar) ? 0.0 : b / reps;
     }
     for (auto& e : pe) (void)hipEventDestroy(e);
     const int32_t nr_used = h->hat_K > 0 && ritz_count(o) > 0 ? h->ritz_nr : 0;

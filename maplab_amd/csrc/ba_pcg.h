@@ -18,7 +18,7 @@ namespace mlba {
 struct PcgBuffers {
   int32_t Pvar, K, nr, gwh;
   int32_t zcap;                // Lanczos vectors kept (iterations), 0: none
-  int32_t partials;            // sum of the group partials: 0 automatic, 1 per SpMV work-group, 2 once
+  int32_t partials;            // two-launch iterations, sum of the group partials: 0 automatic, 1 per SpMV work-group, 2 once
   const int32_t* row_ptr;      // block rows of S
   const int32_t* col_var;
   const double* S;
@@ -45,6 +45,7 @@ struct PcgBuffers {
   double* q;
   double* part;                // Pvar
   double* part2;               // (groups + 1) x (3 + ne): per-group partials, then their sum
+  double* step;                // pcg_step_doubles(Pvar): state of one-launch iterations
   double* Zh;                  // zcap x 6 Pvar: deflated preconditioned residual of iteration k
   double* coef;                // 2 zcap: r'z and alpha of iteration k
   void* state_dev;             // pcg_state_bytes()
@@ -60,6 +61,8 @@ struct PcgBuffers {
 };
 
 size_t pcg_state_bytes();
+// Room for the iterations of one launch each (0: they don't apply).
+size_t pcg_step_doubles(int32_t Pvar);
 int32_t pcg_max_hat_nodes();
 // Recycled dense columns of the deflation space, at most.
 constexpr int kPcgMaxRitz = 16;
@@ -71,9 +74,10 @@ int32_t pcg_update_groups(int32_t Pvar);
 bool pcg_deflation_applied(const void* state_host);
 
 // Deflated PCG solve. The host polls the state after `first` iterations, then
-// every `poll` iterations. With `probe` (three events), k_pcg_spmv and then
-// k_pcg_update of one more iteration are each launched `probe_reps` times
-// back to back after the solve and timed as two batches (block-Jacobi only).
+// every `poll` iterations. With `probe` (three events), the kernels of one more
+// iteration are each launched `probe_reps` times back to back after the solve
+// and timed as two batches (block-Jacobi only; the second is empty where an
+// iteration is one launch).
 // Returns the iteration count (max_iters: not converged) or -1 on a launch
 // error or an unsupported combination.
 int launch_pcg_deflated(hipStream_t s, const PcgBuffers& B, double tol, int32_t max_iters, int32_t first,

@@ -23,8 +23,10 @@
 // is a set of coalesced column dot products.
 //
 // Per LM step: k_defl_sr (SW), k_defl_e and k_defl_dense (E, R'b),
-// k_defl_prep (state, E^-1 by Gauss-Jordan, y = E^-1 W'b), k_defl_init (x0,
-// r0, z0 and the first per-group partials). Per PCG iteration: k_pcg_spmv (sums the previous
+// k_defl_prep (state, E^-1 by Gauss-Jordan, y = E^-1 W'b). Up to 2048 vertices
+// with block-Jacobi k_pcg_start and one launch per iteration, k_pcg_step,
+// follow; otherwise k_defl_init (x0, r0, z0 and the first per-group partials)
+// and two launches per iteration: k_pcg_spmv (sums the previous
 // per-group partials; p = z - W mu + beta p_prev and
 // q = S z + beta S p_prev - (SW) mu) and k_pcg_update (x, r, z and the
 // per-group partials r'z, r'r, E^-1 (SW)'z). Every sum of partials runs in
@@ -109,6 +111,13 @@ struct PcgArgs {
   double* Zh;                  // zcap x 6 Pvar: deflated preconditioned residuals
   double* coef;                // 2 zcap: r'z and alpha per iteration
   PcgState* st;
+  // k_pcg_step: what other rows read is kept twice, iteration k reads copy
+  // k & 1 and writes the other.
+  int32_t wgs, step_G;         // work-groups of k_pcg_step, rows of each
+  double* zvp;                 // 2 x Pvar x 18: z, v = M S p and p of each row
+  double* cvec;                // 2 x kMaxCoarse: (SW)'z
+  double* spart;               // 2 x wgs x (kStepScalars + ne) partials
+  double* zpart;               // wgs x ne: the work-groups' (SW)'z
   const double* linv;          // learned preconditioner (with kmat): L_i^-1, 36 Pvar
   const float* kmat;           // K_ij, 36 nnzb
   const int32_t* diag_pos;
@@ -1117,6 +1126,447 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_pcg_small(PcgArgs a, doubl
   }
 }
 
+// ------------------------------------------------------------ block-Jacobi step
+
+// One PCG iteration in one launch. A launch that reads what the one before it
+// wrote costs several us here whatever it computes (launch, then dependent
+// rounds of global loads), and an iteration as a product and an update was
+// two of them. CG needs a global sum for alpha = r'z / p's (s = S p) and a
+// second one after it, r'z and the deflation's c = (SW)'z of the new z. The
+// second follows from the first by linearity: with v = M s formed at the end
+// of an iteration,
+//   r+ = r - alpha s, z+ = z - alpha v,
+//   r+'z+ = r'z - 2 alpha s'z + alpha^2 s'v,   r+'r+ alike,   c+ = c - alpha (SW)'v,
+// so one launch sums all of these and the next one starts from them: each row
+// takes r+, its own z+ = M r+ (formed anew, so that the recurrences for the
+// scalars run over one iteration only), mu = E^-1 c+ of its window, and the
+// product of its row with z+ = z - alpha v and p as three sums that do not
+// wait for alpha. c is carried over at most kStepRefresh iterations and then
+// summed anew from z: carried through the whole solve, its rounding error stays
+// at 1e-16 of the first c while r falls, and the residual stagnates at 1e-11.
+//
+// A work-group of 1024 threads takes G rows, so that at most 256 work-groups
+// (one a CU) publish the partials that every work-group sums. Component t % 6
+// of every kBlocks-th block of a row is thread t's; with one row a work-group
+// three quarters of the waves have no product and sum the partials meanwhile.
+// A work-group reads about 0.4 MB (its rows of S, E^-1 and 256 x 113 partials),
+// and the kernel is bound by that behind four dependent rounds of loads: more
+// rows with fewer work-groups (500 keyframes: 125 work-groups 18.8 us, 250
+// 15.5 us) and the partials summed once by the work-group that ends last
+// (24 us) are slower. Sums run in a fixed order.
+//
+// An iteration, two launches -> one (MI355X, 15-node space and 16 dense
+// columns from 250 keyframes): 60 keyframes 14.7 -> 7.9 us, 250 19.6 -> 13.4,
+// 500 21.3 -> 15.5, 1000 26.7 -> 21.5, 2000 39.0 -> 30.8. At 5000 (work-groups
+// of 16 rows) 68 -> 91: the product is the larger part there, and three vectors
+// gathered cost it more than the launch; the line is drawn at 2048 vertices.
+constexpr int kStepScalars = 7;  // p's, r'z, s'z, s'v, r'r, r's, s's (k_pcg_start: r'z, r'r, b'b in 1, 4, 5)
+constexpr int kStepStride = kStepScalars + kMaxCoarse;
+constexpr int kStepThreads = 1024;
+constexpr int kStepFlight = 16;  // a thread's partials in flight
+constexpr int kStepVertices = 2048;
+constexpr int kStepRefresh = 8;  // every launch k with k % 8 = 0 sums (SW)'z as well
+static_assert(kStepStride <= 128, "128 threads hold the partials of one work-group");
+
+int32_t step_rows(int32_t Pvar) {
+  return Pvar <= 256 ? 1 : (Pvar <= 512 ? 2 : (Pvar <= 1024 ? 4 : 8));
+}
+int32_t step_wgs(int32_t Pvar) { return (Pvar + step_rows(Pvar) - 1) / step_rows(Pvar); }
+
+template <int G>
+struct StepShape {
+  static constexpr int kProduct = G == 1 ? 256 : kStepThreads;  // threads of the products
+  static constexpr int kT = kProduct / G;                       // threads of a row
+  static constexpr int kBlocks = (kT < 256 ? kT : 256) / 6;     // blocks of a row at once
+  static constexpr int kFirst = kProduct < kStepThreads ? kProduct : 0;  // first thread of the sums
+  static constexpr int kSlices = (kStepThreads - kFirst) / 128;
+  static constexpr int kCols = (kMaxCoarse + kBlocks - 1) / kBlocks;
+  static constexpr int kRitz = (kMaxRitz + kBlocks - 1) / kBlocks;
+};
+
+// Slice sl (the same in a wave) of entry t of the sum of wgs work-groups' partials.
+template <int kSlices>
+__device__ inline double step_slice(const double* part, int wgs, int stride, int t, int sl) {
+  double acc = 0.0;
+  if (t >= stride) return acc;
+  // The loads of a pass differ by a uniform number of bytes.
+  const uint32_t own = 8u * (uint32_t)t;
+  for (int w0 = sl; w0 < wgs; w0 += kStepFlight * kSlices) {
+    double v[kStepFlight];
+#pragma unroll
+    for (int m = 0; m < kStepFlight; ++m) {
+      const int w = w0 + m * kSlices;
+      const char* row = reinterpret_cast<const char*>(part + (size_t)min(w, wgs - 1) * stride);
+      v[m] = *reinterpret_cast<const double*>(row + own);
+      if (w >= wgs) v[m] = 0.0;
+    }
+#pragma unroll
+    for (int m = 0; m < kStepFlight; ++m) acc += v[m];
+  }
+  return acc;
+}
+
+// Coarse column e of the sum over a work-group's rows of the window products
+// tmp[row][window column][component].
+template <int G>
+__device__ inline double step_column(const PcgArgs& a, int i0, int e, const double (*tmp)[kMaxCoarse][6]) {
+  double s = 0.0;
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    if (i0 + g < a.Pvar) {
+      const int lc = e >= a.neh ? a.gwh + (e - a.neh) : e - 6 * a.grp_lo[(i0 + g) / kRowsPerGroup];
+      if (lc >= 0 && lc < a.gw && (e >= a.neh || lc < a.gwh)) {
+        const double* t = tmp[g][lc];
+        s += ((t[0] + t[1]) + (t[2] + t[3])) + (t[4] + t[5]);
+      }
+    }
+  }
+  return s;
+}
+
+// Publishes a work-group's partials: the scalars over its rows' entries
+// (sc[e]) and the coarse columns of tmp.
+template <int G>
+__device__ inline void step_publish(const PcgArgs& a, int i0, const double (*sc)[kStepScalars],
+                                    const double (*tmp)[kMaxCoarse][6], double* part) {
+  const int tid = threadIdx.x, stride = kStepScalars + a.ne;
+  double* out = part + (size_t)blockIdx.x * stride;
+  if (tid < kStepScalars) {
+    double s = 0.0;
+#pragma unroll
+    for (int e = 0; e < 6 * G; ++e) s += sc[e][tid];
+    out[tid] = s;
+  } else if (tid < stride) {
+    out[tid] = step_column<G>(a, i0, tid - kStepScalars, tmp);
+  }
+}
+
+// x0 = W y, r0 = b - (SW) y, z0 = M r0, p = v = s = 0 and the first partials.
+template <int G>
+__global__ __launch_bounds__(kStepThreads) void k_pcg_start(PcgArgs a) {
+  using Sh = StepShape<G>;
+  __shared__ double sc[6 * G][kStepScalars];
+  __shared__ double tmp[G][kMaxCoarse][6];
+  __shared__ double ys[kMaxCoarse], rows[G][6], red[G][Sh::kBlocks][6];
+  const int tid = threadIdx.x, i0 = blockIdx.x * G, ne = a.ne;
+  const int g = min(tid / Sh::kT, G - 1), t = tid - g * Sh::kT, comp = t % 6, bs = t / 6, i = i0 + g;
+  const bool row_ok = i < a.Pvar, lane_in = t < 6 * Sh::kBlocks, lane_ok = row_ok && lane_in;
+  const int gi = row_ok ? i / kRowsPerGroup : 0, c0 = ne ? 6 * a.grp_lo[gi] : 0;
+  for (int c = tid; c < ne; c += kStepThreads) ys[c] = a.y[c];
+  double sw[Sh::kCols] = {};
+  if (ne && lane_ok) {
+#pragma unroll
+    for (int m = 0; m < Sh::kCols; ++m) {
+      const int lc = bs + Sh::kBlocks * m;
+      if (lc < a.gw) sw[m] = sr_col(a, gi, lc)[6 * (i - gi * kRowsPerGroup) + comp];
+    }
+  }
+  __syncthreads();
+  if (lane_in) {
+    double sy = 0.0;
+    if (ne) {
+#pragma unroll
+      for (int m = 0; m < Sh::kCols; ++m) {
+        const int lc = bs + Sh::kBlocks * m, gc = lc < a.gw ? win_col(a, c0, lc) : -1;
+        if (gc >= 0) sy += sw[m] * ys[gc];
+      }
+    }
+    red[g][bs][comp] = sy;
+  }
+  __syncthreads();
+  if (t < 6) {
+    double rv = 0.0, bv = 0.0, zv = 0.0, M[6];
+    const int e = 6 * i + comp;
+    if (row_ok) {
+      double xv = 0.0, s = 0.0;
+      bv = a.b[e];
+      for (int k = 0; k < Sh::kBlocks; ++k) s += red[g][k][comp];
+      if (ne) {
+        const int n0 = a.hat_node[i];
+        const double w0 = a.hat_w[2 * i], w1 = a.hat_w[2 * i + 1];
+        xv = w0 * ys[6 * n0 + comp] + (w1 != 0.0 ? w1 * ys[6 * (n0 + 1) + comp] : 0.0);
+        for (int c = 0; c < a.nr; ++c) xv += a.R[(size_t)c * a.n6 + e] * ys[a.neh + c];
+      }
+      rv = bv - s;
+      a.x[e] = xv;
+      a.r[e] = rv;
+      a.q[e] = 0.0;
+    }
+#pragma unroll
+    for (int c = 0; c < 6; ++c) M[c] = row_ok ? a.Minv[(size_t)36 * i + 6 * comp + c] : 0.0;
+#pragma unroll
+    for (int c = 0; c < 6; ++c) zv += M[c] * __shfl(rv, (tid & 63) - comp + c);
+    if (row_ok) {
+      double* o = a.zvp + (size_t)18 * i + comp;
+      o[0] = zv;
+      o[6] = 0.0;
+      o[12] = 0.0;
+    }
+    rows[g][comp] = zv;
+    double* o = sc[6 * g + comp];
+    o[0] = o[2] = o[3] = o[6] = 0.0;
+    o[1] = rv * zv;
+    o[4] = rv * rv;
+    o[5] = bv * bv;
+  }
+  __syncthreads();
+  if (ne && lane_in) {
+    const double z = rows[g][comp];
+#pragma unroll
+    for (int m = 0; m < Sh::kCols; ++m) {
+      const int lc = bs + Sh::kBlocks * m;
+      if (lc < kMaxCoarse) tmp[g][lc][comp] = sw[m] * z;
+    }
+  }
+  __syncthreads();
+  step_publish<G>(a, i0, sc, tmp, a.spart);
+}
+
+// Iteration k: takes step k - 1 (x, r), then stops when |r|^2 <= tol2 or
+// k = max_iters, else forms direction k and its product.
+template <int G>
+__global__ __launch_bounds__(kStepThreads) void k_pcg_step(PcgArgs a, int32_t k) {
+  using Sh = StepShape<G>;
+  __shared__ double sc[6 * G][kStepScalars];
+  __shared__ double tmp[G][kMaxCoarse][6];
+  __shared__ double lds[Sh::kSlices][128], ldz[Sh::kSlices][128];
+  __shared__ double sums[128], cs[kMaxCoarse], mus[kMaxCoarse], rows[G][6], rowz[G][6], red[G][Sh::kBlocks][6], wred[G][kMaxRitz][6];
+  PcgState* st = a.st;
+  const int odd = k & 1, ne = a.ne, stride = kStepScalars + ne;
+  const double* __restrict__ in = a.zvp + (odd ? (size_t)18 * a.Pvar : 0);
+  double* __restrict__ out = a.zvp + (odd ? 0 : (size_t)18 * a.Pvar);
+  const double* __restrict__ c_in = a.cvec + (odd ? kMaxCoarse : 0);
+  double* __restrict__ c_out = a.cvec + (odd ? 0 : kMaxCoarse);
+  const int tid = threadIdx.x, i0 = blockIdx.x * G;
+  const int g = min(tid / Sh::kT, G - 1), t = tid - g * Sh::kT, comp = t % 6, bs = t / 6, i = i0 + g;
+  const bool row_ok = i < a.Pvar, lane_in = t < 6 * Sh::kBlocks, lane_ok = row_ok && lane_in;
+  const bool fresh = k > 0 && (k - 1) % kStepRefresh == 0;  // (SW)'z of the last launch was summed anew
+  // done is 1 + the iteration that stopped: a work-group of that launch which
+  // starts late still takes the last step.
+  const int32_t done = st->done, max_iters = st->max_iters;
+  const double tol2_prev = st->tol2, tol_rel2 = st->tol_rel2;
+  // Coarse columns of the work-group's windows: hat columns ulo .. ulo + nh, then the dense ones.
+  const int gi = row_ok ? i / kRowsPerGroup : 0;
+  const int c0 = ne ? 6 * a.grp_lo[gi] : 0;
+  int ulo = 0, nh = 0;
+  if (ne) {
+    const int la = 6 * a.grp_lo[i0 / kRowsPerGroup], lb = 6 * a.grp_lo[(min(i0 + G, a.Pvar) - 1) / kRowsPerGroup];
+    ulo = min(la, lb);
+    nh = min(max(la, lb) + a.gwh, a.neh) - ulo;
+  }
+  // Slice of the sums, the same in a wave.
+  const int tc = (tid - Sh::kFirst) & 127;
+  const int sl = __builtin_amdgcn_readfirstlane(tid >= Sh::kFirst ? (tid - Sh::kFirst) >> 7 : kStepThreads);
+  const int nu = nh + a.nr, uc = tc < nh ? ulo + tc : a.neh + (tc - nh);
+  constexpr int kEinvCols = (kMaxCoarse + Sh::kSlices - 1) / Sh::kSlices;
+  double sw[Sh::kCols] = {}, rc[Sh::kRitz] = {}, ei[kEinvCols] = {};
+  double az = 0.0, av = 0.0, ap = 0.0;
+  double xv = 0.0, rv = 0.0, sv = 0.0, pv = 0.0, hw0 = 0.0, hw1 = 0.0, M[6] = {};
+  int hn0 = 0;
+  if (lane_ok) {
+    const int re = a.row_ptr[i + 1];
+#pragma unroll 2
+    for (int kb = a.row_ptr[i] + bs; kb < re; kb += Sh::kBlocks) {
+      const double2* x2 = reinterpret_cast<const double2*>(in + (size_t)18 * a.col_var[kb]);
+      const double2* s2 = reinterpret_cast<const double2*>(a.S + (size_t)36 * kb + 6 * comp);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const double2 sb = s2[c], zz = x2[c], vv = x2[3 + c], pp = x2[6 + c];
+        az += sb.x * zz.x;
+        az += sb.y * zz.y;
+        av += sb.x * vv.x;
+        av += sb.y * vv.y;
+        ap += sb.x * pp.x;
+        ap += sb.y * pp.y;
+      }
+    }
+    if (ne) {
+#pragma unroll
+      for (int m = 0; m < Sh::kCols; ++m) {
+        const int lc = bs + Sh::kBlocks * m;
+        if (lc < a.gw) sw[m] = sr_col(a, gi, lc)[6 * (i - gi * kRowsPerGroup) + comp];
+      }
+#pragma unroll
+      for (int m = 0; m < Sh::kRitz; ++m) {
+        const int c = bs + Sh::kBlocks * m;
+        if (c < a.nr) rc[m] = a.R[(size_t)c * a.n6 + 6 * i + comp];
+      }
+    }
+    if (t < 6) {
+      const int e = 6 * i + comp;
+      xv = a.x[e];
+      rv = a.r[e];
+      sv = a.q[e];
+      pv = in[(size_t)18 * i + 12 + comp];
+#pragma unroll
+      for (int c = 0; c < 6; ++c) M[c] = a.Minv[(size_t)36 * i + 6 * comp + c];
+      if (ne) {
+        hn0 = a.hat_node[i];
+        hw0 = a.hat_w[2 * i];
+        hw1 = a.hat_w[2 * i + 1];
+      }
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if (sl < Sh::kSlices) {
+#pragma unroll
+    for (int m = 0; m < kEinvCols; ++m) {
+      const int c = sl + Sh::kSlices * m;
+      ei[m] = tc < nu && c < ne ? a.Einv[(size_t)c * ne + uc] : 0.0;
+    }
+    if (fresh)
+      ldz[sl][tc] = step_slice<Sh::kSlices>(a.zpart, a.wgs, ne, tc, sl);
+    else if (sl == 0 && tc < ne)
+      cs[tc] = k > 0 ? c_in[tc] : 0.0;
+    lds[sl][tc] = step_slice<Sh::kSlices>(a.spart + (odd ? (size_t)a.wgs * stride : 0), a.wgs, stride, tc, sl);
+  }
+  if (done && done != k + 1) return;  // the same value in every thread
+  __syncthreads();
+  if (tid < stride) {
+    double s = 0.0;
+#pragma unroll
+    for (int q = 0; q < Sh::kSlices; ++q) s += lds[q][tid];
+    sums[tid] = s;
+  }
+  if (fresh && tid < ne) {
+    double s = 0.0;
+#pragma unroll
+    for (int q = 0; q < Sh::kSlices; ++q) s += ldz[q][tid];
+    cs[tid] = s;
+  }
+  __syncthreads();
+  const double rz_old = sums[1];
+  double rz = rz_old, rr = sums[4], alpha = 0.0, beta = 0.0, tol2 = tol2_prev;
+  bool stop;
+  if (k == 0) {
+    const double bb = sums[5];
+    tol2 = tol_rel2 * bb;
+    stop = bb <= 0.0 || max_iters <= 0 || rr <= tol2;
+  } else {
+    alpha = rz_old / sums[0];
+    rz += alpha * (alpha * sums[3] - 2.0 * sums[2]);
+    rr += alpha * (alpha * sums[6] - 2.0 * sums[5]);
+    beta = rz / rz_old;
+    stop = rr <= tol2 || k >= max_iters;
+  }
+  if (t < 6 && lane_ok) {
+    const int e = 6 * i + comp;
+    rv -= alpha * sv;
+    a.x[e] = xv + alpha * pv;
+    a.r[e] = rv;
+  }
+  if (blockIdx.x == 0 && tid == 0) {
+    if (k == 0) {
+      st->bb = sums[5];
+      st->tol2 = tol2;
+    } else if (k - 1 < a.zcap) {
+      a.coef[2 * (k - 1) + 1] = alpha;
+    }
+    if (!stop && k < a.zcap) a.coef[2 * k] = rz;
+    st->iters = k;
+    if (stop) st->done = k + 1;
+  }
+  if (stop) return;  // the same value in every thread
+  // c, and mu = E^-1 c on the work-group's windows.
+  const double ca = k > 0 ? -alpha : 1.0;  // cs is zero at k = 0
+  if (blockIdx.x == 0 && tid < ne) c_out[tid] = cs[tid] + ca * sums[kStepScalars + tid];
+  if (sl < Sh::kSlices) {
+    double mp = 0.0;
+#pragma unroll
+    for (int m = 0; m < kEinvCols; ++m) {
+      const int c = sl + Sh::kSlices * m;
+      if (c < ne) mp += ei[m] * (cs[c] + ca * sums[kStepScalars + c]);
+    }
+    lds[sl][tc] = mp;
+  }
+  __syncthreads();
+  if (tid >= Sh::kFirst && tid - Sh::kFirst < nu) {
+    double m = 0.0;
+#pragma unroll
+    for (int q = 0; q < Sh::kSlices; ++q) m += lds[q][tc];
+    mus[uc] = m;
+  }
+  __syncthreads();
+  if (lane_in) {
+    double y = az - alpha * av + beta * ap;
+    if (ne) {
+#pragma unroll
+      for (int m = 0; m < Sh::kCols; ++m) {
+        const int lc = bs + Sh::kBlocks * m, gc = lc < a.gw ? win_col(a, c0, lc) : -1;
+        if (gc >= 0) y -= sw[m] * mus[gc];
+      }
+#pragma unroll
+      for (int m = 0; m < Sh::kRitz; ++m) {
+        const int c = bs + Sh::kBlocks * m;
+        if (c < kMaxRitz) wred[g][c][comp] = c < a.nr ? rc[m] * mus[a.neh + c] : 0.0;
+      }
+    }
+    red[g][bs][comp] = y;
+  }
+  __syncthreads();
+  if (t < 6) {
+    double q = 0.0, zv = 0.0, vv = 0.0;
+#pragma unroll
+    for (int b = 0; b < Sh::kBlocks; ++b) q += red[g][b][comp];
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+      const int l = (tid & 63) - comp + c;
+      zv += M[c] * __shfl(rv, l);
+      vv += M[c] * __shfl(q, l);
+    }
+    double zh = zv;  // deflated preconditioned residual z - W mu
+    if (ne) {
+      double wm = hw0 != 0.0 ? hw0 * mus[6 * hn0 + comp] : 0.0;
+      if (hw1 != 0.0) wm += hw1 * mus[6 * (hn0 + 1) + comp];
+#pragma unroll
+      for (int c = 0; c < kMaxRitz; ++c) wm += wred[g][c][comp];
+      zh -= wm;
+    }
+    const double pn = zh + beta * pv;
+    if (row_ok) {
+      double* o = out + (size_t)18 * i + comp;
+      o[0] = zv;
+      o[6] = vv;
+      o[12] = pn;
+      a.q[6 * i + comp] = q;
+      if (k < a.zcap) a.Zh[(size_t)k * a.n6 + 6 * i + comp] = zh;
+    }
+    rows[g][comp] = row_ok ? vv : 0.0;
+    rowz[g][comp] = row_ok ? zv : 0.0;
+    double* o = sc[6 * g + comp];
+    o[0] = row_ok ? pn * q : 0.0;
+    o[1] = row_ok ? rv * zv : 0.0;
+    o[2] = row_ok ? q * zv : 0.0;
+    o[3] = row_ok ? q * vv : 0.0;
+    o[4] = row_ok ? rv * rv : 0.0;
+    o[5] = row_ok ? rv * q : 0.0;
+    o[6] = row_ok ? q * q : 0.0;
+  }
+  __syncthreads();
+  if (ne && lane_in) {
+    const double v = rows[g][comp];
+#pragma unroll
+    for (int m = 0; m < Sh::kCols; ++m) {
+      const int lc = bs + Sh::kBlocks * m;
+      if (lc < kMaxCoarse) tmp[g][lc][comp] = sw[m] * v;
+    }
+  }
+  __syncthreads();
+  step_publish<G>(a, i0, sc, tmp, a.spart + (odd ? 0 : (size_t)a.wgs * stride));
+  if (k % kStepRefresh != 0 || ne == 0) return;
+  __syncthreads();
+  if (lane_in) {
+    const double z = rowz[g][comp];
+#pragma unroll
+    for (int m = 0; m < Sh::kCols; ++m) {
+      const int lc = bs + Sh::kBlocks * m;
+      if (lc < kMaxCoarse) tmp[g][lc][comp] = sw[m] * z;
+    }
+  }
+  __syncthreads();
+  if (tid < ne) a.zpart[(size_t)blockIdx.x * ne + tid] = step_column<G>(a, i0, tid, tmp);
+}
+
 // Clears the convergence flag and lifts the iteration limit so that one more
 // iteration runs (kernel timing only).
 __global__ void k_pcg_reopen(PcgState* st) {
@@ -1239,6 +1689,12 @@ static PcgArgs make_args(const PcgBuffers& B) {
   a.part1 = B.part2 + (size_t)a.groups * (3 + a.ne);
   a.reduce1 = B.partials == 0 ? (a.groups > kPartChunk / (3 + a.ne) ? 1 : 0) : (B.partials == 2 ? 1 : 0);
   a.pad4 = 0;
+  a.step_G = step_rows(a.Pvar);
+  a.wgs = step_wgs(a.Pvar);
+  a.zvp = B.step;
+  a.cvec = a.zvp + 36 * (size_t)a.Pvar;
+  a.spart = a.cvec + 2 * kMaxCoarse;
+  a.zpart = a.spart + 2 * (size_t)a.wgs * kStepStride;
   a.st = static_cast<PcgState*>(B.state_dev);
   a.linv = B.linv; a.kmat = B.kmat; a.diag_pos = B.diag_pos; a.tpos = B.tpos; a.t = B.t; a.u = B.u;
   return a;
@@ -1268,6 +1724,32 @@ static void launch_spmv(hipStream_t s, const PcgArgs& a, int32_t k, const double
     k_pcg_spmv<false><<<a.Pvar, 256, 0, s>>>(a, k, p_prev, p_cur);
 }
 
+static void launch_step_start(hipStream_t s, const PcgArgs& a) {
+  switch (a.step_G) {
+    case 1: k_pcg_start<1><<<a.wgs, kStepThreads, 0, s>>>(a); break;
+    case 2: k_pcg_start<2><<<a.wgs, kStepThreads, 0, s>>>(a); break;
+    case 4: k_pcg_start<4><<<a.wgs, kStepThreads, 0, s>>>(a); break;
+    default: k_pcg_start<8><<<a.wgs, kStepThreads, 0, s>>>(a);
+  }
+}
+
+static void launch_step(hipStream_t s, const PcgArgs& a, int32_t k) {
+  switch (a.step_G) {
+    case 1: k_pcg_step<1><<<a.wgs, kStepThreads, 0, s>>>(a, k); break;
+    case 2: k_pcg_step<2><<<a.wgs, kStepThreads, 0, s>>>(a, k); break;
+    case 4: k_pcg_step<4><<<a.wgs, kStepThreads, 0, s>>>(a, k); break;
+    default: k_pcg_step<8><<<a.wgs, kStepThreads, 0, s>>>(a, k);
+  }
+}
+
+// Block-Jacobi iterations as one launch each (k_pcg_step).
+static bool step_applies(const PcgBuffers& B) { return B.kmat == nullptr && B.Pvar <= kStepVertices; }
+
+size_t pcg_step_doubles(int32_t Pvar) {
+  if (Pvar <= 0 || Pvar > kStepVertices) return 0;
+  return 36 * (size_t)Pvar + 2 * kMaxCoarse + (size_t)step_wgs(Pvar) * (2 * kStepStride + kMaxCoarse);
+}
+
 bool pcg_small_applies(const PcgBuffers& B) {
   return B.K == 0 && B.kmat == nullptr && B.Pvar > 0 && B.Pvar <= kSmallVertices;
 }
@@ -1279,17 +1761,18 @@ bool launch_pcg_small(hipStream_t s, const PcgBuffers& B, double tol, int32_t ma
 }
 
 // Deflated PCG solve of S y = b. The host polls the state after `first`
-// iterations, then every `poll` iterations. With `probe` (three events),
-// k_pcg_spmv and then k_pcg_update of one more iteration are each launched
-// `probe_reps` times back to back after the solve and timed as two batches
-// (k_pcg_spmv is idempotent; x, r and z then hold extra steps). Returns the
-// iteration count or -1 on a launch error.
+// iterations, then every `poll` iterations. With `probe` (three events), the
+// kernels of one more iteration (k_pcg_step, or k_pcg_spmv and then
+// k_pcg_update) are each launched `probe_reps` times back to back after the
+// solve and timed as two batches, the second empty with k_pcg_step (x, r and
+// z then hold extra steps). Returns the iteration count or -1 on a launch
+// error.
 int launch_pcg_deflated(hipStream_t s, const PcgBuffers& B, double tol, int32_t max_iters, int32_t first,
                         int32_t poll, const hipEvent_t* probe, int32_t probe_reps) {
   const int32_t Pvar = B.Pvar;
   if (Pvar <= 0) return 0;
   if (B.K > kMaxHatNodes || B.nr > kMaxRitz || B.nr < 0) return -1;
-  const bool learned = B.kmat != nullptr;
+  const bool learned = B.kmat != nullptr, step = step_applies(B);
   if (learned && (B.nr > 0 || B.zcap > 0 || probe || !B.linv || !B.diag_pos || !B.tpos || !B.t || !B.u)) return -1;
   const PcgArgs a = make_args(B);
   double* p0 = B.p0;
@@ -1306,6 +1789,8 @@ int launch_pcg_deflated(hipStream_t s, const PcgBuffers& B, double tol, int32_t 
   if (learned) {
     k_defl_init<true><<<groups, kGroupBlock, 0, s>>>(a);
     launch_learned_z(s, a, 1);
+  } else if (step) {
+    launch_step_start(s, a);
   } else {
     k_defl_init<false><<<groups, kGroupBlock, 0, s>>>(a);
   }
@@ -1314,11 +1799,19 @@ int launch_pcg_deflated(hipStream_t s, const PcgBuffers& B, double tol, int32_t 
   while (true) {
     const int n = std::min(k == 0 ? std::max(first, 1) : poll, max_iters - k);
     for (int j = 0; j < n; ++j, ++k) {
-      launch_spmv(s, a, k, (k & 1) ? p1 : p0, (k & 1) ? p0 : p1);
-      launch_update(s, a, k, (k & 1) ? p0 : p1);
+      if (step) {
+        launch_step(s, a, k);
+      } else {
+        launch_spmv(s, a, k, (k & 1) ? p1 : p0, (k & 1) ? p0 : p1);
+        launch_update(s, a, k, (k & 1) ? p0 : p1);
+      }
     }
-    // At k = max_iters this launch only records the final state.
-    if (k >= max_iters) launch_spmv(s, a, k, p0, p1);
+    // At k = max_iters this launch only records the final state (k_pcg_step
+    // also takes the last step).
+    if (k >= max_iters) {
+      if (step) launch_step(s, a, k);
+      else launch_spmv(s, a, k, p0, p1);
+    }
     if (hipMemcpyAsync(hs, a.st, sizeof(PcgState), hipMemcpyDeviceToHost, s) != hipSuccess) return -1;
     if (hipStreamSynchronize(s) != hipSuccess) return -1;
     if (hs->done || k >= max_iters) break;
@@ -1330,9 +1823,12 @@ int launch_pcg_deflated(hipStream_t s, const PcgBuffers& B, double tol, int32_t 
     k_pcg_reopen<<<1, 1, 0, s>>>(a.st);
     const int kk = iters;
     if (hipEventRecord(probe[0], s) != hipSuccess) return -1;
-    for (int j = 0; j < probe_reps; ++j) launch_spmv(s, a, kk, (kk & 1) ? p1 : p0, (kk & 1) ? p0 : p1);
+    for (int j = 0; j < probe_reps; ++j) {
+      if (step) launch_step(s, a, kk);
+      else launch_spmv(s, a, kk, (kk & 1) ? p1 : p0, (kk & 1) ? p0 : p1);
+    }
     if (hipEventRecord(probe[1], s) != hipSuccess) return -1;
-    for (int j = 0; j < probe_reps; ++j) k_pcg_update<false><<<groups, kGroupBlock, 0, s>>>(a, kk, (kk & 1) ? p0 : p1);
+    for (int j = 0; j < probe_reps && !step; ++j) k_pcg_update<false><<<groups, kGroupBlock, 0, s>>>(a, kk, (kk & 1) ? p0 : p1);
     if (hipEventRecord(probe[2], s) != hipSuccess) return -1;
     if (hipGetLastError() != hipSuccess) return -1;
   }

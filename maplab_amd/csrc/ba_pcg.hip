@@ -23,7 +23,7 @@
 // is a set of coalesced column dot products.
 //
 // Per LM step: k_defl_sr (SW), k_defl_e and k_defl_dense (E, R'b),
-// k_defl_prep (state, E^-1 by Gauss-Jordan, y = E^-1 W'b). Up to 2048 vertices
+// k_defl_prep (state, E^-1 by the sweep operator, y = E^-1 W'b). Up to 2048 vertices
 // with block-Jacobi k_pcg_start and one launch per iteration, k_pcg_step,
 // follow; otherwise k_defl_init (x0, r0, z0 and the first per-group partials)
 // and two launches per iteration: k_pcg_spmv (sums the previous
@@ -303,23 +303,80 @@ __global__ __launch_bounds__(256) void k_defl_dense(PcgArgs a) {
 }
 
 constexpr int kPrepThreads = 1024;
-constexpr int kTri = kMaxCoarse * (kMaxCoarse + 1) / 2;  // entries of the lower triangle
-constexpr int kInvPerThread = (kTri + kPrepThreads - 1) / kPrepThreads;
+constexpr int kInvTile = 16;
+constexpr int kInvTiles = (kMaxCoarse + kInvTile - 1) / kInvTile;  // 7
+constexpr int kInvPad = kInvTile + 1;                              // LDS pitch of a 16-wide panel
+constexpr int kInvWaves = kPrepThreads / 64;
+constexpr int kInvPerWave = (kInvTiles * (kInvTiles + 1) / 2 + kInvWaves - 1) / kInvWaves;  // lower tiles of a wave
+
+typedef double double4v __attribute__((ext_vector_type(4)));  // v_mfma_f64_16x16x4's accumulator
+
+__device__ inline double readlane_f64(double v, int lane) {
+  const int2 u = __builtin_bit_cast(int2, v);
+  return __builtin_bit_cast(double, make_int2(__builtin_amdgcn_readlane(u.x, lane), __builtin_amdgcn_readlane(u.y, lane)));
+}
+// Lane kLane of every 16 lanes.
+template <int kLane>
+__device__ inline double row_lane_f64(double v) {
+  const int2 u = __builtin_bit_cast(int2, v);
+  constexpr int kCtrl = 0x150 + kLane;  // row_newbcast
+  return __builtin_bit_cast(double, make_int2(__builtin_amdgcn_update_dpp(0, u.x, kCtrl, 0xf, 0xf, true),
+                                              __builtin_amdgcn_update_dpp(0, u.y, kCtrl, 0xf, 0xf, true)));
+}
+
+// Sweeps pivots kP .. 15 of a symmetric 16 x 16 tile (lane l, value i: row
+// 4 i + l / 16, column l % 16). False if a pivot is not positive.
+template <int kP>
+__device__ inline bool sweep_tile(double4v& t, int lane) {
+  if constexpr (kP == kInvTile) {
+    return true;
+  } else {
+    constexpr int kI = kP / 4, kG = kP % 4;
+    const double p = readlane_f64(t[kI], 16 * kG + kP), ip = 1.0 / p;
+    const double rowp = __shfl(t[kI], 16 * kG + (lane & 15));  // (p, own column)
+    const double w = rowp * ip;
+    const bool own_col = (lane & 15) == kP;
+    double4v n;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const double colp = row_lane_f64<kP>(t[i]);  // (own row, p)
+      n[i] = own_col ? colp * ip : fma(-colp, w, t[i]);
+    }
+    if ((lane >> 4) == kG) n[kI] = own_col ? -ip : w;
+    t = n;
+    return sweep_tile<kP + 1>(t, lane) && p > 0.0;
+  }
+}
 
 // Solve set-up (one work-group): the PCG state, c = W'b, E^-1 by the sweep
 // operator on the lower triangle (Goodnight, "A tutorial on the SWEEP
 // operator", Amer. Statistician 33, 1979: sweeping pivot k of a symmetric A
 // maps a_kk -> -1/a_kk, a_ik -> a_ik / a_kk, a_ij -> a_ij - a_ik a_kj / a_kk,
 // keeps A symmetric, and sweeping every pivot gives -A^-1; E is SPD, so the
-// pivots are the positive Cholesky pivots and no pivoting is needed). Each
-// thread keeps its lower-triangle entries in registers, pivot column k goes
-// through LDS. Then y = E^-1 c. A non-positive pivot disables deflation for
-// this solve (E^-1 = 0, y = 0, defl_ok = 0).
+// pivots are the positive Cholesky pivots and no pivoting is needed). Then
+// y = E^-1 c. A non-positive pivot disables deflation for this solve (E^-1 = 0,
+// y = 0, defl_ok = 0).
+//
+// Sixteen pivots are swept at once: with the 16 x 16 tile A_kk swept (-P) by
+// its wave, in registers, L_i = A_ik P for the other tile rows i, the panel
+// becomes L and A_ij -= L_i A_jk'. The lower tiles stay in registers, two a
+// wave, as the matrix instruction's accumulators; the panel and L go through
+// LDS. One pivot at a time, every entry a register of one of 1024 threads, is
+// a barrier, a divide and a column through LDS per pivot: 106 columns took
+// about 100 us that way and take 35 so, 34 columns 13. Columns past ne are those
+// of the identity.
 __global__ __launch_bounds__(kPrepThreads) void k_defl_prep(PcgArgs a, double tol, int32_t max_iters) {
-  __shared__ double Ms[kMaxCoarse * kMaxCoarse];
+  __shared__ union {
+    struct {
+      double panel[2][kInvTiles * kInvTile][kInvPad];  // A_ik by row, of step k in panel[k & 1]
+      double l[kInvTiles * kInvTile][kInvPad];
+      double pinv[2][kInvTile][kInvPad];
+    } s;
+    double inv[kMaxCoarse * kMaxCoarse];
+  } sh;
   __shared__ double cpart[kPrepThreads];
   __shared__ double cvec[kMaxCoarse];
-  __shared__ double colb[2][kMaxCoarse];  // column k of the swept matrix in colb[k & 1]
+  __shared__ int bad;
   const int ne = a.ne, tid = threadIdx.x;
   if (tid == 0) {
     PcgState* st = a.st;
@@ -332,8 +389,26 @@ __global__ __launch_bounds__(kPrepThreads) void k_defl_prep(PcgArgs a, double to
     st->max_iters = max_iters;
     st->defl_ok = 0;
     st->arrive = 0;
+    bad = 0;
   }
   if (ne == 0) return;
+  // The wave's lower tiles (ti, tj), ti >= tj, row by row; ti = -1: none.
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nt = (ne + kInvTile - 1) / kInvTile;
+  const int lr = lane >> 4, lc = lane & 15;
+  double4v v[kInvPerWave];
+  int ti[kInvPerWave], tj[kInvPerWave];
+#pragma unroll
+  for (int m = 0; m < kInvPerWave; ++m) {
+    int e = wave + m * kInvWaves, r = 0;
+    while (e > r) e -= ++r;
+    ti[m] = r < nt ? r : -1;
+    tj[m] = e;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = kInvTile * r + 4 * i + lr, col = kInvTile * e + lc;
+      v[m][i] = ti[m] < 0 ? 0.0 : (max(row, col) < ne ? a.E[(size_t)max(row, col) * ne + min(row, col)] : (row == col ? 1.0 : 0.0));
+    }
+  }
   // c = W'b: thread (column, g) sums the support rows lo + g, lo + g + G, ...
   // of a hat column; dense columns come from k_defl_dense.
   {
@@ -355,81 +430,82 @@ __global__ __launch_bounds__(kPrepThreads) void k_defl_prep(PcgArgs a, double to
       cvec[tid] = c;
     }
   }
-  const int nt = ne * (ne + 1) / 2;
-  double v[kInvPerThread];
-  int er[kInvPerThread], ec[kInvPerThread];  // entry (row >= column); -1 past the triangle
+  for (int k = 0; k < nt; ++k) {
+    double(*panel)[kInvPad] = sh.s.panel[k & 1];
+    double(*pinv)[kInvPad] = sh.s.pinv[k & 1];
+    // The panel (the previous step's readers use the other buffer), and the
+    // swept tile by the wave that holds it.
 #pragma unroll
-  for (int m = 0; m < kInvPerThread; ++m) {
-    const int e = tid + m * kPrepThreads;
-    int i = -1, j = -1;
-    if (e < nt) {
-      i = (int)((sqrt(8.0 * e + 1.0) - 1.0) * 0.5);
-      while (i * (i + 1) / 2 > e) --i;
-      while ((i + 1) * (i + 2) / 2 <= e) ++i;
-      j = e - i * (i + 1) / 2;
+    for (int m = 0; m < kInvPerWave; ++m) {
+      if (ti[m] > k && tj[m] == k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) panel[kInvTile * ti[m] + 4 * i + lr][lc] = v[m][i];
+      if (ti[m] == k && tj[m] < k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) panel[kInvTile * tj[m] + lc][4 * i + lr] = v[m][i];
     }
-    er[m] = i;
-    ec[m] = j;
-    v[m] = e < nt ? a.E[(size_t)i * ne + j] : 0.0;
-  }
-  bool ok = true;
-  // One barrier per pivot: step k reads column k from colb[k & 1] and writes
-  // column k + 1 of its result into the other buffer, which nobody reads
-  // until the next step's barrier (its last readers were in step k - 1).
 #pragma unroll
-  for (int m = 0; m < kInvPerThread; ++m) {
-    if (er[m] == 0) colb[0][ec[m]] = v[m];
-    else if (ec[m] == 0) colb[0][er[m]] = v[m];
-  }
-  // Pivot k reads column k from colk and writes column k + 1 into next; the
-  // loop takes two pivots per pass so that each buffer is a fixed LDS address.
-  auto pivot = [&](int k, const double* colk, double* next) -> bool {
-    const double p = colk[k];
-    if (!(p > 0.0)) return false;  // the same value in every thread
-    const double ip = 1.0 / p;
+    for (int m = 0; m < kInvPerWave; ++m)
+      if (ti[m] == k && tj[m] == k) {
+        const bool ok = sweep_tile<0>(v[m], lane);
+        if (!ok && lane == 0) bad = 1;
 #pragma unroll
-    for (int m = 0; m < kInvPerThread; ++m) {
-      const int i = max(er[m], 0), j = max(ec[m], 0);
-      const bool ri = er[m] == k, rj = ec[m] == k;
-      double nv = fma(-colk[i] * ip, colk[j], v[m]);
-      nv = (ri || rj) ? v[m] * ip : nv;
-      v[m] = (ri && rj) ? -ip : nv;
-      if (er[m] == k + 1) next[ec[m]] = v[m];       // (k + 1, j <= k + 1)
-      else if (ec[m] == k + 1) next[er[m]] = v[m];  // (i > k + 1, k + 1)
-    }
-    return true;
-  };
-  for (int k = 0; k < ne; k += 2) {
+        for (int i = 0; i < 4; ++i) pinv[4 * i + lr][lc] = -v[m][i];
+      }
     __syncthreads();
-    if (!pivot(k, colb[0], colb[1])) {
-      ok = false;
-      break;
+    if (wave < nt && wave != k) {  // L_i = A_ik P
+      double4v acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(panel[kInvTile * wave + lc][4 * q + lr], pinv[4 * q + lr][lc], acc,
+                                                   0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sh.s.l[kInvTile * wave + 4 * i + lr][lc] = acc[i];
     }
-    if (k + 1 == ne) break;
     __syncthreads();
-    if (!pivot(k + 1, colb[1], colb[0])) {
-      ok = false;
-      break;
+#pragma unroll
+    for (int m = 0; m < kInvPerWave; ++m) {
+      if (ti[m] < 0 || (ti[m] == k && tj[m] == k)) continue;
+      if (tj[m] == k) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[m][i] = sh.s.l[kInvTile * ti[m] + 4 * i + lr][lc];
+      } else if (ti[m] == k) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[m][i] = sh.s.l[kInvTile * tj[m] + lc][4 * i + lr];
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          v[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(-sh.s.l[kInvTile * ti[m] + lc][4 * q + lr],
+                                                      panel[kInvTile * tj[m] + lc][4 * q + lr], v[m], 0, 0, 0);
+      }
     }
   }
   __syncthreads();
-  // E^-1 = -(swept matrix), both triangles.
+  const bool ok = bad == 0;
+  // E^-1 = -(swept matrix), both triangles (a diagonal tile is symmetric up to
+  // rounding: its lower triangle counts).
 #pragma unroll
-  for (int m = 0; m < kInvPerThread; ++m)
-    if (er[m] >= 0) {
-      const double x = ok ? -v[m] : 0.0;
-      Ms[er[m] * ne + ec[m]] = x;
-      Ms[ec[m] * ne + er[m]] = x;
+  for (int m = 0; m < kInvPerWave; ++m) {
+    if (ti[m] < 0) continue;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = kInvTile * ti[m] + 4 * i + lr, col = kInvTile * tj[m] + lc;
+      if (row < ne && col <= row) {
+        const double x = ok ? -v[m][i] : 0.0;
+        sh.inv[row * ne + col] = x;
+        sh.inv[col * ne + row] = x;
+      }
     }
+  }
   __syncthreads();
   const int n2 = ne * ne;
-  for (int e = tid; e < n2; e += kPrepThreads) a.Einv[e] = Ms[e];
+  for (int e = tid; e < n2; e += kPrepThreads) a.Einv[e] = sh.inv[e];
   if (tid == 0) a.st->defl_ok = ok ? 1 : 0;
   // y = E^-1 c: thread (row, part) sums a contiguous part of the columns.
   const int nparts = kPrepThreads / ne, row = tid % ne, part = tid / ne, len = (ne + nparts - 1) / nparts;
   double yv = 0.0;
   if (part < nparts)
-    for (int c = part * len; c < min(ne, (part + 1) * len); ++c) yv += Ms[row * ne + c] * cvec[c];
+    for (int c = part * len; c < min(ne, (part + 1) * len); ++c) yv += sh.inv[row * ne + c] * cvec[c];
   cpart[tid] = yv;
   __syncthreads();
   if (tid < ne) {
@@ -1156,8 +1232,8 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_pcg_small(PcgArgs a, doubl
 // (24 us) are slower. Sums run in a fixed order.
 //
 // An iteration, two launches -> one (MI355X, 15-node space and 16 dense
-// columns from 250 keyframes): 60 keyframes 14.7 -> 7.9 us, 250 19.6 -> 13.4,
-// 500 21.3 -> 15.5, 1000 26.7 -> 21.5, 2000 39.0 -> 30.8. At 5000 (work-groups
+// columns from 250 keyframes): 60 keyframes 14.7 -> 8.2 us, 250 19.6 -> 13.6,
+// 500 21.3 -> 15.6, 1000 26.7 -> 21.6, 2000 39.0 -> 30.6. At 5000 (work-groups
 // of 16 rows) 68 -> 91: the product is the larger part there, and three vectors
 // gathered cost it more than the launch; the line is drawn at 2048 vertices.
 constexpr int kStepScalars = 7;  // p's, r'z, s'z, s'v, r'r, r's, s's (k_pcg_start: r'z, r'r, b'b in 1, 4, 5)

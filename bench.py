@@ -75,21 +75,21 @@ def kernel_table(sm, kt, n_pcg_total):
         if launches:
             rows[name] = row_of(launches, sm.kernel_ms[kid], bytes_per_launch)
 
-    add("k_linearize", abi.KERNEL_LINEARIZE, N * 196 + L * 176)
+    add("k_linearize", abi.KERNEL_LINEARIZE, N * 132 + L * 176)
     add("k_linearize_cost", abi.KERNEL_COST, N * 36 + L * 32)
-    add("k_schur_factors", abi.KERNEL_SCHUR_FACTORS, n_inc * 352)
+    add("k_schur_factors", abi.KERNEL_SCHUR_FACTORS, n_inc * 96 + kt.schur_factor_blocks * 120)
     tp = kt.schur_tile_pairs
     add("k_schur_blocks", abi.KERNEL_SCHUR_BLOCKS,
-        kt.schur_factor_blocks * 192 + L * 120 + kt.schur_staged_blocks * 8 + tp * 2 + kt.schur_batches * 530
+        kt.schur_factor_blocks * 120 + L * (80 + 144) + kt.schur_staged_blocks * 8 + tp * 2 + kt.schur_batches * 530
         + kt.schur_segments * (1040 + 2 * 86016) + nub * 584 + P * 48)
     if "k_schur_blocks" in rows:
         r = rows["k_schur_blocks"]
-        r["flops"] = int(tp * 216)
-        r["achieved_tflops"] = round(tp * 216 / r["avg_ms"] / 1e9, 3)
+        r["flops"] = int(tp * 198)
+        r["achieved_tflops"] = round(tp * 198 / r["avg_ms"] / 1e9, 3)
         r["staged_factor_blocks"] = int(kt.schur_staged_blocks)
-    add("k_back_substitute", abi.KERNEL_BACK_SUBSTITUTE, N * 160 + L * 216)
+    add("k_back_substitute", abi.KERNEL_BACK_SUBSTITUTE, N * 96 + L * 216)
     add("k_pose_rows", abi.KERNEL_POSE_ROWS)
-    add("k_landmark_prep", abi.KERNEL_LANDMARK_PREP, L * (144 + 24 + 72))
+    add("k_landmark_prep", abi.KERNEL_LANDMARK_PREP, L * (144 + 24 + 80 + 144))
     launches = sm.kernel_launches[abi.KERNEL_PCG]
     if launches and n_pcg_total > 0:
         it_ms = sm.kernel_ms[abi.KERNEL_PCG] / n_pcg_total

@@ -2,20 +2,19 @@
 //
 // One LM iteration on the device (names match the launchers at the bottom):
 //   k_vertex_prep     R_I_M and |q|^2 of every vertex (state or candidate)
-//   k_linearize<1>    per observation: residual, tangent Jacobians, robust
-//                     correction (VisualReprojectionError::Evaluate + ceres
-//                     Corrector); per landmark: V, g reductions in LDS
+//   k_linearize<1>    per observation: residual, its Jacobian by the landmark
+//                     in the IMU frame, robust correction
+//                     (VisualReprojectionError::Evaluate + ceres Corrector);
+//                     per landmark: V, g reductions in LDS
 //   k_linearize<0>    the same chain, cost only (candidate evaluation)
 //   k_pose_rows       per variable vertex: unscaled gradient, diag(F'F) and
 //                     the direct observation block sum Jo^T Jo
-//   k_landmark_prep   per landmark: Z = C (C V C + D^2)^-1 C (Schur pivot)
-//   k_schur_factors   per row incidence, per linearization: W_x, r0_x (and
-//                     the anchor maps A_l)
-//   k_schur_incidences per row incidence, per LM iteration: Q_x and rhs_x
-//   k_schur_items     partial sums of the upper blocks of the reduced camera
-//                     system S over work items of <= 512 incidence pairs
-//   k_schur_finalize  S blocks from the item partials, both triangles
-//   k_schur_rhs       rhs of every S row
+//   k_schur_factors   per factor block, per linearization: P, p and k
+//   k_landmark_prep   per landmark: T of Z = C (C V C + D^2)^-1 C = T'T, T g and
+//                     the anchor's factor and self product
+//   k_schur_tiles     partial sums of the upper blocks of the reduced camera
+//                     system S over segments of 16 x 16-block tiles
+//   k_schur_finalize  S blocks and rhs from the partials, both triangles
 //   k_block_inverse   block-Jacobi preconditioner (6x6 inverses of diag(S))
 //   (ba_pcg.hip)      deflated block-Jacobi PCG on S
 //   k_back_substitute landmark step and the LM model cost change
@@ -237,6 +236,11 @@ __device__ inline double loss_scale(const DevLoss& loss, int32_t type, double si
 // values, so S stays the Schur complement of J'J of one Jacobian; records are
 // Rec32 (residual and p_I in FP64).
 //
+// Records leave through LDS, so that consecutive lanes write consecutive 16
+// bytes: written by its own thread, a record is six stores of which each touches
+// 64 rows of 96 bytes: 188 -> 164 us for 2M observations of 500 keyframes, 358 ->
+// 311 for 1000 (and k_schur_factors, which writes so too, 185 -> 134, 327 -> 229).
+//
 // The landmark sums meet in LDS: nine values per observation (V and g), value-
 // major; thread (run, value) adds its landmark's run of observations in order,
 // the pose-coupled ones and the store vertex's own separately, so all 256
@@ -253,7 +257,11 @@ __global__ __launch_bounds__(kObsTile) void k_linearize(DevTopology t, const dou
                                                          double* __restrict__ lm_acc,
                                                          double* __restrict__ split_part,
                                                          double* __restrict__ tile_cost) {
-  __shared__ double red[kJac ? kLinVals : 1][kJac ? kObsTile + 1 : 1];
+  constexpr int kRecWords = (kF32 ? (int)sizeof(Rec32) : kObsRecord * 8) / 16;  // 16-byte words of a record
+  __shared__ union {
+    double red[kJac ? kLinVals : 1][kJac ? kObsTile + 1 : 1];
+    double2 rec[kJac ? kObsTile * kRecWords : 1];
+  } sh;
   __shared__ int32_t seg[kJac ? kObsTile : 1];    // landmark of each observation
   __shared__ uint8_t own[kJac ? kObsTile : 1];    // made by the store vertex (not pose-coupled)
   __shared__ int16_t head[kJac ? kObsTile + 1 : 1];  // first observation of each run
@@ -320,23 +328,29 @@ __global__ __launch_bounds__(kObsTile) void k_linearize(DevTopology t, const dou
     }
     if (kJac) {
       if (kF32) {
-        Rec32* out = static_cast<Rec32*>(obs_rec) + o;
+        Rec32* out = reinterpret_cast<Rec32*>(sh.rec) + tid;
         for (int i = 0; i < 2; ++i) out->r[i] = rec[i];
         for (int i = 0; i < 3; ++i) out->p[i] = rec[8 + i];
+        out->unused = 0;
         for (int i = 0; i < 6; ++i) {
           const float hi = (float)rec[2 + i];  // the sum rounds back to its parts
           out->K[i] = hi;
           out->lo[i] = bf16_round((float)(rec[2 + i] - (double)hi));
         }
       } else {
-        // Records are 96 bytes and the array is 256-byte aligned.
-        double2* out = reinterpret_cast<double2*>(static_cast<double*>(obs_rec) + (size_t)kObsRecord * o);
-        for (int i = 0; i < kObsRecord / 2; ++i) out[i] = make_double2(rec[2 * i], rec[2 * i + 1]);
+        for (int i = 0; i < kRecWords; ++i) sh.rec[kRecWords * tid + i] = make_double2(rec[2 * i], rec[2 * i + 1]);
       }
     }
   }
   if (kJac) {
-    for (int i = 0; i < kLinVals; ++i) red[i][tid] = acc[i];
+    // Records are 96 or 80 bytes and the array is 256-byte aligned.
+    __syncthreads();
+    double2* out = static_cast<double2*>(obs_rec) + (size_t)kRecWords * b;
+    for (int i = tid; i < kRecWords * (e - b); i += kObsTile) out[i] = sh.rec[i];
+    __syncthreads();
+  }
+  if (kJac) {
+    for (int i = 0; i < kLinVals; ++i) sh.red[i][tid] = acc[i];
     seg[tid] = l;
     own[tid] = pose_coupled ? 0 : 1;
     __syncthreads();
@@ -359,7 +373,7 @@ __global__ __launch_bounds__(kObsTile) void k_linearize(DevTopology t, const dou
       const int k0 = head[run], k1 = head[run + 1];
       double sum = 0.0, sum_own = 0.0;
       for (int k = k0; k < k1; ++k) {
-        const double v = red[c][k];
+        const double v = sh.red[c][k];
         if (own[k]) sum_own += v; else sum += v;
       }
       const int32_t lr = seg[k0];
@@ -607,8 +621,11 @@ __global__ __launch_bounds__(256) void k_schur_factors(
     DevTopology t, int32_t n_g, const int32_t* __restrict__ g_row, const int32_t* __restrict__ g_inc_ptr,
     const int32_t* __restrict__ g_inc, const double* __restrict__ vR, const double* __restrict__ lm,
     const void* __restrict__ obs_rec, double* __restrict__ gf, double* __restrict__ gk) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= n_g) return;
+  // Blocks leave through LDS, as k_linearize's records do.
+  __shared__ double2 sf[256 * kFactor / 2];
+  __shared__ double sk[256 * 3];
+  const int tid = threadIdx.x, g0 = blockIdx.x * 256, n = min(256, n_g - g0);
+  const int g = min(g0 + tid, n_g - 1);  // the last work-group's spare threads repeat the last block
   const int m0 = g_inc_ptr[g], m1 = g_inc_ptr[g + 1];
   double f[kFactor] = {}, k[3] = {0, 0, 0};
   const int32_t x0 = g_inc[m0];
@@ -639,9 +656,12 @@ __global__ __launch_bounds__(256) void k_schur_factors(
         for (int c = 0; c < 3; ++c) f[9 + c] = rec.p(c);
     }
   }
-  double2* out = reinterpret_cast<double2*>(gf + (size_t)kFactor * g);
-  for (int c = 0; c < kFactor / 2; ++c) out[c] = make_double2(f[2 * c], f[2 * c + 1]);
-  for (int c = 0; c < 3; ++c) gk[(size_t)3 * g + c] = k[c];
+  for (int c = 0; c < kFactor / 2; ++c) sf[kFactor / 2 * tid + c] = make_double2(f[2 * c], f[2 * c + 1]);
+  for (int c = 0; c < 3; ++c) sk[3 * tid + c] = k[c];
+  __syncthreads();
+  double2* out = reinterpret_cast<double2*>(gf + (size_t)kFactor * g0);
+  for (int i = tid; i < kFactor / 2 * n; i += 256) out[i] = sf[i];
+  for (int i = tid; i < 3 * n; i += 256) gk[(size_t)3 * g0 + i] = sk[i];
 }
 
 // LDS of one round of a tile: the staged factors of one or two batches (U and

@@ -11,7 +11,7 @@ CSRC = os.path.join(os.path.dirname(HERE), "maplab_amd", "csrc")
 
 
 @pytest.fixture(scope="module")
-def checker(tmp_path_factory):
+def program(tmp_path_factory):
     gxx = shutil.which("g++")
     if gxx is None:
         pytest.skip("g++ is not available")
@@ -23,7 +23,7 @@ def checker(tmp_path_factory):
 
 
 @pytest.mark.parametrize("pvar, landmarks", [(1, 0), (1, 50), (16, 1), (17, 3000), (300, 60000), (40, 40000)])
-def test_decomposition_is_the_same_on_one_cpu(checker, pvar, landmarks):
-    out = subprocess.run([checker, str(pvar), str(landmarks), "3"], capture_output=True, text=True)
+def test_decomposition_is_the_same_on_one_cpu(program, pvar, landmarks):
+    out = subprocess.run([program, str(pvar), str(landmarks), "3"], capture_output=True, text=True)
     print(out.stdout)
     assert out.returncode == 0, out.stdout + out.stderr

@@ -530,19 +530,21 @@ class GnnWorkspace {
   }
 };
 
-GnnWorkspace* gnn_workspace_create(int32_t nodes, int32_t slots, bool for_training) {
+GnnWorkspace* gnn_workspace_create(hipStream_t s, int32_t nodes, int32_t slots, bool for_training) {
   GnnWorkspace* w = new GnnWorkspace();
   w->nodes = nodes;
   w->slots = slots;
   w->m_pad = std::max(128, ((nodes + 127) / 128) * 128);
   w->training = for_training;
   const size_t bytes = w->place(nullptr);
-  if (hipMalloc(&w->base, bytes) != hipSuccess) {
-    w->base = nullptr;
+  if (hipMalloc(&w->base, bytes) != hipSuccess) w->base = nullptr;
+  // Cleared in the order of the stream that goes on to use it: a solver's
+  // stream does not wait for the null stream, where a clear still running
+  // would wipe the weights and gates that the first forward pass writes.
+  if (!w->base || hipMemsetAsync(w->base, 0, bytes, s) != hipSuccess) {
     delete w;
     return nullptr;
   }
-  (void)hipMemset(w->base, 0, bytes);
   (void)w->place(static_cast<char*>(w->base));
   return w;
 }
@@ -753,9 +755,9 @@ int32_t mlba_gnn_evaluate(const mlba_gnn_dataset* data, const float* params, flo
   float* dloss = ds.put<float>(nullptr, 1);
   if (!dp || !dtheta || !dgrad || !dloss) return gnn_fail(MLBA_ENOMEM, "device allocation failed");
   Workspace ws;
-  ws.w = mlba::gnn_workspace_create(n, data->slots, loss || grad);
-  if (!ws.w) return gnn_fail(MLBA_ENOMEM, "workspace allocation failed");
   hipStream_t s = nullptr;
+  ws.w = mlba::gnn_workspace_create(s, n, data->slots, loss || grad);
+  if (!ws.w) return gnn_fail(MLBA_ENOMEM, "workspace allocation failed");
   if (!mlba::gnn_forward(s, ws.w, ds.g, dp, dtheta)) return gnn_fail(MLBA_EDEVICE, "forward launch failed");
   if (loss || grad) {
     if (!mlba::gnn_loss_backward(s, ws.w, ds.g, dp, dtheta, ds.qc, ds.inv_count, dloss, dgrad))
@@ -786,9 +788,9 @@ int32_t mlba_gnn_train(const mlba_gnn_dataset* data, int32_t epochs, float learn
   float* dlosses = ds.put<float>(nullptr, (size_t)std::max(epochs, 1));
   if (!dp || !m || !v || !dtheta || !dgrad || !dlosses) return gnn_fail(MLBA_ENOMEM, "device allocation failed");
   Workspace ws;
-  ws.w = mlba::gnn_workspace_create(n, data->slots, true);
-  if (!ws.w) return gnn_fail(MLBA_ENOMEM, "workspace allocation failed");
   hipStream_t s = nullptr;
+  ws.w = mlba::gnn_workspace_create(s, n, data->slots, true);
+  if (!ws.w) return gnn_fail(MLBA_ENOMEM, "workspace allocation failed");
   for (int ep = 0; ep < epochs; ++ep) {
     if (!mlba::gnn_forward(s, ws.w, ds.g, dp, dtheta) ||
         !mlba::gnn_loss_backward(s, ws.w, ds.g, dp, dtheta, ds.qc, ds.inv_count, dlosses + ep, dgrad))

@@ -982,7 +982,7 @@ int lp_ensure(mlba_handle* h, bool network, bool t2) {
   }
   if (network && h->lp_model && (h->lp_ws_nodes != h->Pvar || h->lp_ws_slots != h->nnzb)) {
     if (h->lp_ws) gnn_workspace_destroy(h->lp_ws);
-    h->lp_ws = gnn_workspace_create(h->Pvar, h->nnzb, false);
+    h->lp_ws = gnn_workspace_create(h->stream, h->Pvar, h->nnzb, false);
     if (!h->lp_ws) { h->lp_ws_nodes = -1; return set_err(h, MLBA_ENOMEM, "network workspace allocation failed"); }
     h->lp_ws_nodes = h->Pvar;
     h->lp_ws_slots = h->nnzb;

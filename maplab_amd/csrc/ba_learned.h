@@ -125,7 +125,9 @@ struct GnnGraph {
 };
 
 class GnnWorkspace;  // activations of one graph batch (ba_gnn.hip)
-GnnWorkspace* gnn_workspace_create(int32_t nodes, int32_t slots, bool for_training);
+// Allocates and, on stream s, clears a workspace; it may be used on s (or on a
+// stream that waits for s). Null when either fails.
+GnnWorkspace* gnn_workspace_create(hipStream_t s, int32_t nodes, int32_t slots, bool for_training);
 void gnn_workspace_destroy(GnnWorkspace* w);
 
 // theta [nodes x 2] = network(graph) with the FP32 parameters `params`

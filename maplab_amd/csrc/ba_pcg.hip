@@ -1242,6 +1242,7 @@ constexpr int kStepThreads = 1024;
 constexpr int kStepFlight = 16;  // a thread's partials in flight
 constexpr int kStepVertices = 2048;
 constexpr int kStepRefresh = 8;  // every launch k with k % 8 = 0 sums (SW)'z as well
+constexpr double kStepCancel = 1e-12;  // r'r by recurrence holds to about 1e-15 of the last one: 3 digits here
 static_assert(kStepStride <= 128, "128 threads hold the partials of one work-group");
 
 int32_t step_rows(int32_t Pvar) {
@@ -1399,7 +1400,9 @@ __global__ __launch_bounds__(kStepThreads) void k_pcg_start(PcgArgs a) {
 }
 
 // Iteration k: takes step k - 1 (x, r), then stops when |r|^2 <= tol2 or
-// k = max_iters, else forms direction k and its product.
+// k = max_iters, else forms direction k and its product. Where |r|^2 was too
+// small a difference to stop on, launch k + 1 finds it summed and stops without
+// a step, after k iterations.
 template <int G>
 __global__ __launch_bounds__(kStepThreads) void k_pcg_step(PcgArgs a, int32_t k) {
   using Sh = StepShape<G>;
@@ -1417,7 +1420,7 @@ __global__ __launch_bounds__(kStepThreads) void k_pcg_step(PcgArgs a, int32_t k)
   const int g = min(tid / Sh::kT, G - 1), t = tid - g * Sh::kT, comp = t % 6, bs = t / 6, i = i0 + g;
   const bool row_ok = i < a.Pvar, lane_in = t < 6 * Sh::kBlocks, lane_ok = row_ok && lane_in;
   const bool fresh = k > 0 && (k - 1) % kStepRefresh == 0;  // (SW)'z of the last launch was summed anew
-  // done is 1 + the iteration that stopped: a work-group of that launch which
+  // done is 1 + the launch that stopped: a work-group of that launch which
   // starts late still takes the last step.
   const int32_t done = st->done, max_iters = st->max_iters;
   const double tol2_prev = st->tol2, tol_rel2 = st->tol_rel2;
@@ -1512,20 +1515,26 @@ __global__ __launch_bounds__(kStepThreads) void k_pcg_step(PcgArgs a, int32_t k)
   }
   __syncthreads();
   const double rz_old = sums[1];
-  double rz = rz_old, rr = sums[4], alpha = 0.0, beta = 0.0, tol2 = tol2_prev;
-  bool stop;
+  double rr = sums[4], alpha = 0.0, beta = 0.0, tol2 = tol2_prev;
+  bool stop, take = k > 0;  // take: step k - 1 is taken
   if (k == 0) {
     const double bb = sums[5];
     tol2 = tol_rel2 * bb;
     stop = bb <= 0.0 || max_iters <= 0 || rr <= tol2;
+  } else if (rr <= tol2) {
+    // The last launch's r'r, summed from r itself, was small enough.
+    stop = true;
+    take = false;
   } else {
     alpha = rz_old / sums[0];
-    rz += alpha * (alpha * sums[3] - 2.0 * sums[2]);
+    // r'r and r'z of the new r are differences of numbers as large as the old
+    // ones. A result below kStepCancel of r'r has few or no digits left and may
+    // come out negative: it stops nothing, this launch sums r'r anew.
     rr += alpha * (alpha * sums[6] - 2.0 * sums[5]);
-    beta = rz / rz_old;
-    stop = rr <= tol2 || k >= max_iters;
+    beta = fmax(rz_old + alpha * (alpha * sums[3] - 2.0 * sums[2]), 0.0) / rz_old;
+    stop = (rr <= tol2 && rr > kStepCancel * sums[4]) || k >= max_iters;
   }
-  if (t < 6 && lane_ok) {
+  if (t < 6 && lane_ok && take) {
     const int e = 6 * i + comp;
     rv -= alpha * sv;
     a.x[e] = xv + alpha * pv;
@@ -1535,11 +1544,11 @@ __global__ __launch_bounds__(kStepThreads) void k_pcg_step(PcgArgs a, int32_t k)
     if (k == 0) {
       st->bb = sums[5];
       st->tol2 = tol2;
-    } else if (k - 1 < a.zcap) {
+    } else if (take && k - 1 < a.zcap) {
+      a.coef[2 * (k - 1)] = rz_old;
       a.coef[2 * (k - 1) + 1] = alpha;
     }
-    if (!stop && k < a.zcap) a.coef[2 * k] = rz;
-    st->iters = k;
+    st->iters = k > 0 && !take ? k - 1 : k;
     if (stop) st->done = k + 1;
   }
   if (stop) return;  // the same value in every thread

@@ -827,6 +827,8 @@ int ritz_queue_vectors(mlba_handle* h) {
   for (int j = 0; j < m; ++j) {
     const double rz = coef[2 * j], al = coef[2 * j + 1];
     if (!(rz > 0.0) || !(al > 0.0) || !std::isfinite(rz) || !std::isfinite(al)) return MLBA_OK;
+    // A one-launch iteration's r'z is a difference: too few digits are left.
+    if (j > 0 && rz <= 1e-12 * coef[2 * (j - 1)]) return MLBA_OK;
     d[j] = 1.0 / al + (j > 0 ? (rz / coef[2 * (j - 1)]) / coef[2 * (j - 1) + 1] : 0.0);
     if (j + 1 < m) e[j] = -std::sqrt(coef[2 * (j + 1)] / rz) / al;
   }

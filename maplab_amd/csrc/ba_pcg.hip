@@ -1515,7 +1515,7 @@ __global__ __launch_bounds__(kStepThreads) void k_pcg_step(PcgArgs a, int32_t k)
   }
   __syncthreads();
   const double rz_old = sums[1];
-  double rr = sums[4], alpha = 0.0, beta = 0.0, tol2 = tol2_prev;
+  double rz = rz_old, rr = sums[4], alpha = 0.0, beta = 0.0, tol2 = tol2_prev;
   bool stop, take = k > 0;  // take: step k - 1 is taken
   if (k == 0) {
     const double bb = sums[5];
@@ -1530,8 +1530,9 @@ __global__ __launch_bounds__(kStepThreads) void k_pcg_step(PcgArgs a, int32_t k)
     // r'r and r'z of the new r are differences of numbers as large as the old
     // ones. A result below kStepCancel of r'r has few or no digits left and may
     // come out negative: it stops nothing, this launch sums r'r anew.
+    rz += alpha * (alpha * sums[3] - 2.0 * sums[2]);
     rr += alpha * (alpha * sums[6] - 2.0 * sums[5]);
-    beta = fmax(rz_old + alpha * (alpha * sums[3] - 2.0 * sums[2]), 0.0) / rz_old;
+    beta = rz < 0.0 ? 0.0 : rz / rz_old;
     stop = (rr <= tol2 && rr > kStepCancel * sums[4]) || k >= max_iters;
   }
   if (t < 6 && lane_ok && take) {
@@ -1545,9 +1546,9 @@ __global__ __launch_bounds__(kStepThreads) void k_pcg_step(PcgArgs a, int32_t k)
       st->bb = sums[5];
       st->tol2 = tol2;
     } else if (take && k - 1 < a.zcap) {
-      a.coef[2 * (k - 1)] = rz_old;
       a.coef[2 * (k - 1) + 1] = alpha;
     }
+    if (!stop && k < a.zcap) a.coef[2 * k] = rz;
     st->iters = k > 0 && !take ? k - 1 : k;
     if (stop) st->done = k + 1;
   }

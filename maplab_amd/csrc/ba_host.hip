@@ -416,66 +416,14 @@ int build_topology(mlba_handle* h) {
     if (!build_schur_tiles(Pvar, L, inc_ptr.data(), inc.data(), h->s_landmark.data(), &st, &terr))
       return set_err(h, MLBA_ENOMEM, terr);
   }
-  // Block structure of S: row i couples with the row of every factor block of
-  // every landmark it has one of. Incidence pairs (x in row i, y in row j >= i,
-  // same landmark) summed into each upper block: two factor blocks of a
-  // landmark multiply their incidence counts. Rows are independent.
-  std::vector<int32_t> row_ptr(Pvar + 1, 0), col_var, diag_pos(Pvar, 0);
-  std::vector<int32_t> upair;
-  int64_t total_pairs = 0;
+  // Block structure of S, the incidence pairs of every upper block.
+  SchurRows sr;
   {
-    const int64_t n_g = (int64_t)st.g_row.size();
-    std::vector<int32_t> row_g_ptr(Pvar + 1, 0), row_g(n_g), row_l(n_g);  // factor blocks and landmarks of each row
-    for (int64_t g = 0; g < n_g; ++g) row_g_ptr[st.g_row[g] + 1]++;
-    for (int i = 0; i < Pvar; ++i) row_g_ptr[i + 1] += row_g_ptr[i];
-    {
-      std::vector<int32_t> fill(row_g_ptr.begin(), row_g_ptr.end() - 1);
-      for (int l = 0; l < L; ++l)
-        for (int g = st.lm_g_ptr[l]; g < st.lm_g_ptr[l + 1]; ++g) {
-          const int k = fill[st.g_row[g]]++;
-          row_g[k] = g;
-          row_l[k] = l;
-        }
-    }
-    std::vector<std::vector<int32_t>> cols(Pvar), counts(Pvar);  // columns of a row; pairs of those >= the row
-    if (!parallel_ranges(Pvar, 4, [&](int64_t i0, int64_t i1) {
-          std::vector<int32_t> mark(Pvar, -1), pairs(Pvar, 0);
-          for (int i = (int)i0; i < (int)i1; ++i) {
-            std::vector<int32_t>& c = cols[i];
-            auto touch = [&](int j) {
-              if (mark[j] != i) {
-                mark[j] = i;
-                pairs[j] = 0;
-                c.push_back(j);
-              }
-            };
-            touch(i);
-            for (int k = row_g_ptr[i]; k < row_g_ptr[i + 1]; ++k) {
-              const int a = row_g[k], l = row_l[k];
-              const int ma = st.g_inc_ptr[a + 1] - st.g_inc_ptr[a];
-              for (int b = st.lm_g_ptr[l]; b < a; ++b) touch(st.g_row[b]);
-              for (int b = a; b < st.lm_g_ptr[l + 1]; ++b) {
-                const int j = st.g_row[b];
-                touch(j);
-                pairs[j] += ma * (st.g_inc_ptr[b + 1] - st.g_inc_ptr[b]);
-              }
-            }
-            std::sort(c.begin(), c.end());
-            for (int j : c)
-              if (j >= i) counts[i].push_back(pairs[j]);
-          }
-        }))
-      return set_err(h, MLBA_ENOMEM, "host allocation failed");
-    h->max_row_blocks = 0;
-    for (int i = 0; i < Pvar; ++i) {
-      diag_pos[i] = (int32_t)(col_var.size() + cols[i].size() - counts[i].size());
-      col_var.insert(col_var.end(), cols[i].begin(), cols[i].end());
-      upair.insert(upair.end(), counts[i].begin(), counts[i].end());
-      row_ptr[i + 1] = (int32_t)col_var.size();
-      h->max_row_blocks = std::max<int32_t>(h->max_row_blocks, (int32_t)cols[i].size());
-    }
-    for (int32_t n : upair) total_pairs += n;
+    std::string terr;
+    if (!build_schur_rows(Pvar, L, st, &sr, &terr)) return set_err(h, MLBA_ENOMEM, terr);
   }
+  const std::vector<int32_t>&row_ptr = sr.row_ptr, &col_var = sr.col, &diag_pos = sr.diag_pos, &upair = sr.upper_pairs;
+  h->max_row_blocks = sr.max_row_blocks;
   h->nnzb = (int32_t)col_var.size();
   h->hat_K = -1;
   h->pcg_last_iters[0] = h->pcg_last_iters[1] = 0;
@@ -498,7 +446,7 @@ int build_topology(mlba_handle* h) {
       ublk.push_back(make_int4(k, kt, i, j));
     }
   h->n_upper = (int32_t)ublk.size();
-  h->schur_pairs = total_pairs;
+  h->schur_pairs = sr.pairs;
   h->n_g = (int32_t)st.g_row.size();
   h->nbands = st.nbands;
   h->n_segs = (int32_t)(st.segs.size() / 4);

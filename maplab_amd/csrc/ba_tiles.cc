@@ -17,15 +17,15 @@ struct Run {
 
 }  // namespace
 
-bool parallel_ranges(int64_t n, int64_t piece, const std::function<void(int64_t, int64_t)>& body) {
+bool parallel_ranges(int64_t n, int64_t piece, const std::function<void(int64_t, int64_t, int)>& body) {
   if (n <= 0) return true;
   piece = std::max<int64_t>(piece, 1);
   std::atomic<int64_t> next{0};
   std::atomic<bool> ok{true};
-  auto work = [&]() {
+  auto work = [&](int thread) {
     for (int64_t b = next.fetch_add(piece); b < n; b = next.fetch_add(piece)) {
       try {
-        body(b, std::min(n, b + piece));
+        body(b, std::min(n, b + piece), thread);
       } catch (...) {
         ok = false;
       }
@@ -35,13 +35,13 @@ bool parallel_ranges(int64_t n, int64_t piece, const std::function<void(int64_t,
   const int64_t hw = std::max(1u, std::thread::hardware_concurrency());
   std::vector<std::thread> pool;
   try {
-    const int64_t extra = std::min<int64_t>({pieces, hw, 8}) - 1;
+    const int64_t extra = std::min<int64_t>({pieces, hw, kMaxHostThreads}) - 1;
     pool.reserve((size_t)std::max<int64_t>(extra, 0));
-    for (int64_t t = 0; t < extra; ++t) pool.emplace_back(work);
+    for (int64_t t = 0; t < extra; ++t) pool.emplace_back(work, (int)t + 1);
   } catch (...) {
     // Fewer threads than wanted: the ones that run take all pieces.
   }
-  work();
+  work(0);
   for (std::thread& t : pool) t.join();
   return ok;
 }
@@ -70,7 +70,7 @@ bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const in
   lm_g.resize((size_t)L + 1);
   lm_g[0] = 0;
   std::atomic<bool> shared{false};
-  bool ok = parallel_ranges(L, kPiece, [&](int64_t l0, int64_t l1) {
+  bool ok = parallel_ranges(L, kPiece, [&](int64_t l0, int64_t l1, int) {
     for (int64_t l = l0; l < l1; ++l) {
       int n = 0, last = -1;
       for (int m = lm_ptr[l]; m < lm_ptr[l + 1]; ++m) {
@@ -94,7 +94,7 @@ bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const in
   T.g_inc_ptr.resize((size_t)n_g + 1);
   T.g_inc.resize((size_t)n_inc);
   T.g_inc_ptr[n_g] = (int32_t)n_inc;
-  ok = ok && parallel_ranges(L, kPiece, [&](int64_t l0, int64_t l1) {
+  ok = ok && parallel_ranges(L, kPiece, [&](int64_t l0, int64_t l1, int) {
     for (int64_t l = l0; l < l1; ++l) {
       int g = lm_g[l], last = -1;
       for (int m = lm_ptr[l]; m < lm_ptr[l + 1]; ++m) {
@@ -121,49 +121,73 @@ bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const in
   };
   // Visits (landmark, first block in I, first in J, blocks in I, in J),
   // grouped by tile in (I, J) order, landmarks ascending in a tile (a
-  // landmark visits a tile at most once; only visited tiles exist): a counting
-  // sort over pieces of the landmarks, each with counts of its own.
+  // landmark visits a tile at most once; only visited tiles exist). Two stable
+  // counting sorts, by I over pieces of the landmarks with counts of their own,
+  // then by J within each I: memory and time grow with the bands and the
+  // visits, not with the square of the bands.
   struct Visit {
-    int64_t key;  // I * nb + J
-    int32_t l, gi, gj, ni, nj;
+    int32_t I, J, l, gi, gj;
+    uint8_t ni, nj;  // <= kTileBand
   };
-  const int64_t keys = nb * nb;
-  const int64_t pieces = std::max<int64_t>(1, std::min<int64_t>({16, (L + kPiece - 1) / kPiece, (1 << 22) / std::max<int64_t>(keys, 1)}));
+  const int64_t pieces = std::max<int64_t>(1, std::min<int64_t>(16, (L + kPiece - 1) / kPiece));
   const int64_t span = (L + pieces - 1) / pieces;
-  std::vector<int64_t> at((size_t)(pieces * keys), 0);  // visits, then the place of the next, by piece and tile
-  ok = ok && parallel_ranges(pieces, 1, [&](int64_t p0, int64_t p1) {
+  std::vector<int64_t> at((size_t)(pieces * nb), 0);  // visits, then the place of the next, by piece and I
+  ok = ok && parallel_ranges(pieces, 1, [&](int64_t p0, int64_t p1, int) {
     std::vector<Run> runs;
     for (int64_t q = p0; q < p1; ++q)
       for (int64_t l = q * span; l < std::min<int64_t>(L, (q + 1) * span); ++l) {
         landmark_runs(l, runs);
-        for (size_t a = 0; a < runs.size(); ++a)
-          for (size_t b = a; b < runs.size(); ++b) at[(size_t)(q * keys + runs[a].band * nb + runs[b].band)]++;
+        for (size_t a = 0; a < runs.size(); ++a) at[(size_t)(q * nb + runs[a].band)] += (int64_t)(runs.size() - a);
       }
   });
+  std::vector<int64_t> band_at((size_t)nb + 1, 0);
   int64_t n_visits = 0;
-  for (int64_t k = 0; k < keys; ++k)
+  for (int64_t k = 0; k < nb; ++k) {
     for (int64_t q = 0; q < pieces; ++q) {
-      const int64_t n = at[(size_t)(q * keys + k)];
-      at[(size_t)(q * keys + k)] = n_visits;
+      const int64_t n = at[(size_t)(q * nb + k)];
+      at[(size_t)(q * nb + k)] = n_visits;
       n_visits += n;
     }
-  UnsetVector<Visit> visits;
+    band_at[(size_t)k + 1] = n_visits;
+  }
+  UnsetVector<Visit> visits, by_band;
   visits.resize((size_t)n_visits);
-  ok = ok && parallel_ranges(pieces, 1, [&](int64_t p0, int64_t p1) {
+  by_band.resize((size_t)n_visits);
+  ok = ok && parallel_ranges(pieces, 1, [&](int64_t p0, int64_t p1, int) {
     std::vector<Run> runs;
     for (int64_t q = p0; q < p1; ++q)
       for (int64_t l = q * span; l < std::min<int64_t>(L, (q + 1) * span); ++l) {
         landmark_runs(l, runs);
         for (size_t a = 0; a < runs.size(); ++a)
-          for (size_t b = a; b < runs.size(); ++b) {
-            const int64_t key = runs[a].band * nb + runs[b].band;
-            visits[(size_t)at[(size_t)(q * keys + key)]++] =
-                Visit{key, (int32_t)l, runs[a].g, runs[b].g, runs[a].n, a == b ? 0 : runs[b].n};
-          }
+          for (size_t b = a; b < runs.size(); ++b)
+            by_band[(size_t)at[(size_t)(q * nb + runs[a].band)]++] =
+                Visit{runs[a].band, runs[b].band, (int32_t)l, runs[a].g, runs[b].g, (uint8_t)runs[a].n,
+                      (uint8_t)(a == b ? 0 : runs[b].n)};
       }
   });
+  std::vector<std::vector<int64_t>> place(kMaxHostThreads);  // by thread: visits of J, then the place of the next
+  ok = ok && parallel_ranges(nb, 1, [&](int64_t i0, int64_t i1, int thread) {
+    std::vector<int64_t>& p = place[thread];
+    if (p.empty()) p.resize((size_t)nb, 0);
+    std::vector<int32_t> touched;
+    for (int64_t i = i0; i < i1; ++i) {
+      touched.clear();
+      for (int64_t k = band_at[i]; k < band_at[i + 1]; ++k)
+        if (p[by_band[k].J]++ == 0) touched.push_back(by_band[k].J);
+      std::sort(touched.begin(), touched.end());
+      int64_t next = band_at[i];
+      for (int32_t J : touched) {
+        const int64_t n = p[J];
+        p[J] = next;
+        next += n;
+      }
+      for (int64_t k = band_at[i]; k < band_at[i + 1]; ++k) visits[(size_t)p[by_band[k].J]++] = by_band[k];
+      for (int32_t J : touched) p[J] = 0;
+    }
+  });
+  UnsetVector<Visit>().swap(by_band);
   if (!ok) {
-    *err = "internal: the Schur decomposition failed";
+    *err = "host allocation failed";
     return false;
   }
   T.visits = n_visits;
@@ -181,6 +205,7 @@ bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const in
   const int64_t segment_slots = staged_all / (kSegmentTarget * rounds);
   auto is_anchor = [&](int g) { return T.g_inc[T.g_inc_ptr[g]] < 0; };
   auto pairs_of = [](const Visit& v) { return v.nj ? v.ni * v.nj : v.ni * (v.ni + 1) / 2; };
+  auto same_tile = [&](int64_t v, const Visit& of) { return v < n_visits && visits[v].I == of.I && visits[v].J == of.J; };
   // Batches (LDS-sized groups of visits) and segments (runs of batches of one
   // tile) of every visited tile, counted first: each tile's slots, pairs
   // (batches start on a 32-bit word), batches and segments then have their
@@ -192,13 +217,13 @@ bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const in
   std::vector<Tile> tiles;
   int64_t n_slots = 0, n_pairs = 0, n_batches = 0, n_segs = 0;
   for (int64_t v = 0; v < n_visits;) {
-    const int64_t key = visits[v].key;
+    const Visit of = visits[v];
     tiles.push_back(Tile{v, v, n_slots, n_pairs, n_batches, n_segs});
     int64_t seg_slots = 0, seg_batches = 0;
     bool open = false;
-    while (v < n_visits && visits[v].key == key) {
+    while (same_tile(v, of)) {
       int64_t slots = 0, np = 0;
-      for (; v < n_visits && visits[v].key == key; ++v) {
+      for (; same_tile(v, of); ++v) {
         const int c = visits[v].ni + visits[v].nj;
         if (slots + c > kBatchSlots) break;
         slots += c;
@@ -224,7 +249,7 @@ bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const in
     }
     if (open) ++n_segs;
     tiles.back().v1 = v;
-    T.tile_key.push_back(key);
+    T.tile_key.push_back(of.I * nb + of.J);
     T.tile_seg.push_back((int32_t)tiles.back().seg);
     T.tile_seg.push_back((int32_t)n_segs);
   }
@@ -298,7 +323,7 @@ bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const in
     }
   };
   auto fill_tile = [&](const Tile& tile) {
-    const int64_t key = visits[tile.v0].key, I = key / nb, J = key % nb;
+    const int64_t I = visits[tile.v0].I, J = visits[tile.v0].J;
     const bool diag = I == J;
     int64_t slot = tile.slot, pair = tile.pair, batch = tile.batch, seg = tile.seg, seg_first = batch, seg_slots = 0;
     uint16_t block[kBatchPairs], list[kBatchPairs];
@@ -351,12 +376,78 @@ bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const in
   };
   // The whole decomposition of 300 keyframes (1.2M observations, 8.4M pairs):
   // 480 ms on one thread of an eight-core host, 69 ms on its eight.
-  if (!parallel_ranges((int64_t)tiles.size(), 1, [&](int64_t b, int64_t e) {
+  if (!parallel_ranges((int64_t)tiles.size(), 1, [&](int64_t b, int64_t e, int) {
         for (int64_t t = b; t < e; ++t) fill_tile(tiles[t]);
       })) {
-    *err = "internal: the Schur decomposition failed";
+    *err = "host allocation failed";
     return false;
   }
+  return true;
+}
+
+bool build_schur_rows(int32_t Pvar, int32_t L, const SchurTiles& T, SchurRows* out, std::string* err) {
+  SchurRows& R = *out;
+  R = SchurRows();
+  R.row_ptr.assign((size_t)Pvar + 1, 0);
+  R.diag_pos.assign((size_t)Pvar, 0);
+  const int64_t n_g = (int64_t)T.g_row.size();
+  std::vector<int32_t> row_g_ptr(Pvar + 1, 0), row_g(n_g), row_l(n_g);  // factor blocks and landmarks of each row
+  for (int64_t g = 0; g < n_g; ++g) row_g_ptr[T.g_row[g] + 1]++;
+  for (int i = 0; i < Pvar; ++i) row_g_ptr[i + 1] += row_g_ptr[i];
+  {
+    std::vector<int32_t> fill(row_g_ptr.begin(), row_g_ptr.end() - 1);
+    for (int l = 0; l < L; ++l)
+      for (int g = T.lm_g_ptr[l]; g < T.lm_g_ptr[l + 1]; ++g) {
+        const int k = fill[T.g_row[g]]++;
+        row_g[k] = g;
+        row_l[k] = l;
+      }
+  }
+  std::vector<std::vector<int32_t>> cols(Pvar), counts(Pvar);  // columns of a row; pairs of those >= the row
+  // By thread: the last row that met a column, and the pairs it has with it.
+  std::vector<std::vector<int32_t>> marks(kMaxHostThreads), pair_sums(kMaxHostThreads);
+  if (!parallel_ranges(Pvar, 4, [&](int64_t i0, int64_t i1, int thread) {
+        std::vector<int32_t>&mark = marks[thread], &pairs = pair_sums[thread];
+        if (mark.empty()) {
+          pairs.resize((size_t)Pvar, 0);
+          mark.resize((size_t)Pvar, -1);
+        }
+        for (int i = (int)i0; i < (int)i1; ++i) {
+          std::vector<int32_t>& c = cols[i];
+          auto touch = [&](int j) {
+            if (mark[j] != i) {
+              mark[j] = i;
+              pairs[j] = 0;
+              c.push_back(j);
+            }
+          };
+          touch(i);
+          for (int k = row_g_ptr[i]; k < row_g_ptr[i + 1]; ++k) {
+            const int a = row_g[k], l = row_l[k];
+            const int ma = T.g_inc_ptr[a + 1] - T.g_inc_ptr[a];
+            for (int b = T.lm_g_ptr[l]; b < a; ++b) touch(T.g_row[b]);
+            for (int b = a; b < T.lm_g_ptr[l + 1]; ++b) {
+              const int j = T.g_row[b];
+              touch(j);
+              pairs[j] += ma * (T.g_inc_ptr[b + 1] - T.g_inc_ptr[b]);
+            }
+          }
+          std::sort(c.begin(), c.end());
+          for (int j : c)
+            if (j >= i) counts[i].push_back(pairs[j]);
+        }
+      })) {
+    *err = "host allocation failed";
+    return false;
+  }
+  for (int i = 0; i < Pvar; ++i) {
+    R.diag_pos[i] = (int32_t)(R.col.size() + cols[i].size() - counts[i].size());
+    R.col.insert(R.col.end(), cols[i].begin(), cols[i].end());
+    R.upper_pairs.insert(R.upper_pairs.end(), counts[i].begin(), counts[i].end());
+    R.row_ptr[i + 1] = (int32_t)R.col.size();
+    R.max_row_blocks = std::max<int32_t>(R.max_row_blocks, (int32_t)cols[i].size());
+  }
+  for (int32_t n : R.upper_pairs) R.pairs += n;
   return true;
 }
 

@@ -69,10 +69,12 @@ struct UnsetAllocator : std::allocator<T> {
 template <class T>
 using UnsetVector = std::vector<T, UnsetAllocator<T>>;
 
-// Runs body(begin, end) over pieces of [0, n) on up to eight threads (the
-// caller's among them), pieces taken in order; rethrows nothing: returns false
-// when a piece threw.
-bool parallel_ranges(int64_t n, int64_t piece, const std::function<void(int64_t, int64_t)>& body);
+constexpr int kMaxHostThreads = 8;  // threads of parallel_ranges, the caller's among them
+
+// Runs body(begin, end, thread) over pieces of [0, n) on up to kMaxHostThreads
+// threads (the caller's is thread 0), pieces taken in order; rethrows nothing:
+// returns false when a piece threw.
+bool parallel_ranges(int64_t n, int64_t piece, const std::function<void(int64_t, int64_t, int)>& body);
 
 struct SchurTiles {
   int32_t nbands = 0;
@@ -98,6 +100,18 @@ struct SchurTiles {
 // when a count overflows the decomposition's index widths.
 bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const int32_t* inc,
                        const int32_t* obs_landmark, SchurTiles* out, std::string* err);
+
+// Block structure of S in rows of ascending columns: row i couples with the row
+// of every factor block of every landmark it has one of, and with itself.
+struct SchurRows {
+  std::vector<int32_t> row_ptr, col;     // Pvar + 1; one per block
+  std::vector<int32_t> diag_pos;         // position of each row's own block
+  std::vector<int32_t> upper_pairs;      // per block with column >= row, in row order: incidence pairs
+                                         // (x in the row, y in the column, same landmark) summed into it
+  int64_t pairs = 0;                     // their sum
+  int32_t max_row_blocks = 0;
+};
+bool build_schur_rows(int32_t Pvar, int32_t L, const SchurTiles& tiles, SchurRows* out, std::string* err);
 
 }  // namespace mlba
 

@@ -260,7 +260,8 @@ int32_t mlba_download_state(const mlba_handle* handle, double* vertex_q_IM__M_p_
 
 /* Deactivate / reactivate landmarks (ProblemInformation::deactivateCostFunction
  * for all observations of a landmark, outlier-rejection-solver.cc:168-177).
- * mask[l] != 0 means active. */
+ * mask[l] != 0 means active. Where it fails (MLBA_ENOMEM, MLBA_EDEVICE), the
+ * calls that run on the device return MLBA_ESTATE until it has succeeded. */
 int32_t mlba_set_landmark_active(mlba_handle* handle, const uint8_t* mask);
 int32_t mlba_get_landmark_active(const mlba_handle* handle, uint8_t* mask);
 

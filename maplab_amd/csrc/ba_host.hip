@@ -247,6 +247,7 @@ struct mlba_handle {
   hipEvent_t scal_ev = nullptr;
   DevTopology topo{};
   SchurTilesDev tdev{};
+  bool topology_ok = false;  // topo and tdev describe the current active landmarks
   // Event pairs bracketing kernels inside the LM loop (kernel id, start, end).
   std::vector<hipEvent_t> ev_pool;
   std::vector<std::pair<int, std::pair<hipEvent_t, hipEvent_t>>> ev_pending;
@@ -272,6 +273,16 @@ namespace {
 int set_err(mlba_handle* h, int code, const std::string& msg) {
   if (h) h->err = msg; else g_create_error = msg;
   return code;
+}
+
+// For the catch blocks of the C entry points: host memory ran out, so the
+// message may not fit either.
+int host_out_of_memory(mlba_handle* h) noexcept {
+  try {
+    return set_err(h, MLBA_ENOMEM, "host allocation failed");
+  } catch (...) {
+    return MLBA_ENOMEM;
+  }
 }
 
 #define HIP_OK(expr)                                                                  \
@@ -323,8 +334,11 @@ int upload_item_order(mlba_handle* h) {
 }
 
 // Build the observation / landmark / vertex topology and the reduced camera
-// system structure for the current active landmark set, and upload it.
+// system structure for the current active landmark set, and upload it. A
+// handle whose last build failed holds a part of each of two structures and
+// runs nothing (check_topology) until a build succeeds.
 int build_topology(mlba_handle* h) {
+  h->topology_ok = false;
   const int N = h->N, L = h->L, P = h->P;
   // Error type per sorted observation (optimization-terms-addition.cc:68-78).
   // Variable vertices: non-constant and in an active pose-coupled residual.
@@ -556,6 +570,11 @@ int build_topology(mlba_handle* h) {
   d.batches = h->t_batches.p; d.slots = h->t_slots.p; d.batch_off = h->t_batch_off.p; d.pairs = h->t_pairs.p;
   d.uslot_ptr = h->t_uslot_ptr.p; d.uslot = h->t_uslot.p; d.n_uslot = (int32_t)uslot.size();
   HIP_OK(hipStreamSynchronize(h->stream));
+  h->topology_ok = true;
+  return MLBA_OK;
+}
+int check_topology(mlba_handle* h) {
+  if (!h->topology_ok) return set_err(h, MLBA_ESTATE, "the last change of the active landmarks failed");
   return MLBA_OK;
 }
 
@@ -1293,7 +1312,7 @@ int validate_options(mlba_handle* h, const mlba_options* o) {
     return set_err(h, MLBA_ESTATE, "learned preconditioner without a model (mlba_set_preconditioner_model)");
   if (!(o->initial_trust_region_radius > 0.0)) return set_err(h, MLBA_EINVAL, "initial_trust_region_radius <= 0");
   if (o->loss_type == MLBA_LOSS_CAUCHY && !(o->loss_scale_px > 0.0)) return set_err(h, MLBA_EINVAL, "loss_scale_px <= 0");
-  return MLBA_OK;
+  return check_topology(h);
 }
 
 int count_active_obs(const mlba_handle* h) {
@@ -1338,8 +1357,8 @@ void mlba_options_init(mlba_options* o) {
 
 const char* mlba_last_error(const mlba_handle* h) { return h ? h->err.c_str() : g_create_error.c_str(); }
 
-int32_t mlba_create(const mlba_problem_desc* d, mlba_handle** out) {
-  mlba_handle* h = nullptr;
+// h is the caller's, who deletes it if this throws.
+static int32_t create_handle(const mlba_problem_desc* d, mlba_handle** out, mlba_handle*& h) {
   if (!d || !out) return set_err(h, MLBA_EINVAL, "NULL argument");
   *out = nullptr;
   const int N = d->num_observations, L = d->num_landmarks, P = d->num_vertices, C = d->num_cameras,
@@ -1488,6 +1507,16 @@ int32_t mlba_create(const mlba_problem_desc* d, mlba_handle** out) {
   return MLBA_OK;
 }
 
+int32_t mlba_create(const mlba_problem_desc* d, mlba_handle** out) {
+  mlba_handle* h = nullptr;
+  try {
+    return create_handle(d, out, h);
+  } catch (...) {
+    delete h;
+    return host_out_of_memory(nullptr);
+  }
+}
+
 int32_t mlba_destroy(mlba_handle* h) {
   if (!h) return MLBA_EINVAL;
   if (h->stream) (void)hipStreamSynchronize(h->stream);
@@ -1523,8 +1552,12 @@ int32_t mlba_download_state(const mlba_handle* hc, double* vertices, double* lan
 
 int32_t mlba_set_landmark_active(mlba_handle* h, const uint8_t* mask) {
   if (!h || !mask) return MLBA_EINVAL;
-  for (int l = 0; l < h->L; ++l) h->lm_active[l] = mask[l] ? 1 : 0;
-  return build_topology(h);
+  try {
+    for (int l = 0; l < h->L; ++l) h->lm_active[l] = mask[l] ? 1 : 0;
+    return build_topology(h);
+  } catch (...) {
+    return host_out_of_memory(h);
+  }
 }
 
 int32_t mlba_get_landmark_active(const mlba_handle* h, uint8_t* mask) {
@@ -1545,6 +1578,7 @@ void mlba_quality_options_init(mlba_quality_options* o) {
 
 int32_t mlba_landmark_quality(mlba_handle* h, const mlba_quality_options* o, uint8_t* good) {
   if (!h || !o || !good) return h ? set_err(h, MLBA_EINVAL, "null argument") : MLBA_EINVAL;
+  if (const int rc = check_topology(h)) return rc;
   if (o->min_observers < 0) return set_err(h, MLBA_EINVAL, "min_observers must be >= 0");
   if (h->L == 0) return MLBA_OK;
   hipStream_t s = h->stream;
@@ -1586,6 +1620,7 @@ int32_t mlba_evaluate(mlba_handle* h, int32_t flags, const mlba_options* options
                       double* const* jacobians, double* cost) {
   if (!h) return MLBA_EINVAL;
   if (flags & ~(MLBA_EVAL_TANGENT | MLBA_EVAL_WITH_XI)) return set_err(h, MLBA_EINVAL, "unknown flags");
+  if (const int rc = check_topology(h)) return rc;
   const bool tangent = (flags & MLBA_EVAL_TANGENT) != 0;
   const int nblocks = (flags & MLBA_EVAL_WITH_XI) ? 10 : 9;
   static const int amb[10] = {3, 7, 7, 7, 7, 4, 3, 4, 4, 1};
@@ -1640,6 +1675,7 @@ int32_t mlba_evaluate_noalloc(mlba_handle* h, int32_t flags, const mlba_options*
                               double* const* jacobians, double* cost) {
   if (!h) return MLBA_EINVAL;
   if (flags & ~(MLBA_EVAL_TANGENT | MLBA_EVAL_WITH_XI)) return set_err(h, MLBA_EINVAL, "unknown flags");
+  if (const int rc = check_topology(h)) return rc;
   if (h->device < 0 || h->device >= kMaxDevices) return set_err(h, MLBA_EINVAL, "device index out of range");
   const bool tangent = (flags & MLBA_EVAL_TANGENT) != 0;
   const int nblocks = (flags & MLBA_EVAL_WITH_XI) ? 10 : 9;
@@ -2407,7 +2443,8 @@ int32_t mlba_set_schedule(mlba_handle* h, const mlba_schedule* sc) {
   h->sched_waves = sc->item_waves;
   h->sched_xcd = sc->xcd_mapping;
   h->sched_pcg = sc->pcg_partials;
-  return reorder ? upload_item_order(h) : MLBA_OK;
+  // A build that is still to come orders its segments itself.
+  return reorder && h->topology_ok ? upload_item_order(h) : MLBA_OK;
 }
 
 int32_t mlba_autotune(mlba_handle* h, const mlba_options* o, int32_t repeats, mlba_schedule* out) {

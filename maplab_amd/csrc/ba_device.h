@@ -86,10 +86,13 @@ constexpr uint32_t kLmConstant = 2u;
 constexpr uint32_t kLmAnchorVar = 4u;   // anchor vertex variable and landmark has pose-coupled obs
 constexpr uint32_t kLmSplit = 8u;       // observations span several linearization tiles
 
-// Observation meta word: bits 0-1 error type, bit 2 observer variable,
-// bits 8.. camera index.
+// Observation meta word: bits 0-1 error type, bit 2 observer variable, bit 3
+// landmark active, bits 8.. camera index.
 __host__ __device__ inline int32_t obs_type(int32_t meta) { return meta & 3; }
 __host__ __device__ inline bool obs_observer_var(int32_t meta) { return (meta >> 2) & 1; }
+// The landmark was active when the topology was built (outlier rejection may
+// have cleared kLmActive since).
+__host__ __device__ inline bool obs_built_active(int32_t meta) { return (meta >> 3) & 1; }
 __host__ __device__ inline int32_t obs_camera(int32_t meta) { return meta >> 8; }
 
 struct DevCamera {

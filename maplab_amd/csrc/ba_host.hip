@@ -398,7 +398,7 @@ int build_topology(mlba_handle* h) {
   for (int o = 0; o < N; ++o) {
     const int type = h->s_type[o];
     const bool ov = type != kTypeKeyframe && vertex_var[h->s_vertex[o]] >= 0;
-    meta[o] = type | (ov ? 4 : 0) | (h->s_camera[o] << 8);
+    meta[o] = type | (ov ? 4 : 0) | (h->lm_active[h->s_landmark[o]] ? 8 : 0) | (h->s_camera[o] << 8);
   }
   // Incidences of each variable vertex row.
   std::vector<int32_t> inc_ptr(Pvar + 1, 0), inc;

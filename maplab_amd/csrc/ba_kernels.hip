@@ -139,17 +139,14 @@ __device__ inline void landmark_to_imu(const DevTopology& t, int32_t type, int32
   mat3_mul(Rv, H, G);
 }
 
-// Residual of one observation and the factors of its Jacobians
-// (visual-error-term-inl.h:13-379).
+// Residual of one observation, of landmark l (anchored in vertex a) by vertex
+// v, and the factors of its Jacobians (visual-error-term-inl.h:13-379).
 template <bool kJac>
-__device__ inline void eval_observation(const DevTopology& t, int o, const double* __restrict__ vert,
-                                        const double* __restrict__ vR, const double* __restrict__ lm,
-                                        ObsEval& e) {
-  const int32_t meta = t.obs_meta[o];
+__device__ inline void eval_observation(const DevTopology& t, int o, int32_t meta, int32_t l, int32_t v, int32_t a,
+                                        const double* __restrict__ vert, const double* __restrict__ vR,
+                                        const double* __restrict__ lm, ObsEval& e) {
   const int32_t type = obs_type(meta);
   const DevCamera& cam = t.cams[obs_camera(meta)];
-  const int32_t l = t.obs_landmark[o];
-  const int32_t v = t.obs_vertex[o];
   const double* pB = lm + 3 * l;
   double* pI = e.pI;
   if (type == kTypeKeyframe) {
@@ -158,7 +155,6 @@ __device__ inline void eval_observation(const DevTopology& t, int o, const doubl
       for (int i = 0; i < 9; ++i) e.G[i] = (i % 4 == 0) ? 1.0 : 0.0;
   } else {
     const double* Rv = vR + 12 * v;
-    const int32_t a = t.lm_anchor[l];
     const double* Ra = vR + 12 * a;        // R_B_LM
     const double* pa = vert + 7 * a + 4;   // p_LM_B
     double pM[3];
@@ -277,21 +273,26 @@ __global__ __launch_bounds__(kObsTile) void k_linearize(DevTopology t, const dou
   bool pose_coupled = true;
   if (o < e) {
     l = t.obs_landmark[o];
+    // What the evaluation's loads start from comes with the flags, so that an
+    // active landmark's evaluation waits one round for them and an inactive
+    // one's is skipped. 500 keyframes, all active / 60 % inactive / three
+    // quarters of the tiles inactive: 138 / 125 / 65 us, cost only 46 / 38 / 18;
+    // evaluated whatever the flags say 138 / 138 / 131 and 47 / 46 / 45; loaded
+    // after the flags 143 / 125 / 67 and 46 / 38 / 19.
+    const int32_t meta = t.obs_meta[o], v = t.obs_vertex[o];
     const uint32_t flags = t.lm_flags[l];
+    const int32_t a = t.lm_anchor[l];
     double rec[kObsRecord] = {};
-    // Evaluated whatever the flags say (an inactive landmark's result is left
-    // out), so that its loads don't wait for them (166 -> 157 us at 500 keyframes).
-    ObsEval ev;
-    eval_observation<kJac>(t, o, vert, vR, lm, ev);
     if (flags & kLmActive) {
-      const int32_t meta = t.obs_meta[o];
+      ObsEval ev;
+      eval_observation<kJac>(t, o, meta, l, v, a, vert, vR, lm, ev);
       const int32_t type = obs_type(meta);
       const double s = ev.r[0] * ev.r[0] + ev.r[1] * ev.r[1];
       double rho[3];
       robust_loss(loss.type, loss_scale(loss, type, t.obs_sinv[o]), s, rho);
       pose_coupled = type != kTypeKeyframe;
       const bool has_var = !(flags & kLmConstant) ||
-                           (pose_coupled && (obs_observer_var(meta) || t.vertex_var[t.lm_anchor[l]] >= 0));
+                           (pose_coupled && (obs_observer_var(meta) || t.vertex_var[a] >= 0));
       if (has_var) cost = 0.5 * rho[0]; else fixed = 0.5 * rho[0];
       if (kJac) {
         // ceres Corrector: J~ = sqrt(rho') (I - alpha r r'/|r|^2) J, r~ = rs r.
@@ -1426,27 +1427,31 @@ __global__ __launch_bounds__(kObsTile) void k_back_substitute(DevTopology t, con
   uint32_t flags = 0;
   double K[6], s[3] = {0, 0, 0}, c[3] = {0, 0, 0}, r[2] = {0, 0};
   const double* Rv = vR;
-  // An inactive landmark's values are left out below: no load waits for its flags. The
-  // observer's variable comes with the observation (obs_col), not through its
-  // vertex (two dependent rounds of loads less: 154 -> 145 us at 500 keyframes,
-  // 268 -> 250 at 1000).
+  // The observation itself says whether its landmark was active when the
+  // structure was built, and brings its observer's variable (obs_col): no load
+  // waits for the landmark's flags. Values of a landmark deactivated since are
+  // left out below. 500 keyframes, all active / 60 % inactive / three quarters of
+  // the tiles inactive: 98 / 64 / 32 us; loaded whatever the landmark's state 97 /
+  // 79 / 47, after its flags 102 / 66 / 33.
   if (o < e) {
     l = t.obs_landmark[o];
-    const RecView<kF32> rec(obs_rec, o);
     const int32_t meta = t.obs_meta[o], col = t.obs_col[o];
     v = t.obs_vertex[o];
-    type = obs_type(meta);
-    for (int k = 0; k < 6; ++k) K[k] = rec.K(k);
-    r[0] = rec.r(0);
-    r[1] = rec.r(1);
-    flags = t.lm_flags[l];
-    if (type != kTypeKeyframe) {
-      Rv = vR + 12 * v;
-      if (col >= 0) {
-        observer_motion(rec, Rv, w + 6 * col, s);
-        const double j0 = K[0] * s[0] + K[1] * s[1] + K[2] * s[2], j1 = K[3] * s[0] + K[4] * s[1] + K[5] * s[2];
-        const double kj[3] = {-(K[0] * j0 + K[3] * j1), -(K[1] * j0 + K[4] * j1), -(K[2] * j0 + K[5] * j1)};
-        rotate_observer(t, type, l, v, Rv, false, kj, c);
+    if (obs_built_active(meta)) {
+      const RecView<kF32> rec(obs_rec, o);
+      flags = t.lm_flags[l];
+      type = obs_type(meta);
+      for (int k = 0; k < 6; ++k) K[k] = rec.K(k);
+      r[0] = rec.r(0);
+      r[1] = rec.r(1);
+      if (type != kTypeKeyframe) {
+        Rv = vR + 12 * v;
+        if (col >= 0) {
+          observer_motion(rec, Rv, w + 6 * col, s);
+          const double j0 = K[0] * s[0] + K[1] * s[1] + K[2] * s[2], j1 = K[3] * s[0] + K[4] * s[1] + K[5] * s[2];
+          const double kj[3] = {-(K[0] * j0 + K[3] * j1), -(K[1] * j0 + K[4] * j1), -(K[2] * j0 + K[5] * j1)};
+          rotate_observer(t, type, l, v, Rv, false, kj, c);
+        }
       }
     }
   }

@@ -386,8 +386,10 @@ typedef struct mlba_kernel_times {
   double schur_blocks_ms;     /* reduced camera system blocks and rhs */
   double block_inverse_ms;    /* block-Jacobi preconditioner */
   double pcg_solve_ms;        /* one whole (deflated) PCG solve at the initial radius */
-  double pcg_spmv_ms;         /* one PCG iteration's S p product (all of the iteration when it is one launch) */
-  double pcg_update_ms;       /* one PCG iteration's vector update and reductions (0 when it is one launch) */
+  double pcg_spmv_ms;         /* one PCG iteration's S p product (all of the iteration when it is one launch,
+                                 0 when the whole solve is one) */
+  double pcg_update_ms;       /* one PCG iteration's vector update and reductions (0 when the iteration or the
+                                 solve is one launch) */
   double back_substitute_ms;  /* landmark step + model cost change */
   int64_t num_observations;
   int64_t num_landmarks;

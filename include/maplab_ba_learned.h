@@ -99,7 +99,9 @@ int32_t mlba_rcs_system(mlba_handle* handle, const mlba_options* options, double
  * PCG iterations to solve the RCS at the current state and radius, with
  * b = its right-hand side, to ||r|| <= tolerance ||b|| with `preconditioner`
  * (MLBA_PRECOND_*; LEARNED and LEARNED_DEFLATED need a model; no fallback
- * and no recycled columns here). iterations: -1 when not converged
+ * and no recycled columns here). DEFLATED iterates by launches here, also
+ * where mlba_solve solves a small system (fewer than 32 variable vertices, no
+ * coarse space) in one. iterations: -1 when not converged
  * within max_iterations. The state is not changed.
  */
 int32_t mlba_rcs_pcg_iterations(mlba_handle* handle, const mlba_options* options, double radius,

@@ -2602,10 +2602,20 @@ int32_t mlba_time_kernels(mlba_handle* h, const mlba_options* o, int32_t repeats
   if (h->Pvar > 0) {
     if ((rc = ensure_coarse_basis(h, o->pcg_coarse_nodes))) return rc;
     int32_t iters = 0;
+    const PcgBuffers B = pcg_buffers(h, ritz_count(o) > 0 ? h->ritz_nr : 0, false);
+    const bool small = pcg_small_applies(B);
     t->pcg_solve_ms = timed([&] {
-      iters = launch_pcg_deflated(s, pcg_buffers(h, ritz_count(o) > 0 ? h->ritz_nr : 0, false),
-                                  o->pcg_relative_tolerance, o->pcg_max_iterations, kPcgPoll, kPcgPoll, nullptr, 0);
+      if (small)
+        iters = launch_pcg_small(s, B, o->pcg_relative_tolerance, o->pcg_max_iterations, h->scal.p + kPcgIters) ? 0 : -1;
+      else
+        iters = launch_pcg_deflated(s, B, o->pcg_relative_tolerance, o->pcg_max_iterations, kPcgPoll, kPcgPoll, nullptr,
+                                    0);
     });
+    if (iters < 0) return set_err(h, MLBA_EDEVICE, "PCG launch failed");
+    if (small) {
+      if ((rc = read_scalars(h))) return rc;
+      iters = (int32_t)h->scal_host[kPcgIters];
+    }
     t->pcg_iterations = iters;
     // One more iteration: each of its kernels (one: pcg_spmv, or two) launched
     // repeats x 8 times back to back between events (launch gaps included),
@@ -2613,9 +2623,8 @@ int32_t mlba_time_kernels(mlba_handle* h, const mlba_options* o, int32_t repeats
     hipEvent_t pe[3];
     for (auto& e : pe) HIP_OK(hipEventCreate(&e));
     const int reps = std::max(1, repeats) * 8;
-    if (iters > 0) {
-      const int it = launch_pcg_deflated(s, pcg_buffers(h, ritz_count(o) > 0 ? h->ritz_nr : 0, false),
-                                         o->pcg_relative_tolerance, std::min<int32_t>(o->pcg_max_iterations, 4),
+    if (iters > 0 && !small) {
+      const int it = launch_pcg_deflated(s, B, o->pcg_relative_tolerance, std::min<int32_t>(o->pcg_max_iterations, 4),
                                          kPcgPoll, kPcgPoll, pe, reps);
       if (it < 0) return set_err(h, MLBA_EDEVICE, "PCG launch failed");
       HIP_OK(hipEventSynchronize(pe[2]));

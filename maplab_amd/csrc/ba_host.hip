@@ -1153,7 +1153,7 @@ int minimize(mlba_handle* h, const mlba_options* o, double initial_radius, mlba_
         if ((rc = ritz_merge(h))) return rc;
         const int32_t nr_used = nritz > 0 ? h->ritz_nr : 0;
         const PcgBuffers B = pcg_buffers(h, nr_used, nritz > 0);
-        if ((pcg_small = pcg_small_applies(B))) {
+        if ((pcg_small = pcg_small_applies(B, o->pcg_max_iterations))) {
           if (!launch_pcg_small(s, B, o->pcg_relative_tolerance, o->pcg_max_iterations, h->scal.p + kPcgIters))
             return set_err(h, MLBA_EDEVICE, "PCG launch failed");
           h->ritz_nr = h->ritz_stage = 0;  // no coarse space to recycle columns for
@@ -2603,7 +2603,7 @@ int32_t mlba_time_kernels(mlba_handle* h, const mlba_options* o, int32_t repeats
     if ((rc = ensure_coarse_basis(h, o->pcg_coarse_nodes))) return rc;
     int32_t iters = 0;
     const PcgBuffers B = pcg_buffers(h, ritz_count(o) > 0 ? h->ritz_nr : 0, false);
-    const bool small = pcg_small_applies(B);
+    const bool small = pcg_small_applies(B, o->pcg_max_iterations);
     t->pcg_solve_ms = timed([&] {
       if (small)
         iters = launch_pcg_small(s, B, o->pcg_relative_tolerance, o->pcg_max_iterations, h->scal.p + kPcgIters) ? 0 : -1;

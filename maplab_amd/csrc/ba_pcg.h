@@ -84,9 +84,9 @@ int launch_pcg_deflated(hipStream_t s, const PcgBuffers& B, double tol, int32_t 
                         int32_t poll, const hipEvent_t* probe, int32_t probe_reps);
 
 // Block-Jacobi PCG of a system without a coarse space (K = 0) and few enough
-// vertices for one work-group: one launch, no host poll. The iteration count
-// goes to iters_out (device).
-bool pcg_small_applies(const PcgBuffers& B);
+// vertices for one work-group, of a bounded number of iterations: one launch,
+// no host poll. The iteration count goes to iters_out (device).
+bool pcg_small_applies(const PcgBuffers& B, int32_t max_iters);
 bool launch_pcg_small(hipStream_t s, const PcgBuffers& B, double tol, int32_t max_iters, double* iters_out);
 
 // Recycling the deflation space after a solve (m Lanczos vectors kept):

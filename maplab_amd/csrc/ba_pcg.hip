@@ -1091,6 +1091,10 @@ __global__ __launch_bounds__(kGroupBlock) void k_defl_partials(PcgArgs a, int32_
 // meet in LDS, and wave 0 keeps the vectors, so an iteration is two barriers.
 // Sums run in a fixed order.
 constexpr int kSmallVertices = 31;
+// A launch that cannot stop early (a residual that is not a number, a tolerance
+// below what 64 bits reach) runs all its iterations: at 6.6 us each at most 0.1 s
+// go into one launch; a larger cap is iterated by launches that the host polls.
+constexpr int kSmallIterations = 16384;
 constexpr int kSmallRows = 192;
 constexpr int kSmallWaves = 16;
 constexpr int kSmallCols = kSmallRows / kSmallWaves;  // two blocks of columns a wave
@@ -1836,12 +1840,12 @@ size_t pcg_step_doubles(int32_t Pvar) {
   return 36 * (size_t)Pvar + 2 * kMaxCoarse + (size_t)step_wgs(Pvar) * (2 * kStepStride + kMaxCoarse);
 }
 
-bool pcg_small_applies(const PcgBuffers& B) {
-  return B.K == 0 && B.kmat == nullptr && B.Pvar > 0 && B.Pvar <= kSmallVertices;
+bool pcg_small_applies(const PcgBuffers& B, int32_t max_iters) {
+  return B.K == 0 && B.kmat == nullptr && B.Pvar > 0 && B.Pvar <= kSmallVertices && max_iters <= kSmallIterations;
 }
 
 bool launch_pcg_small(hipStream_t s, const PcgBuffers& B, double tol, int32_t max_iters, double* iters_out) {
-  if (!pcg_small_applies(B)) return false;
+  if (!pcg_small_applies(B, max_iters)) return false;
   k_pcg_small<<<1, 64 * kSmallWaves, 0, s>>>(make_args(B), tol, max_iters, iters_out);
   return hipGetLastError() == hipSuccess;
 }

@@ -58,3 +58,21 @@ def test_one_launch_iterations_of_small_systems(n, nodes):
         assert abs(got - plain) <= max(1, plain // 50)
     else:
         assert got <= plain + 2
+
+
+def test_an_iteration_cap_too_large_for_one_launch():
+    # Above 16384 iterations a solve is one launch an iteration again: the same
+    # system, sums in another order.
+    out = []
+    for cap in (16384, 16385, 20000):
+        with DeviceProblem(ring(12)) as dev:
+            o = opts(max_num_iterations=4, pcg_max_iterations=cap)
+            one = dev.time_kernels(o, repeats=1).pcg_spmv_ms == 0
+            assert one == (cap == 16384)
+            sm, rows = dev.solve(o)
+            out.append(([r.cost for r in rows], [r.linear_solver_iterations for r in rows], dev.download_state()[0]))
+    for costs, its, v in out[1:]:
+        np.testing.assert_allclose(costs, out[0][0], rtol=1e-9)
+        assert np.abs(np.array(its) - out[0][1]).max() <= 1
+        np.testing.assert_allclose(v, out[0][2], atol=1e-7)
+    assert out[1][0] == out[2][0]

@@ -121,38 +121,42 @@ bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const in
   };
   // Visits (landmark, first block in I, first in J, blocks in I, in J),
   // grouped by tile in (I, J) order, landmarks ascending in a tile (a
-  // landmark visits a tile at most once; only visited tiles exist). Two stable
-  // counting sorts, by I over pieces of the landmarks with counts of their own,
-  // then by J within each I: memory and time grow with the bands and the
-  // visits, not with the square of the bands.
+  // landmark visits a tile at most once; only visited tiles exist): a stable
+  // counting sort over pieces of the landmarks, each with counts of its own. By
+  // tile, unless such counts were more than four a landmark: a long map has far
+  // more pairs of bands than visited tiles (400000 vertices: 5 GB of counts). Then
+  // by I, and by J within each I.
   struct Visit {
     int32_t I, J, l, gi, gj;
     uint8_t ni, nj;  // <= kTileBand
   };
   const int64_t pieces = std::max<int64_t>(1, std::min<int64_t>(16, (L + kPiece - 1) / kPiece));
   const int64_t span = (L + pieces - 1) / pieces;
-  std::vector<int64_t> at((size_t)(pieces * nb), 0);  // visits, then the place of the next, by piece and I
+  const bool by_tile = pieces * nb * nb <= 4 * (int64_t)L;
+  const int64_t keys = by_tile ? nb * nb : nb;
+  auto key_of = [&](int64_t I, int64_t J) { return by_tile ? I * nb + J : I; };
+  std::vector<int64_t> at((size_t)(pieces * keys), 0);  // visits, then the place of the next, by piece and key
   ok = ok && parallel_ranges(pieces, 1, [&](int64_t p0, int64_t p1, int) {
     std::vector<Run> runs;
     for (int64_t q = p0; q < p1; ++q)
       for (int64_t l = q * span; l < std::min<int64_t>(L, (q + 1) * span); ++l) {
         landmark_runs(l, runs);
-        for (size_t a = 0; a < runs.size(); ++a) at[(size_t)(q * nb + runs[a].band)] += (int64_t)(runs.size() - a);
+        for (size_t a = 0; a < runs.size(); ++a)
+          for (size_t b = a; b < runs.size(); ++b) at[(size_t)(q * keys + key_of(runs[a].band, runs[b].band))]++;
       }
   });
-  std::vector<int64_t> band_at((size_t)nb + 1, 0);
+  std::vector<int64_t> key_end((size_t)keys, 0);
   int64_t n_visits = 0;
-  for (int64_t k = 0; k < nb; ++k) {
+  for (int64_t k = 0; k < keys; ++k) {
     for (int64_t q = 0; q < pieces; ++q) {
-      const int64_t n = at[(size_t)(q * nb + k)];
-      at[(size_t)(q * nb + k)] = n_visits;
+      const int64_t n = at[(size_t)(q * keys + k)];
+      at[(size_t)(q * keys + k)] = n_visits;
       n_visits += n;
     }
-    band_at[(size_t)k + 1] = n_visits;
+    key_end[(size_t)k] = n_visits;
   }
-  UnsetVector<Visit> visits, by_band;
+  UnsetVector<Visit> visits;
   visits.resize((size_t)n_visits);
-  by_band.resize((size_t)n_visits);
   ok = ok && parallel_ranges(pieces, 1, [&](int64_t p0, int64_t p1, int) {
     std::vector<Run> runs;
     for (int64_t q = p0; q < p1; ++q)
@@ -160,32 +164,37 @@ bool build_schur_tiles(int32_t Pvar, int32_t L, const int32_t* inc_ptr, const in
         landmark_runs(l, runs);
         for (size_t a = 0; a < runs.size(); ++a)
           for (size_t b = a; b < runs.size(); ++b)
-            by_band[(size_t)at[(size_t)(q * nb + runs[a].band)]++] =
+            visits[(size_t)at[(size_t)(q * keys + key_of(runs[a].band, runs[b].band))]++] =
                 Visit{runs[a].band, runs[b].band, (int32_t)l, runs[a].g, runs[b].g, (uint8_t)runs[a].n,
                       (uint8_t)(a == b ? 0 : runs[b].n)};
       }
   });
-  std::vector<std::vector<int64_t>> place(kMaxHostThreads);  // by thread: visits of J, then the place of the next
-  ok = ok && parallel_ranges(nb, 1, [&](int64_t i0, int64_t i1, int thread) {
-    std::vector<int64_t>& p = place[thread];
-    if (p.empty()) p.resize((size_t)nb, 0);
-    std::vector<int32_t> touched;
-    for (int64_t i = i0; i < i1; ++i) {
-      touched.clear();
-      for (int64_t k = band_at[i]; k < band_at[i + 1]; ++k)
-        if (p[by_band[k].J]++ == 0) touched.push_back(by_band[k].J);
-      std::sort(touched.begin(), touched.end());
-      int64_t next = band_at[i];
-      for (int32_t J : touched) {
-        const int64_t n = p[J];
-        p[J] = next;
-        next += n;
+  if (!by_tile) {
+    UnsetVector<Visit> by_band;
+    by_band.swap(visits);
+    visits.resize((size_t)n_visits);
+    std::vector<std::vector<int64_t>> place(kMaxHostThreads);  // by thread: visits of J, then the place of the next
+    ok = ok && parallel_ranges(nb, 1, [&](int64_t i0, int64_t i1, int thread) {
+      std::vector<int64_t>& p = place[thread];
+      if (p.empty()) p.resize((size_t)nb, 0);
+      std::vector<int32_t> touched;
+      for (int64_t i = i0; i < i1; ++i) {
+        const int64_t begin = i ? key_end[i - 1] : 0, end = key_end[i];
+        touched.clear();
+        for (int64_t k = begin; k < end; ++k)
+          if (p[by_band[k].J]++ == 0) touched.push_back(by_band[k].J);
+        std::sort(touched.begin(), touched.end());
+        int64_t next = begin;
+        for (int32_t J : touched) {
+          const int64_t n = p[J];
+          p[J] = next;
+          next += n;
+        }
+        for (int64_t k = begin; k < end; ++k) visits[(size_t)p[by_band[k].J]++] = by_band[k];
+        for (int32_t J : touched) p[J] = 0;
       }
-      for (int64_t k = band_at[i]; k < band_at[i + 1]; ++k) visits[(size_t)p[by_band[k].J]++] = by_band[k];
-      for (int32_t J : touched) p[J] = 0;
-    }
-  });
-  UnsetVector<Visit>().swap(by_band);
+    });
+  }
   if (!ok) {
     *err = "host allocation failed";
     return false;

@@ -11,16 +11,19 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), "maplab_amd", "csrc")
 
 
-@pytest.fixture(scope="module")
-def program(tmp_path_factory):
+def build(tmp_path_factory, name):
     gxx = shutil.which("g++")
     if gxx is None:
         pytest.skip("g++ is not available")
-    exe = str(tmp_path_factory.mktemp("tiles") / "schur_tiles_memory")
+    exe = str(tmp_path_factory.mktemp("tiles") / name)
     subprocess.run([gxx, "-O2", "-std=c++17", "-pthread", "-I", CSRC, "-o", exe,
-                    os.path.join(HERE, "native", "schur_tiles_memory.cc"), os.path.join(CSRC, "ba_tiles.cc")],
-                   check=True)
+                    os.path.join(HERE, "native", name + ".cc"), os.path.join(CSRC, "ba_tiles.cc")], check=True)
     return exe
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    return build(tmp_path_factory, "schur_tiles_memory")
 
 
 def test_allocations_are_linear_in_the_rows(program):
@@ -34,7 +37,16 @@ def test_allocations_are_linear_in_the_rows(program):
     assert large[1] < 64000 * 4096
 
 
-@pytest.mark.parametrize("rows, per_row", [(1, 1), (2, 5), (15, 3), (16, 3), (17, 3), (33, 1), (500, 4)])
+@pytest.mark.parametrize("rows, per_row", [(1, 1), (2, 5), (15, 3), (16, 3), (17, 3), (33, 1), (500, 4), (2000, 1)])
 def test_rows_match_a_plain_count(program, rows, per_row):
     out = subprocess.run([program, str(rows), str(per_row), "check"], capture_output=True, text=True)
     assert out.returncode == 0, (out.returncode, out.stdout)
+
+
+@pytest.mark.parametrize("rows, landmarks", [(100, 12), (100, 13), (400, 60), (700, 4500)])
+def test_few_landmarks_over_many_bands(tmp_path_factory, rows, landmarks):
+    # Visits sorted by tile row, then by column (fewer than a fourth as many
+    # landmarks as pairs of bands, times the pieces of 4096 landmarks).
+    checker = build(tmp_path_factory, "schur_tiles_check")
+    out = subprocess.run([checker, str(rows), str(landmarks), "8"], capture_output=True, text=True)
+    assert out.returncode == 0, out.stdout + out.stderr

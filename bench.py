@@ -120,7 +120,7 @@ TRAFFIC_PROFILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "prof
 # Bench kernel row -> the kernel whose rocprofv3 FETCH_SIZE / WRITE_SIZE row
 # gives its HBM traffic (the Schur block build is dominated by its tile pass).
 TRAFFIC_KERNEL = {"k_schur_blocks": "mlba::k_schur_tiles", "k_pcg_spmv": "mlba::k_pcg_spmv<false>",
-                  "k_pcg_update": "mlba::k_pcg_update", "k_pcg_step": "mlba::k_pcg_step",
+                  "k_pcg_update": "mlba::k_pcg_update", "k_pcg_step": "mlba::k_pcg_step<2>",
                   "k_schur_factors": "mlba::k_schur_factors<false>", "k_linearize": "mlba::k_linearize<true, false>",
                   "k_back_substitute": "mlba::k_back_substitute<false>"}
 

@@ -234,8 +234,9 @@ __device__ inline double loss_scale(const DevLoss& loss, int32_t type, double si
 //
 // Records leave through LDS, so that consecutive lanes write consecutive 16
 // bytes: written by its own thread, a record is six stores of which each touches
-// 64 rows of 96 bytes: 188 -> 164 us for 2M observations of 500 keyframes, 358 ->
-// 311 for 1000 (and k_schur_factors, which writes so too, 185 -> 134, 327 -> 229).
+// 64 rows of 96 bytes: 188 -> 164 us for 2.9M observations of 500 keyframes, 358
+// -> 311 for 5.1M of 1000 (and k_schur_factors, which writes so too, 185 -> 134,
+// 327 -> 229).
 //
 // The landmark sums meet in LDS: nine values per observation (V and g), value-
 // major; thread (run, value) adds its landmark's run of observations in order,
@@ -1992,8 +1993,11 @@ void launch_schur_blocks(hipStream_t s, const DevTopology& t, const SchurTilesDe
                          int32_t items_per_wg, int32_t xcd_map, hipEvent_t stop) {
   if (t.Pvar <= 0 || nub <= 0) return launch_nothing(s, stop);
   launch_schur_tiles(s, d, gf, gk, lm_z, lm_anc, partial, items_per_wg, xcd_map);
-  // kWide from 24 slots a block on: below that its groups have too few slots
-  // each to hide their latency behind one another.
+  // kWide from 24 slots a block on (MI355X, tiles and this kernel, seven blocks a
+  // work-group against one): 165 slots a block 62 and 24 us, 64 slots 107 and 58,
+  // 28 slots 114 and 86, 19 slots 145 and 129, 13 slots 166 and 162, 8 slots 232
+  // and 240. The two meet near 12; between there and the line the wide form would
+  // save up to a tenth.
   const bool wide = d.n_uslot >= 24 * (int64_t)nub;
   launch(s, stop, wide ? &k_schur_finalize<true> : &k_schur_finalize<false>,
          wide ? nub : (nub + kFinalizeGroups - 1) / kFinalizeGroups, 252, t, nub, ublk, d.uslot_ptr, d.uslot, partial,

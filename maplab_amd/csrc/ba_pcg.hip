@@ -1084,7 +1084,8 @@ __global__ __launch_bounds__(kGroupBlock) void k_defl_partials(PcgArgs a, int32_
 // system of 10 keyframes needs about 40 iterations, and as two launches each
 // they cost 10.5 us an iteration on MI355X (launch and two dependent rounds
 // of global loads, not the 54 x 54 product): 450 us a solve, 3.6 ms of the
-// 6.3 ms that 10 LM iterations took (2.7 ms with this). Here S stays in
+// 6.3 ms that 10 LM iterations took (2.7 ms with this). Here an iteration is
+// 2.0 us (37 of them 75 us, set-up included). S stays in
 // registers, dense: wave w holds columns 12 w .. 12 w + 11 of rows lane,
 // lane + 64 and lane + 128 (36 doubles a thread, which is what 1024 threads
 // leave room for and why 31 vertices are the limit); the waves' sums of a row
@@ -1092,8 +1093,8 @@ __global__ __launch_bounds__(kGroupBlock) void k_defl_partials(PcgArgs a, int32_
 // Sums run in a fixed order.
 constexpr int kSmallVertices = 31;
 // A launch that cannot stop early (a residual that is not a number, a tolerance
-// below what 64 bits reach) runs all its iterations: at 6.6 us each at most 0.1 s
-// go into one launch; a larger cap is iterated by launches that the host polls.
+// below what 64 bits reach) runs all its iterations: at 2 us each at most 33 ms go
+// into one launch; a larger cap is iterated by launches that the host polls.
 constexpr int kSmallIterations = 16384;
 constexpr int kSmallRows = 192;
 constexpr int kSmallWaves = 16;
@@ -1237,9 +1238,12 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_pcg_small(PcgArgs a, doubl
 //
 // An iteration, two launches -> one (MI355X, 15-node space and 16 dense
 // columns from 250 keyframes): 60 keyframes 14.7 -> 8.2 us, 250 19.6 -> 13.6,
-// 500 21.3 -> 15.6, 1000 26.7 -> 21.6, 2000 39.0 -> 30.6. At 5000 (work-groups
-// of 16 rows) 68 -> 91: the product is the larger part there, and three vectors
-// gathered cost it more than the launch; the line is drawn at 2048 vertices.
+// 500 21.3 -> 15.6, 1000 26.7 -> 21.6, 2000 39.0 -> 30.6. The line is drawn at
+// 2048 vertices, 256 work-groups of 8 rows: one more and a compute unit runs two
+// of them after another, in an iteration that is a chain of latencies. Whole
+// solves, two launches -> one, us an iteration: 2000 vertices 37.7 -> 32.6, 2049
+// (257 work-groups) 37.9 -> 32.5, 2300 (288) 39.7 -> 60.1, 3000 47.9 -> 61.6,
+// 4000 57.2 -> 68.6, 5000 64.5 -> 102 (16 rows a work-group: 91 against 68).
 constexpr int kStepScalars = 7;  // p's, r'z, s'z, s'v, r'r, r's, s's (k_pcg_start: r'z, r'r, b'b in 1, 4, 5)
 constexpr int kStepStride = kStepScalars + kMaxCoarse;
 constexpr int kStepThreads = 1024;

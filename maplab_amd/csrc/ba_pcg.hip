@@ -1213,18 +1213,25 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_pcg_small(PcgArgs a, doubl
 // wrote costs several us here whatever it computes (launch, then dependent
 // rounds of global loads), and an iteration as a product and an update was
 // two of them. CG needs a global sum for alpha = r'z / p's (s = S p) and a
-// second one after it, r'z and the deflation's c = (SW)'z of the new z. The
-// second follows from the first by linearity: with v = M s formed at the end
-// of an iteration,
+// second one after it, r'z and the deflation's c = (SW)'z - W'r of the new z and
+// r. The second follows from the first by linearity: with v = M s formed at the
+// end of an iteration,
 //   r+ = r - alpha s, z+ = z - alpha v,
-//   r+'z+ = r'z - 2 alpha s'z + alpha^2 s'v,   r+'r+ alike,   c+ = c - alpha (SW)'v,
+//   r+'z+ = r'z - 2 alpha s'z + alpha^2 s'v,   r+'r+ alike,
+//   c+ = c - alpha ((SW)'v - W's),
 // so one launch sums all of these and the next one starts from them: each row
 // takes r+, its own z+ = M r+ (formed anew, so that the recurrences for the
 // scalars run over one iteration only), mu = E^-1 c+ of its window, and the
 // product of its row with z+ = z - alpha v and p as three sums that do not
 // wait for alpha. c is carried over at most kStepRefresh iterations and then
-// summed anew from z: carried through the whole solve, its rounding error stays
-// at 1e-16 of the first c while r falls, and the residual stagnates at 1e-11.
+// summed anew from z and r: carried through the whole solve, its rounding error
+// stays at 1e-16 of the first c while r falls, and the residual stagnates at
+// 1e-11. W'r is zero but for the errors of the c before it, which reach r through
+// W mu; the direction z - W E^-1 c takes them out again (the A-DEF2 operator of
+// Tang, Nabben, Vuik and Erlangga, J. Sci. Comput. 39, 2009). With c = (SW)'z
+// they stay: a 1500-keyframe ring took 57 iterations for 49, its recycled columns
+// came to depend on the hat functions, and the next solve did not converge. The
+// term costs 0.3 us an iteration.
 //
 // A work-group of 1024 threads takes G rows, so that at most 256 work-groups
 // (one a CU) publish the partials that every work-group sums. Component t % 6
@@ -1291,10 +1298,25 @@ __device__ inline double step_slice(const double* part, int wgs, int stride, int
   return acc;
 }
 
+// A row's hat part of W: its nodes n, n + 1 and their weights.
+struct StepHat {
+  int32_t n;
+  double w0, w1;
+};
+
+// Entry of W in a row's component comp and hat column gc.
+__device__ inline double hat_entry(const StepHat& h, int gc, int comp) {
+  const int node = gc / 6;
+  if (gc - 6 * node != comp) return 0.0;
+  return node == h.n ? h.w0 : (node == h.n + 1 ? h.w1 : 0.0);
+}
+
 // Coarse column e of the sum over a work-group's rows of the window products
-// tmp[row][window column][component].
+// tmp[row][window column][component] and, to be subtracted, the dense columns'
+// den[row][column][component].
 template <int G>
-__device__ inline double step_column(const PcgArgs& a, int i0, int e, const double (*tmp)[kMaxCoarse][6]) {
+__device__ inline double step_column(const PcgArgs& a, int i0, int e, const double (*tmp)[kMaxCoarse][6],
+                                     const double (*den)[kMaxRitz][6]) {
   double s = 0.0;
 #pragma unroll
   for (int g = 0; g < G; ++g) {
@@ -1303,6 +1325,10 @@ __device__ inline double step_column(const PcgArgs& a, int i0, int e, const doub
       if (lc >= 0 && lc < a.gw && (e >= a.neh || lc < a.gwh)) {
         const double* t = tmp[g][lc];
         s += ((t[0] + t[1]) + (t[2] + t[3])) + (t[4] + t[5]);
+        if (e >= a.neh) {
+          const double* d = den[g][e - a.neh];
+          s -= ((d[0] + d[1]) + (d[2] + d[3])) + (d[4] + d[5]);
+        }
       }
     }
   }
@@ -1313,7 +1339,8 @@ __device__ inline double step_column(const PcgArgs& a, int i0, int e, const doub
 // (sc[e]) and the coarse columns of tmp.
 template <int G>
 __device__ inline void step_publish(const PcgArgs& a, int i0, const double (*sc)[kStepScalars],
-                                    const double (*tmp)[kMaxCoarse][6], double* part) {
+                                    const double (*tmp)[kMaxCoarse][6], const double (*den)[kMaxRitz][6],
+                                    double* part) {
   const int tid = threadIdx.x, stride = kStepScalars + a.ne;
   double* out = part + (size_t)blockIdx.x * stride;
   if (tid < kStepScalars) {
@@ -1322,7 +1349,7 @@ __device__ inline void step_publish(const PcgArgs& a, int i0, const double (*sc)
     for (int e = 0; e < 6 * G; ++e) s += sc[e][tid];
     out[tid] = s;
   } else if (tid < stride) {
-    out[tid] = step_column<G>(a, i0, tid - kStepScalars, tmp);
+    out[tid] = step_column<G>(a, i0, tid - kStepScalars, tmp, den);
   }
 }
 
@@ -1332,7 +1359,8 @@ __global__ __launch_bounds__(kStepThreads) void k_pcg_start(PcgArgs a) {
   using Sh = StepShape<G>;
   __shared__ double sc[6 * G][kStepScalars];
   __shared__ double tmp[G][kMaxCoarse][6];
-  __shared__ double ys[kMaxCoarse], rows[G][6], red[G][Sh::kBlocks][6];
+  __shared__ double ys[kMaxCoarse], rows[G][6], rowr[G][6], den[G][kMaxRitz][6], red[G][Sh::kBlocks][6];
+  __shared__ StepHat hat[G];
   const int tid = threadIdx.x, i0 = blockIdx.x * G, ne = a.ne;
   const int g = min(tid / Sh::kT, G - 1), t = tid - g * Sh::kT, comp = t % 6, bs = t / 6, i = i0 + g;
   const bool row_ok = i < a.Pvar, lane_in = t < 6 * Sh::kBlocks, lane_ok = row_ok && lane_in;
@@ -1369,6 +1397,7 @@ __global__ __launch_bounds__(kStepThreads) void k_pcg_start(PcgArgs a) {
       if (ne) {
         const int n0 = a.hat_node[i];
         const double w0 = a.hat_w[2 * i], w1 = a.hat_w[2 * i + 1];
+        if (comp == 0) hat[g] = StepHat{n0, w0, w1};
         xv = w0 * ys[6 * n0 + comp] + (w1 != 0.0 ? w1 * ys[6 * (n0 + 1) + comp] : 0.0);
         for (int c = 0; c < a.nr; ++c) xv += a.R[(size_t)c * a.n6 + e] * ys[a.neh + c];
       }
@@ -1388,6 +1417,7 @@ __global__ __launch_bounds__(kStepThreads) void k_pcg_start(PcgArgs a) {
       o[12] = 0.0;
     }
     rows[g][comp] = zv;
+    rowr[g][comp] = rv;
     double* o = sc[6 * g + comp];
     o[0] = o[2] = o[3] = o[6] = 0.0;
     o[1] = rv * zv;
@@ -1396,15 +1426,20 @@ __global__ __launch_bounds__(kStepThreads) void k_pcg_start(PcgArgs a) {
   }
   __syncthreads();
   if (ne && lane_in) {
-    const double z = rows[g][comp];
+    const double z = rows[g][comp], r = rowr[g][comp];
 #pragma unroll
     for (int m = 0; m < Sh::kCols; ++m) {
       const int lc = bs + Sh::kBlocks * m;
-      if (lc < kMaxCoarse) tmp[g][lc][comp] = sw[m] * z;
+      if (lc < kMaxCoarse) tmp[g][lc][comp] = sw[m] * z - (row_ok && lc < a.gwh ? hat_entry(hat[g], c0 + lc, comp) * r : 0.0);
+    }
+#pragma unroll
+    for (int m = 0; m < Sh::kRitz; ++m) {
+      const int c = bs + Sh::kBlocks * m;
+      if (c < kMaxRitz) den[g][c][comp] = row_ok && c < a.nr ? a.R[(size_t)c * a.n6 + 6 * i + comp] * r : 0.0;
     }
   }
   __syncthreads();
-  step_publish<G>(a, i0, sc, tmp, a.spart);
+  step_publish<G>(a, i0, sc, tmp, den, a.spart);
 }
 
 // Iteration k: takes step k - 1 (x, r), then stops when |r|^2 <= tol2 or
@@ -1417,7 +1452,9 @@ __global__ __launch_bounds__(kStepThreads) void k_pcg_step(PcgArgs a, int32_t k)
   __shared__ double sc[6 * G][kStepScalars];
   __shared__ double tmp[G][kMaxCoarse][6];
   __shared__ double lds[Sh::kSlices][128], ldz[Sh::kSlices][128];
-  __shared__ double sums[128], cs[kMaxCoarse], mus[kMaxCoarse], rows[G][6], rowz[G][6], red[G][Sh::kBlocks][6], wred[G][kMaxRitz][6];
+  __shared__ double sums[128], cs[kMaxCoarse], mus[kMaxCoarse], rows[G][6], rowz[G][6], rowq[G][6], rowr[G][6];
+  __shared__ double red[G][Sh::kBlocks][6], wred[G][kMaxRitz][6];
+  __shared__ StepHat hat[G];
   PcgState* st = a.st;
   const int odd = k & 1, ne = a.ne, stride = kStepScalars + ne;
   const double* __restrict__ in = a.zvp + (odd ? (size_t)18 * a.Pvar : 0);
@@ -1627,6 +1664,9 @@ __global__ __launch_bounds__(kStepThreads) void k_pcg_step(PcgArgs a, int32_t k)
     }
     rows[g][comp] = row_ok ? vv : 0.0;
     rowz[g][comp] = row_ok ? zv : 0.0;
+    rowq[g][comp] = row_ok ? q : 0.0;
+    rowr[g][comp] = row_ok ? rv : 0.0;
+    if (comp == 0) hat[g] = StepHat{hn0, hw0, hw1};
     double* o = sc[6 * g + comp];
     o[0] = row_ok ? pn * q : 0.0;
     o[1] = row_ok ? rv * zv : 0.0;
@@ -1638,27 +1678,39 @@ __global__ __launch_bounds__(kStepThreads) void k_pcg_step(PcgArgs a, int32_t k)
   }
   __syncthreads();
   if (ne && lane_in) {
-    const double v = rows[g][comp];
+    const double v = rows[g][comp], q = rowq[g][comp];
+    const StepHat h = hat[g];
 #pragma unroll
     for (int m = 0; m < Sh::kCols; ++m) {
       const int lc = bs + Sh::kBlocks * m;
-      if (lc < kMaxCoarse) tmp[g][lc][comp] = sw[m] * v;
+      if (lc < kMaxCoarse) tmp[g][lc][comp] = sw[m] * v - (lc < a.gwh ? hat_entry(h, c0 + lc, comp) * q : 0.0);
+    }
+#pragma unroll
+    for (int m = 0; m < Sh::kRitz; ++m) {
+      const int c = bs + Sh::kBlocks * m;
+      if (c < kMaxRitz) wred[g][c][comp] = rc[m] * q;
     }
   }
   __syncthreads();
-  step_publish<G>(a, i0, sc, tmp, a.spart + (odd ? 0 : (size_t)a.wgs * stride));
+  step_publish<G>(a, i0, sc, tmp, wred, a.spart + (odd ? 0 : (size_t)a.wgs * stride));
   if (k % kStepRefresh != 0 || ne == 0) return;
   __syncthreads();
   if (lane_in) {
-    const double z = rowz[g][comp];
+    const double z = rowz[g][comp], r = rowr[g][comp];
+    const StepHat h = hat[g];
 #pragma unroll
     for (int m = 0; m < Sh::kCols; ++m) {
       const int lc = bs + Sh::kBlocks * m;
-      if (lc < kMaxCoarse) tmp[g][lc][comp] = sw[m] * z;
+      if (lc < kMaxCoarse) tmp[g][lc][comp] = sw[m] * z - (lc < a.gwh ? hat_entry(h, c0 + lc, comp) * r : 0.0);
+    }
+#pragma unroll
+    for (int m = 0; m < Sh::kRitz; ++m) {
+      const int c = bs + Sh::kBlocks * m;
+      if (c < kMaxRitz) wred[g][c][comp] = rc[m] * r;
     }
   }
   __syncthreads();
-  if (tid < ne) a.zpart[(size_t)blockIdx.x * ne + tid] = step_column<G>(a, i0, tid, tmp);
+  if (tid < ne) a.zpart[(size_t)blockIdx.x * ne + tid] = step_column<G>(a, i0, tid, tmp, wred);
 }
 
 // Clears the convergence flag and lifts the iteration limit so that one more

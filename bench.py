@@ -106,7 +106,7 @@ def kernel_table(sm, kt, n_pcg_total):
         groups = (P + 41) // 42
         spmv_b = nnzb * 292 + P * 200 + P * 6 * gw * 8
         upd_b = P * 344 + P * 288 + P * 6 * gw * 8 + groups * gw * ne * 8 + groups * (3 + ne) * 8
-        # One launch per iteration up to 2048 vertices, two above.
+        # One launch per iteration (pcg_update_ms 0), or two on dense and large systems.
         step_b = nnzb * 292 + P * (2 * 144 + 288 + 288) + P * 6 * gw * 8 + ne * ne * 8
         two = (("k_pcg_spmv", kt.pcg_spmv_ms, spmv_b), ("k_pcg_update", kt.pcg_update_ms, upd_b))
         for name, ms, b in two if kt.pcg_update_ms > 0 else (("k_pcg_step", kt.pcg_spmv_ms, step_b),):

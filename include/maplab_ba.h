@@ -436,8 +436,9 @@ int32_t mlba_measure_copy(int64_t bytes, int32_t repeats, double* ms_per_copy);
  * (bands of item_band_rows tile rows swept tile column by tile column; 0 =
  * the items with the most work first), how many items a work-group runs
  * (item_waves: 1, 2, 4, 8) and whether work-groups are mapped
- * XCD-contiguously. Where a PCG iteration is two launches (more than 2048
- * vertices, or the learned preconditioner) it sums the per-group partials of
+ * XCD-contiguously. Where a PCG iteration is two launches (dense systems of
+ * more than 512 vertices, all of more than 2048, and the learned
+ * preconditioner) it sums the per-group partials of
  * each iteration (r'z, r'r and the coarse-space product of every
  * 42-row group) in group order, either in every SpMV work-group
  * (pcg_partials 1) or once, in the update work-group that finishes last

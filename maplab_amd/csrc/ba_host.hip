@@ -698,7 +698,7 @@ int ensure_coarse_basis(mlba_handle* h, int32_t requested) {
   if (!h->defl_SR.alloc(groups * gw * (size_t)(6 * gr)) ||
       !h->defl_E.alloc(std::max<size_t>(ne * ne, 1)) || !h->defl_Einv.alloc(std::max<size_t>(ne * ne + groups * gw * ne, 1)) ||
       !h->defl_y.alloc(std::max<size_t>(ne, 1)) || !h->defl_cden.alloc(std::max<size_t>(nr, 1)) ||
-      !h->pcg_part2.alloc((groups + 1) * (3 + ne)) || !h->pcg_step.alloc(std::max<size_t>(pcg_step_doubles(Pvar), 1)))
+      !h->pcg_part2.alloc((groups + 1) * (3 + ne)) || !h->pcg_step.alloc(std::max<size_t>(pcg_step_doubles(Pvar, h->nnzb), 1)))
     return set_err(h, MLBA_ENOMEM, "device allocation failed");
   if (nr > 0) {
     const size_t n6 = 6 * (size_t)Pvar, zc = (size_t)pcg_max_lanczos();
@@ -735,6 +735,7 @@ int32_t ritz_count(const mlba_options* o) {
 PcgBuffers pcg_buffers(mlba_handle* h, int32_t nr, bool keep_lanczos) {
   PcgBuffers B{};
   B.Pvar = h->Pvar;
+  B.nnzb = h->nnzb;
   B.K = std::max(h->hat_K, 0);
   B.nr = B.K > 0 ? nr : 0;
   B.gwh = h->grp_width;
@@ -2632,7 +2633,7 @@ int32_t mlba_time_kernels(mlba_handle* h, const mlba_options* o, int32_t repeats
       HIP_OK(hipEventElapsedTime(&a, pe[0], pe[1]));
       HIP_OK(hipEventElapsedTime(&b, pe[1], pe[2]));
       t->pcg_spmv_ms = a / reps;
-      t->pcg_update_ms = pcg_step_doubles(h->Pvar) ? 0.0 : b / reps;
+      t->pcg_update_ms = pcg_step_applies(B) ? 0.0 : b / reps;
     }
     for (auto& e : pe) (void)hipEventDestroy(e);
     const int32_t nr_used = h->hat_K > 0 && ritz_count(o) > 0 ? h->ritz_nr : 0;

@@ -19,6 +19,7 @@ struct PcgBuffers {
   int32_t Pvar, K, nr, gwh;
   int32_t zcap;                // Lanczos vectors kept (iterations), 0: none
   int32_t partials;            // two-launch iterations, sum of the group partials: 0 automatic, 1 per SpMV work-group, 2 once
+  int64_t nnzb;                // blocks of S
   const int32_t* row_ptr;      // block rows of S
   const int32_t* col_var;
   const double* S;
@@ -45,7 +46,7 @@ struct PcgBuffers {
   double* q;
   double* part;                // Pvar
   double* part2;               // (groups + 1) x (3 + ne): per-group partials, then their sum
-  double* step;                // pcg_step_doubles(Pvar): state of one-launch iterations
+  double* step;                // pcg_step_doubles(Pvar, nnzb): state of one-launch iterations
   double* Zh;                  // zcap x 6 Pvar: deflated preconditioned residual of iteration k
   double* coef;                // 2 zcap: r'z and alpha of iteration k
   void* state_dev;             // pcg_state_bytes()
@@ -61,8 +62,9 @@ struct PcgBuffers {
 };
 
 size_t pcg_state_bytes();
-// Room for the iterations of one launch each (0: they don't apply).
-size_t pcg_step_doubles(int32_t Pvar);
+// Room for the iterations of one launch each (0: they don't pay for a system of
+// Pvar vertices and nnzb blocks).
+size_t pcg_step_doubles(int32_t Pvar, int64_t nnzb);
 int32_t pcg_max_hat_nodes();
 // Recycled dense columns of the deflation space, at most.
 constexpr int kPcgMaxRitz = 16;
@@ -72,6 +74,9 @@ int32_t pcg_update_groups(int32_t Pvar);
 // Whether the last solve's coarse matrix E was positive definite (its
 // deflation was applied); reads the host copy of the state.
 bool pcg_deflation_applied(const void* state_host);
+
+// Whether launch_pcg_deflated takes one launch an iteration.
+bool pcg_step_applies(const PcgBuffers& B);
 
 // Deflated PCG solve. The host polls the state after `first` iterations, then
 // every `poll` iterations. With `probe` (three events), the kernels of one more

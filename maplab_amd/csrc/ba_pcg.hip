@@ -23,9 +23,9 @@
 // is a set of coalesced column dot products.
 //
 // Per LM step: k_defl_sr (SW), k_defl_e and k_defl_dense (E, R'b),
-// k_defl_prep (state, E^-1 by the sweep operator, y = E^-1 W'b). Up to 2048 vertices
-// with block-Jacobi k_pcg_start and one launch per iteration, k_pcg_step,
-// follow; otherwise k_defl_init (x0, r0, z0 and the first per-group partials)
+// k_defl_prep (state, E^-1 by the sweep operator, y = E^-1 W'b). With
+// block-Jacobi k_pcg_start and one launch per iteration, k_pcg_step, follow where
+// that pays (step_pays); otherwise k_defl_init (x0, r0, z0 and the first per-group partials)
 // and two launches per iteration: k_pcg_spmv (sums the previous
 // per-group partials; p = z - W mu + beta p_prev and
 // q = S z + beta S p_prev - (SW) mu) and k_pcg_update (x, r, z and the
@@ -1243,14 +1243,21 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_pcg_small(PcgArgs a, doubl
 // 15.5 us) and the partials summed once by the work-group that ends last
 // (24 us) are slower. Sums run in a fixed order.
 //
-// An iteration, two launches -> one (MI355X, 15-node space and 16 dense
-// columns from 250 keyframes): 60 keyframes 14.7 -> 8.2 us, 250 19.6 -> 13.6,
-// 500 21.3 -> 15.6, 1000 26.7 -> 21.6, 2000 39.0 -> 30.6. The line is drawn at
-// 2048 vertices, 256 work-groups of 8 rows: one more and a compute unit runs two
-// of them after another, in an iteration that is a chain of latencies. Whole
-// solves, two launches -> one, us an iteration: 2000 vertices 37.7 -> 32.6, 2049
-// (257 work-groups) 37.9 -> 32.5, 2300 (288) 39.7 -> 60.1, 3000 47.9 -> 61.6,
-// 4000 57.2 -> 68.6, 5000 64.5 -> 102 (16 rows a work-group: 91 against 68).
+// Where it pays (step_pays; MI355X, whole solves with the 15-node space, two
+// launches -> one, us an iteration). A work-group has G rows of B blocks and
+// takes them side by side, so its product lasts as long as G B blocks, where the
+// two launches give every row a work-group and grow with the vertices:
+//   up to 512 vertices (G <= 2) always: walks 60 vertices 18 -> 12, 500 33.5 ->
+//     27.6; rings that every keyframe sees whole, B = vertices: 120 20.8 -> 15.7,
+//     256 24.3 -> 20.8, 512 34.1 -> 30.3;
+//   up to 1024 (G = 4) from 5 B vertices on: 1000 vertices (B 155) 27.6 -> 24.3,
+//     800 (152) 23.2 -> 23.2, 1000 (201) 31.8 -> 31.6, 600 (150) 22.5 -> 23.6, 800
+//     (211) 28.4 -> 31.0, rings 600 40 -> 45, 1000 79 -> 82;
+//   up to 2048 (G = 8) from 12 B vertices on: 2000 (149) 37.7 -> 32.6, 2040 (186)
+//     46.9 -> 46.3, 1400 (156) 34.2 -> 33.2, 1050 (155) 27.4 -> 31.3, 1600 (172)
+//     38.8 -> 41.2, 1200 (206) 33.2 -> 46.0, rings 1100 136 -> 197, 2000 287 -> 311;
+//   above 2048, 256 work-groups of 8 rows, a compute unit runs two of them one
+//     after the other: 2300 39.7 -> 60.1, 4000 57.2 -> 68.6, 5000 64.5 -> 102.
 constexpr int kStepScalars = 7;  // p's, r'z, s'z, s'v, r'r, r's, s's (k_pcg_start: r'z, r'r, b'b in 1, 4, 5)
 constexpr int kStepStride = kStepScalars + kMaxCoarse;
 constexpr int kStepThreads = 1024;
@@ -1888,11 +1895,19 @@ static void launch_step(hipStream_t s, const PcgArgs& a, int32_t k) {
   }
 }
 
-// Block-Jacobi iterations as one launch each (k_pcg_step).
-static bool step_applies(const PcgBuffers& B) { return B.kmat == nullptr && B.Pvar <= kStepVertices; }
+// Whether an iteration in one launch is the faster form (k_pcg_step): S has at
+// most a fifth, with eight rows a work-group a twelfth, of its blocks.
+static bool step_pays(int32_t Pvar, int64_t nnzb) {
+  if (Pvar <= 0 || Pvar > kStepVertices) return false;
+  const int32_t G = step_rows(Pvar);
+  const int64_t sparse = G <= 2 ? 0 : (G == 4 ? 5 : 12);
+  return (int64_t)Pvar * Pvar >= sparse * nnzb;
+}
 
-size_t pcg_step_doubles(int32_t Pvar) {
-  if (Pvar <= 0 || Pvar > kStepVertices) return 0;
+bool pcg_step_applies(const PcgBuffers& B) { return B.kmat == nullptr && step_pays(B.Pvar, B.nnzb); }
+
+size_t pcg_step_doubles(int32_t Pvar, int64_t nnzb) {
+  if (!step_pays(Pvar, nnzb)) return 0;
   return 36 * (size_t)Pvar + 2 * kMaxCoarse + (size_t)step_wgs(Pvar) * (2 * kStepStride + kMaxCoarse);
 }
 
@@ -1918,7 +1933,7 @@ int launch_pcg_deflated(hipStream_t s, const PcgBuffers& B, double tol, int32_t 
   const int32_t Pvar = B.Pvar;
   if (Pvar <= 0) return 0;
   if (B.K > kMaxHatNodes || B.nr > kMaxRitz || B.nr < 0) return -1;
-  const bool learned = B.kmat != nullptr, step = step_applies(B);
+  const bool learned = B.kmat != nullptr, step = pcg_step_applies(B);
   if (learned && (B.nr > 0 || B.zcap > 0 || probe || !B.linv || !B.diag_pos || !B.tpos || !B.t || !B.u)) return -1;
   const PcgArgs a = make_args(B);
   double* p0 = B.p0;

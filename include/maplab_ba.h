@@ -48,7 +48,8 @@ extern "C" {
 #define MLBA_EINVAL -1   /* invalid argument (sigma <= 0, bad index, ...) */
 #define MLBA_ENOMEM -2   /* device or host allocation failed */
 #define MLBA_EDEVICE -3  /* HIP runtime error */
-#define MLBA_ESTATE -4   /* state violates an invariant (non-unit quaternion) */
+#define MLBA_ESTATE -4   /* state violates an invariant (non-unit quaternion), or a landmark mask
+                          * could not be set (mlba_set_landmark_active) */
 
 /* Distortion models (aslam::Distortion::Type subset). */
 #define MLBA_DISTORTION_NONE 0

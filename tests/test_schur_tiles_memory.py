@@ -47,6 +47,6 @@ def test_rows_match_a_plain_count(program, rows, per_row):
 def test_few_landmarks_over_many_bands(tmp_path_factory, rows, landmarks):
     # Visits sorted by tile row, then by column (fewer than a fourth as many
     # landmarks as pairs of bands, times the pieces of 4096 landmarks).
-    checker = build(tmp_path_factory, "schur_tiles_check")
-    out = subprocess.run([checker, str(rows), str(landmarks), "8"], capture_output=True, text=True)
+    program = build(tmp_path_factory, "schur_tiles_check")
+    out = subprocess.run([program, str(rows), str(landmarks), "8"], capture_output=True, text=True)
     assert out.returncode == 0, out.stdout + out.stderr
